@@ -1,0 +1,85 @@
+"""The weight-streaming kernel for 2 to 64 rows of activations (csrc/gemm_rows.h) against the oracle: every tiling of the
+inner dimension with one slice and with several, row counts at the edges of the 16-row blocks, widths that end inside a
+strip of 16, every epilogue, head-major stores, groups, and the two-launch form of the sliced products."""
+import ctypes
+
+import pytest
+import torch
+
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+# (M, N, K): tiling and slices
+SHAPES = [
+    (17, 16384, 2048),   # A, one slice
+    (33, 8192, 4096),    # A, two
+    (64, 4096, 8192),    # A, four
+    (2, 2048, 1024),     # B, one
+    (5, 50, 1024),       # B, a width inside one group of strips that ends inside a strip
+    (16, 4099, 1024),    # B, a width that no vector store fits
+    (64, 2064, 3072),    # B, three slices, a strip past a multiple of 64
+    (48, 8192, 5120),    # C, one
+    (16, 5120, 10240),   # C, two
+    (40, 2560, 2560),    # D, one
+    (3, 640, 7680),      # D, three
+    (31, 768, 768),      # E, one
+    (8, 784, 2304),      # E, three
+    (49, 16, 768),       # one strip
+]
+
+
+def _s8(g, *shape):
+    return torch.randint(-127, 128, shape, dtype=torch.int8, generator=g)
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_every_epilogue_is_exact(M, N, K):
+    import torch_int._CUDA as C
+    import torch_int._hip_ext as X
+    C._lib.ti_last_kernel.restype = ctypes.c_char_p
+    g = torch.Generator().manual_seed(M * 7 + N + K)
+    x, w = _s8(g, M, K), _s8(g, N, K)
+    b8, bf = _s8(g, N), torch.randn(N, generator=g)
+    b32 = torch.randint(-65535, 65535, (N,), dtype=torch.int32, generator=g)
+    resid = torch.randn(M, N, generator=g) * 3
+    al, be = 3e-4, 0.02
+    acc = orc.gemm_acc_torch(x, w)
+    xd, wd, b8d, bfd, b32d = (t.to(DEV) for t in (x, w, b8, bf, b32))
+    runs = [(lambda: C.linear_a8_w8_b32_o32(xd, wd, b32d), orc.epi_b32_o32(acc, b32)),
+            (lambda: C.linear_a8_w8_b32_o32_with_scaling(xd, wd, b32d, al, be), orc.epi_b32_o32_scaled(acc, b32, al, be)),
+            (lambda: C.linear_a8_w8_bfp32_ofp32(xd, wd, bfd, al, 1.0), orc.epi_bfp32_ofp32(acc, bf, al, 1.0)),
+            (lambda: C.linear_a8_w8_b8_o8(xd, wd, b8d, al, be), orc.epi_b8_o8(acc, b8, al, be)),
+            (lambda: C.linear_relu_a8_w8_b8_o8(xd, wd, b8d, al, be), orc.epi_b8_o8(acc, b8, al, be, relu=True)),
+            (lambda: C._linear_a8_w8_bfp32_ofp32_acc(xd, wd, bfd, al, 1.0, resid.to(DEV)),
+             orc.linear_a8_w8_bfp32_ofp32_acc(x, w, bf, al, 1.0, resid, acc_fn=lambda *_: acc))]
+    for i, (run, want) in enumerate(runs):
+        print("rows epilogue", i, M, N, K, flush=True)
+        outs = [run() for _ in range(2)]
+        assert C._lib.ti_last_kernel().decode() == ("stream" if M <= 16 else "mid_stream")
+        for o in outs:   # twice: the arrival counters and the accumulation buffers are left as they were found
+            assert torch.equal(o.cpu(), want), (i, M, N, K)
+    before = C._lib.ti_fused_splitk(0)   # several slices: the two-launch form, or another kernel where there is no workspace
+    try:
+        assert torch.equal(C.linear_a8_w8_b8_o8(xd, wd, b8d, al, be).cpu(), orc.epi_b8_o8(acc, b8, al, be))
+    finally:
+        C._lib.ti_fused_splitk(before)
+    d = 16 if N % 16 == 0 else 0
+    if d:
+        want = orc.epi_b8_o8(acc, b8, al, be).view(1, M, N // d, d).transpose(1, 2)
+        assert torch.equal(X.linear_a8_w8_b8_o8_heads(xd, wd, b8d, al, be, 1, M, N // d, d).cpu(), want)
+
+
+@pytest.mark.parametrize("M,N,K", [(24, 4096, 4096), (16, 1024, 4096), (7, 2560, 2560), (48, 768, 768), (2, 100, 1024)])
+def test_groups_are_exact(M, N, K):
+    import torch_int._hip_ext as X
+    g = torch.Generator().manual_seed(M + N + K)
+    x, ws, bs = _s8(g, M, K), [_s8(g, N, K) for _ in range(3)], [_s8(g, N) for _ in range(3)]
+    al, be = [3e-4, 2e-4, 5e-4], [0.02, 0.1, 0.05]
+    ref = [orc.linear_a8_w8_b8_o8(x, w, b, a, c, acc_fn=orc.gemm_acc_torch) for w, b, a, c in zip(ws, bs, al, be)]
+    print("rows group", M, N, K, flush=True)
+    for _ in range(2):
+        out = X.linear_a8_w8_b8_o8_group(x.to(DEV), [w.to(DEV) for w in ws], [b.to(DEV) for b in bs], al, be)
+        for o, r in zip(out, ref):
+            assert torch.equal(o.cpu(), r), (M, N, K)

@@ -17,6 +17,8 @@ long long gemm_workspace_bytes(long long M, long long N, long long K) {
     const long long head = M - r <= 1024 ? gemm_workspace_bytes(M - r, N, K) : 0;
     return head > need ? head : need;
   }
+  const RowsPick rows = rows_pick(M, N, K);
+  if (M > 16 && rows.tiling != ROWS_NONE) return rows.slices > 1 ? (long long)rows.slices * M * N * 4 : 0;
   const int s = choose_splits(M, N, K);
   return s > 1 ? (long long)s * M * N * 4 : 0;
 }
@@ -62,6 +64,10 @@ static constexpr int kFusedCounters = 32768;            // per stream: tiles x w
 static constexpr int kFusedTiles = kFusedCounters / 8;  // per stream: one XCC word per tile
 static __device__ __align__(256) int g_fused_arrivals[kFusedStreams * (kFusedCounters + kFusedTiles)];
 
+// Parked tiles of gemm_rows_kernel for up to 16 rows, whose callers hold no workspace: a block per stream slot, used by one
+// launch of that stream at a time and written in full before it is read.
+static __device__ __align__(256) char g_rows_park[kFusedStreams * kRowsParkBytes];
+
 __global__ void xcc_probe_kernel(unsigned* out) {
   if (threadIdx.x == 0) out[blockIdx.x] = __builtin_amdgcn_s_getreg((3 << 11) | 20) & 0xf;  // HW_REG_XCC_ID
 }
@@ -70,6 +76,7 @@ struct FusedDevice {
   std::mutex lock;
   int state = 0;  // 0 = not probed yet, 1 = usable, -1 = off
   int* arrivals = nullptr;
+  char* park = nullptr;
   int* host_words = nullptr;  // [0] = the misplacement flag, [1 .. 256] = the probe's output
   int* host_words_dev = nullptr;
   hipStream_t streams[kFusedStreams] = {};
@@ -234,7 +241,9 @@ int fused_split_prepare(hipStream_t stream, long long counters, GemmParams& q) {
     if (is_capturing(stream)) return 0;
     d.state = -1;
     void* sym = nullptr;
+    void* park = nullptr;
     if (hipGetSymbolAddress(&sym, HIP_SYMBOL(g_fused_arrivals)) != hipSuccess || sym == nullptr) return 0;
+    if (hipGetSymbolAddress(&park, HIP_SYMBOL(g_rows_park)) != hipSuccess || park == nullptr) return 0;
     if (hipHostMalloc(reinterpret_cast<void**>(&d.host_words), 257 * sizeof(int), hipHostMallocMapped) != hipSuccess) {
       d.host_words = nullptr;
       return 0;
@@ -244,6 +253,7 @@ int fused_split_prepare(hipStream_t stream, long long counters, GemmParams& q) {
       return 0;
     if (!probe_placement(d, stream)) return 0;
     d.arrivals = static_cast<int*>(sym);
+    d.park = static_cast<char*>(park);
     d.state = 1;
     probed_now = true;
   }
@@ -268,6 +278,14 @@ int fused_split_prepare(hipStream_t stream, long long counters, GemmParams& q) {
   q.xcc_seen = reinterpret_cast<unsigned*>(q.arrivals + kFusedCounters);
   q.xcc_error = d.host_words_dev;
   return 1;
+}
+
+void* fused_split_park(const GemmParams& q) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
+  FusedDevice& d = g_fused[dev];
+  const long long slot = (q.arrivals - d.arrivals) / (kFusedCounters + kFusedTiles);
+  return d.park + slot * kRowsParkBytes;
 }
 
 int warm_fused_split(void* stream) {
@@ -325,13 +343,19 @@ static int group_prefill_tile(long long M, long long N, long long K, int count) 
 // sizes) rather than a loop over the problems; a caller that holds a split-K workspace does better with separate
 // calls in the second case.
 int gemm_group_is_one_launch(long long M, long long N, long long K, int count) {
-  if (M <= 16) return K % SBK == 0 ? 1 : 0;
+  if (M <= 16 && K % SBK == 0) return 1;
+  if (M <= TI_ROWS_MAX_M && N % 4 == 0) {
+    const RowsPick rows = rows_pick(M, N, K);
+    if (rows.tiling != ROWS_NONE && rows.slices == 1) return 1;  // no workspace needed
+  }
+  if (M <= 16) return 0;
   return group_prefill_tile(M, N, K, count) != 0 ? 1 : 0;
 }
 
 // q/k/v-style group of s8 linears.  Decode shapes (M <= 16, K % 1024 == 0, enough strips) take one launch
 // of the streaming kernel over all the weights; anything else runs problem by problem.
-int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStream_t stream) {
+int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStream_t stream, void* workspace,
+                         long long workspace_bytes) {
   constexpr int KIND = EPI_S8_BIAS;
   if (shape.M == 0 || shape.N == 0 || grp.count == 0) return TI_OK;
   bool ptr_ok = (reinterpret_cast<uintptr_t>(shape.A) & 15) == 0;
@@ -339,6 +363,13 @@ int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStrea
   const bool aligned = ptr_ok && (shape.K % SBK == 0) && shape.K > 0;
   const int spb = (shape.N + 15) / 16;
   const long long strips = (long long)spb * grp.count;
+  if (ptr_ok && shape.M <= TI_ROWS_MAX_M && shape.N % 4 == 0 && !(gemv_takes(shape) && strips >= 256)) {
+    const int rc = launch_rows<KIND, true>(shape, grp, grp.count, workspace, workspace_bytes, stream);
+    if (rc >= 0) {
+      if (rc == TI_OK) g_last_kernel = shape.M <= 16 ? "stream_group" : "mid_stream_group";
+      return rc;
+    }
+  }
   if (aligned && gemv_takes(shape) && strips >= 256) {
     g_last_kernel = "gemv_group";
     return launch_gemv<KIND, true>(shape, grp, grp.count, stream);

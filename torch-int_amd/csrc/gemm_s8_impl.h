@@ -2501,6 +2501,10 @@ static int row_split_rows(long long M, long long N, long long K, long long* rest
   return (int)r;
 }
 
+}  // namespace ti
+#include "gemm_rows.h"
+namespace ti {
+
 template <int KIND, bool GROUPED>
 static int launch_gemv(const GemmParams& p, const GemmGroup& grp, int problems, hipStream_t stream) {
   static std::atomic<unsigned long long> lds_ok{0};
@@ -2532,6 +2536,20 @@ static inline bool stream_deep_pipeline(int M, long long strips, int cus) {
   return false;
 }
 
+// Few, long weight rows (fc2 of a decode step: 1x5120x20480, 1x9216x36864): the view of the problem in which every row is
+// cut into four (two rows of activations: two) parts has that many times the strips, and its rows lie a part instead of
+// a whole row apart, which spreads the 16 rows of a strip over the memory channels (a multiple of 4 KiB between them does
+// not): 1x5120x20480 22.4 -> 19.6 us, 1x9216x36864 58.5 -> 52.2 us, 2x5120x20480 23.9 -> 20.1 us.  Not when the parts are
+// again a multiple of 4 KiB apart (1x4096x16384: 13.5 -> 15.1 us).  1 = no such view.
+static inline int stream_parts(const GemmParams& p) {
+  const int spb = (p.N + 15) / 16;
+  if (!(p.M <= 2 && p.batch == 1 && p.out_d == 0 && p.m_base == 0 && p.lda == p.K && p.ldb == p.K && p.N % 16 == 0 &&
+        p.K >= 8192 && spb >= 256 && spb <= 4 * num_cus()))
+    return 1;
+  if (p.M == 1) return p.K % 4096 == 0 && p.K % 16384 != 0 ? 4 : 1;
+  return p.K % 2048 == 0 && p.K % 8192 != 0 ? 2 : 1;
+}
+
 template <int KIND>
 int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes, hipStream_t stream) {
   using Out = typename Epi<KIND>::Out;
@@ -2546,6 +2564,17 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
     return TI_OK;
+  }
+  // Up to 64 rows: the weight-streaming kernel with the activations in registers.  Not for one row where the dot-product
+  // kernel reads weight rows flat, one or two rows against the few, long weight rows of the view below, ragged widths of a
+  // K that 1024 does not divide, nor up to four rows of a short K (2 x 768 x 768: 3.1 us against the skinny kernel's 2.9).
+  if (p.M <= TI_ROWS_MAX_M && (p.N % 16 == 0 || p.K % SBK == 0) && stream_parts(p) == 1 && (p.M > 4 || p.K >= SBK) &&
+      !(gemv_takes(p) && (p.N + 15) / 16 >= 256)) {
+    const int rc = launch_rows<KIND, false>(p, GemmGroup{}, 1, workspace, workspace_bytes, stream);
+    if (rc >= 0) {
+      if (rc == TI_OK) g_last_kernel = p.M <= 16 ? "stream" : "mid_stream";
+      return rc;
+    }
   }
   if (p.M <= 16 && p.K % SBK == 0 && (long long)((p.N + 15) / 16) * p.batch >= 256) {
     g_last_kernel = "stream";
@@ -2564,17 +2593,7 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
       if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
       return TI_OK;
     };
-    // Few, long weight rows (fc2 of a decode step: 1x5120x20480, 1x9216x36864): the view of the problem in which
-    // every row is cut into four (two rows of activations: two) parts has that many times the strips, and its rows
-    // lie a part instead of a whole row apart, which spreads the 16 rows of a strip over the memory channels
-    // (a multiple of 4 KiB between them does not): 1x5120x20480 22.4 -> 19.6 us, 1x9216x36864 58.5 -> 52.2 us,
-    // 2x5120x20480 23.9 -> 20.1 us.
-    const int parts = p.batch == 1 && p.out_d == 0 && p.m_base == 0 && p.lda == p.K && p.ldb == p.K && p.N % 16 == 0 &&
-                              p.K >= 8192 && spb <= 4 * cus
-                          ? (p.M == 1 && p.K % 4096 == 0 && p.K % 16384 != 0       ? 4
-                             : p.M == 2 && p.K % 2048 == 0 && p.K % 8192 != 0 ? 2
-                                                                              : 1)
-                          : 1;  // not when the parts are again a multiple of 4 KiB apart (1x4096x16384: 13.5 -> 15.1 us)
+    const int parts = stream_parts(p);
     // one row of activations: the flat-reading dot-product kernel, except against the few very long rows where the
     // view with rows cut into parts is ahead (1x9216x36864: 52.2 against 54.6 us; 1x5120x20480: 19.6 against 18.5)
     if (gemv_takes(p) && !(parts > 1 && p.K > 24 * 1024)) {

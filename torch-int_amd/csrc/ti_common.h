@@ -234,7 +234,8 @@ struct GemmGroup {
   float alpha[4], beta[4];
   int count;
 };
-int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStream_t stream);
+int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStream_t stream, void* workspace = nullptr,
+                         long long workspace_bytes = 0);
 
 // Launchers (gemm_s8.hip).  `kind` is an EpiKind.  Returns a TI_* status.
 int launch_gemm(int kind, const GemmParams& p, void* workspace, long long workspace_bytes,
