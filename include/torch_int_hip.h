@@ -441,7 +441,7 @@ int ti_attn_prefill_s8_mc(const int8_t* q, const int8_t* k, const int8_t* vt, co
  * the LayerNorm parameters are fp16 too), updated in place; mask fp32 [B, 1, 1, S] or NULL; k_buf / v_buf the cache
  * buffers [B, heads, cap, head_dim] holding S - 1 positions, S after the call; scratch: device memory of
  * ti_opt_decoder_layer_decode_scratch_bytes(B, embed, ffn) bytes on a 256-byte boundary (the layers of a model can
- * share it: calls on one stream run one after the other).  B <= 16. */
+ * share it: calls on one stream run one after the other).  B <= 64. */
 typedef struct TiOptDecodeLayer {
   int64_t embed, heads, head_dim, ffn;
   int32_t half;                 /* 1: residual stream and LayerNorm parameters are fp16 */

@@ -83,3 +83,31 @@ def test_groups_are_exact(M, N, K):
         out = X.linear_a8_w8_b8_o8_group(x.to(DEV), [w.to(DEV) for w in ws], [b.to(DEV) for b in bs], al, be)
         for o, r in zip(out, ref):
             assert torch.equal(o.cpu(), r), (M, N, K)
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("D,H,bsz", [(768, 12, 17), (1024, 8, 64), (320, 4, 33)])
+def test_decode_step_of_a_large_batch_from_one_call(D, H, bsz, half):
+    """17 to 64 sequences, one new token each: residual stream and caches of the one C call bit for bit those of the
+    modules, with the projections grouped (768), sliced (fc2 of 1024) and on the split-K kernels (320)."""
+    from test_gpu_models import causal_mask, randomize_int8_layer
+    from torch_int.models.opt import Int8OPTDecoderLayer
+    g = torch.Generator().manual_seed(D + bsz)
+    layer = randomize_int8_layer(Int8OPTDecoderLayer(D, H, 4 * D), g).to(DEV)
+    layer = layer.half() if half else layer
+    dt = torch.float16 if half else torch.float32
+    hidden = torch.randn(bsz, 32, D, generator=g).to(DEV).to(dt)
+    out = layer(hidden.clone(), attention_mask=causal_mask(bsz, 32, 32).to(DEV).to(dt), use_cache=True)
+    caches = {True: out[-1], False: tuple(t.clone() for t in out[-1])}
+    for step in range(3):
+        x = torch.randn(bsz, 1, D, generator=g).to(DEV).to(dt)
+        res = {}
+        for one_call in (True, False):
+            layer.decode_in_one_call = one_call
+            print("rows decode", D, bsz, half, step, one_call, flush=True)
+            res[one_call] = layer(x.clone(), past_key_value=caches[one_call], use_cache=True)
+            caches[one_call] = res[one_call][-1]
+        assert torch.equal(res[True][0], res[False][0])
+        for a, b in zip(caches[True], caches[False]):
+            assert torch.equal(a, b)

@@ -422,7 +422,7 @@ int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStrea
     q.C = grp.C[i];
     q.alpha = grp.alpha[i];
     q.beta = grp.beta[i];
-    if (int rc = launch_gemm_kind_3(q, nullptr, 0, stream)) return rc;
+    if (int rc = launch_gemm_kind_3(q, workspace, workspace_bytes, stream)) return rc;
   }
   return TI_OK;
 }

@@ -510,7 +510,7 @@ class Int8OPTDecoderLayer(nn.Module):
         """``forward`` for one new token per sequence over a KV cache, or None when the tensors do not qualify."""
         hs = hidden_states
         dtype = hs.dtype
-        if not (hs.is_cuda and hs.is_contiguous() and hs.shape[0] <= 16
+        if not (hs.is_cuda and hs.is_contiguous() and hs.shape[0] <= 64
                 and (dtype is torch.float32 or dtype is torch.float16)):
             return None
         past_k, past_v = past_key_value
