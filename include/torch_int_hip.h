@@ -441,7 +441,7 @@ int ti_attn_prefill_s8_mc(const int8_t* q, const int8_t* k, const int8_t* vt, co
  * the LayerNorm parameters are fp16 too), updated in place; mask fp32 [B, 1, 1, S] or NULL; k_buf / v_buf the cache
  * buffers [B, heads, cap, head_dim] holding S - 1 positions, S after the call; scratch: device memory of
  * ti_opt_decoder_layer_decode_scratch_bytes(B, embed, ffn) bytes on a 256-byte boundary (the layers of a model can
- * share it: calls on one stream run one after the other).  B <= 64. */
+ * share it: calls on one stream run one after the other).  B <= 16. */
 typedef struct TiOptDecodeLayer {
   int64_t embed, heads, head_dim, ffn;
   int32_t half;                 /* 1: residual stream and LayerNorm parameters are fp16 */
@@ -482,6 +482,20 @@ int ti_opt_decoder_layer_prefill(const TiOptDecodeLayer* layer, void* hidden, co
                                  const uint8_t* mask_classes, int8_t* k_out, int8_t* v_out, int64_t B, int64_t T,
                                  void* scratch, int64_t scratch_bytes, void* workspace, int64_t workspace_bytes,
                                  void* stream);
+
+/* The two calls above for the layers of a model one after the other on one residual stream (Int8OPTDecoder.forward's loop,
+ * torch_int/models/opt.py:302-398): decode steps of up to 64 sequences, prefills of any number of tokens.  carry: fp32
+ * [rows, embed] that belongs to this pass (16-byte aligned; unused with chain = 0).  chain & 2: where the output of fc2 would be
+ * added to the stream by a kernel of its own (an fp16 stream, or more than 4096 rows), leave it in carry instead; chain & 1:
+ * this call's first LayerNorm kernel adds what the call before left there.  Every layer but the last leaves, every layer but
+ * the first adds; the additions and their order are those of the separate calls. */
+int ti_opt_decoder_layer_decode_chained(const TiOptDecodeLayer* layer, void* hidden, const float* mask, int8_t* k_buf,
+                                        int8_t* v_buf, int64_t B, int64_t cap, int64_t S, int chain, float* carry,
+                                        void* scratch, int64_t scratch_bytes, void* stream);
+int ti_opt_decoder_layer_prefill_chained(const TiOptDecodeLayer* layer, void* hidden, const float* mask,
+                                         const uint8_t* mask_classes, int8_t* k_out, int8_t* v_out, int64_t B, int64_t T,
+                                         int chain, float* carry, void* scratch, int64_t scratch_bytes, void* workspace,
+                                         int64_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

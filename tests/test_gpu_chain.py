@@ -1,0 +1,59 @@
+"""The layers of a model chained, one C call each with the last addition left to the next layer's first kernel, against the
+same model going through its modules: logits and key / value caches bit for bit."""
+import pytest
+import torch
+
+from torch_int.models.opt import Int8OPTDecoderLayer, Int8OPTForCausalLM, OPTConfigLite
+from test_gpu_models import randomize_int8_layer
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _generate(lm, ids, attention_mask, steps):
+    results = []
+    out = lm(ids, attention_mask=attention_mask, use_cache=True)
+    for step in range(steps):
+        results.append(out)
+        if attention_mask is not None:
+            attention_mask = torch.cat([attention_mask, attention_mask.new_ones(ids.shape[0], 1)], dim=1)
+        out = lm(ids[:, step:step + 1], attention_mask=attention_mask, past_key_values=out.past_key_values, use_cache=True)
+    return results + [out]
+
+
+# rows of the prefill up to and past the 4096 at which fp32 streams change how they add fc2's output; 1, 3 and 17 sequences in
+# the decode steps; with and without padding
+@torch.no_grad()
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("bsz,T,layers,pad", [(1, 48, 1, False), (3, 16, 3, True), (17, 33, 2, False), (4, 1024, 2, True),
+                                              (3, 1376, 3, True), (5, 1000, 2, False)])
+def test_chained_layers_give_the_modules_values(bsz, T, layers, pad, half):
+    torch.manual_seed(0)
+    g = torch.Generator().manual_seed(T)
+    lm = Int8OPTForCausalLM(OPTConfigLite(hidden_size=128, num_hidden_layers=layers, ffn_dim=512, num_attention_heads=2, vocab_size=64,
+                                          max_position_embeddings=2048))
+    for layer in lm.model.decoder.layers:
+        randomize_int8_layer(layer, g)
+    lm = lm.to(DEV)
+    lm = lm.half() if half else lm
+    ids = torch.randint(2, 64, (bsz, T), generator=g).to(DEV)
+    keep = torch.ones(bsz, T, dtype=torch.long, device=DEV) if pad else None
+    if pad:
+        keep[1, :5] = 0
+        keep[2, T // 2:] = 0
+    print("chained", bsz, T, layers, pad, half, flush=True)
+    chained = _generate(lm, ids, keep, 3)
+    seen = []
+    hook = lm.model.decoder.layers[-1].register_forward_hook(lambda *a: seen.append(1))
+    hooked = _generate(lm, ids, keep, 3)     # the hooked layer is called as a module
+    hook.remove()
+    assert len(seen) == 4
+    try:
+        Int8OPTDecoderLayer.prefill_in_one_call = Int8OPTDecoderLayer.decode_in_one_call = False
+        modules = _generate(lm, ids, keep, 3)
+    finally:
+        Int8OPTDecoderLayer.prefill_in_one_call = Int8OPTDecoderLayer.decode_in_one_call = True
+    for a, h, b in zip(chained, hooked, modules):
+        assert torch.equal(a.logits, b.logits) and torch.equal(h.logits, b.logits)
+        for (ka, va), (kb, vb) in zip(a.past_key_values, b.past_key_values):
+            assert torch.equal(ka, kb) and torch.equal(va, vb)

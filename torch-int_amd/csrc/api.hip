@@ -721,64 +721,107 @@ int ti_transpose_last2_s8(const int8_t* src, int8_t* dst, int64_t B, int64_t R, 
   return launch_transpose_last2_s8(src, dst, B, R, C, static_cast<hipStream_t>(stream));
 }
 
-// One decoder layer of a decode step: the seven (fp16 stream: eight) calls an Int8OPTDecoderLayer makes for one new
-// token per sequence, issued from one C call.  Each step IS the public entry point the Python modules call, with
-// the arguments they pass, so the values are theirs.
+// ---------------------------------------------------------------- a decoder layer from one C call
+// A decoder layer, one new token per sequence or a prefill: the calls that Int8OPTDecoderLayer's modules make, each of them
+// the public entry point with the arguments the modules pass, so the values are theirs.  In a chain of layers (CHAIN_*, the
+// layers of a model one after the other) one thing is moved: on an fp16 residual stream, and on an fp32 one
+// beyond 4096 rows, where the GEMM's accumulating epilogue costs more than it saves, the output of fc2 is added by the NEXT
+// layer's LayerNorm kernel, which reads the stream anyway, instead of by a kernel of its own (3 us of a decode layer, 6.3 us
+// at 2048 x 2048: a launch, and the stream read and written once more).  Same additions, same order.
+}  // extern "C"
+namespace {
+enum Chain : int { CHAIN_ADD = 1, CHAIN_LEAVE = 2 };  // add what the previous layer left in `carry` / leave fc2's output there
+
+inline int64_t up256(int64_t n) { return (n + 255) / 256 * 256; }
+
+struct Carver {  // consecutive 256-byte aligned pieces of the caller's scratch
+  char* at;
+  template <class T>
+  T* take(int64_t bytes) {
+    T* r = reinterpret_cast<T*>(at);
+    at += up256(bytes);
+    return r;
+  }
+};
+
+// LayerNorm-quantise the residual stream, first adding `pending` (fp32, or NULL) into it
+int layernorm(const TiOptDecodeLayer* L, const float* pending, void* hidden, const void* gamma, const void* beta, float eps,
+              int8_t* out, int64_t rows, void* stream) {
+  const int64_t E = L->embed;
+  if (!L->half)
+    return ti_add_layernorm_q(pending, static_cast<float*>(hidden), static_cast<const float*>(gamma),
+                              static_cast<const float*>(beta), eps, out, rows, E, stream);
+  return pending == nullptr ? ti_add_layernorm_q_f16(nullptr, hidden, gamma, beta, eps, out, rows, E, stream)
+                            : ti_add_layernorm_q_f16_xf32(pending, hidden, gamma, beta, eps, out, rows, E, stream);
+}
+
+// whether fc2's output is added by a later kernel rather than in the GEMM's epilogue
+bool adds_later(const TiOptDecodeLayer* L, int64_t rows) { return L->half || rows > 4096; }
+
+// out_proj, the second LayerNorm, fc1 and fc2 of a layer
+int after_attention(const TiOptDecodeLayer* L, const int8_t* ctx, float* f32, int8_t* x, int8_t* h, void* hidden,
+                    int64_t rows, int chain, float* carry, void* ws, int64_t ws_bytes, void* stream) {
+  const int64_t E = L->embed, F = L->ffn;
+  int rc;
+  if ((rc = ti_linear_a8_w8_bfp32_ofp32(ctx, L->wo, L->bo, f32, rows, E, E, L->alpha_o, 1.0f, ws, ws_bytes, stream))) return rc;
+  if ((rc = layernorm(L, f32, hidden, L->ln2_gamma, L->ln2_beta, L->ln2_eps, x, rows, stream))) return rc;
+  if ((rc = ti_linear_relu_a8_w8_b8_o8(x, L->w1, L->b1, h, rows, F, E, L->alpha_1, L->beta_1, ws, ws_bytes, stream))) return rc;
+  if (!adds_later(L, rows))
+    return ti_linear_a8_w8_bfp32_ofp32_acc(h, L->w2, L->b2, static_cast<float*>(hidden), rows, E, F, L->alpha_2, 1.0f, ws,
+                                           ws_bytes, stream);
+  float* out = chain & CHAIN_LEAVE ? carry : f32;
+  if ((rc = ti_linear_a8_w8_bfp32_ofp32(h, L->w2, L->b2, out, rows, E, F, L->alpha_2, 1.0f, ws, ws_bytes, stream))) return rc;
+  if (chain & CHAIN_LEAVE) return TI_OK;
+  if (L->half) return ti_add_f16_xf32(f32, hidden, rows * E, stream);
+  return launch_add_f32(f32, static_cast<float*>(hidden), rows * E, static_cast<hipStream_t>(stream));
+}
+
+int check_layer(const char* op, const TiOptDecodeLayer* L) {
+  if (L == nullptr) return fail(TI_ERR_INVALID_ARG, "%s: no layer description", op);
+  if (L->embed <= 0 || L->heads <= 0 || L->head_dim <= 0 || L->ffn <= 0 || L->heads * L->head_dim != L->embed)
+    return fail(TI_ERR_INVALID_ARG, "%s: needs embed = heads * head_dim > 0 and ffn > 0 (got %lld, %lld x %lld, %lld)", op,
+                (long long)L->embed, (long long)L->heads, (long long)L->head_dim, (long long)L->ffn);
+  return TI_OK;
+}
+
 // Workspace of the largest of a decode step's linears (slices of a long inner dimension, see ti_linear_workspace_bytes);
 // the three projections of the group share one.
-static int64_t decode_workspace_bytes(int64_t B, int64_t embed, int64_t ffn) {
-  const int64_t need[4] = {3 * gemm_workspace_bytes(B, embed, embed), gemm_workspace_bytes(B, embed, embed),
-                           gemm_workspace_bytes(B, ffn, embed), gemm_workspace_bytes(B, embed, ffn)};
+int64_t decode_workspace_bytes(int64_t B, int64_t embed, int64_t ffn) {
+  if (B <= 16) return 0;
+  const int64_t need[3] = {3 * gemm_workspace_bytes(B, embed, embed), gemm_workspace_bytes(B, ffn, embed),
+                           gemm_workspace_bytes(B, embed, ffn)};
   int64_t most = 0;
   for (int64_t n : need) most = n > most ? n : most;
-  return B > 16 ? most : 0;
+  return most;
 }
 
-int64_t ti_opt_decoder_layer_decode_scratch_bytes(int64_t B, int64_t embed, int64_t ffn) {
-  if (B <= 0 || embed <= 0 || ffn <= 0) return 0;
-  auto up = [](int64_t n) { return (n + 255) / 256 * 256; };
-  return 5 * up(B * embed) + up(4 * B * embed) + up(B * ffn) + up(decode_workspace_bytes(B, embed, ffn));
-}
-
-int ti_opt_decoder_layer_decode(const TiOptDecodeLayer* L, void* hidden, const float* mask, int8_t* k_buf, int8_t* v_buf,
-                                int64_t B, int64_t cap, int64_t S, void* scratch, int64_t scratch_bytes, void* stream) {
-  g_err[0] = 0;
-  const char* op = "opt_decoder_layer_decode";
-  if (L == nullptr) return fail(TI_ERR_INVALID_ARG, "%s: no layer description", op);
+int decode_layer(const char* op, const TiOptDecodeLayer* L, void* hidden, const float* mask, int8_t* k_buf, int8_t* v_buf,
+                 int64_t B, int64_t cap, int64_t S, int chain, float* carry, void* scratch, int64_t scratch_bytes,
+                 void* stream, int64_t most) {
+  if (int rc = check_layer(op, L)) return rc;
   const int64_t E = L->embed, H = L->heads, d = L->head_dim, F = L->ffn;
-  if (E <= 0 || H <= 0 || d <= 0 || F <= 0 || H * d != E)
-    return fail(TI_ERR_INVALID_ARG, "%s: needs embed = heads * head_dim > 0 and ffn > 0 (got %lld, %lld x %lld, %lld)", op,
-                (long long)E, (long long)H, (long long)d, (long long)F);
-  if (B < 0 || B > 64) return fail(TI_ERR_INVALID_ARG, "%s: 0 to 64 sequences, one new token each (got %lld)", op, (long long)B);
+  if (B < 0 || B > most)
+    return fail(TI_ERR_INVALID_ARG, "%s: 0 to %lld sequences, one new token each (got %lld)", op, (long long)most, (long long)B);
   if (B == 0) return TI_OK;
   if (int rc = check_ptr(op, "hidden", hidden, L->half ? 2 : 4, true)) return rc;
+  if (int rc = check_ptr(op, "carry", carry, 16, chain != 0)) return rc;
   if (int rc = check_ptr(op, "scratch", scratch, 256, true)) return rc;
-  if (scratch_bytes < ti_opt_decoder_layer_decode_scratch_bytes(B, E, F))
-    return fail(TI_ERR_INVALID_ARG, "%s: scratch of %lld bytes, needs %lld", op, (long long)scratch_bytes,
-                (long long)ti_opt_decoder_layer_decode_scratch_bytes(B, E, F));
-  auto up = [](int64_t n) { return (n + 255) / 256 * 256; };
-  char* at = static_cast<char*>(scratch);
-  auto take = [&](int64_t bytes) {
-    char* r = at;
-    at += up(bytes);
-    return r;
-  };
-  int8_t* x = reinterpret_cast<int8_t*>(take(B * E));      // LayerNorm-quantised input of the projections, then of fc1
-  int8_t* q = reinterpret_cast<int8_t*>(take(B * E));
-  int8_t* k = reinterpret_cast<int8_t*>(take(B * E));
-  int8_t* v = reinterpret_cast<int8_t*>(take(B * E));
-  int8_t* ctx = reinterpret_cast<int8_t*>(take(B * E));
-  float* f32 = reinterpret_cast<float*>(take(4 * B * E));   // output of out_proj, then (fp16 stream) of fc2
-  int8_t* h = reinterpret_cast<int8_t*>(take(B * F));
+  const int64_t need = ti_opt_decoder_layer_decode_scratch_bytes(B, E, F);
+  if (scratch_bytes < need)
+    return fail(TI_ERR_INVALID_ARG, "%s: scratch of %lld bytes, needs %lld", op, (long long)scratch_bytes, (long long)need);
+  Carver carve{static_cast<char*>(scratch)};
+  int8_t* x = carve.take<int8_t>(B * E);      // LayerNorm-quantised input of the projections, then of fc1
+  int8_t* q = carve.take<int8_t>(B * E);
+  int8_t* k = carve.take<int8_t>(B * E);
+  int8_t* v = carve.take<int8_t>(B * E);
+  int8_t* ctx = carve.take<int8_t>(B * E);
+  float* f32 = carve.take<float>(4 * B * E);  // output of out_proj, then of fc2
+  int8_t* h = carve.take<int8_t>(B * F);
   const int64_t ws_bytes = decode_workspace_bytes(B, E, F);
-  void* ws = ws_bytes > 0 ? take(ws_bytes) : nullptr;
+  void* ws = ws_bytes > 0 ? carve.take<void>(ws_bytes) : nullptr;
+  const float* pending = (chain & CHAIN_ADD) && adds_later(L, B) ? carry : nullptr;
   int rc;
-  // self_attn_layer_norm
-  rc = L->half ? ti_add_layernorm_q_f16(nullptr, hidden, L->ln1_gamma, L->ln1_beta, L->ln1_eps, x, B, E, stream)
-               : ti_add_layernorm_q(nullptr, static_cast<float*>(hidden), static_cast<const float*>(L->ln1_gamma),
-                                    static_cast<const float*>(L->ln1_beta), L->ln1_eps, x, B, E, stream);
-  if (rc) return rc;
-  // q, k, v projections
+  if ((rc = layernorm(L, pending, hidden, L->ln1_gamma, L->ln1_beta, L->ln1_eps, x, B, stream))) return rc;
   const int8_t* w3[3] = {L->wq, L->wk, L->wv};
   const int8_t* b3[3] = {L->bq, L->bk, L->bv};
   int8_t* o3[3] = {q, k, v};
@@ -789,73 +832,40 @@ int ti_opt_decoder_layer_decode(const TiOptDecodeLayer* L, void* hidden, const f
   if ((rc = ti_decode_attn_s8(q, k, v, k_buf, v_buf, mask, ctx, nullptr, B * H, 1, d, cap, S, H, L->alpha_qk, L->alpha_pv,
                               stream)))
     return rc;
-  // out_proj, then the residual update fused with final_layer_norm
-  if ((rc = ti_linear_a8_w8_bfp32_ofp32(ctx, L->wo, L->bo, f32, B, E, E, L->alpha_o, 1.0f, ws, ws_bytes, stream))) return rc;
-  rc = L->half ? ti_add_layernorm_q_f16_xf32(f32, hidden, L->ln2_gamma, L->ln2_beta, L->ln2_eps, x, B, E, stream)
-               : ti_add_layernorm_q(f32, static_cast<float*>(hidden), static_cast<const float*>(L->ln2_gamma),
-                                    static_cast<const float*>(L->ln2_beta), L->ln2_eps, x, B, E, stream);
-  if (rc) return rc;
-  // fc1 (ReLU), fc2 added into the residual stream
-  if ((rc = ti_linear_relu_a8_w8_b8_o8(x, L->w1, L->b1, h, B, F, E, L->alpha_1, L->beta_1, ws, ws_bytes, stream))) return rc;
-  if (L->half) {
-    if ((rc = ti_linear_a8_w8_bfp32_ofp32(h, L->w2, L->b2, f32, B, E, F, L->alpha_2, 1.0f, ws, ws_bytes, stream))) return rc;
-    return ti_add_f16_xf32(f32, hidden, B * E, stream);
-  }
-  return ti_linear_a8_w8_bfp32_ofp32_acc(h, L->w2, L->b2, static_cast<float*>(hidden), B, E, F, L->alpha_2, 1.0f, ws, ws_bytes,
-                                         stream);
+  return after_attention(L, ctx, f32, x, h, hidden, B, chain, carry, ws, ws_bytes, stream);
 }
 
-// One decoder layer of a prefill (no cache yet): the launches an Int8OPTDecoderLayer makes for T > 16 tokens per
-// sequence when its attention takes the one-launch prefill kernel, issued from one C call through the public entry
-// points, with the arguments the modules pass.
-int64_t ti_opt_decoder_layer_prefill_scratch_bytes(int64_t rows, int64_t embed, int64_t ffn) {
-  if (rows <= 0 || embed <= 0 || ffn <= 0) return 0;
-  auto up = [](int64_t n) { return (n + 255) / 256 * 256; };
-  return 4 * up(rows * embed) + up(4 * rows * embed) + up(rows * ffn);
-}
-
-int ti_opt_decoder_layer_prefill(const TiOptDecodeLayer* L, void* hidden, const float* mask, const uint8_t* mask_classes,
-                                 int8_t* k_out, int8_t* v_out, int64_t B, int64_t T, void* scratch, int64_t scratch_bytes,
-                                 void* workspace, int64_t workspace_bytes, void* stream) {
-  g_err[0] = 0;
-  const char* op = "opt_decoder_layer_prefill";
-  if (L == nullptr) return fail(TI_ERR_INVALID_ARG, "%s: no layer description", op);
+int prefill_layer(const char* op, const TiOptDecodeLayer* L, void* hidden, const float* mask, const uint8_t* mask_classes,
+                  int8_t* k_out, int8_t* v_out, int64_t B, int64_t T, int chain, float* carry, void* scratch,
+                  int64_t scratch_bytes, void* workspace, int64_t workspace_bytes, void* stream, int64_t most) {
+  if (int rc = check_layer(op, L)) return rc;
   const int64_t E = L->embed, H = L->heads, d = L->head_dim, F = L->ffn;
-  if (E <= 0 || H <= 0 || d <= 0 || F <= 0 || H * d != E)
-    return fail(TI_ERR_INVALID_ARG, "%s: needs embed = heads * head_dim > 0 and ffn > 0 (got %lld, %lld x %lld, %lld)", op,
-                (long long)E, (long long)H, (long long)d, (long long)F);
   if (B < 0 || T < 0 || B > 65535 || T > 4096) return fail(TI_ERR_INVALID_ARG, "%s: needs 0 <= B <= 65535, 0 <= T <= 4096", op);
   const int64_t M = B * T;
   if (M == 0) return TI_OK;
-  if (M > 4096) return fail(TI_ERR_INVALID_ARG, "%s: up to 4096 tokens in all (got %lld x %lld)", op, (long long)B, (long long)T);
+  if (M > most)
+    return fail(TI_ERR_INVALID_ARG, "%s: up to %lld tokens in all (got %lld x %lld)", op, (long long)most, (long long)B, (long long)T);
   if (!attn_prefill_supported(T, T, d))
     return fail(TI_ERR_INVALID_ARG, "%s: %lld tokens per sequence at head size %lld: needs a multiple of 16 up to 4096 and a "
                 "head size that is a multiple of 16 up to 128", op, (long long)T, (long long)d);
   if (int rc = check_ptr(op, "hidden", hidden, L->half ? 2 : 4, true)) return rc;
   if (int rc = check_ptr(op, "k_out", k_out, 16, true)) return rc;
   if (int rc = check_ptr(op, "v_out", v_out, 16, true)) return rc;
+  if (int rc = check_ptr(op, "carry", carry, 16, chain != 0)) return rc;
   if (int rc = check_ptr(op, "scratch", scratch, 256, true)) return rc;
-  if (scratch_bytes < ti_opt_decoder_layer_prefill_scratch_bytes(M, E, F))
-    return fail(TI_ERR_INVALID_ARG, "%s: scratch of %lld bytes, needs %lld", op, (long long)scratch_bytes,
-                (long long)ti_opt_decoder_layer_prefill_scratch_bytes(M, E, F));
-  auto up = [](int64_t n) { return (n + 255) / 256 * 256; };
-  char* at = static_cast<char*>(scratch);
-  auto take = [&](int64_t bytes) {
-    char* r = at;
-    at += up(bytes);
-    return r;
-  };
-  int8_t* x = reinterpret_cast<int8_t*>(take(M * E));     // LayerNorm-quantised input of the projections, then of fc1
-  int8_t* q = reinterpret_cast<int8_t*>(take(M * E));     // [B, heads, T, head_dim]
-  int8_t* vt = reinterpret_cast<int8_t*>(take(M * E));    // [B * heads, head_dim, T]
-  int8_t* ctx = reinterpret_cast<int8_t*>(take(M * E));   // [B, T, embed]
-  float* f32 = reinterpret_cast<float*>(take(4 * M * E)); // output of out_proj, then (fp16 stream) of fc2
-  int8_t* h = reinterpret_cast<int8_t*>(take(M * F));
+  const int64_t need = ti_opt_decoder_layer_prefill_scratch_bytes(M, E, F);
+  if (scratch_bytes < need)
+    return fail(TI_ERR_INVALID_ARG, "%s: scratch of %lld bytes, needs %lld", op, (long long)scratch_bytes, (long long)need);
+  Carver carve{static_cast<char*>(scratch)};
+  int8_t* x = carve.take<int8_t>(M * E);      // LayerNorm-quantised input of the projections, then of fc1
+  int8_t* q = carve.take<int8_t>(M * E);      // [B, heads, T, head_dim]
+  int8_t* vt = carve.take<int8_t>(M * E);     // [B * heads, head_dim, T]
+  int8_t* ctx = carve.take<int8_t>(M * E);    // [B, T, embed]
+  float* f32 = carve.take<float>(4 * M * E);  // output of out_proj, then of fc2
+  int8_t* h = carve.take<int8_t>(M * F);
+  const float* pending = (chain & CHAIN_ADD) && adds_later(L, M) ? carry : nullptr;
   int rc;
-  rc = L->half ? ti_add_layernorm_q_f16(nullptr, hidden, L->ln1_gamma, L->ln1_beta, L->ln1_eps, x, M, E, stream)
-               : ti_add_layernorm_q(nullptr, static_cast<float*>(hidden), static_cast<const float*>(L->ln1_gamma),
-                                    static_cast<const float*>(L->ln1_beta), L->ln1_eps, x, M, E, stream);
-  if (rc) return rc;
+  if ((rc = layernorm(L, pending, hidden, L->ln1_gamma, L->ln1_beta, L->ln1_eps, x, M, stream))) return rc;
   // q, k, v stored head-major by the projections themselves: one grouped launch where the library has one, else one
   // call per projection with the split-K workspace (the choice the attention module makes)
   const int8_t* w3[3] = {L->wq, L->wk, L->wv};
@@ -876,24 +886,50 @@ int ti_opt_decoder_layer_prefill(const TiOptDecodeLayer* L, void* hidden, const 
   if ((rc = ti_attn_prefill_s8_mc(q, k_out, vt, mask, mask_classes, ctx, B * H, T, T, d, T * d, T * d, H, L->alpha_qk,
                                   L->alpha_pv, stream)))
     return rc;
-  if ((rc = ti_linear_a8_w8_bfp32_ofp32(ctx, L->wo, L->bo, f32, M, E, E, L->alpha_o, 1.0f, workspace, workspace_bytes,
-                                        stream)))
-    return rc;
-  rc = L->half ? ti_add_layernorm_q_f16_xf32(f32, hidden, L->ln2_gamma, L->ln2_beta, L->ln2_eps, x, M, E, stream)
-               : ti_add_layernorm_q(f32, static_cast<float*>(hidden), static_cast<const float*>(L->ln2_gamma),
-                                    static_cast<const float*>(L->ln2_beta), L->ln2_eps, x, M, E, stream);
-  if (rc) return rc;
-  if ((rc = ti_linear_relu_a8_w8_b8_o8(x, L->w1, L->b1, h, M, F, E, L->alpha_1, L->beta_1, workspace, workspace_bytes,
-                                       stream)))
-    return rc;
-  if (L->half) {
-    if ((rc = ti_linear_a8_w8_bfp32_ofp32(h, L->w2, L->b2, f32, M, E, F, L->alpha_2, 1.0f, workspace, workspace_bytes,
-                                          stream)))
-      return rc;
-    return ti_add_f16_xf32(f32, hidden, M * E, stream);
-  }
-  return ti_linear_a8_w8_bfp32_ofp32_acc(h, L->w2, L->b2, static_cast<float*>(hidden), M, E, F, L->alpha_2, 1.0f, workspace,
-                                         workspace_bytes, stream);
+  return after_attention(L, ctx, f32, x, h, hidden, M, chain, carry, workspace, workspace_bytes, stream);
+}
+}  // namespace
+extern "C" {
+
+int64_t ti_opt_decoder_layer_decode_scratch_bytes(int64_t B, int64_t embed, int64_t ffn) {
+  if (B <= 0 || embed <= 0 || ffn <= 0) return 0;
+  return 5 * up256(B * embed) + up256(4 * B * embed) + up256(B * ffn) + up256(decode_workspace_bytes(B, embed, ffn));
+}
+
+int ti_opt_decoder_layer_decode(const TiOptDecodeLayer* L, void* hidden, const float* mask, int8_t* k_buf, int8_t* v_buf,
+                                int64_t B, int64_t cap, int64_t S, void* scratch, int64_t scratch_bytes, void* stream) {
+  g_err[0] = 0;
+  return decode_layer("opt_decoder_layer_decode", L, hidden, mask, k_buf, v_buf, B, cap, S, 0, nullptr, scratch, scratch_bytes, stream, 16);
+}
+
+int ti_opt_decoder_layer_decode_chained(const TiOptDecodeLayer* L, void* hidden, const float* mask, int8_t* k_buf,
+                                        int8_t* v_buf, int64_t B, int64_t cap, int64_t S, int chain, float* carry,
+                                        void* scratch, int64_t scratch_bytes, void* stream) {
+  g_err[0] = 0;
+  return decode_layer("opt_decoder_layer_decode_chained", L, hidden, mask, k_buf, v_buf, B, cap, S, chain, carry, scratch,
+                      scratch_bytes, stream, 64);
+}
+
+int64_t ti_opt_decoder_layer_prefill_scratch_bytes(int64_t rows, int64_t embed, int64_t ffn) {
+  if (rows <= 0 || embed <= 0 || ffn <= 0) return 0;
+  return 4 * up256(rows * embed) + up256(4 * rows * embed) + up256(rows * ffn);
+}
+
+int ti_opt_decoder_layer_prefill(const TiOptDecodeLayer* L, void* hidden, const float* mask, const uint8_t* mask_classes,
+                                 int8_t* k_out, int8_t* v_out, int64_t B, int64_t T, void* scratch, int64_t scratch_bytes,
+                                 void* workspace, int64_t workspace_bytes, void* stream) {
+  g_err[0] = 0;
+  return prefill_layer("opt_decoder_layer_prefill", L, hidden, mask, mask_classes, k_out, v_out, B, T, 0, nullptr, scratch,
+                       scratch_bytes, workspace, workspace_bytes, stream, 4096);
+}
+
+int ti_opt_decoder_layer_prefill_chained(const TiOptDecodeLayer* L, void* hidden, const float* mask,
+                                         const uint8_t* mask_classes, int8_t* k_out, int8_t* v_out, int64_t B, int64_t T,
+                                         int chain, float* carry, void* scratch, int64_t scratch_bytes, void* workspace,
+                                         int64_t workspace_bytes, void* stream) {
+  g_err[0] = 0;
+  return prefill_layer("opt_decoder_layer_prefill_chained", L, hidden, mask, mask_classes, k_out, v_out, B, T, chain, carry, scratch,
+                       scratch_bytes, workspace, workspace_bytes, stream, 1 << 20);
 }
 
 }  // extern "C"

@@ -196,42 +196,104 @@ static PyObject* fc_decode_attn(PyObject* self, PyObject* const* a, Py_ssize_t n
                                            (float)apv, st));
 }
 
-/* opt_layer_decode(layer, hidden, mask, k_buf, v_buf, B, cap, S, scratch, scratch_bytes, stream) -> status;
+/* opt_layer_decode(layer, hidden, mask, k_buf, v_buf, B, cap, S, chain, carry, scratch, scratch_bytes, stream) -> status;
  * layer = address of a TiOptDecodeLayer that the caller keeps alive */
 static PyObject* fc_opt_layer_decode(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   (void)self;
-  if (n != 11) {
-    PyErr_SetString(PyExc_TypeError, "opt_layer_decode expects 11 arguments");
+  if (n != 13) {
+    PyErr_SetString(PyExc_TypeError, "opt_layer_decode expects 13 arguments");
     return NULL;
   }
   void *layer = as_ptr(a[0]), *hidden = as_ptr(a[1]), *mask = as_ptr(a[2]), *kb = as_ptr(a[3]), *vb = as_ptr(a[4]);
-  int64_t B = as_i64(a[5]), cap = as_i64(a[6]), S = as_i64(a[7]);
-  void* scratch = as_ptr(a[8]);
-  int64_t sb = as_i64(a[9]);
-  void* st = as_ptr(a[10]);
+  int64_t B = as_i64(a[5]), cap = as_i64(a[6]), S = as_i64(a[7]), chain = as_i64(a[8]);
+  void *carry = as_ptr(a[9]), *scratch = as_ptr(a[10]);
+  int64_t sb = as_i64(a[11]);
+  void* st = as_ptr(a[12]);
   if (PyErr_Occurred()) return NULL;
-  return PyLong_FromLong(ti_opt_decoder_layer_decode((const TiOptDecodeLayer*)layer, hidden, (const float*)mask, kb, vb, B,
-                                                     cap, S, scratch, sb, st));
+  return PyLong_FromLong(ti_opt_decoder_layer_decode_chained((const TiOptDecodeLayer*)layer, hidden, (const float*)mask, kb,
+                                                             vb, B, cap, S, (int)chain, carry, scratch, sb, st));
 }
 
-/* opt_layer_prefill(layer, hidden, mask, classes, k_out, v_out, B, T, scratch, scratch_bytes, ws, ws_bytes, stream) -> status */
+/* opt_layer_prefill(layer, hidden, mask, classes, k_out, v_out, B, T, chain, carry, scratch, scratch_bytes, ws, ws_bytes, stream) -> status */
 static PyObject* fc_opt_layer_prefill(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   (void)self;
-  if (n != 13) {
-    PyErr_SetString(PyExc_TypeError, "opt_layer_prefill expects 13 arguments");
+  if (n != 15) {
+    PyErr_SetString(PyExc_TypeError, "opt_layer_prefill expects 15 arguments");
     return NULL;
   }
   void *layer = as_ptr(a[0]), *hidden = as_ptr(a[1]), *mask = as_ptr(a[2]), *cls = as_ptr(a[3]);
   void *ko = as_ptr(a[4]), *vo = as_ptr(a[5]);
-  int64_t B = as_i64(a[6]), T = as_i64(a[7]);
-  void* scratch = as_ptr(a[8]);
-  int64_t sb = as_i64(a[9]);
-  void* ws = as_ptr(a[10]);
-  int64_t wsb = as_i64(a[11]);
-  void* st = as_ptr(a[12]);
+  int64_t B = as_i64(a[6]), T = as_i64(a[7]), chain = as_i64(a[8]);
+  void *carry = as_ptr(a[9]), *scratch = as_ptr(a[10]);
+  int64_t sb = as_i64(a[11]);
+  void* ws = as_ptr(a[12]);
+  int64_t wsb = as_i64(a[13]);
+  void* st = as_ptr(a[14]);
   if (PyErr_Occurred()) return NULL;
-  return PyLong_FromLong(ti_opt_decoder_layer_prefill((const TiOptDecodeLayer*)layer, hidden, (const float*)mask,
-                                                      (const uint8_t*)cls, ko, vo, B, T, scratch, sb, ws, wsb, st));
+  return PyLong_FromLong(ti_opt_decoder_layer_prefill_chained((const TiOptDecodeLayer*)layer, hidden, (const float*)mask,
+                                                              (const uint8_t*)cls, ko, vo, B, T, (int)chain, carry, scratch, sb,
+                                                              ws, wsb, st));
+}
+
+/* t = (dict, name, object, ...) of `size` items: 1 when dict[name] is that object, 0 when not, -1 with an exception set */
+static int still_held(PyObject* t, Py_ssize_t size) {
+  if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != size) {
+    PyErr_SetString(PyExc_TypeError, "plan_current: (dict, name, tensor, version) and (dict, name, module) tuples");
+    return -1;
+  }
+  PyObject* held = PyObject_GetItem(PyTuple_GET_ITEM(t, 0), PyTuple_GET_ITEM(t, 1));
+  if (held == NULL) {
+    if (!PyErr_ExceptionMatches(PyExc_KeyError)) return -1;
+    PyErr_Clear();
+    return 0;
+  }
+  Py_DECREF(held); /* only compared from here on; the tuple keeps its own object alive */
+  return held == PyTuple_GET_ITEM(t, 2);
+}
+
+/* plan_current(sources, modules) -> bool.  sources: tuple of (dict, name, tensor, version): every dict still holds that
+ * tensor under that name and nothing has written to it since; modules: tuple of (dict, name, module): likewise, and the
+ * module has no forward hooks. */
+static PyObject* fc_plan_current(PyObject* self, PyObject* const* a, Py_ssize_t n) {
+  (void)self;
+  static PyObject *s_version, *s_hooks, *s_pre;
+  if (n != 2 || !PyTuple_Check(a[0]) || !PyTuple_Check(a[1])) {
+    PyErr_SetString(PyExc_TypeError, "plan_current expects two tuples");
+    return NULL;
+  }
+  if (s_version == NULL) {
+    s_version = PyUnicode_InternFromString("_version");
+    s_hooks = PyUnicode_InternFromString("_forward_hooks");
+    s_pre = PyUnicode_InternFromString("_forward_pre_hooks");
+    if (s_version == NULL || s_hooks == NULL || s_pre == NULL) return NULL;
+  }
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(a[0]); ++i) {
+    PyObject* t = PyTuple_GET_ITEM(a[0], i);
+    const int held = still_held(t, 4);
+    if (held < 0) return NULL;
+    if (!held) Py_RETURN_FALSE;
+    PyObject* version = PyObject_GetAttr(PyTuple_GET_ITEM(t, 2), s_version);
+    if (version == NULL) return NULL;
+    const int same = PyObject_RichCompareBool(version, PyTuple_GET_ITEM(t, 3), Py_EQ);
+    Py_DECREF(version);
+    if (same < 0) return NULL;
+    if (!same) Py_RETURN_FALSE;
+  }
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(a[1]); ++i) {
+    PyObject* t = PyTuple_GET_ITEM(a[1], i);
+    const int held = still_held(t, 3);
+    if (held < 0) return NULL;
+    if (!held) Py_RETURN_FALSE;
+    for (int k = 0; k < 2; ++k) {
+      PyObject* hooks = PyObject_GetAttr(PyTuple_GET_ITEM(t, 2), k ? s_pre : s_hooks);
+      if (hooks == NULL) return NULL;
+      const Py_ssize_t count = PyObject_Size(hooks);
+      Py_DECREF(hooks);
+      if (count < 0) return NULL;
+      if (count > 0) Py_RETURN_FALSE;
+    }
+  }
+  Py_RETURN_TRUE;
 }
 
 static PyObject* fc_last_error(PyObject* self, PyObject* noargs) {
@@ -251,8 +313,9 @@ static PyMethodDef methods[] = {
     {"linear_group3", (PyCFunction)(void (*)(void))fc_linear_group3, METH_FASTCALL, "forward to ti_linear_a8_w8_b8_o8_group"},
     {"kv_append", (PyCFunction)(void (*)(void))fc_kv_append, METH_FASTCALL, "forward to ti_kv_append_s8"},
     {"decode_attn", (PyCFunction)(void (*)(void))fc_decode_attn, METH_FASTCALL, "forward to ti_decode_attn_s8"},
-    {"opt_layer_decode", (PyCFunction)(void (*)(void))fc_opt_layer_decode, METH_FASTCALL, "forward to ti_opt_decoder_layer_decode"},
-    {"opt_layer_prefill", (PyCFunction)(void (*)(void))fc_opt_layer_prefill, METH_FASTCALL, "forward to ti_opt_decoder_layer_prefill"},
+    {"opt_layer_decode", (PyCFunction)(void (*)(void))fc_opt_layer_decode, METH_FASTCALL, "forward to ti_opt_decoder_layer_decode_chained"},
+    {"opt_layer_prefill", (PyCFunction)(void (*)(void))fc_opt_layer_prefill, METH_FASTCALL, "forward to ti_opt_decoder_layer_prefill_chained"},
+    {"plan_current", (PyCFunction)(void (*)(void))fc_plan_current, METH_FASTCALL, "tensors and hooks as a plan found them"},
     {"last_error", fc_last_error, METH_NOARGS, "ti_last_error()"},
     {NULL, NULL, 0, NULL}};
 

@@ -321,34 +321,39 @@ int launch_add_layernorm_q_f16(const void* x, void* residual, const void* gamma,
                              q_out, rows, H, stream);
 }
 
-// residual (fp16) += fp16(x), elementwise, for an fp32 x: `residual.add_(x.to(residual.dtype))` in one pass (what the
-// decoder layer does with the fp32 output of fc2 on an fp16 stream).  Chunks of four elements; a scalar tail.
-__global__ __launch_bounds__(256) void add_f16_xf32_kernel(const float* __restrict__ x, _Float16* residual, long long n,
-                                                           bool vec) {
+// residual += x, elementwise, for an fp32 x (an fp16 residual: += fp16(x), `residual.add_(x.to(residual.dtype))` in one
+// pass): what a decoder layer does with the fp32 output of fc2.  Chunks of four elements; a scalar tail.
+template <class T>
+__global__ __launch_bounds__(256) void add_xf32_kernel(const float* __restrict__ x, T* residual, long long n, bool vec) {
   const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
   if (c * 4 >= n) return;
   if (vec && c * 4 + 4 <= n) {
     const v4f a = reinterpret_cast<const v4f*>(x)[c];
-    const v4h h = reinterpret_cast<const v4h*>(residual)[c];
-    v4h o;
+    v4f o = load4(residual, (int)c);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = (_Float16)as_stored<_Float16>((float)h[j] + as_stored<_Float16>(a[j]));
-    reinterpret_cast<v4h*>(residual)[c] = o;
+    for (int j = 0; j < 4; ++j) o[j] = as_stored<T>(o[j] + as_stored<T>(a[j]));
+    store4(residual, (int)c, o);
   } else {
-    for (long long i = c * 4; i < n && i < c * 4 + 4; ++i)
-      residual[i] = (_Float16)as_stored<_Float16>((float)residual[i] + as_stored<_Float16>(x[i]));
+    for (long long i = c * 4; i < n && i < c * 4 + 4; ++i) residual[i] = (T)as_stored<T>((float)residual[i] + as_stored<T>(x[i]));
   }
 }
 
-int launch_add_f16_xf32(const float* x, void* residual, long long n, hipStream_t stream) {
+template <class T>
+static int launch_add_xf32(const float* x, T* residual, long long n, hipStream_t stream) {
   if (n == 0) return TI_OK;
-  const bool vec = (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(residual) & 7) == 0;
+  const bool vec = (reinterpret_cast<uintptr_t>(x) & 15) == 0 &&
+                   (reinterpret_cast<uintptr_t>(residual) & (4 * sizeof(T) - 1)) == 0 && n < (1LL << 32);
   const long long chunks = (n + 3) / 4;
-  hipLaunchKernelGGL(add_f16_xf32_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, stream, x,
-                     static_cast<_Float16*>(residual), n, vec);
+  hipLaunchKernelGGL(add_xf32_kernel<T>, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, stream, x, residual, n, vec);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "add_f16_xf32 launch: %s", hipGetErrorString(e));
+  if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "add_xf32 launch: %s", hipGetErrorString(e));
   return TI_OK;
+}
+int launch_add_f16_xf32(const float* x, void* residual, long long n, hipStream_t stream) {
+  return launch_add_xf32(x, static_cast<_Float16*>(residual), n, stream);
+}
+int launch_add_f32(const float* x, float* residual, long long n, hipStream_t stream) {
+  return launch_add_xf32(x, residual, n, stream);
 }
 
 // residual (fp16) += fp16(x) for an fp32 x, then the LayerNorm-quantiser: `residual.add_(x.to(residual.dtype))`

@@ -113,9 +113,15 @@ _lib.ti_opt_decoder_layer_prefill_scratch_bytes.argtypes = [_i64, _i64, _i64]
 _lib.ti_opt_decoder_layer_prefill_scratch_bytes.restype = _i64
 _lib.ti_opt_decoder_layer_prefill.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp, _i64, _vp, _i64, _vp]
 _lib.ti_opt_decoder_layer_prefill.restype = ctypes.c_int
+_lib.ti_opt_decoder_layer_decode_chained.argtypes = [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, ctypes.c_int, _vp, _vp, _i64,
+                                                     _vp]
+_lib.ti_opt_decoder_layer_decode_chained.restype = ctypes.c_int
+_lib.ti_opt_decoder_layer_prefill_chained.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, ctypes.c_int, _vp, _vp, _i64,
+                                                      _vp, _i64, _vp]
+_lib.ti_opt_decoder_layer_prefill_chained.restype = ctypes.c_int
 _raw_stream = torch._C._cuda_getCurrentRawStream
-_fast_opt_layer_decode = getattr(_CUDA._fast, "opt_layer_decode", None)
-_fast_opt_layer_prefill = getattr(_CUDA._fast, "opt_layer_prefill", None)
+_opt_layer_decode = getattr(_CUDA._fast, "opt_layer_decode", None) or _lib.ti_opt_decoder_layer_decode_chained
+_opt_layer_prefill = getattr(_CUDA._fast, "opt_layer_prefill", None) or _lib.ti_opt_decoder_layer_prefill_chained
 _fast = _CUDA._fast if getattr(_CUDA._fast, "kv_append", None) is not None else None
 _fast_decode_attn = getattr(_CUDA._fast, "decode_attn", None)
 _fast_group3 = getattr(_CUDA._fast, "linear_group3", None)
@@ -585,13 +591,17 @@ def _scratch_for(dev, stream, nbytes):
 _layer_scratch_need = {}
 
 
-def opt_layer_decode(plan, hidden, mask, k_buf, v_buf, S):
-    """One decode step of one decoder layer from one C call (``ti_opt_decoder_layer_decode``): ``hidden`` [B, 1, embed]
-    (fp32, or fp16 when the plan says half) is updated in place, the new key and value rows are appended to the cache
-    buffers, which hold S - 1 positions before the call.  ``plan`` carries ``addr`` (the address of an ``OptDecodeLayer``
-    that the caller filled from tensors it keeps alive), ``embed`` and ``ffn``; the caller has checked shapes, dtypes,
-    devices and contiguity (the decoder layer does).  The scratch memory is one buffer per device, stream and size,
-    shared by every layer."""
+#: bits of ``chain``: this layer adds what the layer before left in ``carry`` / leaves its own fc2 output there
+CHAIN_ADD, CHAIN_LEAVE = 1, 2
+
+
+def opt_layer_decode(plan, hidden, mask, k_buf, v_buf, S, chain=0, carry=None):
+    """One decode step of one decoder layer from one C call (``ti_opt_decoder_layer_decode_chained``): ``hidden`` [B, 1, embed]
+    (fp32, or fp16 when the plan says half; up to 64 sequences) is updated in place, the new key and value rows are appended
+    to the cache buffers, which hold S - 1 positions before the call.  ``plan`` carries ``addr`` (the address of an
+    ``OptDecodeLayer`` that the caller filled from tensors it keeps alive), ``embed`` and ``ffn``; the caller has checked
+    shapes, dtypes, devices and contiguity (the decoder layer does).  The scratch memory is one buffer per device, stream
+    and size, shared by every layer; ``chain`` and ``carry`` (fp32 [B, embed], of this pass) tie the layers of one forward pass together."""
     dev = hidden.device
     B = hidden.shape[0]
     with _on(dev):
@@ -601,52 +611,64 @@ def opt_layer_decode(plan, hidden, mask, k_buf, v_buf, S):
         if need is None:
             need = _layer_scratch_need[key] = _lib.ti_opt_decoder_layer_decode_scratch_bytes(B, plan.embed, plan.ffn)
         scratch = _scratch_for(dev, stream, need)
-        if _fast_opt_layer_decode is not None:
-            rc = _fast_opt_layer_decode(plan.addr, hidden.data_ptr(),
-                                        mask.data_ptr() if mask is not None else 0, k_buf.data_ptr(), v_buf.data_ptr(),
-                                        B, k_buf.shape[2], S, scratch.data_ptr(), scratch.numel(), stream)
-        else:
-            rc = _lib.ti_opt_decoder_layer_decode(plan.addr, hidden.data_ptr(),
-                                                  mask.data_ptr() if mask is not None else None, k_buf.data_ptr(),
-                                                  v_buf.data_ptr(), B, k_buf.shape[2], S, scratch.data_ptr(),
-                                                  scratch.numel(), stream or None)
+        rc = _opt_layer_decode(plan.addr, hidden.data_ptr(), mask.data_ptr() if mask is not None else 0, k_buf.data_ptr(),
+                               v_buf.data_ptr(), B, k_buf.shape[2], S, chain, carry.data_ptr() if chain else 0, scratch.data_ptr(),
+                               scratch.numel(), stream)
     if rc:
         raise RuntimeError(f"torch_int._hip_ext.opt_layer_decode: {_lib.ti_last_error().decode()} (status {rc})")
     return hidden
 
 
-def opt_layer_prefill(plan, hidden, mask, k_out, v_out):
-    """A prefill through one decoder layer from one C call (``ti_opt_decoder_layer_prefill``): ``hidden`` [B, T, embed]
+def opt_prefill_scratch(plan, hidden):
+    """The scratch memory and the split-K workspace of the layers of one prefill: (tensor, workspace pointer, its bytes).
+    More than 64 MiB of scratch come from torch's allocator for the pass instead of staying with the stream."""
+    dev = hidden.device
+    M, E, F = hidden.shape[0] * hidden.shape[1], plan.embed, plan.ffn
+    stream = _raw_stream(dev.index)
+    key = (1, M, E, F)
+    need = _layer_scratch_need.get(key)
+    if need is None:
+        if len(_layer_scratch_need) > 4096:
+            _layer_scratch_need.clear()
+        need = _layer_scratch_need[key] = (
+            _lib.ti_opt_decoder_layer_prefill_scratch_bytes(M, E, F),
+            max(_CUDA._ws_bytes(M, E, E), _CUDA._ws_bytes(M, F, E), _CUDA._ws_bytes(M, E, F)))
+    scratch = (_scratch_for(dev, stream, need[0]) if need[0] <= 64 << 20
+               else torch.empty(need[0], dtype=torch.uint8, device=dev))
+    return (scratch,) + _CUDA._workspace(dev.index, stream, need[1])
+
+
+def opt_layer_prefill(plan, hidden, mask, k_out, v_out, chain=0, carry=None, memory=None):
+    """A prefill through one decoder layer from one C call (``ti_opt_decoder_layer_prefill_chained``): ``hidden`` [B, T, embed]
     is updated in place, ``k_out`` / ``v_out`` (int8 [B, heads, T, head_dim], contiguous) receive the layer's key and
-    value rows.  ``plan`` as for ``opt_layer_decode``; the caller has checked shapes, dtypes, devices and contiguity."""
+    value rows.  ``plan``, ``chain`` and ``carry`` as for ``opt_layer_decode``; the caller has checked shapes, dtypes, devices and
+    contiguity.  Layers of one chain share ``memory`` (``opt_prefill_scratch``)."""
     dev = hidden.device
     B, T = hidden.shape[0], hidden.shape[1]
-    M, E, F = B * T, plan.embed, plan.ffn
     with _on(dev):
-        stream = _raw_stream(dev.index)
-        key = (1, M, E, F)
-        need = _layer_scratch_need.get(key)
-        if need is None:
-            if len(_layer_scratch_need) > 4096:
-                _layer_scratch_need.clear()
-            need = _layer_scratch_need[key] = (
-                _lib.ti_opt_decoder_layer_prefill_scratch_bytes(M, E, F),
-                max(_CUDA._ws_bytes(M, E, E), _CUDA._ws_bytes(M, F, E), _CUDA._ws_bytes(M, E, F)))
-        scratch = _scratch_for(dev, stream, need[0])
-        ws_ptr, ws_bytes = _CUDA._workspace(dev.index, stream, need[1])
+        scratch, ws_ptr, ws_bytes = memory if memory is not None else opt_prefill_scratch(plan, hidden)
         cls = _classes_ptr(mask, T) if mask is not None else None
-        if _fast_opt_layer_prefill is not None:
-            rc = _fast_opt_layer_prefill(plan.addr, hidden.data_ptr(), mask.data_ptr() if mask is not None else 0,
-                                         cls or 0, k_out.data_ptr(), v_out.data_ptr(), B, T, scratch.data_ptr(),
-                                         scratch.numel(), ws_ptr, ws_bytes, stream)
-        else:
-            rc = _lib.ti_opt_decoder_layer_prefill(plan.addr, hidden.data_ptr(),
-                                                   mask.data_ptr() if mask is not None else None, cls, k_out.data_ptr(),
-                                                   v_out.data_ptr(), B, T, scratch.data_ptr(), scratch.numel(),
-                                                   ws_ptr or None, ws_bytes, stream or None)
+        rc = _opt_layer_prefill(plan.addr, hidden.data_ptr(), mask.data_ptr() if mask is not None else 0, cls or 0,
+                                k_out.data_ptr(), v_out.data_ptr(), B, T, chain, carry.data_ptr() if chain else 0, scratch.data_ptr(),
+                                scratch.numel(), ws_ptr, ws_bytes, _raw_stream(dev.index))
     if rc:
         raise RuntimeError(f"torch_int._hip_ext.opt_layer_prefill: {_lib.ti_last_error().decode()} (status {rc})")
     return hidden
+
+
+def _plan_current(sources, modules):
+    for holder, name, tensor, version in sources:
+        if holder.get(name) is not tensor or tensor._version != version:
+            return False
+    for holder, name, mod in modules:
+        if holder.get(name) is not mod or mod._forward_hooks or mod._forward_pre_hooks:
+            return False
+    return True
+
+
+#: (sources, modules) -> bool: every (dict, name, tensor, version) and (dict, name, module) of a plan still holds, and no module
+#: has a forward hook (which wants to see that module's call)
+plan_current = getattr(_CUDA._fast, "plan_current", None) or _plan_current
 
 
 def decode_attention_devlen(q, k_new, v_new, k_buf, v_buf, length, max_length, alpha_qk, alpha_pv):

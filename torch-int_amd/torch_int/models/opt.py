@@ -16,6 +16,7 @@ import torch
 from torch import nn
 
 from .. import _hip_ext
+from ..nn._scalars import read_scalars
 from ..nn.bmm import BMM_S8T_S8N_F32T, BMM_S8T_S8N_S8T
 from ..nn.fused import LayerNormQ
 from ..nn.linear import W8A8B8O8Linear, W8A8B8O8LinearReLU, W8A8BFP32OFP32Linear
@@ -61,8 +62,18 @@ def _kv_fresh(past, T):
     return _KVBuffer(buf, S)
 
 
+def _kv_rooms(past):
+    """Buffers of a layer's (key, value) cache with room for one more position, or None when a kernel cannot write there."""
+    kk = _kv_room_for(past[0], 1) or _kv_fresh(past[0], 1)
+    vv = _kv_room_for(past[1], 1) or _kv_fresh(past[1], 1)
+    kb, vb = kk.buf, vv.buf
+    if kb.data_ptr() % 16 or vb.data_ptr() % 16 or not (kb.is_contiguous() and vb.is_contiguous() and kb.shape == vb.shape):
+        return None
+    return kk, vv
+
+
 def _kv_view(kv, n):
-    out = kv.buf[:, :, :n]
+    out = kv.buf.narrow(2, 0, n)
     out._ti_kv = kv
     return out
 
@@ -358,22 +369,33 @@ class Int8OPTAttention(nn.Module):
 
 class _DecodePlan:
     """``Int8OPTDecoderLayer`` flattened into the structure ``ti_opt_decoder_layer_decode`` reads, plus what it was
-    built from: (dict that holds the tensor, its name, the tensor, its version) for every buffer, so that a replaced
-    or rewritten buffer is noticed."""
+    built from: (dict that holds the tensor, its name, the tensor, its version) for every buffer and (dict, name, module)
+    for every sub-module, so that a replaced or rewritten buffer and a replaced module are noticed."""
     __slots__ = ("ok", "half", "device", "struct", "addr", "sources", "modules", "embed", "heads", "head_dim", "ffn")
+
+    def __reduce__(self):   # a copied or pickled layer makes a plan of its own tensors
+        return _no_plan, ()
+
+    def new_cache(self, hidden):
+        """Empty key and value tensors [bsz, heads, tokens, head_dim] for a prefill of ``hidden``."""
+        shape = (hidden.shape[0], self.heads, hidden.shape[1], self.head_dim)
+        return (torch.empty(shape, dtype=torch.int8, device=self.device), torch.empty(shape, dtype=torch.int8, device=self.device))
 
     @staticmethod
     def build(layer, half, device):
         plan = _DecodePlan()
-        plan.ok, plan.half, plan.device, plan.sources = False, half, device, []
+        plan.ok, plan.half, plan.device = False, half, device
+        sources = []
         at = layer.self_attn
-        plan.modules = (at, at.q_proj, at.k_proj, at.v_proj, at.out_proj, at.qk_bmm, at.pv_bmm, layer.fc1, layer.fc2,
-                        layer.self_attn_layer_norm, layer.final_layer_norm)
+        plan.modules = tuple((holder._modules, name, getattr(holder, name)) for holder, names in (
+            (layer, ("self_attn", "fc1", "fc2", "self_attn_layer_norm", "final_layer_norm")),
+            (at, ("q_proj", "k_proj", "v_proj", "out_proj", "qk_bmm", "pv_bmm"))) for name in names)
         stock = (type(at.q_proj) is W8A8B8O8Linear and type(at.k_proj) is W8A8B8O8Linear
                  and type(at.v_proj) is W8A8B8O8Linear and type(at.out_proj) is W8A8BFP32OFP32Linear
                  and type(layer.fc1) is W8A8B8O8LinearReLU and type(layer.fc2) is W8A8BFP32OFP32Linear
                  and type(at.qk_bmm) is BMM_S8T_S8N_F32T and type(at.pv_bmm) is BMM_S8T_S8N_S8T
                  and type(layer.self_attn_layer_norm) is LayerNormQ and type(layer.final_layer_norm) is LayerNormQ)
+        plan.sources = ()
         if not stock:
             return plan
         E, H, d, F = at.embed_dim, at.num_heads, at.head_dim, layer.fc1.out_features
@@ -385,19 +407,21 @@ class _DecodePlan:
             if not (isinstance(t, torch.Tensor) and t.device == device and t.dtype is dtype and t.is_contiguous()
                     and t.numel() == numel and t.data_ptr() % 16 == 0):
                 raise _NotStock
-            plan.sources.append((holder, name, t, t._version))
+            sources.append((holder, name, t, t._version))
             return t.data_ptr()
 
         def scalar(mod, name):
             value = mod._scalar(name)
             t = mod._buffers.get(name)
             if isinstance(t, torch.Tensor):
-                plan.sources.append((mod._buffers, name, t, t._version))
+                sources.append((mod._buffers, name, t, t._version))
             else:
                 raise _NotStock   # a scale that is not a registered buffer cannot be watched
             return value
 
         try:
+            qkv1 = (at.q_proj, at.k_proj, at.v_proj, layer.fc1)
+            read_scalars([(m, "a") for m in qkv1 + (at.qk_bmm, at.pv_bmm, at.out_proj, layer.fc2)] + [(m, "b") for m in qkv1])
             for lin in (at.out_proj, layer.fc2):   # their fp32 bias may still be in the dtype a cast left (see _run)
                 _, bias = lin._wb()
                 if bias.dtype is not torch.float32:
@@ -421,6 +445,8 @@ class _DecodePlan:
             st.alpha_2 = scalar(layer.fc2, "a")
         except _NotStock:
             return plan
+        finally:
+            plan.sources = tuple(sources)
         if H * d != E or at.q_proj.in_features != E or layer.fc2.in_features != F:
             return plan
         plan.struct, plan.addr = st, ctypes.addressof(st)
@@ -431,6 +457,10 @@ class _DecodePlan:
 
 class _NotStock(Exception):
     pass
+
+
+def _no_plan():
+    return None
 
 
 def _mask_as_fp32(mask):
@@ -490,84 +520,81 @@ class Int8OPTDecoderLayer(nn.Module):
         """The layer as ``ti_opt_decoder_layer_decode`` reads it, built once and rebuilt when a tensor it was built from
         has been replaced or written to; None when the layer is not the stock int8 block on ``device``."""
         plan = self.__dict__.get("_ti_decode_plan")
-        if plan is not None and plan.half == half and plan.device == device:
-            for holder, name, tensor, version in plan.sources:
-                if holder.get(name) is not tensor or tensor._version != version:
-                    plan = None
-                    break
-        else:
-            plan = None
-        if plan is None:
+        if plan is None or plan.half != half or plan.device != device or not _hip_ext.plan_current(plan.sources, plan.modules):
+            if plan is not None and any(m._forward_hooks or m._forward_pre_hooks for _, _, m in plan.modules):
+                return None   # a hook on a sub-module wants to see that module's call
             plan = self.__dict__["_ti_decode_plan"] = _DecodePlan.build(self, half, device)
-        if not plan.ok or _GLOBAL_FORWARD_HOOKS or _GLOBAL_FORWARD_PRE_HOOKS:
-            return None
-        for mod in plan.modules:   # a hook on a sub-module wants to see that module's call
-            if mod._forward_hooks or mod._forward_pre_hooks:
+            if not _hip_ext.plan_current(plan.sources, plan.modules):
                 return None
-        return plan
+        return plan if plan.ok and not _GLOBAL_FORWARD_HOOKS and not _GLOBAL_FORWARD_PRE_HOOKS else None
+
+    def _decode_checks(self, hs, mask, past_key_value):
+        """(plan, positions after this step) when one new token per sequence over this KV cache can be issued from one C
+        call, else None.  ``mask`` fp32 on the device or None."""
+        past_k, past_v = past_key_value
+        shape = past_k.shape
+        if not (len(shape) == 4 and past_v.shape == shape and past_k.dtype is torch.int8 and past_v.dtype is torch.int8
+                and past_k.device == hs.device and past_v.device == hs.device):
+            return None
+        plan = self._decode_plan(hs.dtype is torch.float16, hs.device)
+        bsz, S = hs.shape[0], shape[2] + 1
+        if (plan is None or shape[0] != bsz or shape[1] != plan.heads or shape[3] != plan.head_dim or hs.shape[2] != plan.embed
+                or not _hip_ext.decode_attention_shape_ok_cached(1, S, plan.head_dim)
+                or (mask is not None and mask.shape != (bsz, 1, 1, S))):
+            return None
+        return plan, S
+
+    @staticmethod
+    def _one_call_tensors(hs, attention_mask):
+        """(whether the residual stream and the mask qualify for the C calls, the mask as they read it)."""
+        if not (hs.is_cuda and hs.is_contiguous() and (hs.dtype is torch.float32 or hs.dtype is torch.float16)):
+            return False, None
+        if attention_mask is None:
+            return True, None
+        mask = _mask_as_fp32(attention_mask)
+        return (mask is not None and mask.is_contiguous() and mask.device == hs.device and mask.data_ptr() % 16 == 0), mask
 
     def _decode_in_one_call(self, hidden_states, attention_mask, past_key_value, use_cache):
         """``forward`` for one new token per sequence over a KV cache, or None when the tensors do not qualify."""
-        hs = hidden_states
-        dtype = hs.dtype
-        if not (hs.is_cuda and hs.is_contiguous() and hs.shape[0] <= 64
-                and (dtype is torch.float32 or dtype is torch.float16)):
+        ok, mask = self._one_call_tensors(hidden_states, attention_mask)
+        if not ok or hidden_states.shape[0] > 64:
             return None
-        past_k, past_v = past_key_value
-        bsz = hs.shape[0]
-        if not (past_k.dim() == 4 and past_v.shape == past_k.shape and past_k.dtype is torch.int8
-                and past_v.dtype is torch.int8 and past_k.device == hs.device and past_v.device == hs.device
-                and past_k.shape[0] == bsz):
+        found = self._decode_checks(hidden_states, mask, past_key_value)
+        rooms = found and _kv_rooms(past_key_value)
+        if not rooms:
             return None
-        plan = self._decode_plan(dtype is torch.float16, hs.device)
-        if plan is None or past_k.shape[1] != plan.heads or past_k.shape[3] != plan.head_dim or hs.shape[2] != plan.embed:
-            return None
-        S = past_k.shape[2] + 1
-        if not _hip_ext.decode_attention_shape_ok_cached(1, S, plan.head_dim):
-            return None
-        mask = attention_mask
-        if mask is not None:
-            mask = _mask_as_fp32(mask)
-            if not (mask is not None and mask.is_contiguous() and mask.shape == (bsz, 1, 1, S) and mask.device == hs.device):
-                return None
-        kk = _kv_room_for(past_k, 1) or _kv_fresh(past_k, 1)
-        vv = _kv_room_for(past_v, 1) or _kv_fresh(past_v, 1)
-        if kk.buf.data_ptr() % 16 or vv.buf.data_ptr() % 16 or not (kk.buf.is_contiguous() and vv.buf.is_contiguous()
-                                                                    and kk.buf.shape == vv.buf.shape):
-            return None
-        _hip_ext.opt_layer_decode(plan, hs, mask, kk.buf, vv.buf, S)
+        (plan, S), (kk, vv) = found, rooms
+        _hip_ext.opt_layer_decode(plan, hidden_states, mask, kk.buf, vv.buf, S)
         kk.filled = vv.filled = S
         if use_cache:
-            return hs, (_kv_view(kk, S), _kv_view(vv, S))
-        return (hs,)
+            return hidden_states, (_kv_view(kk, S), _kv_view(vv, S))
+        return (hidden_states,)
 
-    #: a prefill of up to 4096 tokens in all (more than 16 per sequence, a multiple of 16): likewise one C call
-    #: (``ti_opt_decoder_layer_prefill``); at those sizes a layer's kernels take less time than eight trips through Python
+    #: a prefill (more than 16 tokens per sequence, a multiple of 16) likewise: up to 4096 tokens a layer's kernels take less
+    #: time than eight trips through Python (``ti_opt_decoder_layer_prefill``); as part of a model, any number of tokens
     prefill_in_one_call = True
+
+    def _prefill_checks(self, hs, mask):
+        """The plan when a prefill without a cache can be issued from one C call, else None."""
+        bsz, T = hs.shape[0], hs.shape[1]
+        if T % 16 or bsz == 0 or (mask is not None and mask.shape != (bsz, 1, T, T)):
+            return None
+        plan = self._decode_plan(hs.dtype is torch.float16, hs.device)
+        if plan is None or hs.shape[2] != plan.embed or not _hip_ext.attn_prefill_shape_ok_cached(T, T, plan.head_dim):
+            return None
+        return plan
 
     def _prefill_in_one_call(self, hidden_states, attention_mask, use_cache):
         """``forward`` without a cache on T > 16 tokens per sequence, or None when the tensors do not qualify."""
-        hs = hidden_states
-        dtype = hs.dtype
-        bsz, T = hs.shape[0], hs.shape[1]
-        if not (hs.is_cuda and hs.is_contiguous() and T % 16 == 0 and 0 < bsz * T <= 4096
-                and (dtype is torch.float32 or dtype is torch.float16)):
+        ok, mask = self._one_call_tensors(hidden_states, attention_mask)
+        plan = self._prefill_checks(hidden_states, mask) if ok and hidden_states.shape[0] * hidden_states.shape[1] <= 4096 else None
+        if plan is None:
             return None
-        plan = self._decode_plan(dtype is torch.float16, hs.device)
-        if plan is None or hs.shape[2] != plan.embed or not _hip_ext.attn_prefill_shape_ok_cached(T, T, plan.head_dim):
-            return None
-        mask = attention_mask
-        if mask is not None:
-            mask = _mask_as_fp32(mask)
-            if not (mask is not None and mask.is_contiguous() and mask.shape == (bsz, 1, T, T) and mask.device == hs.device
-                    and mask.data_ptr() % 16 == 0):
-                return None
-        key = torch.empty((bsz, plan.heads, T, plan.head_dim), dtype=torch.int8, device=hs.device)
-        value = torch.empty((bsz, plan.heads, T, plan.head_dim), dtype=torch.int8, device=hs.device)
-        _hip_ext.opt_layer_prefill(plan, hs, mask, key, value)
+        key, value = plan.new_cache(hidden_states)
+        _hip_ext.opt_layer_prefill(plan, hidden_states, mask, key, value)
         if use_cache:
-            return hs, (key, value)
-        return (hs,)
+            return hidden_states, (key, value)
+        return (hidden_states,)
 
     def decode_step_devlen(self, hidden_states, k_buf, v_buf, length, max_length):
         """``forward`` for one new token per sequence with the cache length read on the device (see
@@ -730,6 +757,54 @@ class Int8OPTDecoder(nn.Module):
             q.layers[i] = Int8OPTDecoderLayer.from_float(layer, **decoder_layer_scales[i])
         return q
 
+    def _chain_layers(self, hidden, attention_mask, past_key_values, use_cache):
+        """The loop over the layers with one C call per layer and the last addition of a layer left to the next one's first
+        kernel (``chain`` in ``_hip_ext.opt_layer_decode``): updates ``hidden`` in place and returns the cache, or None
+        when a layer, its hooks or the tensors want the ordinary calls.  Values of the loop over ``layer(hidden, ...)``."""
+        layers = list(self.layers)
+        count, decode = len(layers), bool(past_key_values)
+        if count == 0 or (hidden.shape[1] != 1 or hidden.shape[0] > 64 if decode else hidden.shape[1] <= 16):
+            return None
+        ok, mask = Int8OPTDecoderLayer._one_call_tensors(hidden, attention_mask)
+        if not ok or (decode and len(past_key_values) != count):
+            return None
+        found = []
+        for i, layer in enumerate(layers):
+            if (type(layer) is not Int8OPTDecoderLayer or layer._forward_hooks or layer._forward_pre_hooks
+                    or "forward" in layer.__dict__):
+                return None
+            attn = layer.self_attn
+            if not (type(attn) is Int8OPTAttention and attn.fused_softmax and (attn.kv_cache_in_place or not decode)
+                    and (layer.decode_in_one_call if decode else layer.prefill_in_one_call)):
+                return None
+            hit = layer._decode_checks(hidden, mask, past_key_values[i]) if decode else layer._prefill_checks(hidden, mask)
+            if hit is None:
+                return None
+            found.append(hit)
+        # fc2's output on its way from one layer to the next; memory of this pass, so that passes of other threads on the same
+        # stream do not meet in it
+        carry = torch.empty((hidden.shape[0] * hidden.shape[1], hidden.shape[2]), dtype=torch.float32, device=hidden.device)
+        cache = []
+        if decode:
+            rooms = [_kv_rooms(past) for past in past_key_values]
+            if not all(rooms):
+                return None
+            for i, ((plan, S), (kk, vv)) in enumerate(zip(found, rooms)):
+                chain = (_hip_ext.CHAIN_ADD if i else 0) | (_hip_ext.CHAIN_LEAVE if i + 1 < count else 0)
+                _hip_ext.opt_layer_decode(plan, hidden, mask, kk.buf, vv.buf, S, chain=chain, carry=carry)
+                kk.filled = vv.filled = S
+                if use_cache:
+                    cache.append((_kv_view(kk, S), _kv_view(vv, S)))
+        else:
+            memory = _hip_ext.opt_prefill_scratch(found[0], hidden)
+            for i, plan in enumerate(found):
+                chain = (_hip_ext.CHAIN_ADD if i else 0) | (_hip_ext.CHAIN_LEAVE if i + 1 < count else 0)
+                key, value = plan.new_cache(hidden)
+                _hip_ext.opt_layer_prefill(plan, hidden, mask, key, value, chain=chain, carry=carry, memory=memory)
+                if use_cache:
+                    cache.append((key, value))
+        return tuple(cache)
+
     @torch.no_grad()
     def forward(self, input_ids: torch.LongTensor = None, attention_mask: Optional[torch.Tensor] = None,
                 head_mask: Optional[torch.Tensor] = None,
@@ -765,7 +840,12 @@ class Int8OPTDecoder(nn.Module):
         all_hidden = () if output_hidden_states else None
         all_attn = () if output_attentions else None
         cache = () if use_cache else None
-        for i, layer in enumerate(self.layers):
+        chained = None
+        if head_mask is None and not output_attentions and not output_hidden_states:
+            chained = self._chain_layers(hidden, mask, past_key_values, use_cache)
+        if chained is not None:
+            cache = chained if use_cache else None
+        for i, layer in enumerate(self.layers if chained is None else ()):
             if output_hidden_states:
                 all_hidden += (hidden.clone(),)
             out = layer(hidden, attention_mask=mask,
