@@ -1,11 +1,12 @@
-// Attention for incremental decoding in one launch: per (batch, head) one workgroup appends the new
+// Attention for incremental decoding in one launch (two kernels: one for a single new token, decode_attn_one_kernel, and
+// one for up to four): per (batch, head) one workgroup appends the new
 // key / value rows to the KV cache, computes alpha_qk * Q.K^T over the whole cache, turns the scores into
 // int8 probabilities (mask, clamp, softmax, *127, round: the arithmetic and the summation order of
 // attn_softmax_q) and multiplies them with V as the cache stores it ([len, head_dim] rows).  It replaces
 // the append, skinny Q.K^T, softmax and row-major P.V launches of a decode step; the scores and the
 // probabilities stay in LDS.  HBM-bound on the 2 * len * head_dim bytes of cache per (batch, head).
 //
-// 256 threads.  A cache row is read by head_dim/16 adjacent lanes (16 bytes each), so one load
+// A cache row is read by head_dim/16 adjacent lanes (16 bytes each), so one load
 // instruction of a wave covers 64*16/head_dim whole rows; partial dot products meet through lane
 // shuffles (integers: any order gives the same bits).
 #include "ti_common.h"
@@ -32,12 +33,219 @@ __device__ __forceinline__ int row_sum(int a) {
   return a;
 }
 
+// This wave's LDS traffic is done, then the workgroup's barrier; loads of the cache stay in flight across it.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// One new token (T == 1): the whole cache of the (batch, head) is in flight at once.  NW waves, at most NI row groups
+// each; row s of the cache is row slot s % RPW of wave (s / RPW) % NW, group s / (RPW * NW).
+//
+// Bound by HBM for a batch of users, by the chain load - maximum - sum - product - sum for a single one, and laid out for
+// both: all key loads are issued up front and all value loads before the softmax, which covers their latency;
+// a lane keeps "its" scores (group u belongs to lane u % LPR of the row) in registers from the product to the
+// exponential, so the maximum and the exponentials need no pass over the LDS; probabilities become the bytes of a
+// v_dot4 operand and four value rows are transposed in registers (8 v_perm_b32 for 16 bytes of four rows), 12
+// instructions for 16 products instead of 32; the row slots of a wave meet through v_permlane swaps, which halve the
+// values left at every step.
+// Measured, cold caches, us (before: decode_attn_kernel): head size 128, heads x positions, 40 x 508 10.7 -> 5.6, 32 x 108
+// 7.8 -> 3.8, 128 x 904 21.5 -> 10.3, 768 x 250 20.0 -> 10.9, 768 x 904 36.5 -> 32.1 (5.5 TB/s), 128 x 2000 40.4 -> 18.3; head size
+// 64, 12 x 108 7.7 -> 3.6, 576 x 500 20.0 -> 10.8.
+// LDS: exponentials [Sp], maxima [NW], scale, probabilities as bytes [NW][RPW][NIP], partial outputs [NW][D].
+template <int D, int NW, int NI, bool PART>
+__global__ __launch_bounds__(NW * 64, 4) void decode_attn_one_kernel(
+    const int8_t* __restrict__ q, const int8_t* __restrict__ k_new, const int8_t* __restrict__ v_new, int8_t* k_buf,
+    int8_t* v_buf, const float* __restrict__ mask, int8_t* __restrict__ ctx, int8_t* __restrict__ probs_out, int S_arg,
+    long long cap, int heads, float alpha_qk, float alpha_pv, const int* __restrict__ s_dev, int dr_arg) {
+  constexpr int LPR = D / 16;                // lanes per cache row
+  constexpr int RPW = 64 / LPR;              // rows per wave per load
+  constexpr int STEP = NW * RPW;             // rows per group
+  constexpr int NJ = (NI + LPR - 1) / LPR;   // scores a lane keeps
+  constexpr int NIP = (NI + 3) / 4 * 4;
+  __shared__ __attribute__((aligned(16))) float ex[NI * STEP];
+  __shared__ __attribute__((aligned(16))) float wmax[NW];
+  __shared__ float scale_of_row;
+  __shared__ __attribute__((aligned(16))) int8_t pb[NW * RPW * NIP];
+  __shared__ __attribute__((aligned(16))) int red[NW * D];
+
+  const int dr = PART ? dr_arg : D;
+  int S = S_arg;
+  if (s_dev != nullptr) {  // clamped to the contract, as below
+    S = s_dev[0];
+    S = S < 1 ? 1 : S;
+    S = S > S_arg ? S_arg : S;
+  }
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rs = lane / LPR, cs = lane % LPR;
+  const bool in_row = !PART || cs * 16 < dr;
+  const long long bh = blockIdx.x;
+  const bool grow = k_new != nullptr;         // the last row comes from k_new / v_new and goes into the cache
+  const int S_old = grow ? S - 1 : S;
+  int8_t* kb = k_buf + bh * cap * dr;
+  int8_t* vb = v_buf + bh * cap * dr;
+  const v4i zero = {0, 0, 0, 0};
+  const int col = in_row ? cs * 16 : 0;
+
+  const v4i qr = in_row ? *reinterpret_cast<const v4i*>(q + bh * dr + col) : zero;
+  v4i fresh_k = zero, fresh_v = zero;
+  if (grow) {
+    fresh_k = *reinterpret_cast<const v4i*>(k_new + bh * dr + col);
+    fresh_v = *reinterpret_cast<const v4i*>(v_new + bh * dr + col);
+  }
+  // Rows past the end re-read the last cached row (row 0 of an empty cache); groups past the end are not loaded.
+  const int base = wave * RPW;
+  const int last = S_old > 0 ? S_old - 1 : 0;
+  auto load_rows = [&](v4i (&dst)[NI], const int8_t* buf) {
+#pragma unroll
+    for (int u = 0; u < NI; ++u) {
+      dst[u] = zero;
+      if (base + u * STEP < S) {  // the same for every lane of the wave
+        int s = base + u * STEP + rs;
+        s = s < last ? s : last;
+        dst[u] = *reinterpret_cast<const v4i*>(buf + (unsigned)(s * dr + col));
+      }
+    }
+  };
+  v4i kv[NI], vv[NI];
+  load_rows(kv, kb);
+  // the additive mask of the scores this lane keeps, fetched together with the cache rows
+  float mk[NJ];
+  const float* msk = mask != nullptr ? mask + (bh / heads) * (long long)S : nullptr;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int u = j * LPR + cs, s = base + u * STEP + rs;
+    mk[j] = msk != nullptr && u < NI && s < S ? msk[s] : 0.0f;
+  }
+
+  // ---- scores: max(alpha_qk * (q . k) + mask, most negative finite float)
+  const float lowest = -3.402823466e+38f;
+  int own[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) own[j] = 0;
+#pragma unroll
+  for (int u = 0; u < NI; ++u) {
+    if (base + u * STEP >= S) break;  // the same for every lane of the wave
+    if (base + u * STEP <= S_old && S_old < base + u * STEP + RPW && rs == S_old - base - u * STEP) kv[u] = fresh_k;
+    const int a = row_sum<LPR>(in_row ? dot16(kv[u], qr, 0) : 0);
+    if (cs == u % LPR) own[u / LPR] = a;
+  }
+  load_rows(vv, vb);  // on their way during the softmax; together with the keys they only cost registers
+  float x[NJ], m = lowest;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int u = j * LPR + cs, s = base + u * STEP + rs;
+    float y = Epi<EPI_F32_SCALE>::apply(own[j], 0.0f, alpha_qk);
+    if (msk != nullptr) y = y + mk[j];
+    x[j] = u < NI && s < S && y > lowest ? y : lowest;
+    m = m > x[j] ? m : x[j];
+  }
+  m = wave_max(m);
+  if (lane == 0) wmax[wave] = m;
+  lds_barrier();
+#pragma unroll
+  for (int w = 0; w < NW; ++w) m = m > wmax[w] ? m : wmax[w];
+
+  // ---- exponentials; positions S .. the next multiple of 4 hold zeros, which change no sum
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int u = j * LPR + cs, s = base + u * STEP + rs;
+    x[j] = exp_nonpos(x[j] - m);
+    if (u < NI) ex[s] = s < S ? x[j] : 0.0f;
+  }
+  lds_barrier();
+  // ---- the sum, by one wave in the order of attn_softmax_q (chunk c of four elements belongs to lane c % 64, a lane
+  // adds its elements in ascending order, lanes combine with a xor butterfly 32..1)
+  if (wave == 0) {
+    const int nchunks = (S + 3) >> 2;
+    float sum = 0.0f;
+    for (int c = lane; c < nchunks; c += 64) {
+      const v4f e4 = reinterpret_cast<const v4f*>(ex)[c];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sum = sum + e4[j];
+    }
+    sum = wave_sum(sum);
+    if (lane == 0) scale_of_row = 127.0f / sum;
+  }
+  lds_barrier();
+  const float scale = scale_of_row;
+  // ---- probabilities: a byte per position, to the lanes of the same row of the same wave (no barrier)
+  int8_t* my_pb = pb + (wave * RPW + rs) * NIP;
+#pragma unroll
+  for (int j = 0; j < (NIP + LPR - 1) / LPR; ++j) {
+    const int u = j * LPR + cs, s = base + u * STEP + rs;
+    const bool live = j < NJ && u < NI && s < S;
+    const int8_t pq = live ? (int8_t)(int)__builtin_rintf(x[j < NJ ? j : 0] * scale) : (int8_t)0;
+    if (u < NIP) my_pb[u] = pq;
+    if (live && probs_out != nullptr) probs_out[bh * (long long)S + s] = pq;
+  }
+  __builtin_amdgcn_wave_barrier();
+
+  // ---- ctx[n] = s8(alpha_pv * sum_s p[s] * v[s][n]); the lane owns columns cs*16 .. +15
+  int acc[16];
+#pragma unroll
+  for (int c = 0; c < 16; ++c) acc[c] = 0;
+#pragma unroll
+  for (int u0 = 0; u0 < NI; u0 += 4) {
+    if (base + u0 * STEP >= S) break;  // the same for every lane of the wave
+    const int p4 = *reinterpret_cast<const int*>(my_pb + u0);
+    v4i r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int u = u0 + i;
+      r[i] = u < NI ? vv[u < NI ? u : 0] : zero;
+      if (u < NI && base + u * STEP <= S_old && S_old < base + u * STEP + RPW && rs == S_old - base - u * STEP)
+        r[i] = fresh_v;
+    }
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const unsigned r0 = r[0][w], r1 = r[1][w], r2 = r[2][w], r3 = r[3][w];
+      const unsigned a = __builtin_amdgcn_perm(r1, r0, 0x05010400), b = __builtin_amdgcn_perm(r3, r2, 0x05010400);
+      const unsigned c = __builtin_amdgcn_perm(r1, r0, 0x07030602), d = __builtin_amdgcn_perm(r3, r2, 0x07030602);
+      acc[4 * w + 0] = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_perm(b, a, 0x05040100), p4, acc[4 * w + 0], false);
+      acc[4 * w + 1] = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_perm(b, a, 0x07060302), p4, acc[4 * w + 1], false);
+      acc[4 * w + 2] = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_perm(d, c, 0x05040100), p4, acc[4 * w + 2], false);
+      acc[4 * w + 3] = __builtin_amdgcn_sdot4((int)__builtin_amdgcn_perm(d, c, 0x07060302), p4, acc[4 * w + 3], false);
+    }
+  }
+  // The row slots of a wave: the upper half of the lanes takes columns 8..15, the odd rows of 16 lanes 4..7 and 12..15,
+  // then the lanes of a row of 16 that hold the same columns.
+  int h8[8], h4[4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const auto s = __builtin_amdgcn_permlane32_swap((unsigned)acc[i], (unsigned)acc[i + 8], false, false);
+    h8[i] = (int)(s[0] + s[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const auto s = __builtin_amdgcn_permlane16_swap((unsigned)h8[i], (unsigned)h8[i + 4], false, false);
+    h4[i] = (int)(s[0] + s[1]);
+    h4[i] += __builtin_amdgcn_mov_dpp(h4[i], 0x128, 0xf, 0xf, true);                 // row_ror:8
+    if (LPR == 4) h4[i] += __builtin_amdgcn_mov_dpp(h4[i], 0x124, 0xf, 0xf, true);   // row_ror:4
+  }
+  if ((lane & 15) < LPR) {
+    const int c0 = cs * 16 + ((lane >> 4) & 1) * 4 + (lane >> 5) * 8;
+    *reinterpret_cast<v4i*>(red + wave * D + c0) = v4i{h4[0], h4[1], h4[2], h4[3]};
+  }
+  lds_barrier();
+  if (tid < dr) {
+    int sum = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) sum += red[w * D + tid];
+    ctx[bh * dr + tid] = Epi<EPI_S8_SCALE>::apply(sum, 0.0f, alpha_pv);
+  }
+  // the new row goes into the cache last: no load of this launch reads it from there
+  if (grow && rs == 0 && in_row) {
+    if (wave == NW - 1) *reinterpret_cast<v4i*>(kb + (long long)S_old * dr + col) = fresh_k;
+    if (wave == NW - 2) *reinterpret_cast<v4i*>(vb + (long long)S_old * dr + col) = fresh_v;
+  }
+}
+
 // Bytes of dynamic LDS: fp32 scores [T][Sp], int8 probabilities [T][Sp], partial outputs [4][T][D].
 __host__ __device__ inline long long decode_attn_lds(long long T, long long S, long long D) {
   const long long Sp = (S + 3) / 4 * 4;
   return T * Sp * 4 + T * Sp + 4 * T * D * 4;
 }
 
+// 256 threads.  For two to four new tokens, and for one where decode_attn_one_kernel does not apply.
 // NI > 0: the whole cache of the (batch, head) is at most NI row groups per lane and all of its loads are
 // issued up front (keys and values, 16 bytes each per lane), so the kernel waits for memory once.
 // NI == 0: any length, four row groups in flight at a time.
@@ -277,8 +485,35 @@ int launch_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_
   const dim3 grid((unsigned)BH), block(256);
   const int lanes_d = D <= 64 ? 64 : 128;  // the kernel variant: bytes of a cache row that its lanes cover
   const size_t lds = (size_t)decode_attn_lds(T, S, lanes_d);
-  // caches of at most 20 row groups per lane (640 positions at head size 128) with one or two query rows take
-  // the variant that issues all loads up front
+  // One new token: the form with the fewest waves and groups that hold the cache (rows groups of 8 rows at head size 128, 16 at
+  // 64), us, head size 128, cold: 250 positions, 768 heads: 4 waves x 8 groups 10.9, 8 x 8 11.3, 16 x 8 16.2; 500 positions,
+  // 40 heads: 8 x 8 5.6, 16 x 8 5.8.  Between 96 and 128 groups sixteen waves are ahead while every workgroup has a CU to
+  // itself (904 positions: 32 heads 7.3 against 8.0, 128 heads 10.2 / 10.4, 768 heads 38.0 / 32.1).  Beyond 128 groups only one
+  // workgroup fits a CU, which leaves it without loads during the softmax: with more heads than two rounds of 256 the
+  // streaming form, several small workgroups per CU, is level or ahead (1400 positions, 768 heads: 51.7 against 52.5; 128
+  // heads 29.1 / 13.8).
+  const long long groups = (S + 64 / (lanes_d / 16) - 1) / (64 / (lanes_d / 16));
+#define TI_DA1(DD, NW, NI)                                                                                             \
+  do {                                                                                                                 \
+    if (D == DD)                                                                                                       \
+      hipLaunchKernelGGL((decode_attn_one_kernel<DD, NW, NI, false>), grid, dim3(NW * 64), 0, stream, q, k_new, v_new, \
+                         k_buf, v_buf, mask, ctx, probs_out, (int)S, cap, (int)heads, alpha_qk, alpha_pv, s_dev, (int)D); \
+    else                                                                                                               \
+      hipLaunchKernelGGL((decode_attn_one_kernel<DD, NW, NI, true>), grid, dim3(NW * 64), 0, stream, q, k_new, v_new,  \
+                         k_buf, v_buf, mask, ctx, probs_out, (int)S, cap, (int)heads, alpha_qk, alpha_pv, s_dev, (int)D); \
+  } while (0)
+#define TI_DA1_FORMS(DD)                                            \
+  do {                                                              \
+    if (groups <= 8) TI_DA1(DD, 4, 2);                              \
+    else if (groups <= 16) TI_DA1(DD, 4, 4);                        \
+    else if (groups <= 32) TI_DA1(DD, 4, 8);                        \
+    else if (groups <= 64) TI_DA1(DD, 8, 8);                        \
+    else if (groups <= 96) TI_DA1(DD, 8, 12);                       \
+    else if (groups <= 128 && BH > 256) TI_DA1(DD, 8, 16);          \
+    else if (groups <= 128) TI_DA1(DD, 16, 8);                      \
+    else if (groups <= 192) TI_DA1(DD, 16, 12);                     \
+    else TI_DA1(DD, 16, 16);                                        \
+  } while (0)
 #define TI_DA(TQ, DD, NI)                                                                                              \
   do {                                                                                                                 \
     if (D == DD)                                                                                                       \
@@ -288,16 +523,23 @@ int launch_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_
       hipLaunchKernelGGL((decode_attn_kernel<TQ, DD, NI, true>), grid, block, lds, stream, q, k_new, v_new, k_buf,     \
                          v_buf, mask, ctx, probs_out, (int)T, (int)S, cap, (int)heads, alpha_qk, alpha_pv, s_dev, (int)D); \
   } while (0)
-  const bool resident = T <= 2 && S <= 20 * 4 * (64 / (lanes_d / 16));
+  const bool one = T == 1 && (groups <= 128 || (groups <= 256 && BH <= 512));
+  // caches of at most 20 row groups per lane (640 positions at head size 128) with two query rows take
+  // the variant that issues all loads up front
+  const bool resident = T == 2 && S <= 20 * 4 * (64 / (lanes_d / 16));
   if (lanes_d == 128) {
-    if (T == 1) { if (resident) TI_DA(1, 128, 20); else TI_DA(1, 128, 0); }
+    if (one) TI_DA1_FORMS(128);
+    else if (T == 1) TI_DA(1, 128, 0);
     else if (T == 2) { if (resident) TI_DA(2, 128, 20); else TI_DA(2, 128, 0); }
     else TI_DA(4, 128, 0);
   } else {
-    if (T == 1) { if (resident) TI_DA(1, 64, 20); else TI_DA(1, 64, 0); }
+    if (one) TI_DA1_FORMS(64);
+    else if (T == 1) TI_DA(1, 64, 0);
     else if (T == 2) { if (resident) TI_DA(2, 64, 20); else TI_DA(2, 64, 0); }
     else TI_DA(4, 64, 0);
   }
+#undef TI_DA1_FORMS
+#undef TI_DA1
 #undef TI_DA
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "decode_attn launch: %s", hipGetErrorString(e));
