@@ -57,3 +57,21 @@ def test_chained_layers_give_the_modules_values(bsz, T, layers, pad, half):
         assert torch.equal(a.logits, b.logits) and torch.equal(h.logits, b.logits)
         for (ka, va), (kb, vb) in zip(a.past_key_values, b.past_key_values):
             assert torch.equal(ka, kb) and torch.equal(va, vb)
+
+
+@torch.no_grad()
+def test_layers_handed_one_cache_keep_their_own_rows():
+    g = torch.Generator().manual_seed(1)
+    lm = Int8OPTForCausalLM(OPTConfigLite(hidden_size=128, num_hidden_layers=3, ffn_dim=512, num_attention_heads=2, vocab_size=64,
+                                          max_position_embeddings=64))
+    for layer in lm.model.decoder.layers:
+        randomize_int8_layer(layer, g)
+    lm = lm.to(DEV)
+    ids = torch.randint(2, 64, (2, 21), generator=g).to(DEV)
+    # the cache of a decode step has room behind it, and all layers would append there
+    first = lm(ids[:, 19:20], past_key_values=lm(ids[:, :19], use_cache=True).past_key_values, use_cache=True).past_key_values[0]
+    out = lm(ids[:, 20:], past_key_values=[first] * 3, use_cache=True)
+    alone = lm(ids[:, 20:], past_key_values=[tuple(t.clone() for t in first) for _ in range(3)], use_cache=True)
+    assert torch.equal(out.logits, alone.logits)
+    for kept, want in zip(out.past_key_values, alone.past_key_values):
+        assert all(torch.equal(a, b) for a, b in zip(kept, want))
