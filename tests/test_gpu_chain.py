@@ -75,3 +75,10 @@ def test_layers_handed_one_cache_keep_their_own_rows():
     assert torch.equal(out.logits, alone.logits)
     for kept, want in zip(out.past_key_values, alone.past_key_values):
         assert all(torch.equal(a, b) for a, b in zip(kept, want))
+
+
+@pytest.mark.parametrize("bsz,T,taken", [(64, 16, True), (65536, 16, False), (1025, 1024, False)])
+def test_prefills_beyond_what_the_c_call_takes_go_to_the_modules(bsz, T, taken):
+    layer = randomize_int8_layer(Int8OPTDecoderLayer(128, 2, 512), torch.Generator().manual_seed(2)).to(DEV)
+    hidden = torch.empty((1, 1, 128), device=DEV).expand(bsz, T, 128)
+    assert (layer._prefill_checks(hidden, None) is not None) == taken

@@ -577,7 +577,7 @@ class Int8OPTDecoderLayer(nn.Module):
     def _prefill_checks(self, hs, mask):
         """The plan when a prefill without a cache can be issued from one C call, else None."""
         bsz, T = hs.shape[0], hs.shape[1]
-        if T % 16 or bsz == 0 or (mask is not None and mask.shape != (bsz, 1, T, T)):
+        if T % 16 or bsz == 0 or bsz > 65535 or bsz * T > 1 << 20 or (mask is not None and mask.shape != (bsz, 1, T, T)):
             return None
         plan = self._decode_plan(hs.dtype is torch.float16, hs.device)
         if plan is None or hs.shape[2] != plan.embed or not _hip_ext.attn_prefill_shape_ok_cached(T, T, plan.head_dim):
