@@ -111,3 +111,21 @@ def test_decode_step_of_a_large_batch_from_one_call(D, H, bsz, half):
         assert torch.equal(res[True][0], res[False][0])
         for a, b in zip(caches[True], caches[False]):
             assert torch.equal(a, b)
+
+
+def test_a_group_too_wide_for_its_bias_in_the_lds():
+    """The biases of a workgroup's strips (64 bytes each) lie beside the weight rings, which leave 24 to 30 KiB where a workgroup
+    has a CU to itself: the widest groups of four go problem by problem."""
+    import torch_int._hip_ext as X
+    M, N, K = 2, 524272, 4096
+    g = torch.Generator(device=DEV).manual_seed(5)
+    x = torch.randint(-127, 128, (M, K), dtype=torch.int8, device=DEV, generator=g)
+    w = torch.randint(-127, 128, (N, K), dtype=torch.int8, device=DEV, generator=g)
+    bs = [torch.randint(-127, 128, (N,), dtype=torch.int8, device=DEV, generator=g) for _ in range(4)]
+    al, be = [3e-4, 2e-4, 5e-4, 1e-4], [0.02, 0.1, 0.05, 0.3]
+    print("rows wide group", M, N, K, flush=True)
+    out = X.linear_a8_w8_b8_o8_group(x, [w] * 4, bs, al, be)
+    some = torch.cat([torch.arange(2048), torch.arange(N - 2048, N)]).to(DEV)
+    for o, b, a, c in zip(out, bs, al, be):
+        want = orc.linear_a8_w8_b8_o8(x.cpu(), w[some].cpu(), b[some].cpu(), a, c, acc_fn=orc.gemm_acc_torch)
+        assert torch.equal(o[:, some].cpu(), want)

@@ -440,6 +440,7 @@ static int launch_rows_cfg(const GemmParams& p, const GemmGroup& grp, int strips
   const int grid = need < slots ? (int)need : slots;
   const int groups = grid / 8 / p.splits * 8;
   const int lds = Cfg::LDS_BYTES + ((strips + groups - 1) / groups + 3) / 4 * 256;
+  if (lds > 160 * 1024) return -1;  // so wide an output that the bias of a workgroup's strips leaves the ring no room
   static std::atomic<unsigned long long> lds_ok{0};
   if (int rc = allow_lds(gemm_rows_kernel<Cfg>, 160 * 1024, lds_ok)) return rc;
   hipLaunchKernelGGL(gemm_rows_kernel<Cfg>, dim3((unsigned)grid), dim3(Cfg::NT), lds, stream, p, grp, strips, per_problem);
