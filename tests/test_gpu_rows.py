@@ -129,3 +129,10 @@ def test_a_group_too_wide_for_its_bias_in_the_lds():
     for o, b, a, c in zip(out, bs, al, be):
         want = orc.linear_a8_w8_b8_o8(x.cpu(), w[some].cpu(), b[some].cpu(), a, c, acc_fn=orc.gemm_acc_torch)
         assert torch.equal(o[:, some].cpu(), want)
+
+
+@pytest.mark.parametrize("N,K,sliced", [(1000, 2560, True), (1008, 2560, False), (1000, 2048, False)])
+def test_workspace_is_that_of_the_kernel_that_runs(N, K, sliced):
+    """Widths that 16 does not divide go to the tiled kernels where 1024 does not divide the inner dimension, which slice it."""
+    import torch_int._CUDA as C
+    assert (C._lib.ti_linear_workspace_bytes(48, N, K) > 0) == sliced

@@ -18,7 +18,7 @@ long long gemm_workspace_bytes(long long M, long long N, long long K) {
     return head > need ? head : need;
   }
   const RowsPick rows = rows_pick(M, N, K);
-  if (M > 16 && rows.tiling != ROWS_NONE) return rows.slices > 1 ? (long long)rows.slices * M * N * 4 : 0;
+  if (M > 16 && rows.tiling != ROWS_NONE && (N % 16 == 0 || K % SBK == 0)) return rows.slices > 1 ? (long long)rows.slices * M * N * 4 : 0;
   const int s = choose_splits(M, N, K);
   return s > 1 ? (long long)s * M * N * 4 : 0;
 }
