@@ -2272,8 +2272,14 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmParams p, const 
 // 128x5120x5120: 19.6 -> 16.4 us), although a workgroup of this shape multiplies at half the rate of a 256x160 one
 // (its four waves read 7 fragments from the LDS per 10 MFMAs); with K = 20480 the larger tiles win
 // (512x5120x20480: 79 against 64 us).  More than three LDS stages did not help it (four to six: +1 to +3 %).
+//
+// 160x160 tiles (four waves of 80x80, 10 fragment reads per 25 MFMAs; raw-int32 slices only) for the row counts that they
+// cover with fewer padded rows than 128-row tiles do: 129 to 160, 257 to 320, 385 to 480, 769 to 800.  257 rows on three
+// 128-row tiles multiply half as much padding as rows.  Bound by the matrix pipe and by the partial tiles' way through the
+// last-level cache, cold weights, us: 257x5120x20480 57.3 -> 48.7, 300x5120x20480 59.1 -> 54.8, 320x5120x20480 60.3 -> 58.8.  Priced
+// at 0.36 us per 64-byte step they are not taken at 5120x5120 or 20480x5120, where few rows of tiles fill the chip anyway.
 enum SplitTile { SPLIT_128 = 0, SPLIT_256 = 1, SPLIT_256x160 = 2, SPLIT_256x288 = 3, SPLIT_128x160 = 4, SPLIT_128x288 = 5,
-                 SPLIT_128x80 = 6, SPLIT_128x192 = 7, SPLIT_256x192 = 8 };
+                 SPLIT_128x80 = 6, SPLIT_128x192 = 7, SPLIT_256x192 = 8, SPLIT_160x160 = 9 };
 // `batch` > 1: a batched product (A and B per batch); every tile count, byte count and the streaming floor scale with
 // it, the one-launch form is not available, and the tile shapes are those that exist for every epilogue of the
 // raw-int32 kernels.
@@ -2294,24 +2300,26 @@ static int choose_splits(long long M, long long N, long long K, int* tile_kind =
   // (256x192 tiles, unsplit only: 256 x 49152 or 1024 x 12288 outputs are exactly 256 of them.  Their two LDS stages
   // leave weights that come from HBM one step of cover, and the split forms lost to the 128x192 tiles: 512 x 12288 x
   // 49152 in two slices 319 against 309 us, 512 x 49152 x 12288 331 against 290 us for 256x128 tiles)
-  const int order[9] = {SPLIT_128x80, SPLIT_128x160, SPLIT_128x192, SPLIT_128x288, SPLIT_128, SPLIT_256, SPLIT_256x160,
-                        SPLIT_256x192, SPLIT_256x288};
-  for (int oi = 0; oi < 9; ++oi) {
+  const int order[10] = {SPLIT_128x80, SPLIT_128x160, SPLIT_160x160, SPLIT_128x192, SPLIT_128x288, SPLIT_128, SPLIT_256,
+                         SPLIT_256x160, SPLIT_256x192, SPLIT_256x288};
+  for (int oi = 0; oi < 10; ++oi) {
     const int kind = order[oi];
     const bool wide192 = kind == SPLIT_128x192;
     const bool tall192 = kind == SPLIT_256x192;
     const bool half = kind == SPLIT_128x160 || kind == SPLIT_128x288;  // 128-row forms of the two tall tiles
     const bool small = kind == SPLIT_128x80;
-    const int bm = kind == SPLIT_128 || half || small || wide192 ? 128 : 256;
+    const bool square = kind == SPLIT_160x160;
+    const int bm = square ? 160 : kind == SPLIT_128 || half || small || wide192 ? 128 : 256;
     const int bn = small ? 80 : wide192 || tall192 ? 192 : kind == SPLIT_128 ? 128 : kind == SPLIT_256 ? 256
                    : kind == SPLIT_256x288 || kind == SPLIT_128x288 ? 288 : 160;
     if (kind >= SPLIT_256x160 && N % bn != 0) continue;
+    if (square && (batch > 1 || (M + 159) / 160 * 160 >= (M + 127) / 128 * 128)) continue;  // only where it saves rows
     if ((wide192 || tall192) && (N % 160 == 0 || N % 288 == 0)) continue;  // those widths keep their tuned tiles
     const double tiles = (double)((M + bm - 1) / bm) * (double)((N + bn - 1) / bn) * (double)batch;
     for (int s = 1; s <= 16; ++s) {
       if (steps % s != 0 || steps / s < 4) continue;
       if (kind >= SPLIT_256x160 && (K / s) % QBK != 0) continue;  // these tiles step 128 bytes at a time
-      if (half && s == 1) continue;                                // exist as raw-int32 kernels only
+      if ((half || square) && s == 1) continue;                    // exist as raw-int32 kernels only
       if (tall192 && s > 1) continue;
       if (batch > 1 && s == 1 && (small || wide192 || tall192)) continue;  // unsplit batched products keep their dispatch
       // an unsplit candidate stands for what the ordinary dispatch would launch, which takes the 256-row tiles only
@@ -2330,14 +2338,14 @@ static int choose_splits(long long M, long long N, long long K, int* tile_kind =
       } else {
         rounds = (double)(long long)((wgs + cus - 1) / cus);
         step_us = kind == SPLIT_256 ? 0.85 : kind == SPLIT_256x160 ? 0.55 : kind == SPLIT_256x288 ? 0.92
-                  : kind == SPLIT_128x160 ? 0.375 : wide192 ? 0.41 : tall192 ? 0.66 : 0.6;
+                  : kind == SPLIT_128x160 ? 0.375 : square ? 0.36 : wide192 ? 0.41 : tall192 ? 0.66 : 0.6;
         if (half) fixed_us = kind == SPLIT_128x160 ? 4.0 : 5.0;  // fewer panel rows to fetch first, half the tile to store
-        if (wide192) fixed_us = 4.5;
+        if (wide192 || square) fixed_us = 4.5;
       }
       double t = rounds * ((double)(steps / s) * step_us + fixed_us);
       // The weights come from HBM: a workgroup keeps about `ahead` K steps of its weight rows in flight, and what
       // all resident workgroups have in flight over a 2 us round trip bounds the streaming rate (5 TB/s at most).
-      const double ahead = kind == SPLIT_128 ? 4.0 : kind == SPLIT_256x160 || half || small || wide192 ? 2.5 : 1.5;
+      const double ahead = kind == SPLIT_128 ? 4.0 : kind == SPLIT_256x160 || half || small || wide192 || square ? 2.5 : 1.5;
       const double step_bytes = (double)bn * (kind == SPLIT_128 ? 64.0 : 128.0);
       const double resident = wgs < cus * (kind == SPLIT_128 ? 2 : 1) ? wgs : cus * (kind == SPLIT_128 ? 2 : 1);
       double rate = resident * ahead * step_bytes / 2.0;  // bytes per us
@@ -2351,7 +2359,7 @@ static int choose_splits(long long M, long long N, long long K, int* tile_kind =
       if (t < t_stream) t = t_stream;
       // the slices' partial tiles: written once and read once (they mostly stay in the last-level cache) plus the
       // second launch; in the one-launch form they stay in the XCD's L2 and the reading is the last workgroup's tail
-      const bool one_launch = batch == 1 && kind >= SPLIT_256x160 && M % bm == 0 && s <= (kind == SPLIT_256x288 ? 2 : 4);
+      const bool one_launch = batch == 1 && kind >= SPLIT_256x160 && !square && M % bm == 0 && s <= (kind == SPLIT_256x288 ? 2 : 4);
       if (s > 1 && one_launch) t += (double)(2 * s - 1) * M * N * 4.0 / 8.0e6 + 1.0;
       else if (s > 1) t += (double)batch * (double)(2 * s + 1) * M * N * 4.0 / 5.5e6 + 3.0;  // at 5.5 TB/s, in us
       if (t < best_t * 0.97) {  // prefer fewer slices and the smaller tile unless the gain is clear
@@ -2724,6 +2732,7 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
                       : tile == SPLIT_128x288 ? "splitk_128x288"
                       : tile == SPLIT_128x80  ? "splitk_128x80"
                       : tile == SPLIT_128x192 ? "splitk_128x192"
+                      : tile == SPLIT_160x160 ? "splitk_160x160"
                                               : "splitk_256x288";
       // not for the accumulating epilogue: its reads of the old outputs, done by one workgroup per tile instead of
       // by the whole chip in the reduction kernel, cost more than the launch saved (512x9216x36864: 288 against
