@@ -1,0 +1,43 @@
+"""Who holds the device memory whose address a launch is handed: scratch and workspaces of the Python layer, with the
+allocations done in host memory (no kernel runs)."""
+import types
+import weakref
+
+import pytest
+import torch
+
+from torch_int import _CUDA, _hip_ext
+
+
+@pytest.fixture
+def host_memory(monkeypatch):
+    """torch.empty and the stream queries of the two modules without a HIP device."""
+    def empty(*shape, device=None, **kw):
+        return torch.zeros(*shape, **kw)
+    fake = types.SimpleNamespace(**{n: getattr(torch, n) for n in ("uint8", "int8", "float32", "device", "Tensor")}, empty=empty,
+                                 cuda=types.SimpleNamespace(is_current_stream_capturing=lambda: False))
+    for mod in (_CUDA, _hip_ext):
+        monkeypatch.setattr(mod, "torch", fake)
+        monkeypatch.setattr(mod, "_raw_stream", lambda index: 7)
+    monkeypatch.setattr(_CUDA, "_workspaces", {})
+    monkeypatch.setattr(_hip_ext, "_layer_scratch", {})
+    monkeypatch.setattr(_hip_ext, "_layer_scratch_need", {})
+    return fake
+
+
+def _hidden(rows, width):
+    return types.SimpleNamespace(device=types.SimpleNamespace(index=0), shape=(1, rows, width))
+
+
+def test_a_prefill_holds_its_workspace_while_another_thread_replaces_the_streams(host_memory):
+    # 256 rows at these widths are split over K, so the pass has a workspace; a second thread on the same stream asks for
+    # a larger one between two layers
+    plan = types.SimpleNamespace(embed=5120, ffn=20480)
+    memory = _hip_ext.opt_prefill_scratch(plan, _hidden(256, 5120))
+    held = weakref.ref(_CUDA._workspaces[(0, 7)])
+    address = held().data_ptr()
+    assert address in [v for v in memory if type(v) is int]
+    _CUDA._workspace(0, 7, held().numel() + 1)
+    assert held() is not None and held().data_ptr() == address and held() is not _CUDA._workspaces[(0, 7)]
+    del memory
+    assert held() is None

@@ -161,15 +161,17 @@ def _bmm_ws_bytes(batch, M, N, K):
 
 def _workspace(dev_index, stream, nbytes):
     """Split-K scratch (int32 partial tiles; contents need no initialisation).  One buffer per
-    (device, stream), grown on demand, so that calls on different streams never share it."""
+    (device, stream), grown on demand, so that calls on different streams never share it.  Returns (tensor, its
+    pointer, its bytes): whoever launches with the pointer keeps the tensor until then, since a larger request of
+    another thread on the same stream replaces it here, and the memory then goes to the stream's next allocation."""
     if nbytes <= 0:
-        return 0, 0
+        return None, 0, 0
     key = (dev_index, stream)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.empty(int(nbytes), dtype=torch.uint8, device=torch.device("cuda", dev_index))
         _workspaces[key] = ws
-    return ws.data_ptr(), ws.numel()
+    return ws, ws.data_ptr(), ws.numel()
 
 
 def _pad_inner(a, b, K, macs, weight=False):
@@ -240,7 +242,7 @@ def _linear(op, kind, x, w, bias, bias_dtype, out_dtype, alpha, beta, inout=None
     try:
         stream = _raw_stream(idx)
         # split-K scratch is only ever wanted for mid-sized M (see choose_splits in csrc/gemm_s8.hip)
-        ws_ptr, ws_bytes = _workspace(idx, stream, _ws_bytes(M, N, K)) if M > 16 else (0, 0)
+        ws, ws_ptr, ws_bytes = _workspace(idx, stream, _ws_bytes(M, N, K)) if M > 16 else (None, 0, 0)
         if _fast is not None:
             rc = _fast.linear(kind, x.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), M, N, K,
                               alpha, beta, ws_ptr, ws_bytes, stream)
@@ -311,7 +313,7 @@ def _bmm(op, kind, a, b, out_dtype, alpha):
         # few output tiles and a long inner dimension (never an attention product): split-K with a workspace
         need = _bmm_ws_bytes(batch, M, N, K) if K >= 1024 and M > 16 else 0
         if need:
-            ws_ptr, ws_bytes = _workspace(idx, stream, need)
+            ws, ws_ptr, ws_bytes = _workspace(idx, stream, need)
             scal = () if kind == _K_BMM_S32 else (alpha,)
             rc = _BMM_WS_CTYPES[kind](a.data_ptr(), b.data_ptr(), out.data_ptr(), batch, M, N, K, *scal, ws_ptr, ws_bytes,
                                       stream or None)

@@ -620,7 +620,8 @@ def opt_layer_decode(plan, hidden, mask, k_buf, v_buf, S, chain=0, carry=None):
 
 
 def opt_prefill_scratch(plan, hidden):
-    """The scratch memory and the split-K workspace of the layers of one prefill: (tensor, workspace pointer, its bytes).
+    """The scratch memory and the split-K workspace of the layers of one prefill: (scratch tensor, workspace tensor, its
+    pointer, its bytes).  Held for the pass: between two of its layers another thread may replace the stream's workspace.
     More than 64 MiB of scratch come from torch's allocator for the pass instead of staying with the stream."""
     dev = hidden.device
     M, E, F = hidden.shape[0] * hidden.shape[1], plan.embed, plan.ffn
@@ -646,7 +647,7 @@ def opt_layer_prefill(plan, hidden, mask, k_out, v_out, chain=0, carry=None, mem
     dev = hidden.device
     B, T = hidden.shape[0], hidden.shape[1]
     with _on(dev):
-        scratch, ws_ptr, ws_bytes = memory if memory is not None else opt_prefill_scratch(plan, hidden)
+        scratch, ws, ws_ptr, ws_bytes = memory if memory is not None else opt_prefill_scratch(plan, hidden)
         cls = _classes_ptr(mask, T) if mask is not None else None
         rc = _opt_layer_prefill(plan.addr, hidden.data_ptr(), mask.data_ptr() if mask is not None else 0, cls or 0,
                                 k_out.data_ptr(), v_out.data_ptr(), B, T, chain, carry.data_ptr() if chain else 0, scratch.data_ptr(),
@@ -799,7 +800,7 @@ def linear_a8_w8_b8_o8_heads(x, w, bias, alpha, beta, bsz, seq_len, heads, head_
     idx = x.device.index
     with _on(x.device):
         stream = _raw_stream(idx)
-        ws_ptr, ws_bytes = _CUDA._workspace(idx, stream, _CUDA._ws_bytes(M, N, K)) if M > 16 else (0, 0)
+        ws, ws_ptr, ws_bytes = _CUDA._workspace(idx, stream, _CUDA._ws_bytes(M, N, K)) if M > 16 else (None, 0, 0)
         rc = _lib.ti_linear_a8_w8_b8_o8_heads(x.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), M, N, K,
                                               float(alpha), float(beta), seq_len, head_dim, ws_ptr or None, ws_bytes,
                                               stream or None)
