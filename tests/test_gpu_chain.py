@@ -82,3 +82,42 @@ def test_prefills_beyond_what_the_c_call_takes_go_to_the_modules(bsz, T, taken):
     layer = randomize_int8_layer(Int8OPTDecoderLayer(128, 2, 512), torch.Generator().manual_seed(2)).to(DEV)
     hidden = torch.empty((1, 1, 128), device=DEV).expand(bsz, T, 128)
     assert (layer._prefill_checks(hidden, None) is not None) == taken
+
+
+@torch.no_grad()
+def test_recorded_passes_keep_their_memory():
+    """The layers of a prefill and of a decode step recorded into a graph after eager passes on the recording stream: later
+    eager passes there need more scratch and workspace, which replaces the stream's buffers, and run between the replays."""
+    g = torch.Generator().manual_seed(3)
+    lm = Int8OPTForCausalLM(OPTConfigLite(hidden_size=512, num_hidden_layers=2, ffn_dim=8192, num_attention_heads=4, vocab_size=64,
+                                          max_position_embeddings=512))
+    for layer in lm.model.decoder.layers:
+        randomize_int8_layer(layer, g)
+    lm = lm.to(DEV).half()
+    dec = lm.model.decoder
+    prompt, one, more = (torch.randn(*shape, 512, generator=g).to(DEV).half() for shape in ((2, 80), (20, 1), (8, 128)))
+    past = dec._chain_layers(torch.randn(20, 48, 512, generator=g).to(DEV).half(), None, None, True)
+
+    def layers(hidden, cache):
+        hidden = hidden.clone()
+        return (hidden, *(t for kv in dec._chain_layers(hidden, None, cache, True) for t in kv))
+    want, want_more = layers(prompt, None) + layers(one, past), layers(more, None)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        layers(prompt, None) + layers(one, past)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    print("recording", flush=True)
+    with torch.cuda.graph(graph, stream=side):
+        got = layers(prompt, None) + layers(one, past)
+    for replay in range(4):
+        print("replay", replay, flush=True)
+        with torch.cuda.stream(side):
+            eager = layers(more, None)
+            filled = [torch.full((1 << 20,), 7, dtype=torch.uint8, device=DEV) for _ in range(16)]
+        side.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(eager, want_more)) and all(bool((f == 7).all()) for f in filled)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))

@@ -15,10 +15,11 @@ def host_memory(monkeypatch):
     def empty(*shape, device=None, **kw):
         return torch.zeros(*shape, **kw)
     fake = types.SimpleNamespace(**{n: getattr(torch, n) for n in ("uint8", "int8", "float32", "device", "Tensor")}, empty=empty,
-                                 cuda=types.SimpleNamespace(is_current_stream_capturing=lambda: False))
+                                 cuda=types.SimpleNamespace(is_current_stream_capturing=lambda: fake.capturing), capturing=False)
     for mod in (_CUDA, _hip_ext):
         monkeypatch.setattr(mod, "torch", fake)
         monkeypatch.setattr(mod, "_raw_stream", lambda index: 7)
+    monkeypatch.setattr(_hip_ext, "_current_device", lambda: 0)
     monkeypatch.setattr(_CUDA, "_workspaces", {})
     monkeypatch.setattr(_hip_ext, "_layer_scratch", {})
     monkeypatch.setattr(_hip_ext, "_layer_scratch_need", {})
@@ -41,3 +42,19 @@ def test_a_prefill_holds_its_workspace_while_another_thread_replaces_the_streams
     assert held() is not None and held().data_ptr() == address and held() is not _CUDA._workspaces[(0, 7)]
     del memory
     assert held() is None
+
+
+@pytest.mark.parametrize("get", [lambda n: _CUDA._workspace(0, 7, n)[0],
+                                 lambda n: _hip_ext._scratch_for(types.SimpleNamespace(index=0), 7, n)])
+def test_a_recording_gets_memory_that_the_stream_does_not_keep(host_memory, get):
+    # a graph holds the address for its life; the stream's buffer goes back to the allocator when a call needs a larger one,
+    # and is written by every eager call beside a replay
+    eager = get(4096)
+    host_memory.capturing = True
+    first, second = get(1024), get(1024)
+    assert len({eager.data_ptr(), first.data_ptr(), second.data_ptr()}) == 3
+    held = weakref.ref(first)
+    del first
+    assert held() is None
+    host_memory.capturing = False
+    assert get(1024) is eager

@@ -168,9 +168,11 @@ def _workspace(dev_index, stream, nbytes):
         return None, 0, 0
     key = (dev_index, stream)
     ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
+    capturing = torch.cuda.is_current_stream_capturing()
+    if capturing or ws is None or ws.numel() < nbytes:
         ws = torch.empty(int(nbytes), dtype=torch.uint8, device=torch.device("cuda", dev_index))
-        _workspaces[key] = ws
+        if not capturing:   # a graph keeps the address for its life: memory of its own pool, which nobody else is handed
+            _workspaces[key] = ws
     return ws, ws.data_ptr(), ws.numel()
 
 

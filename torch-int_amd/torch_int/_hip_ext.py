@@ -576,12 +576,14 @@ _layer_scratch = {}   # (device, stream) -> uint8 tensor: the intermediate tenso
 
 def _scratch_for(dev, stream, nbytes):
     """One buffer per device and stream, grown on demand and shared by every layer (calls on one stream run one
-    after the other).  Memory allocated while the stream is capturing belongs to that graph's pool and is not kept."""
+    after the other).  While the stream is capturing, memory of the graph's pool that is not kept: the graph holds the
+    address for its life, the stream's buffer is replaced when a call needs a larger one."""
     key = (dev.index, stream)
     buf = _layer_scratch.get(key)
-    if buf is None or buf.numel() < nbytes:
+    capturing = torch.cuda.is_current_stream_capturing()
+    if capturing or buf is None or buf.numel() < nbytes:
         buf = torch.empty(int(nbytes), dtype=torch.uint8, device=dev)
-        if not torch.cuda.is_current_stream_capturing():
+        if not capturing:
             if len(_layer_scratch) >= 64:
                 _layer_scratch.clear()
             _layer_scratch[key] = buf
@@ -595,22 +597,33 @@ _layer_scratch_need = {}
 CHAIN_ADD, CHAIN_LEAVE = 1, 2
 
 
-def opt_layer_decode(plan, hidden, mask, k_buf, v_buf, S, chain=0, carry=None):
+def opt_decode_scratch(plans, hidden):
+    """The scratch memory of the layers of one decode step, enough for each of ``plans``."""
+    dev, B = hidden.device, hidden.shape[0]
+    need = 0
+    for E, F in {(plan.embed, plan.ffn) for plan in plans}:
+        key = (0, B, E, F)
+        n = _layer_scratch_need.get(key)
+        if n is None:
+            n = _layer_scratch_need[key] = _lib.ti_opt_decoder_layer_decode_scratch_bytes(B, E, F)
+        need = max(need, n)
+    with _on(dev):
+        return _scratch_for(dev, _raw_stream(dev.index), need)
+
+
+def opt_layer_decode(plan, hidden, mask, k_buf, v_buf, S, chain=0, carry=None, scratch=None):
     """One decode step of one decoder layer from one C call (``ti_opt_decoder_layer_decode_chained``): ``hidden`` [B, 1, embed]
     (fp32, or fp16 when the plan says half; up to 64 sequences) is updated in place, the new key and value rows are appended
     to the cache buffers, which hold S - 1 positions before the call.  ``plan`` carries ``addr`` (the address of an
     ``OptDecodeLayer`` that the caller filled from tensors it keeps alive), ``embed`` and ``ffn``; the caller has checked
-    shapes, dtypes, devices and contiguity (the decoder layer does).  The scratch memory is one buffer per device, stream
-    and size, shared by every layer; ``chain`` and ``carry`` (fp32 [B, embed], of this pass) tie the layers of one forward pass together."""
+    shapes, dtypes, devices and contiguity (the decoder layer does).  ``chain`` and ``carry`` (fp32 [B, embed], of this pass)
+    tie the layers of one forward pass together, which share ``scratch`` (``opt_decode_scratch``)."""
     dev = hidden.device
     B = hidden.shape[0]
     with _on(dev):
         stream = _raw_stream(dev.index)
-        key = (0, B, plan.embed, plan.ffn)
-        need = _layer_scratch_need.get(key)
-        if need is None:
-            need = _layer_scratch_need[key] = _lib.ti_opt_decoder_layer_decode_scratch_bytes(B, plan.embed, plan.ffn)
-        scratch = _scratch_for(dev, stream, need)
+        if scratch is None:
+            scratch = opt_decode_scratch((plan,), hidden)
         rc = _opt_layer_decode(plan.addr, hidden.data_ptr(), mask.data_ptr() if mask is not None else 0, k_buf.data_ptr(),
                                v_buf.data_ptr(), B, k_buf.shape[2], S, chain, carry.data_ptr() if chain else 0, scratch.data_ptr(),
                                scratch.numel(), stream)
@@ -634,9 +647,10 @@ def opt_prefill_scratch(plan, hidden):
         need = _layer_scratch_need[key] = (
             _lib.ti_opt_decoder_layer_prefill_scratch_bytes(M, E, F),
             max(_CUDA._ws_bytes(M, E, E), _CUDA._ws_bytes(M, F, E), _CUDA._ws_bytes(M, E, F)))
-    scratch = (_scratch_for(dev, stream, need[0]) if need[0] <= 64 << 20
-               else torch.empty(need[0], dtype=torch.uint8, device=dev))
-    return (scratch,) + _CUDA._workspace(dev.index, stream, need[1])
+    with _on(dev):
+        scratch = (_scratch_for(dev, stream, need[0]) if need[0] <= 64 << 20
+                   else torch.empty(need[0], dtype=torch.uint8, device=dev))
+        return (scratch,) + _CUDA._workspace(dev.index, stream, need[1])
 
 
 def opt_layer_prefill(plan, hidden, mask, k_out, v_out, chain=0, carry=None, memory=None):

@@ -789,9 +789,10 @@ class Int8OPTDecoder(nn.Module):
             rooms = [_kv_rooms(past) for past in past_key_values]
             if not all(rooms) or len({id(kv) for pair in rooms for kv in pair}) < 2 * count:
                 return None   # layers that were handed one and the same cache must not append to one buffer
+            scratch = _hip_ext.opt_decode_scratch([plan for plan, _ in found], hidden)
             for i, ((plan, S), (kk, vv)) in enumerate(zip(found, rooms)):
                 chain = (_hip_ext.CHAIN_ADD if i else 0) | (_hip_ext.CHAIN_LEAVE if i + 1 < count else 0)
-                _hip_ext.opt_layer_decode(plan, hidden, mask, kk.buf, vv.buf, S, chain=chain, carry=carry)
+                _hip_ext.opt_layer_decode(plan, hidden, mask, kk.buf, vv.buf, S, chain=chain, carry=carry, scratch=scratch)
                 kk.filled = vv.filled = S
                 if use_cache:
                     cache.append((_kv_view(kk, S), _kv_view(vv, S)))
