@@ -47,13 +47,13 @@ const char* ti_last_error(void);
  * TI_ERR_NO_DEVICE.  Optional: every entry point works without it.  It also does, for the current device, the two
  * one-time steps that the first calls would otherwise do: it resolves the address of the built-in scratch buffer
  * of ti_linear_a8_w8_b8_o8_noalloc, and it runs the placement probe of the one-launch split-K (ti_fused_splitk;
- * one small kernel on the null stream, 1 KB of mapped host memory, one synchronisation). */
+ * two small kernels on the null stream, 35 KB of mapped host memory, synchronised with). */
 int ti_init(void);
 
 /* Bytes of scratch the linear entry points can use for (M,N,K) to split the K
  * loop over workgroups when the output has too few tiles to fill the chip
  * (16 < M <= 1024 with a long K, or the last rows of a larger M: see ti_linear_row_split; 0 up to 16 rows, whose slices
- * meet in memory of the library's own, 16 MiB per device);
+ * meet in memory of the library's own, 67 MiB per device: 2 MiB for each of 33 streams);
  * 0 when no split is worthwhile.  Passing a smaller or NULL workspace is always legal and
  * only selects a non-split kernel. */
 int64_t ti_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
@@ -75,10 +75,17 @@ int ti_linear_row_split(int64_t M, int64_t N, int64_t K);
  * "" before the first call).  Benchmarks use it to label their rows. */
 const char* ti_last_kernel(void);
 
+/* Diagnostic: what the calling thread's last linear or group did in the weight-streaming kernel of up to 64 rows: 0 = it
+ * took another kernel, 1 = one slice of the inner dimension, 2 = several that met in one launch, 3 = several and a
+ * reduction launch; *tiling = 1 .. 8 for the tilings A .. H of csrc/gemm_rows.h, *slices = their number. */
+int ti_last_rows(int* tiling, int* slices);
+
 /* Switch (no counterpart in the reference): split-K linears whose tile is one of the 16x16-block kernel's and
  * divides M run as ONE launch ("fusedk_*" in ti_last_kernel): the K slices of an output tile run on workgroups
  * of one XCD and meet in its L2, the last wave to arrive adds them up and applies the epilogue; same bits as the
  * two-launch form ("splitk_*": raw int32 slices + a reduction kernel), which everything else takes.
+ * Linears of up to 64 rows whose inner dimension the weight-streaming kernel slices meet in one launch as well, with
+ * state of their own: see "Up to 64 rows" below.
  * enable = 1 / 0 turns the one-launch form on / off for the process, -1 leaves it; returns the setting before
  * the call.  Default on, or off with the environment variable TORCH_INT_FUSED_SPLITK=0.  The form also stays off
  * on a device whose workgroup placement is not "ids congruent mod 8 share an XCD" (probed at the first use),
@@ -89,9 +96,14 @@ const char* ti_last_kernel(void);
  * not from ti_linear_a8_w8_b8_o8_noalloc); ti_init() does it for the null stream.
  * Workspace: the one-launch form needs `workspace` on a 256-byte boundary (a 16-byte aligned one takes the
  * two-launch form).
- * HIP graphs: a launch recorded into a graph keeps the arrival counters (and the caller's workspace) of the stream
- * it was recorded on.  Replays of such a graph must therefore not overlap in time with other split-K linears
+ * HIP graphs: a launch of more than 64 rows recorded into a graph keeps the arrival counters (and the caller's workspace)
+ * of the stream it was recorded on.  Replays of such a graph must therefore not overlap in time with other such linears
  * issued on the recording stream, nor with replays of another graph recorded on that same stream.
+ * Up to 64 rows: each of the first 33 streams of a device that issue such a linear keeps a block of state for the life
+ * of the process; its first call starts the probe on it, without waiting for work queued before, and calls take the other forms (the
+ * two-launch form with a workspace, up to 16 rows without one the kernels that do not slice) until the probe has
+ * run.  So do all calls on further streams, on hipStreamPerThread and while the stream is being captured: a graph
+ * records nothing of this state, and such a linear in a graph needs no care beyond the caller's own workspace.
  * Misplacement: every one-launch GEMM checks that the workgroups of a tile ran on one XCD.  If one did not, the
  * output of THAT call cannot be trusted although it returned TI_OK (the check runs on the device, after the call
  * has returned): the next linear / bmm call on the device, whatever its shape, returns TI_ERR_LAUNCH once, naming
@@ -112,6 +124,10 @@ int ti_fused_splitk_faulted(void);
 int ti_selftest_fused_flag_action(int state, int flag, int enabled, int64_t counters, int64_t max_counters);
 int ti_selftest_fused_slot(int64_t* table, uint32_t* live_mask, int cap, int64_t stream, uint32_t busy_mask,
                            int* fresh);
+/* ... and of the weight-streaming kernel's: the block of `stream` in a table of `cap` (state[i] != 0 = taken), which is taken;
+ * what 256 placement words say (1 = eight XCDs in turn, -1 = another placement, 0 = a word is still -1). */
+int ti_selftest_rows_slot(int64_t* table, signed char* state, int cap, int64_t stream, int* fresh);
+int ti_selftest_placement(const int32_t* words);
 
 /* Diagnostic (no counterpart in the reference; computes nothing): one launch that issues the instruction mix of
  * the tiled GEMM mainloop `iters` times per wave on the first MiB of `data` (device memory, at least 1 MiB, 16-byte

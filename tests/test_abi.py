@@ -335,3 +335,37 @@ def test_only_the_256x288_gemm_tiles_spill_registers():
     for k, v in kernels.items():
         if "gemm_pipe" in k or "attn_qk_softmax_q_kernel" in k or "attn_long_kernel" in k:
             assert v["occupancy_waves_per_simd"] >= 2 and v["vgprs"] + v.get("agprs", 0) <= 256, (k, v)
+
+
+def test_rows_blocks_are_never_handed_on():
+    # a block of state per stream for the slices of up to 64 rows: a stream keeps its own, new ones take the next vacant
+    # one, and with all taken there is none (a launch that is on its way cannot lose its counters to another stream)
+    import torch_int._CUDA as C
+    lib = ctypes.CDLL(C.LIB_PATH)
+    fn = lib.ti_selftest_rows_slot
+    fn.argtypes = [ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_byte), ctypes.c_int, ctypes.c_int64,
+                   ctypes.POINTER(ctypes.c_int)]
+    table, state, fresh = (ctypes.c_int64 * 4)(), (ctypes.c_byte * 4)(), ctypes.c_int(0)
+
+    def slot(stream):
+        s = fn(table, state, 4, stream, ctypes.byref(fresh))
+        return s, fresh.value
+    assert slot(0) == (0, 1) and slot(0) == (0, 0)     # the null stream does not match an empty block
+    assert [slot(1000 + i) for i in range(3)] == [(1, 1), (2, 1), (3, 1)]
+    assert slot(2000) == (-1, 1) and slot(2000) == (-1, 1)
+    assert [slot(s) for s in (1001, 0, 1002)] == [(2, 0), (0, 0), (3, 0)]
+
+
+def test_placement_of_the_probe_words():
+    import torch_int._CUDA as C
+    lib = ctypes.CDLL(C.LIB_PATH)
+
+    def placement(words):
+        return lib.ti_selftest_placement((ctypes.c_int32 * 256)(*words))
+    good = [(i + 3) % 8 for i in range(256)]
+    assert placement(good) == 1
+    assert placement([-1] * 256) == 0 and placement(good[:-1] + [-1]) == 0 and placement([-1] + good[1:]) == 0
+    assert placement(good[:200] + [good[200] ^ 1] + good[201:]) == -1     # a workgroup that ran elsewhere
+    assert placement([0] * 256) == -1                                     # one XCD for all
+    assert placement([0, 1, 2, 3, 0, 1, 2, 3] * 32) == -1                 # two classes on one
+    assert placement([16] + good[1:]) == -1

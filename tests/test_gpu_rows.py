@@ -136,3 +136,94 @@ def test_workspace_is_that_of_the_kernel_that_runs(N, K, sliced):
     """Widths that 16 does not divide go to the tiled kernels where 1024 does not divide the inner dimension, which slice it."""
     import torch_int._CUDA as C
     assert (C._lib.ti_linear_workspace_bytes(48, N, K) > 0) == sliced
+
+
+def _sliced(M, N, K, seed):
+    """A sliced linear of M rows: (call, the oracle's output)."""
+    import torch_int._CUDA as C
+    g = torch.Generator().manual_seed(seed)
+    x, w, b = _s8(g, M, K), _s8(g, N, K), _s8(g, N)
+    want = orc.linear_a8_w8_b8_o8(x, w, b, 3e-4, 0.02, acc_fn=orc.gemm_acc_torch).to(DEV)
+    xd, wd, bd = x.to(DEV), w.to(DEV), b.to(DEV)
+    return lambda: C.linear_a8_w8_b8_o8(xd, wd, bd, 3e-4, 0.02), want
+
+
+def _form():
+    import torch_int._CUDA as C
+    t, s = ctypes.c_int(0), ctypes.c_int(0)
+    return C._lib.ti_last_rows(ctypes.byref(t), ctypes.byref(s))
+
+
+@pytest.mark.parametrize("M,recorded", [(8, 0), (24, 3)])
+def test_graphs_of_sliced_linears_replay_on_two_streams_beside_eager_work(M, recorded):
+    """Two graphs recorded on one stream, replayed on two others while the recording stream runs the same linears eagerly:
+    what is recorded keeps no state of the stream."""
+    call, want = _sliced(M, 2560, 10240, 1)
+    side, others = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            call()
+        assert _form() == 2    # eagerly the slices meet in one launch
+    torch.cuda.synchronize()
+    graphs, outs = [torch.cuda.CUDAGraph() for _ in range(2)], []
+    for graph in graphs:
+        print("recording", M, flush=True)
+        with torch.cuda.graph(graph, stream=side):
+            outs.append([call() for _ in range(6)])
+            assert _form() == recorded
+    torch.cuda.synchronize()
+    for round_ in range(3):
+        print("replays", M, round_, flush=True)
+        eager = []
+        for _ in range(8):
+            for graph, stream in zip(graphs, others):
+                with torch.cuda.stream(stream):
+                    graph.replay()
+            with torch.cuda.stream(side):
+                eager.append(call())
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, want) for o in outs[0] + outs[1] + eager)
+
+
+def test_forty_streams_of_sliced_linears():
+    """More streams than there are blocks of state, all with work queued at once, twice over: exact on every one."""
+    import torch_int._CUDA as C
+    call, want = _sliced(8, 2560, 10240, 2)
+    big, want_big = _sliced(40, 2048, 8192, 3)
+    streams = []
+    for _ in range(40):
+        h = ctypes.c_void_p()
+        assert C._lib.hipStreamCreate(ctypes.byref(h)) == 0   # the HIP runtime that the library is linked to
+        streams.append(torch.cuda.ExternalStream(h.value))
+    torch.cuda.synchronize()
+    forms = set()
+    for turn in range(2):
+        print("forty streams", turn, flush=True)
+        outs = []
+        for s in streams:
+            with torch.cuda.stream(s):
+                outs.append((call(), want))
+                forms.add((8, _form()))
+                outs.append((big(), want_big))
+                forms.add((40, _form()))
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, w) for o, w in outs)
+    assert forms == {(8, 0), (8, 2), (40, 3), (40, 2)}
+
+
+def test_a_stream_of_every_thread_keeps_no_state():
+    """hipStreamPerThread is one handle for a stream of each thread."""
+    import torch_int._CUDA as C
+    g = torch.Generator().manual_seed(4)
+    x, w, b = _s8(g, 40, 8192).to(DEV), _s8(g, 2048, 8192).to(DEV), _s8(g, 2048).to(DEV)
+    out, want = torch.empty((40, 2048), dtype=torch.int8, device=DEV), C.linear_a8_w8_b8_o8(x, w, b, 3e-4, 0.02)
+    need = C._lib.ti_linear_workspace_bytes(40, 2048, 8192)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    torch.cuda.synchronize()
+    for _ in range(2):
+        rc = C._lib.ti_linear_a8_w8_b8_o8(x.data_ptr(), w.data_ptr(), b.data_ptr(), out.data_ptr(), 40, 2048, 8192, 3e-4, 0.02,
+                                          ws.data_ptr(), need, 2)
+        assert rc == 0 and _form() == 3
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)

@@ -140,7 +140,7 @@ int ti_init(void) {
     return fail(TI_ERR_NO_DEVICE, "device %d is %s; this library holds gfx950 code only", dev, prop.gcnArchName);
   void* ptr = nullptr;  // resolve the no-allocation entry point's scratch here, outside any capture or hot loop
   if (int rc = scratch_address("ti_init", &ptr)) return rc;
-  (void)warm_fused_split(nullptr);  // and probe the workgroup placement the one-launch split-K relies on
+  (void)warm_fused_split(nullptr);  // and probe the workgroup placement the one-launch forms rely on
   return TI_OK;
 }
 
@@ -435,6 +435,7 @@ int ti_attn_softmax_q(const float* scores, const float* mask, int8_t* probs, int
 }
 
 const char* ti_last_kernel(void) { return last_gemm_kernel(); }
+int ti_last_rows(int* tiling, int* slices) { return last_rows(tiling, slices); }
 
 int ti_fused_splitk(int enable) { return set_fused_split(enable); }
 int ti_fused_splitk_faulted(void) { return fused_split_faulted(); }
@@ -447,6 +448,11 @@ int ti_selftest_fused_slot(int64_t* table, uint32_t* live_mask, int cap, int64_t
   return fused_slot_for_test(reinterpret_cast<long long*>(table), reinterpret_cast<unsigned*>(live_mask), cap, stream,
                              busy_mask, fresh);
 }
+
+int ti_selftest_rows_slot(int64_t* table, signed char* state, int cap, int64_t stream, int* fresh) {
+  return rows_slot_for_test(reinterpret_cast<long long*>(table), state, cap, stream, fresh);
+}
+int ti_selftest_placement(const int32_t* words) { return placement_of(words); }
 
 int64_t ti_diag_mfma_loop_ops(int64_t iters) { return iters > 0 ? diag_mfma_loop_ops(iters) : 0; }
 

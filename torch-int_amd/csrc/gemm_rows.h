@@ -466,10 +466,16 @@ static int launch_rows_mx(int tiling, const GemmParams& p, const GemmGroup& grp,
   }
 }
 
-// Library-owned home for the parked tiles of launches of up to 16 rows, one block per stream slot of the fused form (see
-// gemm_s8.hip): nullptr when the stream has none.
+// Library-owned home for the parked tiles of launches of up to 16 rows, one block per stream (see gemm_s8.hip).
 static constexpr long long kRowsParkBytes = 2 << 20;
-void* fused_split_park(const GemmParams& q);
+int rows_split_prepare(hipStream_t stream, GemmParams& q, void** park);
+
+// What the calling thread's last linear did here: form 0 = it ran on another kernel, 1 = one slice, 2 = slices that meet in
+// one launch, 3 = two launches.
+struct RowsLast {
+  int form, tiling, slices;
+};
+extern thread_local RowsLast g_rows_last;
 
 // The linear (or GROUPED: up to four linears of one shape on the same activations) through gemm_rows_kernel.  Returns a
 // TI_* status, or -1 when the shape, the alignment or the workspace does not allow it (the caller goes on to the other
@@ -492,11 +498,12 @@ static int launch_rows(const GemmParams& p_in, const GemmGroup& grp, int problem
     const bool given = workspace != nullptr && workspace_bytes >= park && (reinterpret_cast<uintptr_t>(workspace) & 255) == 0;
     const bool own = p.M <= 16 && park <= kRowsParkBytes;
     if (!given && !own) return -1;
-    const int usable = fused_split_prepare(stream, 2 * num_cus() * 8, p);  // arrivals: workgroups x waves at most
+    void* home = nullptr;
+    const int usable = rows_split_prepare(stream, p, &home);
     if (usable < 0) return -usable;
     if (usable) {
-      p.parts = given ? workspace : fused_split_park(p);
-    } else {
+      p.parts = given ? workspace : home;
+    } else {  // without a workspace the kernels that keep no state, as in every graph: 16 x 5120 x 20480 31.8 us against 20.7
       if (!given) return -1;
       p.arrivals = nullptr;
       p.parts = workspace;
@@ -510,6 +517,7 @@ static int launch_rows(const GemmParams& p_in, const GemmGroup& grp, int problem
     case 3: rc = launch_rows_mx<KIND, GROUPED, 3>(pick.tiling, p, grp, strips, per_problem, stream); break;
     default: rc = launch_rows_mx<KIND, GROUPED, 4>(pick.tiling, p, grp, strips, per_problem, stream); break;
   }
+  if (rc == TI_OK) g_rows_last = {two_launches ? 3 : pick.slices > 1 ? 2 : 1, pick.tiling, pick.slices};
   if (rc || !two_launches) return rc;
   for (int i = 0; i < problems; ++i) {
     GemmParams q = p_in;

@@ -44,6 +44,12 @@ long long bmm_workspace_bytes(long long batch, long long M, long long N, long lo
 
 thread_local const char* g_last_kernel = "";
 const char* last_gemm_kernel() { return g_last_kernel; }
+thread_local RowsLast g_rows_last = {0, 0, 0};
+int last_rows(int* tiling, int* slices) {
+  *tiling = g_rows_last.tiling;
+  *slices = g_rows_last.slices;
+  return g_rows_last.form;
+}
 
 // ---------------------------------------------------------------------------
 // State of the one-launch split-K (the FUSED form of gemm_pipe16q_kernel), per device.
@@ -64,21 +70,36 @@ static constexpr int kFusedCounters = 32768;            // per stream: tiles x w
 static constexpr int kFusedTiles = kFusedCounters / 8;  // per stream: one XCC word per tile
 static __device__ __align__(256) int g_fused_arrivals[kFusedStreams * (kFusedCounters + kFusedTiles)];
 
-// Parked tiles of gemm_rows_kernel for up to 16 rows, whose callers hold no workspace: a block per stream slot, used by one
-// launch of that stream at a time and written in full before it is read.
-static __device__ __align__(256) char g_rows_park[kFusedStreams * kRowsParkBytes];
+// State of gemm_rows_kernel's slices, apart from that of the form above: decoding goes through it on every stream, and a
+// graph that holds a block of counters from above must not meet eager decoding there.  A block per stream, used by one
+// launch of that stream at a time: counters and placement words, and for up to 16 rows, whose callers hold no workspace,
+// the parked tiles (written in full before they are read).  A stream keeps its block for the life of the process, so
+// that no launch on its way can lose it, and launches that a graph records get none: a replay is not bound to the stream
+// it was recorded on.  33 blocks, as many as a program gets streams of from torch (the default one and a pool of 32);
+// further streams take the other forms.
+static constexpr int kRowsStreams = 33;
+static constexpr int kRowsCounters = 4096, kRowsWords = 4096;  // rows_pick: at most 256 groups x 8 waves, 256 words 64 bytes apart
+static __device__ __align__(256) int g_rows_arrivals[kRowsStreams * (kRowsCounters + kRowsWords)];
+static __device__ __align__(256) char g_rows_park[kRowsStreams * kRowsParkBytes];
 
 __global__ void xcc_probe_kernel(unsigned* out) {
-  if (threadIdx.x == 0) out[blockIdx.x] = __builtin_amdgcn_s_getreg((3 << 11) | 20) & 0xf;  // HW_REG_XCC_ID
+  if (threadIdx.x == 0)
+    __hip_atomic_store(out + blockIdx.x, __builtin_amdgcn_s_getreg((3 << 11) | 20) & 0xf, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);  // HW_REG_XCC_ID
 }
+static constexpr int kProbeWords = 256;
+enum RowsSlot : signed char { ROWS_VACANT = 0, ROWS_PROBING, ROWS_USABLE, ROWS_REFUSED };
 
 struct FusedDevice {
   std::mutex lock;
   int state = 0;  // 0 = not probed yet, 1 = usable, -1 = off
   int* arrivals = nullptr;
-  char* park = nullptr;
-  int* host_words = nullptr;  // [0] = the misplacement flag, [1 .. 256] = the probe's output
+  int* host_words = nullptr;  // [0] = the misplacement flag, [1 .. 256] = the probe's output, then 256 words per rows slot
   int* host_words_dev = nullptr;
+  int* rows_arrivals = nullptr;
+  char* rows_park = nullptr;
+  hipStream_t rows_streams[kRowsStreams] = {};
+  RowsSlot rows_state[kRowsStreams] = {};
   hipStream_t streams[kFusedStreams] = {};
   bool live[kFusedStreams] = {};
   bool pinned[kFusedStreams] = {};  // a launch with this slot's counters was recorded into a graph: never handed on
@@ -100,27 +121,56 @@ int set_fused_split(int enable) {
 }
 static bool fused_enabled() { return set_fused_split(-1) != 0; }
 
-// The first use on a device allocates 1 KB of host memory and synchronises; a thread that must not allocate (the
+// The first use on a device allocates 35 KB of host memory and synchronises; a thread that must not allocate (the
 // entry point that promises it) clears this around its call and then only uses a device that is ready.
 static thread_local bool g_fused_may_probe = true;
 void allow_fused_split_probe(bool allow) { g_fused_may_probe = allow; }
 
-// Runs the placement probe on `stream` (which must not be capturing) and waits for it: true when the 256 probe
-// workgroups show one XCC per residue class of the workgroup id mod 8, eight different ones.
-static bool probe_placement(FusedDevice& d, hipStream_t stream) {
-  for (int i = 0; i < 256; ++i) d.host_words[1 + i] = -1;
-  hipLaunchKernelGGL(xcc_probe_kernel, dim3(256), dim3(64), 0, stream, reinterpret_cast<unsigned*>(d.host_words_dev + 1));
-  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(stream) != hipSuccess) return false;
+// What 256 probe words say: 1 = one XCC per residue class of the workgroup id mod 8, eight different ones; -1 = another
+// placement; 0 = not all of them are there yet.  Free of HIP calls so that it can be tested on the CPU.
+int placement_of(const volatile int* words) {
+  for (int i = 0; i < kProbeWords; ++i)
+    if (words[i] == -1) return 0;
   unsigned seen = 0;
-  for (int i = 0; i < 256; ++i) {
-    const int xcc = d.host_words[1 + i];
-    if (xcc < 0 || xcc > 15 || xcc != d.host_words[1 + (i & 7)]) return false;
-  }
+  for (int i = 0; i < kProbeWords; ++i)
+    if (words[i] < 0 || words[i] > 15 || words[i] != words[i & 7]) return -1;
   for (int i = 0; i < 8; ++i) {
-    const unsigned xcc = (unsigned)d.host_words[1 + i];
-    if (seen & (1u << xcc)) return false;  // two residue classes on one XCD: not the placement this needs
-    seen |= 1u << xcc;
+    if (seen & (1u << words[i])) return -1;  // two residue classes on one XCD: not the placement this needs
+    seen |= 1u << words[i];
   }
+  return 1;
+}
+
+// Starts the placement probe on `stream` (which must not be capturing); its words are at `at` of the host words.
+static bool start_probe(FusedDevice& d, int at, hipStream_t stream) {
+  for (int i = 0; i < kProbeWords; ++i) d.host_words[at + i] = -1;
+  hipLaunchKernelGGL(xcc_probe_kernel, dim3(kProbeWords), dim3(64), 0, stream, reinterpret_cast<unsigned*>(d.host_words_dev + at));
+  return hipGetLastError() == hipSuccess;
+}
+static bool probe_placement(FusedDevice& d, hipStream_t stream) {  // ... and waits for it
+  return start_probe(d, 1, stream) && hipStreamSynchronize(stream) == hipSuccess && placement_of(d.host_words + 1) == 1;
+}
+
+// Host words and device addresses of the current device, once.
+static bool fused_memory(FusedDevice& d) {
+  if (d.host_words != nullptr) return d.rows_park != nullptr;
+  void *arrivals = nullptr, *rows = nullptr, *park = nullptr;
+  int* words = nullptr;
+  if (hipGetSymbolAddress(&arrivals, HIP_SYMBOL(g_fused_arrivals)) != hipSuccess || arrivals == nullptr) return false;
+  if (hipGetSymbolAddress(&rows, HIP_SYMBOL(g_rows_arrivals)) != hipSuccess || rows == nullptr) return false;
+  if (hipGetSymbolAddress(&park, HIP_SYMBOL(g_rows_park)) != hipSuccess || park == nullptr) return false;
+  if (hipHostMalloc(reinterpret_cast<void**>(&words), (1 + (1 + kRowsStreams) * kProbeWords) * sizeof(int),
+                    hipHostMallocMapped) != hipSuccess)
+    return false;
+  words[0] = 0;
+  if (hipHostGetDevicePointer(reinterpret_cast<void**>(&d.host_words_dev), words, 0) != hipSuccess) {
+    (void)hipHostFree(words);
+    return false;
+  }
+  d.arrivals = static_cast<int*>(arrivals);
+  d.rows_arrivals = static_cast<int*>(rows);
+  d.rows_park = static_cast<char*>(park);
+  d.host_words = words;
   return true;
 }
 
@@ -240,20 +290,7 @@ int fused_split_prepare(hipStream_t stream, long long counters, GemmParams& q) {
     // first use on this device: not while the stream records a graph (the probe allocates and synchronises)
     if (is_capturing(stream)) return 0;
     d.state = -1;
-    void* sym = nullptr;
-    void* park = nullptr;
-    if (hipGetSymbolAddress(&sym, HIP_SYMBOL(g_fused_arrivals)) != hipSuccess || sym == nullptr) return 0;
-    if (hipGetSymbolAddress(&park, HIP_SYMBOL(g_rows_park)) != hipSuccess || park == nullptr) return 0;
-    if (hipHostMalloc(reinterpret_cast<void**>(&d.host_words), 257 * sizeof(int), hipHostMallocMapped) != hipSuccess) {
-      d.host_words = nullptr;
-      return 0;
-    }
-    d.host_words[0] = 0;
-    if (hipHostGetDevicePointer(reinterpret_cast<void**>(&d.host_words_dev), d.host_words, 0) != hipSuccess)
-      return 0;
-    if (!probe_placement(d, stream)) return 0;
-    d.arrivals = static_cast<int*>(sym);
-    d.park = static_cast<char*>(park);
+    if (!fused_memory(d) || !probe_placement(d, stream)) return 0;
     d.state = 1;
     probed_now = true;
   }
@@ -280,17 +317,82 @@ int fused_split_prepare(hipStream_t stream, long long counters, GemmParams& q) {
   return 1;
 }
 
-void* fused_split_park(const GemmParams& q) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
-  FusedDevice& d = g_fused[dev];
-  const long long slot = (q.arrivals - d.arrivals) / (kFusedCounters + kFusedTiles);
-  return d.park + slot * kRowsParkBytes;
+// Slot of `stream` among `cap`: its own (fresh = false), else the first vacant one (fresh = true), else -1.  Slots are
+// never handed on.  Free of HIP calls so that it can be tested on the CPU.
+int pick_rows_slot(const hipStream_t* streams, const RowsSlot* state, int cap, hipStream_t stream, bool& fresh) {
+  fresh = false;
+  for (int i = 0; i < cap && state[i] != ROWS_VACANT; ++i)
+    if (streams[i] == stream) return i;
+  fresh = true;
+  for (int i = 0; i < cap; ++i)
+    if (state[i] == ROWS_VACANT) return i;
+  return -1;
 }
 
+// Makes q ready for slices that meet in one launch of gemm_rows_kernel on `stream`: 1 = ready, *park = the stream's home
+// for parked tiles; 0 = take another form; < 0 = minus the status of a misplacement to report.  Never waits for work that
+// is queued: a stream's first call starts the placement probe on it and waits for that only where nothing is ahead of it
+// (some 20 us); else calls take the other forms until the probe's words are there.
+int rows_split_prepare(hipStream_t stream, GemmParams& q, void** park) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  FusedDevice& d = g_fused[dev];
+  std::lock_guard<std::mutex> guard(d.lock);
+  const int flag = d.host_words != nullptr ? *reinterpret_cast<volatile int*>(d.host_words) : 0;
+  const int action = fused_flag_action(d.state, flag, fused_enabled(), 0, kFusedCounters);
+  if (action < 0 && d.state == 1) {
+    d.state = -1;
+    return -fail(TI_ERR_LAUNCH, "%s", kMisplacedMsg);
+  }
+  // hipStreamPerThread is one handle for a stream of every thread
+  if (action <= 0 || stream == hipStreamPerThread || is_capturing(stream)) return 0;
+  if (d.host_words == nullptr && !g_fused_may_probe) return 0;  // the first use on a device allocates host memory
+  if (!fused_memory(d)) return 0;
+  bool fresh = false;
+  const int slot = pick_rows_slot(d.rows_streams, d.rows_state, kRowsStreams, stream, fresh);
+  if (slot < 0) return 0;
+  const int words = 1 + (1 + slot) * kProbeWords;
+  if (fresh) {
+    const bool idle = g_fused_may_probe && hipStreamQuery(stream) == hipSuccess;
+    (void)hipGetLastError();  // a busy stream leaves "not ready" behind
+    d.rows_streams[slot] = stream;
+    d.rows_state[slot] = start_probe(d, words, stream) ? ROWS_PROBING : ROWS_REFUSED;
+    if (idle) (void)hipStreamSynchronize(stream);
+  }
+  if (d.rows_state[slot] == ROWS_PROBING) {
+    const int placement = placement_of(d.host_words + words);
+    if (placement == 0) return 0;
+    d.rows_state[slot] = placement > 0 ? ROWS_USABLE : ROWS_REFUSED;
+    if (placement > 0 && d.state == 0) d.state = 1;  // a launch of this form reports a misplacement like any other
+  }
+  if (d.rows_state[slot] != ROWS_USABLE) return 0;
+  q.arrivals = d.rows_arrivals + (long long)slot * (kRowsCounters + kRowsWords);
+  q.xcc_seen = reinterpret_cast<unsigned*>(q.arrivals + kRowsCounters);
+  q.xcc_error = d.host_words_dev;
+  *park = d.rows_park + slot * kRowsParkBytes;
+  return 1;
+}
+
+// CPU-testable face of pick_rows_slot: streams are plain integers, state[i] != 0 = slot i is taken; takes the slot.
+int rows_slot_for_test(long long* table, signed char* state, int cap, long long stream, int* fresh) {
+  bool f = false;
+  static_assert(sizeof(hipStream_t) == sizeof(long long) && sizeof(RowsSlot) == 1, "plain tables");
+  const int slot = pick_rows_slot(reinterpret_cast<const hipStream_t*>(table), reinterpret_cast<const RowsSlot*>(state), cap,
+                                  reinterpret_cast<hipStream_t>(stream), f);
+  if (slot >= 0) {
+    table[slot] = stream;
+    state[slot] = ROWS_USABLE;
+  }
+  *fresh = f ? 1 : 0;
+  return slot;
+}
+
+// The probes of both forms on `stream` now rather than at its first calls.
 int warm_fused_split(void* stream) {
   GemmParams unused;
+  void* park = nullptr;
   const int rc = fused_split_prepare(static_cast<hipStream_t>(stream), 0, unused);
+  if (rc > 0) (void)rows_split_prepare(static_cast<hipStream_t>(stream), unused, &park);
   return rc > 0 ? 1 : 0;
 }
 
@@ -359,6 +461,7 @@ int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStrea
                          long long workspace_bytes) {
   constexpr int KIND = EPI_S8_BIAS;
   if (shape.M == 0 || shape.N == 0 || grp.count == 0) return TI_OK;
+  g_rows_last = {0, 0, 0};
   bool ptr_ok = (reinterpret_cast<uintptr_t>(shape.A) & 15) == 0;
   for (int i = 0; i < grp.count; ++i) ptr_ok = ptr_ok && (reinterpret_cast<uintptr_t>(grp.B[i]) & 15) == 0;
   const bool aligned = ptr_ok && (shape.K % SBK == 0) && shape.K > 0;
@@ -430,6 +533,7 @@ int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStrea
 
 int launch_gemm(int kind, const GemmParams& p, void* ws, long long ws_bytes, hipStream_t stream) {
   if (p.M == 0 || p.N == 0 || p.batch == 0) return TI_OK;
+  g_rows_last = {0, 0, 0};
   if (int rc = fused_split_check()) return rc;
   switch (kind) {
     case EPI_S32_BIAS: return launch_gemm_kind_0(p, ws, ws_bytes, stream);
