@@ -59,6 +59,35 @@ def test_chained_layers_give_the_modules_values(bsz, T, layers, pad, half):
             assert torch.equal(ka, kb) and torch.equal(va, vb)
 
 
+def _against_the_modules(lm, ids):
+    """A cached prefill and three decode steps, chained and through the modules: logits and caches bit for bit."""
+    chained = _generate(lm, ids, None, 3)
+    try:
+        Int8OPTDecoderLayer.prefill_in_one_call = Int8OPTDecoderLayer.decode_in_one_call = False
+        modules = _generate(lm, ids, None, 3)
+    finally:
+        Int8OPTDecoderLayer.prefill_in_one_call = Int8OPTDecoderLayer.decode_in_one_call = True
+    for a, b in zip(chained, modules):
+        assert torch.equal(a.logits, b.logits)
+        for (ka, va), (kb, vb) in zip(a.past_key_values, b.past_key_values):
+            assert torch.equal(ka, kb) and torch.equal(va, vb)
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("widths,bsz,T", [((256, 2048, 1024), 2, 160), ((1024, 256), 20, 48), ((128, 8192), 5, 32)])
+def test_layers_of_different_widths(widths, bsz, T):
+    """Layers whose fc1 has been pruned or widened one by one: the memory of a pass is that of the widest."""
+    g = torch.Generator().manual_seed(T)
+    lm = Int8OPTForCausalLM(OPTConfigLite(hidden_size=128, num_hidden_layers=len(widths), ffn_dim=512, num_attention_heads=2,
+                                          vocab_size=64, max_position_embeddings=512))
+    layers = lm.model.decoder.layers
+    for i, width in enumerate(widths):
+        layers[i] = randomize_int8_layer(Int8OPTDecoderLayer(128, 2, width), g)
+    lm = lm.to(DEV).half()
+    print("widths", widths, bsz, T, flush=True)
+    _against_the_modules(lm, torch.randint(2, 64, (bsz, T), generator=g).to(DEV))
+
+
 @torch.no_grad()
 def test_layers_handed_one_cache_keep_their_own_rows():
     g = torch.Generator().manual_seed(1)

@@ -34,7 +34,7 @@ def test_a_prefill_holds_its_workspace_while_another_thread_replaces_the_streams
     # 256 rows at these widths are split over K, so the pass has a workspace; a second thread on the same stream asks for
     # a larger one between two layers
     plan = types.SimpleNamespace(embed=5120, ffn=20480)
-    memory = _hip_ext.opt_prefill_scratch(plan, _hidden(256, 5120))
+    memory = _hip_ext.opt_prefill_scratch([plan], _hidden(256, 5120))
     held = weakref.ref(_CUDA._workspaces[(0, 7)])
     address = held().data_ptr()
     assert address in [v for v in memory if type(v) is int]
@@ -58,3 +58,13 @@ def test_a_recording_gets_memory_that_the_stream_does_not_keep(host_memory, get)
     assert held() is None
     host_memory.capturing = False
     assert get(1024) is eager
+
+
+def test_memory_of_a_pass_fits_its_widest_layer(host_memory):
+    # 304 rows of a 20480 wide layer are split over K and need a workspace; the narrow first layer needs none
+    plans = [types.SimpleNamespace(embed=5120, ffn=f) for f in (512, 20480, 1024)]
+    scratch, _, _, ws_bytes = _hip_ext.opt_prefill_scratch(plans, _hidden(304, 5120))
+    assert scratch.numel() >= _hip_ext._lib.ti_opt_decoder_layer_prefill_scratch_bytes(304, 5120, 20480)
+    assert ws_bytes >= _CUDA._ws_bytes(304, 5120, 20480) > 0
+    one = types.SimpleNamespace(device=types.SimpleNamespace(index=0), shape=(40, 1, 5120))
+    assert _hip_ext.opt_decode_scratch(plans, one).numel() >= _hip_ext._lib.ti_opt_decoder_layer_decode_scratch_bytes(40, 5120, 20480)

@@ -632,25 +632,28 @@ def opt_layer_decode(plan, hidden, mask, k_buf, v_buf, S, chain=0, carry=None, s
     return hidden
 
 
-def opt_prefill_scratch(plan, hidden):
-    """The scratch memory and the split-K workspace of the layers of one prefill: (scratch tensor, workspace tensor, its
-    pointer, its bytes).  Held for the pass: between two of its layers another thread may replace the stream's workspace.
-    More than 64 MiB of scratch come from torch's allocator for the pass instead of staying with the stream."""
+def opt_prefill_scratch(plans, hidden):
+    """The scratch memory and the split-K workspace of the layers of one prefill, enough for each of ``plans``: (scratch
+    tensor, workspace tensor, its pointer, its bytes).  Held for the pass: between two of its layers another thread may
+    replace the stream's workspace.  More than 64 MiB of scratch come from torch's allocator for the pass instead of
+    staying with the stream."""
     dev = hidden.device
-    M, E, F = hidden.shape[0] * hidden.shape[1], plan.embed, plan.ffn
-    stream = _raw_stream(dev.index)
-    key = (1, M, E, F)
-    need = _layer_scratch_need.get(key)
-    if need is None:
-        if len(_layer_scratch_need) > 4096:
-            _layer_scratch_need.clear()
-        need = _layer_scratch_need[key] = (
-            _lib.ti_opt_decoder_layer_prefill_scratch_bytes(M, E, F),
-            max(_CUDA._ws_bytes(M, E, E), _CUDA._ws_bytes(M, F, E), _CUDA._ws_bytes(M, E, F)))
+    M = hidden.shape[0] * hidden.shape[1]
+    need = need_ws = 0
+    for E, F in {(plan.embed, plan.ffn) for plan in plans}:
+        key = (1, M, E, F)
+        n = _layer_scratch_need.get(key)
+        if n is None:
+            if len(_layer_scratch_need) > 4096:
+                _layer_scratch_need.clear()
+            n = _layer_scratch_need[key] = (
+                _lib.ti_opt_decoder_layer_prefill_scratch_bytes(M, E, F),
+                max(_CUDA._ws_bytes(M, E, E), _CUDA._ws_bytes(M, F, E), _CUDA._ws_bytes(M, E, F)))
+        need, need_ws = max(need, n[0]), max(need_ws, n[1])
     with _on(dev):
-        scratch = (_scratch_for(dev, stream, need[0]) if need[0] <= 64 << 20
-                   else torch.empty(need[0], dtype=torch.uint8, device=dev))
-        return (scratch,) + _CUDA._workspace(dev.index, stream, need[1])
+        stream = _raw_stream(dev.index)
+        scratch = _scratch_for(dev, stream, need) if need <= 64 << 20 else torch.empty(need, dtype=torch.uint8, device=dev)
+        return (scratch,) + _CUDA._workspace(dev.index, stream, need_ws)
 
 
 def opt_layer_prefill(plan, hidden, mask, k_out, v_out, chain=0, carry=None, memory=None):
@@ -661,7 +664,7 @@ def opt_layer_prefill(plan, hidden, mask, k_out, v_out, chain=0, carry=None, mem
     dev = hidden.device
     B, T = hidden.shape[0], hidden.shape[1]
     with _on(dev):
-        scratch, ws, ws_ptr, ws_bytes = memory if memory is not None else opt_prefill_scratch(plan, hidden)
+        scratch, ws, ws_ptr, ws_bytes = memory if memory is not None else opt_prefill_scratch((plan,), hidden)
         cls = _classes_ptr(mask, T) if mask is not None else None
         rc = _opt_layer_prefill(plan.addr, hidden.data_ptr(), mask.data_ptr() if mask is not None else 0, cls or 0,
                                 k_out.data_ptr(), v_out.data_ptr(), B, T, chain, carry.data_ptr() if chain else 0, scratch.data_ptr(),

@@ -797,7 +797,7 @@ class Int8OPTDecoder(nn.Module):
                 if use_cache:
                     cache.append((_kv_view(kk, S), _kv_view(vv, S)))
         else:
-            memory = _hip_ext.opt_prefill_scratch(found[0], hidden)
+            memory = _hip_ext.opt_prefill_scratch(found, hidden)
             for i, plan in enumerate(found):
                 chain = (_hip_ext.CHAIN_ADD if i else 0) | (_hip_ext.CHAIN_LEAVE if i + 1 < count else 0)
                 key, value = plan.new_cache(hidden)
