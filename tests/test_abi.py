@@ -369,3 +369,17 @@ def test_placement_of_the_probe_words():
     assert placement([0] * 256) == -1                                     # one XCD for all
     assert placement([0, 1, 2, 3, 0, 1, 2, 3] * 32) == -1                 # two classes on one
     assert placement([16] + good[1:]) == -1
+
+
+def test_prefill_of_more_than_65535_sequences_times_heads_is_refused_before_any_launch():
+    # the transpose of the values takes that many matrices; with a null LayerNorm parameter the first step would refuse too
+    import torch_int._CUDA as C
+    import torch_int._hip_ext as X
+    st = X.OptDecodeLayer()
+    st.embed, st.heads, st.head_dim, st.ffn = 640, 40, 16, 64
+    buf = ctypes.create_string_buffer(512)
+    p = (ctypes.addressof(buf) + 255) // 256 * 256
+    call = X._lib.ti_opt_decoder_layer_prefill_chained
+    for bsz, message in ((1638, b"gamma is NULL"), (1639, b"65535 sequences x heads")):
+        assert call(ctypes.addressof(st), p, None, None, p, p, bsz, 32, 0, None, p, 1 << 40, None, 0, None) == 1
+        assert message in C._lib.ti_last_error()

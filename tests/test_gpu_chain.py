@@ -106,6 +106,21 @@ def test_layers_handed_one_cache_keep_their_own_rows():
         assert all(torch.equal(a, b) for a, b in zip(kept, want))
 
 
+@torch.no_grad()
+@pytest.mark.parametrize("bsz", [1638, 1639])   # 40 heads: 65520 and 65560 matrices of values to transpose
+def test_prefills_around_65535_sequences_times_heads(bsz):
+    g = torch.Generator().manual_seed(bsz)
+    lm = Int8OPTForCausalLM(OPTConfigLite(hidden_size=640, num_hidden_layers=2, ffn_dim=64, num_attention_heads=40, vocab_size=64,
+                                          max_position_embeddings=64))
+    for layer in lm.model.decoder.layers:
+        randomize_int8_layer(layer, g)
+    lm = lm.to(DEV).half()
+    print("sequences", bsz, flush=True)
+    assert (lm.model.decoder.layers[0]._prefill_checks(torch.empty((bsz, 32, 640), dtype=torch.float16, device=DEV), None)
+            is not None) == (bsz * 40 <= 65535)
+    _against_the_modules(lm, torch.randint(2, 64, (bsz, 32), generator=g).to(DEV))
+
+
 @pytest.mark.parametrize("bsz,T,taken", [(64, 16, True), (65536, 16, False), (1025, 1024, False)])
 def test_prefills_beyond_what_the_c_call_takes_go_to_the_modules(bsz, T, taken):
     layer = randomize_int8_layer(Int8OPTDecoderLayer(128, 2, 512), torch.Generator().manual_seed(2)).to(DEV)

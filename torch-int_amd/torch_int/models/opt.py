@@ -580,7 +580,9 @@ class Int8OPTDecoderLayer(nn.Module):
         if T % 16 or bsz == 0 or bsz > 65535 or bsz * T > 1 << 20 or (mask is not None and mask.shape != (bsz, 1, T, T)):
             return None
         plan = self._decode_plan(hs.dtype is torch.float16, hs.device)
-        if plan is None or hs.shape[2] != plan.embed or not _hip_ext.attn_prefill_shape_ok_cached(T, T, plan.head_dim):
+        # one transpose of all values: up to 65535 matrices (beyond, ``_hip_ext.transpose_last2`` leaves them to torch)
+        if (plan is None or hs.shape[2] != plan.embed or bsz * plan.heads > 65535
+                or not _hip_ext.attn_prefill_shape_ok_cached(T, T, plan.head_dim)):
             return None
         return plan
 
