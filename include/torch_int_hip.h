@@ -504,7 +504,9 @@ int ti_opt_decoder_layer_prefill(const TiOptDecodeLayer* layer, void* hidden, co
  * [rows, embed] that belongs to this pass (16-byte aligned; unused with chain = 0).  chain & 2: where the output of fc2 would be
  * added to the stream by a kernel of its own (an fp16 stream, or more than 4096 rows), leave it in carry instead; chain & 1:
  * this call's first LayerNorm kernel adds what the call before left there.  Every layer but the last leaves, every layer but
- * the first adds; the additions and their order are those of the separate calls. */
+ * the first adds; the additions and their order are those of the separate calls.  A prefill with chain != 0 keeps the output of
+ * out_proj in carry too and does with less scratch: ti_opt_decoder_layer_prefill_chained_scratch_bytes(B * T, embed, ffn). */
+int64_t ti_opt_decoder_layer_prefill_chained_scratch_bytes(int64_t rows, int64_t embed, int64_t ffn);
 int ti_opt_decoder_layer_decode_chained(const TiOptDecodeLayer* layer, void* hidden, const float* mask, int8_t* k_buf,
                                         int8_t* v_buf, int64_t B, int64_t cap, int64_t S, int chain, float* carry,
                                         void* scratch, int64_t scratch_bytes, void* stream);

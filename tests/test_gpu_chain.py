@@ -89,6 +89,32 @@ def test_layers_of_different_widths(widths, bsz, T):
 
 
 @torch.no_grad()
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("bsz,T", [(2, 512), (16, 1024)])   # scratch of the stream and of the pass
+def test_a_chained_prefill_needs_hardly_more_memory_than_the_modules(bsz, T, half):
+    """A byte per token and channel more, where the scratch is not the stream's: 9 (x 1, h 4, the carry 4) against 8 (h and
+    fc2's output; x is gone by then)."""
+    lm = Int8OPTForCausalLM(OPTConfigLite(hidden_size=1024, num_hidden_layers=3, ffn_dim=4096, num_attention_heads=8, vocab_size=64,
+                                          max_position_embeddings=1024)).to(DEV)
+    model = (lm.half() if half else lm).model
+    ids = torch.randint(2, 64, (bsz, T), device=DEV)
+    peak = {}
+    try:
+        for chained in (False, True):
+            Int8OPTDecoderLayer.prefill_in_one_call = chained
+            print("memory", bsz, T, half, chained, flush=True)
+            model(ids, use_cache=True)   # the stream's kept buffers are there
+            torch.cuda.synchronize()
+            torch.cuda.reset_peak_memory_stats()
+            before = torch.cuda.memory_allocated()
+            model(ids, use_cache=True)
+            peak[chained] = torch.cuda.max_memory_allocated() - before
+    finally:
+        Int8OPTDecoderLayer.prefill_in_one_call = True
+    assert peak[True] <= peak[False] + (bsz * T * 1024 if bsz * T > 4096 else 0)
+
+
+@torch.no_grad()
 def test_layers_handed_one_cache_keep_their_own_rows():
     g = torch.Generator().manual_seed(1)
     lm = Int8OPTForCausalLM(OPTConfigLite(hidden_size=128, num_hidden_layers=3, ffn_dim=512, num_attention_heads=2, vocab_size=64,

@@ -64,7 +64,7 @@ def test_memory_of_a_pass_fits_its_widest_layer(host_memory):
     # 304 rows of a 20480 wide layer are split over K and need a workspace; the narrow first layer needs none
     plans = [types.SimpleNamespace(embed=5120, ffn=f) for f in (512, 20480, 1024)]
     scratch, _, _, ws_bytes = _hip_ext.opt_prefill_scratch(plans, _hidden(304, 5120))
-    assert scratch.numel() >= _hip_ext._lib.ti_opt_decoder_layer_prefill_scratch_bytes(304, 5120, 20480)
+    assert scratch.numel() >= _hip_ext._lib.ti_opt_decoder_layer_prefill_chained_scratch_bytes(304, 5120, 20480)
     assert ws_bytes >= _CUDA._ws_bytes(304, 5120, 20480) > 0
     one = types.SimpleNamespace(device=types.SimpleNamespace(index=0), shape=(40, 1, 5120))
     assert _hip_ext.opt_decode_scratch(plans, one).numel() >= _hip_ext._lib.ti_opt_decoder_layer_decode_scratch_bytes(40, 5120, 20480)

@@ -861,16 +861,19 @@ int prefill_layer(const char* op, const TiOptDecodeLayer* L, void* hidden, const
   if (int rc = check_ptr(op, "v_out", v_out, 16, true)) return rc;
   if (int rc = check_ptr(op, "carry", carry, 16, chain != 0)) return rc;
   if (int rc = check_ptr(op, "scratch", scratch, 256, true)) return rc;
-  const int64_t need = ti_opt_decoder_layer_prefill_scratch_bytes(M, E, F);
+  const int64_t need = chain != 0 ? ti_opt_decoder_layer_prefill_chained_scratch_bytes(M, E, F)
+                                  : ti_opt_decoder_layer_prefill_scratch_bytes(M, E, F);
   if (scratch_bytes < need)
     return fail(TI_ERR_INVALID_ARG, "%s: scratch of %lld bytes, needs %lld", op, (long long)scratch_bytes, (long long)need);
   Carver carve{static_cast<char*>(scratch)};
   int8_t* x = carve.take<int8_t>(M * E);      // LayerNorm-quantised input of the projections, then of fc1
+  // output of out_proj, then of fc2; in a chain the carry, which nothing else uses between the first LayerNorm, which adds
+  // what the layer before left there, and fc2
+  float* f32 = chain != 0 ? carry : carve.take<float>(4 * M * E);
+  int8_t* h = reinterpret_cast<int8_t*>(carve.at);  // M * F bytes; the next three are done with when fc1 writes it
   int8_t* q = carve.take<int8_t>(M * E);      // [B, heads, T, head_dim]
   int8_t* vt = carve.take<int8_t>(M * E);     // [B * heads, head_dim, T]
   int8_t* ctx = carve.take<int8_t>(M * E);    // [B, T, embed]
-  float* f32 = carve.take<float>(4 * M * E);  // output of out_proj, then of fc2
-  int8_t* h = carve.take<int8_t>(M * F);
   const float* pending = (chain & CHAIN_ADD) && adds_later(L, M) ? carry : nullptr;
   int rc;
   if ((rc = layernorm(L, pending, hidden, L->ln1_gamma, L->ln1_beta, L->ln1_eps, x, M, stream))) return rc;
@@ -921,6 +924,12 @@ int ti_opt_decoder_layer_decode_chained(const TiOptDecodeLayer* L, void* hidden,
 int64_t ti_opt_decoder_layer_prefill_scratch_bytes(int64_t rows, int64_t embed, int64_t ffn) {
   if (rows <= 0 || embed <= 0 || ffn <= 0) return 0;
   return 4 * up256(rows * embed) + up256(4 * rows * embed) + up256(rows * ffn);
+}
+
+int64_t ti_opt_decoder_layer_prefill_chained_scratch_bytes(int64_t rows, int64_t embed, int64_t ffn) {
+  if (rows <= 0 || embed <= 0 || ffn <= 0) return 0;
+  const int64_t attention = 3 * up256(rows * embed), h = up256(rows * ffn);
+  return up256(rows * embed) + (attention > h ? attention : h);
 }
 
 int ti_opt_decoder_layer_prefill(const TiOptDecodeLayer* L, void* hidden, const float* mask, const uint8_t* mask_classes,

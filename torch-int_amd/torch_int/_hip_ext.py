@@ -111,6 +111,8 @@ _lib.ti_opt_decoder_layer_decode.argtypes = [_vp, _vp, _vp, _vp, _vp, _i64, _i64
 _lib.ti_opt_decoder_layer_decode.restype = ctypes.c_int
 _lib.ti_opt_decoder_layer_prefill_scratch_bytes.argtypes = [_i64, _i64, _i64]
 _lib.ti_opt_decoder_layer_prefill_scratch_bytes.restype = _i64
+_lib.ti_opt_decoder_layer_prefill_chained_scratch_bytes.argtypes = [_i64, _i64, _i64]
+_lib.ti_opt_decoder_layer_prefill_chained_scratch_bytes.restype = _i64
 _lib.ti_opt_decoder_layer_prefill.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp, _i64, _vp, _i64, _vp]
 _lib.ti_opt_decoder_layer_prefill.restype = ctypes.c_int
 _lib.ti_opt_decoder_layer_decode_chained.argtypes = [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, ctypes.c_int, _vp, _vp, _i64,
@@ -633,21 +635,24 @@ def opt_layer_decode(plan, hidden, mask, k_buf, v_buf, S, chain=0, carry=None, s
 
 
 def opt_prefill_scratch(plans, hidden):
-    """The scratch memory and the split-K workspace of the layers of one prefill, enough for each of ``plans``: (scratch
-    tensor, workspace tensor, its pointer, its bytes).  Held for the pass: between two of its layers another thread may
-    replace the stream's workspace.  More than 64 MiB of scratch come from torch's allocator for the pass instead of
-    staying with the stream."""
+    """The scratch memory and the split-K workspace of one layer's prefill, or of the layers of a chained one (several
+    ``plans``; they have a carry too), enough for each: (scratch tensor, workspace tensor, its pointer, its bytes).  Held
+    for the pass: between two of its layers another thread may replace the stream's workspace.  More than 64 MiB of
+    scratch come from torch's allocator for the pass instead of staying with the stream."""
     dev = hidden.device
     M = hidden.shape[0] * hidden.shape[1]
     need = need_ws = 0
+    chained = len(plans) > 1
+    scratch_bytes = (_lib.ti_opt_decoder_layer_prefill_chained_scratch_bytes if chained
+                     else _lib.ti_opt_decoder_layer_prefill_scratch_bytes)
     for E, F in {(plan.embed, plan.ffn) for plan in plans}:
-        key = (1, M, E, F)
+        key = (1 + chained, M, E, F)
         n = _layer_scratch_need.get(key)
         if n is None:
             if len(_layer_scratch_need) > 4096:
                 _layer_scratch_need.clear()
             n = _layer_scratch_need[key] = (
-                _lib.ti_opt_decoder_layer_prefill_scratch_bytes(M, E, F),
+                scratch_bytes(M, E, F),
                 max(_CUDA._ws_bytes(M, E, E), _CUDA._ws_bytes(M, F, E), _CUDA._ws_bytes(M, E, F)))
         need, need_ws = max(need, n[0]), max(need_ws, n[1])
     with _on(dev):

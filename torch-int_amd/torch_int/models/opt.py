@@ -783,25 +783,28 @@ class Int8OPTDecoder(nn.Module):
             if hit is None:
                 return None
             found.append(hit)
-        # fc2's output on its way from one layer to the next; memory of this pass, so that passes of other threads on the same
-        # stream do not meet in it
-        carry = torch.empty((hidden.shape[0] * hidden.shape[1], hidden.shape[2]), dtype=torch.float32, device=hidden.device)
+        # The carry: fc2's output on its way from one layer to the next, and in a prefill out_proj's too; memory of this pass, so
+        # that passes of other threads on the same stream do not meet in it.  A decode step on an fp32 stream has none (fc2's
+        # GEMM adds its output itself).
+        carry = None
+        if count > 1 and not (decode and hidden.dtype is torch.float32):
+            carry = torch.empty((hidden.shape[0] * hidden.shape[1], hidden.shape[2]), dtype=torch.float32, device=hidden.device)
+        links = [0 if carry is None else (_hip_ext.CHAIN_ADD if i else 0) | (_hip_ext.CHAIN_LEAVE if i + 1 < count else 0)
+                 for i in range(count)]
         cache = []
         if decode:
             rooms = [_kv_rooms(past) for past in past_key_values]
             if not all(rooms) or len({id(kv) for pair in rooms for kv in pair}) < 2 * count:
                 return None   # layers that were handed one and the same cache must not append to one buffer
             scratch = _hip_ext.opt_decode_scratch([plan for plan, _ in found], hidden)
-            for i, ((plan, S), (kk, vv)) in enumerate(zip(found, rooms)):
-                chain = (_hip_ext.CHAIN_ADD if i else 0) | (_hip_ext.CHAIN_LEAVE if i + 1 < count else 0)
+            for (plan, S), (kk, vv), chain in zip(found, rooms, links):
                 _hip_ext.opt_layer_decode(plan, hidden, mask, kk.buf, vv.buf, S, chain=chain, carry=carry, scratch=scratch)
                 kk.filled = vv.filled = S
                 if use_cache:
                     cache.append((_kv_view(kk, S), _kv_view(vv, S)))
         else:
             memory = _hip_ext.opt_prefill_scratch(found, hidden)
-            for i, plan in enumerate(found):
-                chain = (_hip_ext.CHAIN_ADD if i else 0) | (_hip_ext.CHAIN_LEAVE if i + 1 < count else 0)
+            for plan, chain in zip(found, links):
                 key, value = plan.new_cache(hidden)
                 _hip_ext.opt_layer_prefill(plan, hidden, mask, key, value, chain=chain, carry=carry, memory=memory)
                 if use_cache:
