@@ -191,3 +191,29 @@ def test_recorded_passes_keep_their_memory():
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(eager, want_more)) and all(bool((f == 7).all()) for f in filled)
         assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("where", ["instance", "class", "layer"])
+@pytest.mark.parametrize("bsz,T", [(20, 32), (3, 1376)])
+def test_replaced_forwards_are_called(bsz, T, where, monkeypatch):
+    g = torch.Generator().manual_seed(7)
+    lm = Int8OPTForCausalLM(OPTConfigLite(hidden_size=128, num_hidden_layers=2, ffn_dim=512, num_attention_heads=2, vocab_size=64,
+                                          max_position_embeddings=2048))
+    for layer in lm.model.decoder.layers:
+        randomize_int8_layer(layer, g)
+    lm = lm.to(DEV).half()
+    ids = torch.randint(2, 64, (bsz, T), generator=g).to(DEV)
+    fc1, seen = lm.model.decoder.layers[1].fc1, []
+    want = _generate(lm, ids, None, 1)
+    holder = {"instance": fc1, "class": type(fc1), "layer": Int8OPTDecoderLayer}[where]
+    stock = holder.forward
+
+    def forward(*a, **k):
+        seen.append(1)
+        return stock(*a, **k)
+    monkeypatch.setattr(holder, "forward", forward)
+    print("replaced", where, bsz, T, flush=True)
+    got = _generate(lm, ids, None, 1)
+    assert len(seen) == (2 if where == "instance" else 4)   # a prefill and a decode step of one layer or both
+    assert all(torch.equal(a.logits, b.logits) for a, b in zip(got, want))

@@ -1,0 +1,52 @@
+"""What the one-call paths of torch_int.models.opt stand for and what they leave to the modules, on the CPU (nothing is
+launched: a plan is built from CPU tensors, and the checks before a call take stand-ins)."""
+import types
+
+import pytest
+import torch
+
+from torch_int import _hip_ext
+from torch_int.models.opt import Int8OPTAttention, Int8OPTDecoderLayer
+from torch_int.nn.fused import LayerNormQ
+from torch_int.nn.linear import W8A8B8O8LinearReLU
+
+
+def _layer():
+    g = torch.Generator().manual_seed(6)
+    layer = Int8OPTDecoderLayer(128, 2, 512)
+    for lin in (layer.self_attn.q_proj, layer.self_attn.k_proj, layer.self_attn.v_proj, layer.self_attn.out_proj, layer.fc1, layer.fc2):
+        lin.weight = torch.randint(-127, 128, lin.weight.shape, dtype=torch.int8, generator=g)
+    return layer
+
+
+@pytest.mark.parametrize("name", ["self_attn", "fc1", "fc2", "self_attn_layer_norm", "final_layer_norm", "self_attn.q_proj",
+                                  "self_attn.out_proj", "self_attn.qk_bmm"])
+@pytest.mark.parametrize("native", [True, False])
+def test_a_forward_of_a_modules_own_is_not_passed_by(name, native, monkeypatch):
+    """The plan behind the one-call paths (CPU tensors do for building it) does not stand for a layer one of whose modules has
+    had its forward replaced, and does again once it is taken back."""
+    if not native:
+        monkeypatch.setattr(_hip_ext, "plan_current", _hip_ext._plan_current)
+    layer, dev = _layer(), torch.device("cpu")
+    mod = layer.get_submodule(name)
+    assert layer._decode_plan(False, dev) is not None
+    mod.forward = lambda *a, **k: None
+    assert layer._decode_plan(False, dev) is None and layer._decode_plan(False, dev) is None
+    del mod.forward
+    assert layer._decode_plan(False, dev) is not None
+    mod.forward = lambda *a, **k: None   # ... also where no plan was there before
+    del layer.__dict__["_ti_decode_plan"]
+    assert layer._decode_plan(False, dev) is None
+    del mod.forward
+    hook = mod.register_forward_hook(lambda *a: None)
+    assert layer._decode_plan(False, dev) is None
+    hook.remove()
+    assert layer._decode_plan(False, dev) is not None
+
+
+@pytest.mark.parametrize("cls", [Int8OPTAttention, LayerNormQ, W8A8B8O8LinearReLU])
+def test_a_forward_replaced_on_a_class_is_not_passed_by(cls, monkeypatch):
+    stream = types.SimpleNamespace(is_cuda=True, is_contiguous=lambda: True, dtype=torch.float32)
+    assert Int8OPTDecoderLayer._one_call_tensors(stream, None) == (True, None)
+    monkeypatch.setattr(cls, "forward", lambda *a, **k: None)
+    assert Int8OPTDecoderLayer._one_call_tensors(stream, None)[0] is False

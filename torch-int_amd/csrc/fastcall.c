@@ -253,10 +253,10 @@ static int still_held(PyObject* t, Py_ssize_t size) {
 
 /* plan_current(sources, modules) -> bool.  sources: tuple of (dict, name, tensor, version): every dict still holds that
  * tensor under that name and nothing has written to it since; modules: tuple of (dict, name, module): likewise, and the
- * module has no forward hooks. */
+ * module has no forward hooks and no `forward` of its own. */
 static PyObject* fc_plan_current(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   (void)self;
-  static PyObject *s_version, *s_hooks, *s_pre;
+  static PyObject *s_version, *s_hooks, *s_pre, *s_forward;
   if (n != 2 || !PyTuple_Check(a[0]) || !PyTuple_Check(a[1])) {
     PyErr_SetString(PyExc_TypeError, "plan_current expects two tuples");
     return NULL;
@@ -265,7 +265,8 @@ static PyObject* fc_plan_current(PyObject* self, PyObject* const* a, Py_ssize_t 
     s_version = PyUnicode_InternFromString("_version");
     s_hooks = PyUnicode_InternFromString("_forward_hooks");
     s_pre = PyUnicode_InternFromString("_forward_pre_hooks");
-    if (s_version == NULL || s_hooks == NULL || s_pre == NULL) return NULL;
+    s_forward = PyUnicode_InternFromString("forward");
+    if (s_version == NULL || s_hooks == NULL || s_pre == NULL || s_forward == NULL) return NULL;
   }
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(a[0]); ++i) {
     PyObject* t = PyTuple_GET_ITEM(a[0], i);
@@ -284,14 +285,16 @@ static PyObject* fc_plan_current(PyObject* self, PyObject* const* a, Py_ssize_t 
     const int held = still_held(t, 3);
     if (held < 0) return NULL;
     if (!held) Py_RETURN_FALSE;
-    for (int k = 0; k < 2; ++k) {
-      PyObject* hooks = PyObject_GetAttr(PyTuple_GET_ITEM(t, 2), k ? s_pre : s_hooks);
-      if (hooks == NULL) return NULL;
-      const Py_ssize_t count = PyObject_Size(hooks);
-      Py_DECREF(hooks);
-      if (count < 0) return NULL;
-      if (count > 0) Py_RETURN_FALSE;
+    PyObject* own = PyObject_GenericGetDict(PyTuple_GET_ITEM(t, 2), NULL); /* where a Module keeps its hooks */
+    if (own == NULL) return NULL;
+    int plain = PyDict_GetItemWithError(own, s_forward) == NULL && !PyErr_Occurred();
+    for (int k = 0; k < 2 && plain; ++k) {
+      PyObject* hooks = PyDict_GetItemWithError(own, k ? s_pre : s_hooks);
+      plain = hooks != NULL && PyObject_Size(hooks) == 0;
     }
+    Py_DECREF(own);
+    if (PyErr_Occurred()) return NULL;
+    if (!plain) Py_RETURN_FALSE;
   }
   Py_RETURN_TRUE;
 }

@@ -684,13 +684,13 @@ def _plan_current(sources, modules):
         if holder.get(name) is not tensor or tensor._version != version:
             return False
     for holder, name, mod in modules:
-        if holder.get(name) is not mod or mod._forward_hooks or mod._forward_pre_hooks:
+        if holder.get(name) is not mod or mod._forward_hooks or mod._forward_pre_hooks or "forward" in mod.__dict__:
             return False
     return True
 
 
 #: (sources, modules) -> bool: every (dict, name, tensor, version) and (dict, name, module) of a plan still holds, and no module
-#: has a forward hook (which wants to see that module's call)
+#: has a forward hook (which wants to see that module's call) or a ``forward`` of its own
 plan_current = getattr(_CUDA._fast, "plan_current", None) or _plan_current
 
 

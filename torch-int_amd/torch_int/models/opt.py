@@ -521,8 +521,9 @@ class Int8OPTDecoderLayer(nn.Module):
         has been replaced or written to; None when the layer is not the stock int8 block on ``device``."""
         plan = self.__dict__.get("_ti_decode_plan")
         if plan is None or plan.half != half or plan.device != device or not _hip_ext.plan_current(plan.sources, plan.modules):
-            if plan is not None and any(m._forward_hooks or m._forward_pre_hooks for _, _, m in plan.modules):
-                return None   # a hook on a sub-module wants to see that module's call
+            if plan is not None and any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__
+                                        for _, _, m in plan.modules):
+                return None   # a hook on a sub-module, or a forward that replaces its own, wants to see that module's call
             plan = self.__dict__["_ti_decode_plan"] = _DecodePlan.build(self, half, device)
             if not _hip_ext.plan_current(plan.sources, plan.modules):
                 return None
@@ -547,6 +548,9 @@ class Int8OPTDecoderLayer(nn.Module):
     @staticmethod
     def _one_call_tensors(hs, attention_mask):
         """(whether the residual stream and the mask qualify for the C calls, the mask as they read it)."""
+        for cls, forward in _STOCK_FORWARDS:
+            if cls.forward is not forward:   # replaced for all modules of that class
+                return False, None
         if not (hs.is_cuda and hs.is_contiguous() and (hs.dtype is torch.float32 or hs.dtype is torch.float16)):
             return False, None
         if attention_mask is None:
@@ -645,6 +649,13 @@ class Int8OPTDecoderLayer(nn.Module):
         if use_cache:
             outputs += (present,)
         return outputs
+
+
+#: the calls that a layer's one C call stands for, as their classes define them; the chain stands for the layer's own too
+_STOCK_FORWARDS = tuple((cls, cls.forward) for cls in (
+    Int8OPTAttention, LayerNormQ, W8A8B8O8Linear, W8A8B8O8LinearReLU, W8A8BFP32OFP32Linear, BMM_S8T_S8N_F32T,
+    BMM_S8T_S8N_S8T))
+_STOCK_LAYER_FORWARD = Int8OPTDecoderLayer.forward
 
 
 # --------------------------------------------------------------------------------------
@@ -768,7 +779,7 @@ class Int8OPTDecoder(nn.Module):
         if count == 0 or (hidden.shape[1] != 1 or hidden.shape[0] > 64 if decode else hidden.shape[1] <= 16):
             return None
         ok, mask = Int8OPTDecoderLayer._one_call_tensors(hidden, attention_mask)
-        if not ok or (decode and len(past_key_values) != count):
+        if not ok or Int8OPTDecoderLayer.forward is not _STOCK_LAYER_FORWARD or (decode and len(past_key_values) != count):
             return None
         found = []
         for i, layer in enumerate(layers):
