@@ -383,3 +383,21 @@ def test_prefill_of_more_than_65535_sequences_times_heads_is_refused_before_any_
     for bsz, message in ((1638, b"gamma is NULL"), (1639, b"65535 sequences x heads")):
         assert call(ctypes.addressof(st), p, None, None, p, p, bsz, 32, 0, None, p, 1 << 40, None, 0, None) == 1
         assert message in C._lib.ti_last_error()
+
+
+def test_rows_slices_fit_the_devices_xcds():
+    # the workgroups of all slices of a strip run on one XCD (an eighth of the compute units, one workgroup each at least):
+    # a device of few compute units takes no more slices than that, where the group count would come out as zero
+    import torch_int._CUDA as C
+    lib = ctypes.CDLL(C.LIB_PATH)
+    pick = lib.ti_selftest_rows_pick
+    pick.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
+    tiling = ctypes.c_int(0)
+    sliced = 0
+    for cus in (1, 7, 8, 16, 24, 32, 38, 64, 128, 228, 256, 304):
+        for M in (2, 16, 17, 64):
+            for K in range(768, 32768, 128):
+                slices = pick(M, 2048, K, cus, ctypes.byref(tiling))
+                assert (slices == 0) == (tiling.value == 0) and slices <= cus // 8, (cus, M, K, slices)
+                sliced += slices > 1
+    assert sliced > 0 and pick(17, 2048, 25600, 256, ctypes.byref(tiling)) == 5

@@ -449,6 +449,9 @@ int ti_selftest_fused_slot(int64_t* table, uint32_t* live_mask, int cap, int64_t
                              busy_mask, fresh);
 }
 
+int ti_selftest_rows_pick(int64_t M, int64_t N, int64_t K, int cus, int* tiling) {
+  return rows_pick_for_test(M, N, K, cus, tiling);
+}
 int ti_selftest_rows_slot(int64_t* table, signed char* state, int cap, int64_t stream, int* fresh) {
   return rows_slot_for_test(reinterpret_cast<long long*>(table), state, cap, stream, fresh);
 }

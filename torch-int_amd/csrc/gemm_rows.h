@@ -413,7 +413,7 @@ struct RowsPick {
   int tiling;
   int slices;
 };
-static inline RowsPick rows_pick(long long M, long long N, long long K) {
+static inline RowsPick rows_pick(long long M, long long N, long long K, int cus = num_cus()) {
   if (M < 1 || M > TI_ROWS_MAX_M || N < 1 || K < 768 || K > (1 << 20)) return {ROWS_NONE, 1};
   RowsPick pick{ROWS_NONE, 1};
   if (K == 4096) pick = {ROWS_F, 1};
@@ -425,10 +425,11 @@ static inline RowsPick rows_pick(long long M, long long N, long long K) {
   else if (K % 1024 == 0) pick = {ROWS_B, (int)(K / 1024)};
   else if (K % 768 == 0) pick = {ROWS_E, (int)(K / 768)};
   else return {ROWS_NONE, 1};
-  // The parked tiles of all slices stay a fraction of the weights; an XCD has room for one workgroup of every slice; the
-  // placement words of the groups, 64 bytes apart, fit a stream's block of 4096; only whole strips are parked.
+  if (cus / 8 < pick.slices) return {ROWS_NONE, 1};  // an XCD has room for one workgroup of every slice
+  // The parked tiles of all slices stay a fraction of the weights; the placement words of the groups, 64 bytes apart,
+  // fit a stream's block of 4096; only whole strips are parked.
   if (pick.slices > 1 &&
-      (pick.slices > 16 || 2 * num_cus() / pick.slices > 256 || 8 * pick.slices * M > K || N % 16 != 0))
+      (pick.slices > 16 || 2 * cus / pick.slices > 256 || 8 * pick.slices * M > K || N % 16 != 0))
     return {ROWS_NONE, 1};
   return pick;
 }

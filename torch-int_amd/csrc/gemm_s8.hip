@@ -373,6 +373,13 @@ int rows_split_prepare(hipStream_t stream, GemmParams& q, void** park) {
   return 1;
 }
 
+// CPU-testable face of rows_pick: slices (0 = the kernel does not take the shape) on a device of `cus` compute units.
+int rows_pick_for_test(long long M, long long N, long long K, int cus, int* tiling) {
+  const RowsPick pick = rows_pick(M, N, K, cus);
+  *tiling = pick.tiling;
+  return pick.tiling == ROWS_NONE ? 0 : pick.slices;
+}
+
 // CPU-testable face of pick_rows_slot: streams are plain integers, state[i] != 0 = slot i is taken; takes the slot.
 int rows_slot_for_test(long long* table, signed char* state, int cap, long long stream, int* fresh) {
   bool f = false;

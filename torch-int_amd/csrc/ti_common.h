@@ -250,6 +250,7 @@ int fused_split_faulted();                 // 1 = a one-launch split-K on the cu
 int fused_flag_action(int state, int flag, bool enabled, long long counters, long long max_counters);
 int fused_slot_for_test(long long* table, unsigned* live_mask, int cap, long long stream, unsigned busy_mask, int* fresh);
 int set_fused_split(int enable);  // one-launch split-K on (1) / off (0) / unchanged (-1); returns the previous setting
+int rows_pick_for_test(long long M, long long N, long long K, int cus, int* tiling);
 int rows_slot_for_test(long long* table, signed char* state, int cap, long long stream, int* fresh);
 int placement_of(const volatile int* words);
 int last_rows(int* tiling, int* slices);
