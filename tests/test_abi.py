@@ -401,3 +401,12 @@ def test_rows_slices_fit_the_devices_xcds():
                 assert (slices == 0) == (tiling.value == 0) and slices <= cus // 8, (cus, M, K, slices)
                 sliced += slices > 1
     assert sliced > 0 and pick(17, 2048, 25600, 256, ctypes.byref(tiling)) == 5
+
+
+@pytest.mark.parametrize("M,N,K,slices", [(800, 2560, 10240, 0), (770, 6400, 5120, 0), (480, 12800, 5120, 0), (272, 3200, 20480, 4),
+                                          (300, 5120, 20480, 4), (258, 10240, 10240, 2), (160, 20480, 5120, 2)])
+def test_square_split_tiles_only_where_they_are_ahead(M, N, K, slices):
+    # 800x2560x10240 and 770x6400x5120 run unsplit on other tiles (no workspace), 272x3200x20480 in four slices on 128x160 ones
+    # where 160x160 tiles would make five; the last three are ahead on them
+    import torch_int._CUDA as C
+    assert C._lib.ti_linear_workspace_bytes(M, N, K) == slices * M * N * 4

@@ -2276,8 +2276,12 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmParams p, const 
 // 160x160 tiles (four waves of 80x80, 10 fragment reads per 25 MFMAs; raw-int32 slices only) for the row counts that they
 // cover with fewer padded rows than 128-row tiles do: 129 to 160, 257 to 320, 385 to 480, 769 to 800.  257 rows on three
 // 128-row tiles multiply half as much padding as rows.  Bound by the matrix pipe and by the partial tiles' way through the
-// last-level cache, cold weights, us: 257x5120x20480 57.3 -> 48.7, 300x5120x20480 59.1 -> 54.8, 320x5120x20480 60.3 -> 58.8.  Priced
-// at 0.36 us per 64-byte step they are not taken at 5120x5120 or 20480x5120, where few rows of tiles fill the chip anyway.
+// last-level cache, cold weights, us: 257x5120x20480 57.3 -> 48.7, 300x5120x20480 59.1 -> 54.8, 320x5120x20480 60.3 -> 58.8.
+// The prices come out some 6 % low for these tiles and 8 % high for the split ones they are up against, so they have to
+// be 15 % cheaper: of 520 shapes (widths 1280 to 20480, 129 to 800 rows) the 212 that this takes run at 0.69 to 1.06 times what
+// they would, while without it 800x2560x10240 took 44.4 us instead of 39.8 and 770x6400x5120 55.3 instead of 36.5.  One row of
+// tiles in two slices (129 to 160 rows) is priced evenly against the 256-row tiles it replaces: 130x20480x5120 0.82 times
+// their time, 160x20480x5120 0.95; with more slices 160x7680x20480 lost 13 %.
 enum SplitTile { SPLIT_128 = 0, SPLIT_256 = 1, SPLIT_256x160 = 2, SPLIT_256x288 = 3, SPLIT_128x160 = 4, SPLIT_128x288 = 5,
                  SPLIT_128x80 = 6, SPLIT_128x192 = 7, SPLIT_256x192 = 8, SPLIT_160x160 = 9 };
 // `batch` > 1: a batched product (A and B per batch); every tile count, byte count and the streaming floor scale with
@@ -2291,7 +2295,8 @@ static int choose_splits(long long M, long long N, long long K, int* tile_kind =
   const double cus = num_cus();
   const long long steps = K / PBK;
   int best = 1, best_kind = SPLIT_128;
-  double best_t = 1e30;
+  double best_t = 1e30, square_t = 1e30;
+  int square_s = 1;
   // the 128-row forms of the tall tiles first, then by size: a later candidate must be clearly faster to replace
   // an earlier one
   // (128x192 tiles: widths that 192 divides but neither 160 nor 288 nor 80 does - 12288 and 49152, the GPT-3-sized
@@ -2362,12 +2367,24 @@ static int choose_splits(long long M, long long N, long long K, int* tile_kind =
       const bool one_launch = batch == 1 && kind >= SPLIT_256x160 && !square && M % bm == 0 && s <= (kind == SPLIT_256x288 ? 2 : 4);
       if (s > 1 && one_launch) t += (double)(2 * s - 1) * M * N * 4.0 / 8.0e6 + 1.0;
       else if (s > 1) t += (double)batch * (double)(2 * s + 1) * M * N * 4.0 / 5.5e6 + 3.0;  // at 5.5 TB/s, in us
+      if (square) {  // weighed against the best of the others below
+        if (t < square_t * 0.97) {
+          square_t = t;
+          square_s = s;
+        }
+        continue;
+      }
       if (t < best_t * 0.97) {  // prefer fewer slices and the smaller tile unless the gain is clear
         best_t = t;
         best = s;
         best_kind = kind;
       }
     }
+  }
+  if (M <= 160 ? square_s == 2 && square_t < best_t : square_t < 0.85 * best_t) {
+    best_t = square_t;
+    best = square_s;
+    best_kind = SPLIT_160x160;
   }
   if (tile_kind) *tile_kind = best_kind;
   if (time_us && best_t < 1e29) *time_us = best_t;
