@@ -410,3 +410,14 @@ def test_square_split_tiles_only_where_they_are_ahead(M, N, K, slices):
     # where 160x160 tiles would make five; the last three are ahead on them
     import torch_int._CUDA as C
     assert C._lib.ti_linear_workspace_bytes(M, N, K) == slices * M * N * 4
+
+
+@pytest.mark.parametrize("M,N,K,slices", [(64, 20480, 13312, 0), (17, 9216, 13312, 0), (64, 20480, 1536, 0), (64, 5120, 11264, 0),
+                                          (24, 4096, 16384, 8), (64, 5120, 20480, 4), (48, 2560, 10240, 2), (40, 2048, 8192, 4),
+                                          (64, 4096, 4096, 1)])
+def test_rows_in_slices_only_where_they_are_ahead(M, N, K, slices):
+    # the first four took up to 2.6 times as long in slices that meet as on the kernels they had before
+    import torch_int._CUDA as C
+    pick = C._lib.ti_selftest_rows_pick
+    pick.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
+    assert pick(M, N, K, 256, ctypes.byref(ctypes.c_int(0))) == slices

@@ -402,8 +402,11 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::NW == 16 ? 4 : 2) void gemm_rows_kern
 //   F  16 waves x 256 bytes, one per CU: K == 4096
 //   G  8 waves x 384 bytes, one per CU: K % 3072 == 0
 //   H  8 waves x 448 bytes, one per CU: K % 3584 == 0
-// The longest slice that divides K comes first: slices that meet cost 2 to 2.5 us a launch (park, count, add), which only a
-// long K repays.  us, cold weights, 16 / 32 / 64 rows: 5120 x 5120 C 8.9 / 10.5 / 13.3, B in five slices 9.5 / 11.7 / 15.4;
+// A divisor of K that is a whole slice comes first (C, F, H, then A, G, D, B, E): slices that meet cost 2 to 2.5 us a launch (park,
+// count, add), which only a long K repays.  Several slices take the first tiling in that order; the pairs that are measured
+// below compare one slice with several.  A K whose first divisor makes too many slices goes to the other kernels, also where
+// another tiling would fit (36864: 18 of A, 12 of G; 49152: 24 of A, 16 of G).
+// us, cold weights, 16 / 32 / 64 rows: 5120 x 5120 C 8.9 / 10.5 / 13.3, B in five slices 9.5 / 11.7 / 15.4;
 // 4096 x 4096 F 6.3 / 7.8 / 9.7, A in two 7.2 / 8.7 / 10.5; 16384 x 4096 F 13.1 / 14.6 / 17.6, A in two 14.4 / 16.7 / 21.3 (F with 64
 // rows: 8 waves of 512 bytes, 16 waves have too few registers for the fragments and spill, 21.8); 768 x 3072 G
 // 4.6 / 5.5 / 6.8, E in four 5.1 / 5.6 / 6.5; 2048 x 2048 A 3.6 / 4.0 / 5.2, B in two 5.1 / 5.5 / 6.6.  Pieces of whole 128-byte lines where
@@ -413,7 +416,35 @@ struct RowsPick {
   int tiling;
   int slices;
 };
-static inline RowsPick rows_pick(long long M, long long N, long long K, int cus = num_cus()) {
+// Whether several slices, `pick`, beat the kernel that would run instead.  What they cost is the end: the wave that arrives
+// last adds up its tiles one after the other, four slices a round trip (64 x 20480 x 13312 in thirteen slices: 51 us of
+// weights, 100 us of that).
+static inline bool rows_slices_ahead(RowsPick pick, long long M, long long N, long long K, int problems, int cus) {
+  // waves, workgroups per CU; us per MB of weights and per round of the end, fitted to 875 shapes within 8 %
+  static constexpr struct {
+    int waves, per_cu;
+    double us_per_mb, us_per_round;
+  } cost[] = {{0, 0, 0.0, 0.0},      {4, 2, 0.148, 0.70}, {4, 2, 0.124, 0.65}, {8, 1, 0.118, 2.20}, {4, 2, 0.125, 1.95},
+              {4, 2, 0.172, 1.10},   {8, 1, 0.118, 2.00}, {8, 1, 0.123, 1.95}, {8, 1, 0.118, 2.15}};
+  const auto& c = cost[pick.tiling];
+  const long long strips = (N + 15) / 16 * problems, row_blocks = (M + 15) / 16;
+  int tile = SPLIT_128;
+  double others = -1.0;
+  (void)choose_splits(M, N, K, &tile, &others);
+  if (others <= 0.0) return true;  // no price to compare with
+  // at these few rows that model, made for more of them, is too low for 256x256 tiles and for short runs of 128x80 ones
+  if (tile == SPLIT_256) others *= 1.25;
+  else if (tile == SPLIT_128x80 && others < 14.0) others *= 1.15;
+  const long long slots = (long long)cus * c.per_cu / 8, need = (strips + 7) / 8 * pick.slices;
+  const long long groups = (need < slots ? need : slots) / pick.slices * 8;
+  const long long strips_each = (strips + groups - 1) / groups;
+  const long long rounds = (strips_each * row_blocks + c.waves - 1) / c.waves * ((pick.slices + 3) / 4);
+  // Both prices are good to some 10 %.  Of those 875 shapes (17 to 64 rows) 96 were slower than before in slices, up to 2.6 times
+  // (64 x 20480 x 13312 58.2 -> 151.4 us); of the 730 that this takes three are, by up to 8 %, the others run at 0.38 to 1.02 times.
+  return 5.6 + c.us_per_mb * N * K * problems * 1e-6 + c.us_per_round * rounds <= 0.8 * others * problems;
+}
+
+static inline RowsPick rows_pick(long long M, long long N, long long K, int cus = num_cus(), int problems = 1) {
   if (M < 1 || M > TI_ROWS_MAX_M || N < 1 || K < 768 || K > (1 << 20)) return {ROWS_NONE, 1};
   RowsPick pick{ROWS_NONE, 1};
   if (K == 4096) pick = {ROWS_F, 1};
@@ -431,6 +462,7 @@ static inline RowsPick rows_pick(long long M, long long N, long long K, int cus 
   if (pick.slices > 1 &&
       (pick.slices > 16 || 2 * cus / pick.slices > 256 || 8 * pick.slices * M > K || N % 16 != 0))
     return {ROWS_NONE, 1};
+  if (pick.slices > 1 && M > 16 && !rows_slices_ahead(pick, M, N, K, problems, cus)) return {ROWS_NONE, 1};
   return pick;
 }
 
@@ -485,7 +517,7 @@ template <int KIND, bool GROUPED>
 static int launch_rows(const GemmParams& p_in, const GemmGroup& grp, int problems, void* workspace,
                        long long workspace_bytes, hipStream_t stream) {
   if (p_in.batch != 1 || p_in.lda != p_in.K || p_in.ldb != p_in.K) return -1;
-  const RowsPick pick = rows_pick(p_in.M, p_in.N, p_in.K);
+  const RowsPick pick = rows_pick(p_in.M, p_in.N, p_in.K, num_cus(), problems);
   if (pick.tiling == ROWS_NONE) return -1;
   GemmParams p = p_in;
   p.splits = pick.slices;
