@@ -444,6 +444,25 @@ static inline bool rows_slices_ahead(RowsPick pick, long long M, long long N, lo
   return 5.6 + c.us_per_mb * N * K * problems * 1e-6 + c.us_per_round * rounds <= 0.8 * others * problems;
 }
 
+// The same up to 16 rows, where the streaming kernel (it needs K % 1024 == 0 and 256 strips) or the skinny one would run; what the
+// slices cost shows against the shortest launches and the fewest rows.  Times relative to those kernels, cold weights:
+//   B's many slices (11264, 13312) 1.08 to 1.41 against the streaming kernel, whatever the rows;
+//   A's eight and more at 448 strips and beyond 1.06 to 1.15 (7168 x 16384), at 256 and 320 strips 0.81 to 0.99;
+//   up to 4 rows at 384 strips and beyond 1.00 to 1.12 (7168 x 7168 11.2 -> 12.3 us), from K = 20480 on 0.85 to 0.96;
+//   5 to 8 rows at 384 to 448 strips of up to 7168 bytes 1.01 to 1.05;
+//   E's slices (a K that 1024 does not divide) on 64 strips and more 0.93 to 1.45 against the skinny kernel, 1.18 on average (8 x
+//   4096 x 1536 4.4 -> 6.2 us), K = 1536 on fewer strips too; it runs a group problem by problem, which takes twice as long.
+//   Longer K on fewer than 64 strips keeps them (8 x 768 x 2304 4.6 -> 5.4 us).
+static inline bool few_rows_slices_ahead(RowsPick pick, long long M, long long N, long long K, int problems) {
+  const long long strips = (N + 15) / 16 * problems;
+  if (K % SBK != 0 || strips < 256) return pick.tiling != ROWS_E || problems > 1 || (strips < 64 && K > 1536);
+  if (pick.tiling == ROWS_B) return false;
+  if (strips <= 320) return true;
+  if (pick.tiling == ROWS_A && pick.slices >= 8) return false;
+  if (M <= 4) return K >= 20480;
+  return M > 8 || K > 7168 || strips > 512;
+}
+
 static inline RowsPick rows_pick(long long M, long long N, long long K, int cus = num_cus(), int problems = 1) {
   if (M < 1 || M > TI_ROWS_MAX_M || N < 1 || K < 768 || K > (1 << 20)) return {ROWS_NONE, 1};
   RowsPick pick{ROWS_NONE, 1};
@@ -462,7 +481,9 @@ static inline RowsPick rows_pick(long long M, long long N, long long K, int cus 
   if (pick.slices > 1 &&
       (pick.slices > 16 || 2 * cus / pick.slices > 256 || 8 * pick.slices * M > K || N % 16 != 0))
     return {ROWS_NONE, 1};
-  if (pick.slices > 1 && M > 16 && !rows_slices_ahead(pick, M, N, K, problems, cus)) return {ROWS_NONE, 1};
+  if (pick.slices > 1 && !(M <= 16 ? few_rows_slices_ahead(pick, M, N, K, problems)
+                                   : rows_slices_ahead(pick, M, N, K, problems, cus)))
+    return {ROWS_NONE, 1};
   return pick;
 }
 
