@@ -55,3 +55,25 @@ def test_one_new_token_is_exact(B, H, d, S, masked):
     assert torch.equal(kd.cpu().view(B * H, cap, d), k_ref) and torch.equal(vd.cpu().view(B * H, cap, d), v_ref)
     again, none = X.decode_attention(*args, a_qk, a_pv)
     assert none is None and torch.equal(again.cpu(), ctx)
+
+
+@pytest.mark.parametrize("d,heads", [(128, 256), (128, 260), (80, 260)])   # the rule for a length on the device: 256 heads, d > 96
+def test_a_length_on_the_device_gives_the_values_of_one_on_the_host(d, heads):
+    import torch_int._hip_ext as X
+    g = torch.Generator(device=DEV).manual_seed(d + heads)
+    cap, bound = 1056, 1049
+
+    def s8(*shape):
+        return torch.randint(-127, 128, shape, dtype=torch.int8, device=DEV, generator=g)
+
+    q, kn, vn = (s8(heads // 4, 4, 1, d) for _ in range(3))
+    kb, vb = s8(heads // 4, 4, cap, d), s8(heads // 4, 4, cap, d)
+    length = torch.zeros(1, dtype=torch.int32, device=DEV)
+    for n in (1, 20, 513, bound):
+        print("length on the device", d, heads, n, flush=True)
+        length.fill_(n)
+        caches = [(kb.clone(), vb.clone()) for _ in range(2)]
+        got = X.decode_attention_devlen(q, kn, vn, *caches[0], length, bound, 3e-4, 4e-3)
+        want, _ = X.decode_attention(q, kn, vn, *caches[1], n - 1, None, 3e-4, 4e-3)
+        assert torch.equal(got, want)
+        assert torch.equal(caches[0][0], caches[1][0]) and torch.equal(caches[0][1], caches[1][1])

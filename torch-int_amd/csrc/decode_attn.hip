@@ -491,7 +491,9 @@ int launch_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_
   // itself (904 positions: 32 heads 7.3 against 8.0, 128 heads 10.2 / 10.4, 768 heads 38.0 / 32.1).  Beyond 128 groups only one
   // workgroup fits a CU, which leaves it without loads during the softmax: with more heads than two rounds of 256 the
   // streaming form, several small workgroups per CU, is level or ahead (1400 positions, 768 heads: 51.7 against 52.5; 128
-  // heads 29.1 / 13.8).
+  // heads 29.1 / 13.8).  So it is at head size 128 with more than one round of heads where the kernel reads the length and S is
+  // only its bound: 320 heads, bound 2048, length 20 / 512 / 1024 / 2048 9.1 / 13.7 / 25.4 / 44.9 us, streaming 5.6 / 13.0 /
+  // 25.0 / 44.4 (a length the host knows, 300 heads x 2040: 40.3, streaming 44.0; head size 80 keeps it, 18.0 against 25.9 at 1024).
   const long long groups = (S + 64 / (lanes_d / 16) - 1) / (64 / (lanes_d / 16));
 #define TI_DA1(DD, NW, NI)                                                                                             \
   do {                                                                                                                 \
@@ -523,7 +525,7 @@ int launch_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_
       hipLaunchKernelGGL((decode_attn_kernel<TQ, DD, NI, true>), grid, block, lds, stream, q, k_new, v_new, k_buf,     \
                          v_buf, mask, ctx, probs_out, (int)T, (int)S, cap, (int)heads, alpha_qk, alpha_pv, s_dev, (int)D); \
   } while (0)
-  const bool one = T == 1 && (groups <= 128 || (groups <= 256 && BH <= 512));
+  const bool one = T == 1 && (groups <= 128 || (groups <= 256 && BH <= (s_dev != nullptr && D > 96 ? 256 : 512)));
   // caches of at most 20 row groups per lane (640 positions at head size 128) with two query rows take
   // the variant that issues all loads up front
   const bool resident = T == 2 && S <= 20 * 4 * (64 / (lanes_d / 16));
