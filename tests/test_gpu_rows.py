@@ -12,29 +12,43 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 # (M, N, K): tiling and slices
-SHAPES = [
-    (17, 16384, 2048),   # A, one slice
-    (33, 8192, 4096),    # A, two
-    (64, 4096, 8192),    # A, four
-    (2, 2048, 1024),     # B, one
-    (5, 50, 1024),       # B, a width inside one group of strips that ends inside a strip
-    (16, 4099, 1024),    # B, a width that no vector store fits
-    (64, 2064, 3072),    # B, three slices, a strip past a multiple of 64
-    (48, 8192, 5120),    # C, one
-    (16, 5120, 10240),   # C, two
-    (40, 2560, 2560),    # D, one
-    (3, 640, 7680),      # D, three
-    (31, 768, 768),      # E, one
-    (8, 784, 2304),      # E, three
-    (49, 16, 768),       # one strip
-]
+SHAPES = {
+    (17, 16384, 2048): "A1",
+    (33, 8192, 4096): "F1",
+    (64, 4096, 8192): "A4",
+    (2, 2048, 1024): "B1",
+    (5, 50, 1024): "B1",       # a width inside one group of strips that ends inside a strip
+    (16, 4099, 1024): "B1",    # a width that no vector store fits
+    (64, 2064, 3072): "G1",    # a strip past a multiple of 64
+    (48, 8192, 5120): "C1",
+    (16, 5120, 10240): "C2",
+    (40, 2560, 2560): "D1",
+    (3, 640, 7680): "D3",
+    (31, 768, 768): "E1",
+    (8, 784, 2304): "E3",
+    (49, 16, 768): "E1",       # one strip
+    (64, 1024, 4096): "F1",    # 49 to 64 rows: eight waves instead of sixteen
+    (24, 5120, 20480): "C4",
+    (20, 1040, 3584): "H1",
+    (33, 1024, 7168): "H2",
+    (48, 1024, 9216): "G3",
+    (17, 1024, 11264): "B11",
+}
+
+
+def _last():
+    """The weight-streaming kernel's last launch: (form, tiling and slices)."""
+    import torch_int._CUDA as C
+    t, s = ctypes.c_int(0), ctypes.c_int(0)
+    form = C._lib.ti_last_rows(ctypes.byref(t), ctypes.byref(s))
+    return form, " ABCDEFGH"[t.value].strip() + str(s.value)
 
 
 def _s8(g, *shape):
     return torch.randint(-127, 128, shape, dtype=torch.int8, generator=g)
 
 
-@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("M,N,K", list(SHAPES))
 def test_every_epilogue_is_exact(M, N, K):
     import torch_int._CUDA as C
     import torch_int._hip_ext as X
@@ -58,6 +72,7 @@ def test_every_epilogue_is_exact(M, N, K):
         print("rows epilogue", i, M, N, K, flush=True)
         outs = [run() for _ in range(2)]
         assert C._lib.ti_last_kernel().decode() == ("stream" if M <= 16 else "mid_stream")
+        assert _last() == (1 if SHAPES[M, N, K][1:] == "1" else 2, SHAPES[M, N, K])
         for o in outs:   # twice: the arrival counters and the accumulation buffers are left as they were found
             assert torch.equal(o.cpu(), want), (i, M, N, K)
     before = C._lib.ti_fused_splitk(0)   # several slices: the two-launch form, or another kernel where there is no workspace
@@ -69,6 +84,24 @@ def test_every_epilogue_is_exact(M, N, K):
     if d:
         want = orc.epi_b8_o8(acc, b8, al, be).view(1, M, N // d, d).transpose(1, 2)
         assert torch.equal(X.linear_a8_w8_b8_o8_heads(xd, wd, b8d, al, be, 1, M, N // d, d).cpu(), want)
+
+
+@pytest.mark.parametrize("N,K,want", [(272, 768, "E1"), (272, 1024, "B1"), (272, 2048, "A1"), (272, 2560, "D1"), (272, 3072, "G1"),
+                                      (272, 3584, "H1"), (272, 4096, "F1"), (272, 5120, "C1"), (272, 2304, "E3"),
+                                      (272, 6144, "A3"), (272, 7168, "H2"), (272, 7680, "D3"), (272, 9216, "G3"),
+                                      (272, 11264, "B11"), (272, 20480, "C4")])
+def test_every_tiling_at_every_number_of_row_blocks(N, K, want):
+    """One to four blocks of 16 rows, the last one full and with a single row: a kernel of its own each."""
+    import torch_int._CUDA as C
+    g = torch.Generator().manual_seed(N + K)
+    x, w, b = _s8(g, 64, K), _s8(g, N, K), _s8(g, N)
+    ref = orc.linear_a8_w8_b8_o8(x, w, b, 3e-4, 0.02, acc_fn=orc.gemm_acc_torch)
+    xd, wd, bd = x.to(DEV), w.to(DEV), b.to(DEV)
+    for M in (9, 16, 17, 32, 33, 48, 49, 64):
+        print("rows tiling", want, M, N, K, flush=True)
+        for _ in range(2):
+            assert torch.equal(C.linear_a8_w8_b8_o8(xd[:M], wd, bd, 3e-4, 0.02).cpu(), ref[:M]), M
+        assert _last() == (1 if want[1:] == "1" else 2, want), M
 
 
 @pytest.mark.parametrize("M,N,K", [(24, 4096, 4096), (16, 1024, 4096), (7, 2560, 2560), (48, 768, 768), (2, 100, 1024)])
@@ -87,10 +120,10 @@ def test_groups_are_exact(M, N, K):
 
 @torch.no_grad()
 @pytest.mark.parametrize("half", [False, True])
-@pytest.mark.parametrize("D,H,bsz", [(768, 12, 17), (1024, 8, 64), (320, 4, 33)])
+@pytest.mark.parametrize("D,H,bsz", [(768, 12, 17), (1024, 8, 64), (320, 4, 33), (2048, 16, 24)])
 def test_decode_step_of_a_large_batch_from_one_call(D, H, bsz, half):
     """17 to 64 sequences, one new token each: residual stream and caches of the one C call bit for bit those of the
-    modules, with the projections grouped (768), sliced (fc2 of 1024) and on the split-K kernels (320)."""
+    modules, with the projections grouped (768, 1024, 2048), fc2 in four slices (2048) and on the split-K kernels (320)."""
     from test_gpu_models import causal_mask, randomize_int8_layer
     from torch_int.models.opt import Int8OPTDecoderLayer
     g = torch.Generator().manual_seed(D + bsz)
@@ -108,6 +141,8 @@ def test_decode_step_of_a_large_batch_from_one_call(D, H, bsz, half):
             print("rows decode", D, bsz, half, step, one_call, flush=True)
             res[one_call] = layer(x.clone(), past_key_value=caches[one_call], use_cache=True)
             caches[one_call] = res[one_call][-1]
+            if one_call and not (half or D == 320):   # fc2 comes last
+                assert _last() == {768: (1, "G1"), 1024: (1, "F1"), 2048: (2, "A4")}[D]
         assert torch.equal(res[True][0], res[False][0])
         for a, b in zip(caches[True], caches[False]):
             assert torch.equal(a, b)
@@ -149,9 +184,7 @@ def _sliced(M, N, K, seed):
 
 
 def _form():
-    import torch_int._CUDA as C
-    t, s = ctypes.c_int(0), ctypes.c_int(0)
-    return C._lib.ti_last_rows(ctypes.byref(t), ctypes.byref(s))
+    return _last()[0]
 
 
 @pytest.mark.parametrize("M,recorded", [(8, 0), (24, 3)])
