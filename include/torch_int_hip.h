@@ -124,9 +124,9 @@ int ti_fused_splitk_faulted(void);
 int ti_selftest_fused_flag_action(int state, int flag, int enabled, int64_t counters, int64_t max_counters);
 int ti_selftest_fused_slot(int64_t* table, uint32_t* live_mask, int cap, int64_t stream, uint32_t busy_mask,
                            int* fresh);
-/* ... and of the weight-streaming kernel's: the block of `stream` in a table of `cap` (state[i] != 0 = taken), which is taken;
- * what 256 placement words say (1 = eight XCDs in turn, -1 = another placement, 0 = a word is still -1). */
-/* (and its tiling of a shape on a device of `cus` compute units: slices, 0 = it does not take the shape) */
+/* ... and of the weight-streaming kernel's: its tiling of a shape on a device of `cus` compute units (returns the slices, 0 = it
+ * does not take the shape); the block of `stream` in a table of `cap` (state[i] != 0 = taken), which is taken; what 256
+ * placement words say (1 = eight XCDs in turn, -1 = another placement, 0 = a word is still -1). */
 int ti_selftest_rows_pick(int64_t M, int64_t N, int64_t K, int cus, int* tiling);
 int ti_selftest_rows_slot(int64_t* table, signed char* state, int cap, int64_t stream, int* fresh);
 int ti_selftest_placement(const int32_t* words);

@@ -462,8 +462,9 @@ int gemm_group_is_one_launch(long long M, long long N, long long K, int count) {
   return group_prefill_tile(M, N, K, count) != 0 ? 1 : 0;
 }
 
-// q/k/v-style group of s8 linears.  Decode shapes (M <= 16, K % 1024 == 0, enough strips) take one launch
-// of the streaming kernel over all the weights; anything else runs problem by problem.
+// q/k/v-style group of s8 linears.  One launch over all the weights: one row on the dot-product kernel, up to 64 rows on the
+// weight-streaming kernel of gemm_rows.h where its tilings divide K, else up to 16 rows on the streaming kernel (K % 1024 == 0),
+// and prefills whose tiles group_prefill_tile finds; anything else runs problem by problem.
 int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStream_t stream, void* workspace,
                          long long workspace_bytes) {
   constexpr int KIND = EPI_S8_BIAS;
