@@ -219,6 +219,49 @@ def test_graphs_of_sliced_linears_replay_on_two_streams_beside_eager_work(M, rec
         assert all(torch.equal(o, want) for o in outs[0] + outs[1] + eager)
 
 
+def test_a_first_call_on_a_stream_while_another_thread_records():
+    """A thread that records a graph does not disturb another one's linears on a stream that has no block of state yet, nor do
+    they disturb the recording."""
+    import threading
+    import torch_int._CUDA as C
+    cases = []
+    for M, N, K in ((8, 2560, 10240), (40, 2048, 8192)):
+        g = torch.Generator().manual_seed(M)
+        x, w, b = _s8(g, M, K).to(DEV), _s8(g, N, K).to(DEV), _s8(g, N).to(DEV)
+        need = C._lib.ti_linear_workspace_bytes(M, N, K)
+        cases.append((M, N, K, x, w, b, torch.empty((M, N), dtype=torch.int8, device=DEV), need,
+                      torch.empty(max(need, 1), dtype=torch.uint8, device=DEV), C.linear_a8_w8_b8_o8(x, w, b, 3e-4, 0.02)))
+    h = ctypes.c_void_p()
+    assert C._lib.hipStreamCreate(ctypes.byref(h)) == 0
+    recording, done, status = threading.Event(), threading.Event(), []
+
+    def other():
+        recording.wait(60)
+        for M, N, K, x, w, b, out, need, ws, _ in cases:
+            status.append(C._lib.ti_linear_a8_w8_b8_o8(x.data_ptr(), w.data_ptr(), b.data_ptr(), out.data_ptr(), M, N, K, 3e-4, 0.02,
+                                                       ws.data_ptr() if need else None, need, h.value))
+        done.set()
+
+    thread = threading.Thread(target=other)
+    thread.start()
+    graph, y = torch.cuda.CUDAGraph(), torch.ones(64, device=DEV)
+    torch.cuda.synchronize()
+    print("recording beside another thread", flush=True)
+    with torch.cuda.graph(graph):
+        y.add_(1)
+        recording.set()
+        assert done.wait(60)
+        y.add_(1)
+    thread.join()
+    torch.cuda.synchronize()
+    assert status == [0, 0]
+    assert all(torch.equal(c[6], c[9]) for c in cases)
+    for turn in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, torch.full_like(y, 3 + 2 * turn))
+
+
 def test_forty_streams_of_sliced_linears():
     """More streams than there are blocks of state, all with work queued at once, twice over: exact on every one."""
     import torch_int._CUDA as C

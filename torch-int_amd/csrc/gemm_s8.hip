@@ -126,6 +126,16 @@ static bool fused_enabled() { return set_fused_split(-1) != 0; }
 static thread_local bool g_fused_may_probe = true;
 void allow_fused_split_probe(bool allow) { g_fused_may_probe = allow; }
 
+// While a thread records a graph in the global mode (torch's default), a query, a wait or an allocation by any other thread is
+// an error there and here: it ends the recording.  Ours concern neither, so they are made in the relaxed mode.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  RelaxedCapture(const RelaxedCapture&) = delete;
+  RelaxedCapture& operator=(const RelaxedCapture&) = delete;
+};
+
 // What 256 probe words say: 1 = one XCC per residue class of the workgroup id mod 8, eight different ones; -1 = another
 // placement; 0 = not all of them are there yet.  Free of HIP calls so that it can be tested on the CPU.
 int placement_of(const volatile int* words) {
@@ -148,12 +158,14 @@ static bool start_probe(FusedDevice& d, int at, hipStream_t stream) {
   return hipGetLastError() == hipSuccess;
 }
 static bool probe_placement(FusedDevice& d, hipStream_t stream) {  // ... and waits for it
+  RelaxedCapture relaxed;
   return start_probe(d, 1, stream) && hipStreamSynchronize(stream) == hipSuccess && placement_of(d.host_words + 1) == 1;
 }
 
 // Host words and device addresses of the current device, once.
 static bool fused_memory(FusedDevice& d) {
   if (d.host_words != nullptr) return d.rows_park != nullptr;
+  RelaxedCapture relaxed;
   void *arrivals = nullptr, *rows = nullptr, *park = nullptr;
   int* words = nullptr;
   if (hipGetSymbolAddress(&arrivals, HIP_SYMBOL(g_fused_arrivals)) != hipSuccess || arrivals == nullptr) return false;
@@ -296,7 +308,10 @@ int fused_split_prepare(hipStream_t stream, long long counters, GemmParams& q) {
   }
   bool fresh = false;
   const int slot = pick_stream_slot(d.streams, d.live, kFusedStreams, stream,
-                                    [&](int i) { return d.pinned[i] || hipStreamQuery(d.streams[i]) == hipErrorNotReady; },
+                                    [&](int i) {
+                                      RelaxedCapture relaxed;
+                                      return d.pinned[i] || hipStreamQuery(d.streams[i]) == hipErrorNotReady;
+                                    },
                                     fresh);
   (void)hipGetLastError();  // a query of a destroyed stream leaves an error behind; the slot counts as idle
   if (slot < 0) return 0;
@@ -347,12 +362,16 @@ int rows_split_prepare(hipStream_t stream, GemmParams& q, void** park) {
   // hipStreamPerThread is one handle for a stream of every thread
   if (action <= 0 || stream == hipStreamPerThread || is_capturing(stream)) return 0;
   if (d.host_words == nullptr && !g_fused_may_probe) return 0;  // the first use on a device allocates host memory
-  if (!fused_memory(d)) return 0;
+  if (!fused_memory(d)) {
+    (void)hipGetLastError();  // not the launch's
+    return 0;
+  }
   bool fresh = false;
   const int slot = pick_rows_slot(d.rows_streams, d.rows_state, kRowsStreams, stream, fresh);
   if (slot < 0) return 0;
   const int words = 1 + (1 + slot) * kProbeWords;
   if (fresh) {
+    RelaxedCapture relaxed;
     const bool idle = g_fused_may_probe && hipStreamQuery(stream) == hipSuccess;
     (void)hipGetLastError();  // a busy stream leaves "not ready" behind
     d.rows_streams[slot] = stream;
