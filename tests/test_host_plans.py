@@ -50,3 +50,17 @@ def test_a_forward_replaced_on_a_class_is_not_passed_by(cls, monkeypatch):
     assert Int8OPTDecoderLayer._one_call_tensors(stream, None) == (True, None)
     monkeypatch.setattr(cls, "forward", lambda *a, **k: None)
     assert Int8OPTDecoderLayer._one_call_tensors(stream, None)[0] is False
+
+
+def test_two_continuations_of_one_past_get_rooms_of_their_own():
+    """A decode step takes the position behind a past before its launches, not after them: another thread that continues the same
+    past meanwhile, or another layer handed the same cache, gets a copy; a step that is not taken gives the position back."""
+    from torch_int.models import opt
+    past = tuple(opt._kv_view(opt._KVBuffer(torch.zeros(2, 3, 32, 16, dtype=torch.int8), 10), 10) for _ in range(2))
+    first, second = opt._kv_rooms(past), opt._kv_rooms(past)
+    assert first[0] is past[0]._ti_kv and first[1] is past[1]._ti_kv
+    assert len({id(kv) for kv in first + second}) == 4 and all(kv.filled == 11 for kv in first + second)
+    both = opt._kv_rooms((past[0], past[0]))   # a key tensor handed as the value tensor too
+    assert both[0] is not both[1]
+    opt._kv_give_back(first)
+    assert opt._kv_rooms(past)[0] is first[0]

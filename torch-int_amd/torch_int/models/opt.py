@@ -9,6 +9,7 @@ particular ``transformers`` release; any object with OPTConfig's field names
 works as ``config``.
 """
 import ctypes
+import threading
 from dataclasses import dataclass
 from typing import List, Optional, Tuple
 
@@ -62,14 +63,36 @@ def _kv_fresh(past, T):
     return _KVBuffer(buf, S)
 
 
+_kv_lock = threading.Lock()
+
+
+def _kv_claim(past):
+    """A buffer with room for one more position behind ``past``, taken: it counts as filled from here on, so that nobody else
+    who continues the same past (another thread, while this one's layers are on their way) is given the same position."""
+    S = past.shape[2]
+    with _kv_lock:
+        kv = _kv_room_for(past, 1)
+        if kv is not None:
+            kv.filled = S + 1
+            return kv
+    kv = _kv_fresh(past, 1)
+    kv.filled = S + 1
+    return kv
+
+
 def _kv_rooms(past):
-    """Buffers of a layer's (key, value) cache with room for one more position, or None when a kernel cannot write there."""
-    kk = _kv_room_for(past[0], 1) or _kv_fresh(past[0], 1)
-    vv = _kv_room_for(past[1], 1) or _kv_fresh(past[1], 1)
+    """``_kv_claim`` for a layer's (key, value) cache, or None when a kernel cannot write there."""
+    kk, vv = _kv_claim(past[0]), _kv_claim(past[1])
     kb, vb = kk.buf, vv.buf
     if kb.data_ptr() % 16 or vb.data_ptr() % 16 or not (kb.is_contiguous() and vb.is_contiguous() and kb.shape == vb.shape):
+        _kv_give_back((kk, vv))
         return None
     return kk, vv
+
+
+def _kv_give_back(rooms):
+    for kv in rooms:
+        kv.filled -= 1
 
 
 def _kv_view(kv, n):
@@ -569,7 +592,6 @@ class Int8OPTDecoderLayer(nn.Module):
             return None
         (plan, S), (kk, vv) = found, rooms
         _hip_ext.opt_layer_decode(plan, hidden_states, mask, kk.buf, vv.buf, S)
-        kk.filled = vv.filled = S
         if use_cache:
             return hidden_states, (_kv_view(kk, S), _kv_view(vv, S))
         return (hidden_states,)
@@ -805,12 +827,12 @@ class Int8OPTDecoder(nn.Module):
         cache = []
         if decode:
             rooms = [_kv_rooms(past) for past in past_key_values]
-            if not all(rooms) or len({id(kv) for pair in rooms for kv in pair}) < 2 * count:
-                return None   # layers that were handed one and the same cache must not append to one buffer
+            if not all(rooms):
+                _kv_give_back(kv for pair in rooms if pair for kv in pair)
+                return None
             scratch = _hip_ext.opt_decode_scratch([plan for plan, _ in found], hidden)
             for (plan, S), (kk, vv), chain in zip(found, rooms, links):
                 _hip_ext.opt_layer_decode(plan, hidden, mask, kk.buf, vv.buf, S, chain=chain, carry=carry, scratch=scratch)
-                kk.filled = vv.filled = S
                 if use_cache:
                     cache.append((_kv_view(kk, S), _kv_view(vv, S)))
         else:
