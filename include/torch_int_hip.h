@@ -55,7 +55,7 @@ int ti_init(void);
  * (16 < M <= 1024 with a long K, or the last rows of a larger M: see ti_linear_row_split; 0 up to 16 rows, whose slices
  * meet in memory of the library's own, 67 MiB per device: 2 MiB for each of 33 streams);
  * 0 when no split is worthwhile.  Passing a smaller or NULL workspace is always legal and
- * only selects a non-split kernel. */
+ * only selects another kernel, one that needs less or does not split. */
 int64_t ti_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /* Diagnostic: the number r of rows that a linear of this shape cuts off its end and runs as a second, small
@@ -207,7 +207,8 @@ int ti_linear_a8_w8_b8_o8(const int8_t* x, const int8_t* w, const int8_t* bias, 
  * Same arguments minus the workspace, same bytes out.  The split-K partial products go to a buffer of
  * TI_NOALLOC_SCRATCH_BYTES that is part of the library's device image (one copy per GPU, held until the
  * process ends); the call allocates and frees nothing.  Shapes whose split needs more
- * (ti_linear_workspace_bytes(M, N, K) > TI_NOALLOC_SCRATCH_BYTES) are refused with TI_ERR_INVALID_ARG.
+ * (ti_linear_workspace_bytes(M, N, K) > TI_NOALLOC_SCRATCH_BYTES) are refused with TI_ERR_INVALID_ARG, but for those that
+ * need that much only for the weight-streaming kernel's slices or for 160x160 tiles: they run on the kernels that need less.
  * Every call on a GPU shares that GPU's buffer: calls that may overlap in time on one GPU (different
  * streams, different threads) race and must be serialised by the caller.  The buffer needs no clearing
  * between calls (every partial product is written before it is read).  ti_init() resolves the buffer's address

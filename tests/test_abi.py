@@ -426,3 +426,15 @@ def test_rows_in_slices_only_where_they_are_ahead(M, N, K, slices):
     pick = C._lib.ti_selftest_rows_pick
     pick.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
     assert pick(M, N, K, 256, ctypes.byref(ctypes.c_int(0))) == slices
+
+
+@pytest.mark.parametrize("M,N,K,refused", [(64, 50272, 11264, False), (19, 50272, 11264, False), (257, 11040, 16640, False), (300, 28800, 28672, False),
+                                           (1024, 9216, 36864, True), (512, 9216, 9216, False)])
+def test_the_no_allocation_entry_point_takes_what_kernels_of_less_scratch_run(M, N, K, refused):
+    # the slices of the weight-streaming kernel or of 160x160 tiles would not fit the built-in scratch in the first four, but
+    # those of the kernels that ran such shapes before them do; no pointers, so nothing is launched
+    import torch_int._CUDA as C
+    call = C._lib.ti_linear_a8_w8_b8_o8_noalloc
+    call.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int64] * 3 + [ctypes.c_float] * 2 + [ctypes.c_void_p]
+    assert call(None, None, None, None, M, N, K, 1.0, 1.0, None) != 0
+    assert (b"split-K scratch, the built-in buffer" in C._lib.ti_last_error()) == refused

@@ -189,7 +189,8 @@ int ti_linear_a8_w8_b8_o8_noalloc(const int8_t* x, const int8_t* w, const int8_t
   const char* op = "linear_a8_w8_b8_o8_noalloc";
   g_err[0] = 0;
   if (int rc = check_dims(op, 1, M, N, K)) return rc;
-  const int64_t need = gemm_workspace_bytes(M, N, K);
+  int64_t need = gemm_workspace_bytes(M, N, K);
+  if (need > (int64_t)TI_NOALLOC_SCRATCH_BYTES) need = gemm_workspace_bytes(M, N, K, true);
   if (need > (int64_t)TI_NOALLOC_SCRATCH_BYTES)
     return fail(TI_ERR_INVALID_ARG,
                 "%s: M=%lld N=%lld K=%lld needs %lld bytes of split-K scratch, the built-in buffer holds %lld; "

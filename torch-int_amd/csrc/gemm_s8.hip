@@ -8,18 +8,18 @@
 
 namespace ti {
 
-long long gemm_workspace_bytes(long long M, long long N, long long K) {
+long long gemm_workspace_bytes(long long M, long long N, long long K, bool least) {
   if (M > 1024) {  // the rows beyond the last multiple of 256 as a small problem of their own (row_split_rows)
     long long need = 0;
     const int r = row_split_rows(M, N, K, &need);
     if (r <= 0) return 0;
     // the first rows are a problem of their own too: at exactly 1024 of them they may split K themselves
-    const long long head = M - r <= 1024 ? gemm_workspace_bytes(M - r, N, K) : 0;
+    const long long head = M - r <= 1024 ? gemm_workspace_bytes(M - r, N, K, least) : 0;
     return head > need ? head : need;
   }
-  const RowsPick rows = rows_pick(M, N, K);
+  const RowsPick rows = least ? RowsPick{ROWS_NONE, 1} : rows_pick(M, N, K);
   if (M > 16 && rows.tiling != ROWS_NONE && (N % 16 == 0 || K % SBK == 0)) return rows.slices > 1 ? (long long)rows.slices * M * N * 4 : 0;
-  const int s = choose_splits(M, N, K);
+  const int s = choose_splits(M, N, K, nullptr, nullptr, 1, !least);
   return s > 1 ? (long long)s * M * N * 4 : 0;
 }
 

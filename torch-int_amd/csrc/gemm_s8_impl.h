@@ -2288,7 +2288,7 @@ enum SplitTile { SPLIT_128 = 0, SPLIT_256 = 1, SPLIT_256x160 = 2, SPLIT_256x288 
 // it, the one-launch form is not available, and the tile shapes are those that exist for every epilogue of the
 // raw-int32 kernels.
 static int choose_splits(long long M, long long N, long long K, int* tile_kind = nullptr, double* time_us = nullptr,
-                         long long batch = 1) {
+                         long long batch = 1, bool square_tiles = true) {
   if (tile_kind) *tile_kind = SPLIT_128;
   if (time_us) *time_us = -1.0;  // no estimate
   if (M <= 16 || M > 1024 || K % PBK != 0 || K < 1024) return 1;
@@ -2318,7 +2318,7 @@ static int choose_splits(long long M, long long N, long long K, int* tile_kind =
     const int bn = small ? 80 : wide192 || tall192 ? 192 : kind == SPLIT_128 ? 128 : kind == SPLIT_256 ? 256
                    : kind == SPLIT_256x288 || kind == SPLIT_128x288 ? 288 : 160;
     if (kind >= SPLIT_256x160 && N % bn != 0) continue;
-    if (square && (batch > 1 || (M + 159) / 160 * 160 >= (M + 127) / 128 * 128)) continue;  // only where it saves rows
+    if (square && (!square_tiles || batch > 1 || (M + 159) / 160 * 160 >= (M + 127) / 128 * 128)) continue;  // only where it saves rows
     if ((wide192 || tall192) && (N % 160 == 0 || N % 288 == 0)) continue;  // those widths keep their tuned tiles
     const double tiles = (double)((M + bm - 1) / bm) * (double)((N + bn - 1) / bn) * (double)batch;
     for (int s = 1; s <= 16; ++s) {
@@ -2727,8 +2727,12 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
   }
   if (p.batch == 1 && p.lda == p.K && p.ldb == p.K) {
     int tile = SPLIT_128;
-    const int splits = choose_splits(p.M, p.N, p.K, &tile);
-    const long long need = (long long)splits * p.M * p.N * 4;
+    int splits = choose_splits(p.M, p.N, p.K, &tile);
+    long long need = (long long)splits * p.M * p.N * 4;
+    if (tile == SPLIT_160x160 && (workspace == nullptr || workspace_bytes < need)) {  // the best of the others, which may do with less
+      splits = choose_splits(p.M, p.N, p.K, &tile, nullptr, 1, false);
+      need = (long long)splits * p.M * p.N * 4;
+    }
     if (splits == 1 && tile == SPLIT_128x80) {
       g_last_kernel = "pipe16_128x80";
       return launch_pipe16q<Pipe16QCfg<128, 80, 4, 1, KIND>>(p, stream);

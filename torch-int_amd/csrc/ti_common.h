@@ -240,7 +240,8 @@ int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStrea
 // Launchers (gemm_s8.hip).  `kind` is an EpiKind.  Returns a TI_* status.
 int launch_gemm(int kind, const GemmParams& p, void* workspace, long long workspace_bytes,
                 hipStream_t stream);
-long long gemm_workspace_bytes(long long M, long long N, long long K);
+// `least`: of the kernels that run where the workspace does not hold the slices of the weight-streaming kernel or of 160x160 tiles
+long long gemm_workspace_bytes(long long M, long long N, long long K, bool least = false);
 int gemm_group_is_one_launch(long long M, long long N, long long K, int count);
 int gemm_row_split(long long M, long long N, long long K);
 long long bmm_workspace_bytes(long long batch, long long M, long long N, long long K);  // split-K scratch of a batched product  // rows a linear cuts off its end and runs as a second problem
