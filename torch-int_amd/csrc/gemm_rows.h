@@ -428,6 +428,12 @@ static inline bool rows_slices_ahead(RowsPick pick, long long M, long long N, lo
               {4, 2, 0.172, 1.10},   {8, 1, 0.118, 2.00}, {8, 1, 0.123, 1.95}, {8, 1, 0.118, 2.15}};
   const auto& c = cost[pick.tiling];
   const long long strips = (N + 15) / 16 * problems, row_blocks = (M + 15) / 16;
+  const long long slots = (long long)cus * c.per_cu / 8, need = (strips + 7) / 8 * pick.slices;
+  const long long groups = (need < slots ? need : slots) / pick.slices * 8;
+  const long long strips_each = (strips + groups - 1) / groups;
+  const long long rounds = (strips_each * row_blocks + c.waves - 1) / c.waves * ((pick.slices + 3) / 4);
+  const double weights_us = c.us_per_mb * N * K * problems * 1e-6, end_us = c.us_per_round * rounds;
+  if (end_us <= 2.0 + 0.2 * weights_us) return true;  // an end this short: none of 475 such shapes was slower
   int tile = SPLIT_128;
   double others = -1.0;
   (void)choose_splits(M, N, K, &tile, &others);
@@ -435,13 +441,9 @@ static inline bool rows_slices_ahead(RowsPick pick, long long M, long long N, lo
   // at these few rows that model, made for more of them, is too low for 256x256 tiles and for short runs of 128x80 ones
   if (tile == SPLIT_256) others *= 1.25;
   else if (tile == SPLIT_128x80 && others < 14.0) others *= 1.15;
-  const long long slots = (long long)cus * c.per_cu / 8, need = (strips + 7) / 8 * pick.slices;
-  const long long groups = (need < slots ? need : slots) / pick.slices * 8;
-  const long long strips_each = (strips + groups - 1) / groups;
-  const long long rounds = (strips_each * row_blocks + c.waves - 1) / c.waves * ((pick.slices + 3) / 4);
   // Both prices are good to some 10 %.  Of those 875 shapes (17 to 64 rows) 96 were slower than before in slices, up to 2.6 times
   // (64 x 20480 x 13312 58.2 -> 151.4 us); of the 730 that this takes three are, by up to 8 %, the others run at 0.38 to 1.02 times.
-  return 5.6 + c.us_per_mb * N * K * problems * 1e-6 + c.us_per_round * rounds <= 0.8 * others * problems;
+  return 5.6 + weights_us + end_us <= 0.8 * others * problems;
 }
 
 // The same up to 16 rows, where the streaming kernel (it needs K % 1024 == 0 and 256 strips) or the skinny one would run; what the
