@@ -438,7 +438,7 @@ int launch_splitk_raw(int tile, const GemmParams& q, hipStream_t stream) {
 // Tile width of the one persistent launch that runs a group of `count` [M,K] x [N,K] s8 linears at prefill sizes
 // (160, 288 or 128), or 0 when the problems run one after the other.
 static int group_prefill_tile(long long M, long long N, long long K, int count) {
-  if (!(M > 128 && K % QBK == 0 && K >= QBK && count > 1)) return 0;
+  if (!(M > 128 && K % QBK == 0 && K >= QBK && K <= PANEL_MAX_LD && count > 1)) return 0;
   const long long cus = num_cus();
   auto fill = [&](long long tiles) { return (double)tiles / (double)(((tiles + cus - 1) / cus) * cus); };
   const long long rows256 = (M + 255) / 256;

@@ -673,6 +673,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::MIN_WAVES) void gemm_pipe_kernel(Gemm
 // the stage just released, read the first slice of the next step and multiply
 // the last slice of this one.
 static constexpr int QBK = 128;
+static constexpr int PANEL_MAX_LD = 1 << 23;  // bytes between panel rows up to which 32-bit panel offsets reach
 
 template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int KIND_, bool SWAP_>
 struct Pipe2Cfg {
@@ -997,6 +998,45 @@ __device__ __forceinline__ void store_tile16(v4i (&acc)[Cfg::TM][Cfg::TN], const
       return;
     }
   }
+  if constexpr (sizeof(Out) == 4 && !E::kAccumulate && TN % 2 == 0) {
+    // 32-bit outputs of a wave tile that lies inside the matrix: two column blocks of a row are one 128-byte line.  Lanes
+    // er and er ^ 8 swap one block each, so that a store instruction writes eight rows x 128 bytes instead of sixteen x 64
+    // (256x128 tiles, 2048x12288x12288: 281 -> 276 us).
+    const int nw = tile_n * BN + wave_n * Cfg::WTN;
+    if (vec_ok && bias_al && nw + Cfg::WTN <= N) {
+      const bool upper = er >= 8;
+      BiasT bv[TN][4] = {};
+      if (E::kHasBias) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const v4i w = *reinterpret_cast<const v4i*>(bias + nw + j * 16 + 4 * eg);
+          __builtin_memcpy(bv[j], &w, 16);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int m = tile_m * BM + wave_m * Cfg::WTM + i * 16 + (er & 7);
+        Out* dst = C + out_index(p, m, nw + (upper ? 16 : 0) + 4 * eg);
+        Out* dst8 = dst + 8ll * N;
+#pragma unroll
+        for (int j = 0; j < TN; j += 2) {
+          v4i lo, hi;  // rows 0..7 and 8..15 of the block row
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const Out a = E::apply(acc[i][j][v], E::bias_term(bv[j][v], p.beta), p.alpha);
+            const Out b2 = E::apply(acc[i][j + 1][v], E::bias_term(bv[j + 1][v], p.beta), p.alpha);
+            const int x0 = __builtin_bit_cast(int, a), x1 = __builtin_bit_cast(int, b2);
+            const int got = __builtin_amdgcn_mov_dpp(upper ? x0 : x1, 0x128, 0xf, 0xf, true);  // row_ror:8
+            lo[v] = upper ? got : x0;
+            hi[v] = upper ? x1 : got;
+          }
+          if (m < M) *reinterpret_cast<v4i*>(dst + j * 16) = lo;
+          if (m + 8 < M) *reinterpret_cast<v4i*>(dst8 + j * 16) = hi;
+        }
+      }
+      return;
+    }
+  }
   // accumulate-into-output kind: fetch what the tile holds now, the loads in flight together before the
   // first use -- the whole wave tile when its TM*TN*4 registers fit, else one column block at a time
   constexpr bool HOLD_ALL = E::kAccumulate && TM * TN <= 12;
@@ -1299,6 +1339,7 @@ struct Pipe16QCfg {
   static constexpr int TAIL_ROWS = RPW % 8;
   static constexpr int COPIES = RPW / 8 + (TAIL_ROWS ? 1 : 0);
   static constexpr bool SINGLE_B = 4 * TM * TN + 8 * (TM + TN) >= 224;  // as in Pipe16Cfg
+  static constexpr bool PANEL_COPIES = RPW % 8 == 0 && BM % 8 == 0;
   static_assert(WTM % 16 == 0 && WTN % 16 == 0, "wave tile must be made of 16x16 blocks");
   static_assert((BM + BN) % NWAVES == 0 && RPW % 2 == 0, "a wave must copy whole pairs of rows");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
@@ -1359,7 +1400,13 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_pipe16q_kernel(GemmParams p, 
   mark_xcc(first);
 
   // ---- copy stream: copy j of this wave fills panel rows wave*RPW + 8j .. +7 of [A panel | B panel]
-  const TI_GLOBAL_AS int8_t* src[COPIES];
+  // Where a wave's rows are whole groups of eight (Cfg::PANEL_COPIES), a copy instruction reads one panel: the panel's
+  // address is scalar and a lane holds 32-bit offsets, half the registers of full addresses and no 64-bit additions in
+  // the loop (the 256x256 tiles spill without it).
+  constexpr bool PANEL = Cfg::PANEL_COPIES;
+  const TI_GLOBAL_AS int8_t* src[PANEL ? 1 : COPIES];
+  unsigned off[PANEL ? COPIES : 1];
+  const TI_GLOBAL_AS int8_t *a_panel = nullptr, *b_panel = nullptr;
   auto set_copy_item = [&](int item) {
     int b, tile_id;
     decode_item(item, b, tile_id);
@@ -1368,6 +1415,20 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_pipe16q_kernel(GemmParams p, 
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     const int8_t* A = Cfg::GROUPED ? p.A : a_of_batch(p, b);
     const int8_t* B = Cfg::GROUPED ? grp.B[b] : b_of_batch(p, b);
+    if constexpr (PANEL) {
+      a_panel = (const TI_GLOBAL_AS int8_t*)(A + (size_t)m0 * p.lda);
+      b_panel = (const TI_GLOBAL_AS int8_t*)(B + (size_t)n0 * p.ldb);
+#pragma unroll
+      for (int j = 0; j < COPIES; ++j) {
+        const int slab = wave * Cfg::RPW + j * 8;  // uniform over the wave
+        const bool in_a = slab < BM;
+        const int row = slab - (in_a ? 0 : BM) + (lane >> 3);
+        const int last = (in_a ? M - m0 : N - n0) - 1;  // edge rows re-read the last row; never stored
+        off[j] = (unsigned)(row < last ? row : last) * (unsigned)(in_a ? p.lda : p.ldb) +
+                 (unsigned)(((lane & 7) ^ ((row >> 1) & 7)) << 4);
+      }
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < COPIES; ++j) {
       int prow = wave * Cfg::RPW + j * 8 + (lane >> 3);
@@ -1376,12 +1437,12 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_pipe16q_kernel(GemmParams p, 
       if (prow < BM) {
         const int chunk = pos ^ ((prow >> 1) & 7);
         const int gr = m0 + prow < M ? m0 + prow : M - 1;  // edge rows re-read the last row; never stored
-        src[j] = (const TI_GLOBAL_AS int8_t*)(A + (size_t)gr * p.lda + chunk * 16);
+        src[PANEL ? 0 : j] = (const TI_GLOBAL_AS int8_t*)(A + (size_t)gr * p.lda + chunk * 16);
       } else {
         const int br = prow - BM;
         const int chunk = pos ^ ((br >> 1) & 7);
         const int gr = n0 + br < N ? n0 + br : N - 1;
-        src[j] = (const TI_GLOBAL_AS int8_t*)(B + (size_t)gr * p.ldb + chunk * 16);
+        src[PANEL ? 0 : j] = (const TI_GLOBAL_AS int8_t*)(B + (size_t)gr * p.ldb + chunk * 16);
       }
     }
   };
@@ -1392,7 +1453,11 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_pipe16q_kernel(GemmParams p, 
     TI_LDS_AS char* dst = (TI_LDS_AS char*)smem + c_slot * Cfg::STAGE_BYTES + wave * Cfg::RPW * QBK;
 #pragma unroll
     for (int j = 0; j < COPIES; ++j) {
-      if (Cfg::TAIL_ROWS == 0 || j + 1 < COPIES || lane < Cfg::TAIL_ROWS * 8)
+      if constexpr (PANEL)
+        __builtin_amdgcn_global_load_lds(
+            (const TI_GLOBAL_AS void*)((wave * Cfg::RPW + j * 8 < BM ? a_panel : b_panel) + c_kt * QBK + off[j]),
+            (TI_LDS_AS void*)(dst + j * 1024), 16, 0, 0);
+      else if (Cfg::TAIL_ROWS == 0 || j + 1 < COPIES || lane < Cfg::TAIL_ROWS * 8)
         __builtin_amdgcn_global_load_lds((const TI_GLOBAL_AS void*)(src[j] + c_kt * QBK),
                                          (TI_LDS_AS void*)(dst + j * 1024), 16, 0, 0);
     }
@@ -2669,6 +2734,12 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
     if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
     return TI_OK;
   }
+  constexpr bool SWAP = sizeof(Out) == 1;  // 8-bit outputs take the orientation whose lanes own 16 consecutive columns
+  // The kernels with 128-byte steps hold 32-bit offsets into a panel of at most 288 rows.
+  if ((p.lda > PANEL_MAX_LD || p.ldb > PANEL_MAX_LD) && p.K % PBK == 0) {
+    g_last_kernel = "pipe_128x128";
+    return launch_pipe<PipeCfg<128, 128, 2, 2, 4, KIND, SWAP>>(p, stream);
+  }
   if (p.batch > 1 && p.batch <= 65535 && p.lda == p.K && p.ldb == p.K && p.out_d == 0 && workspace != nullptr &&
       (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
     // A batched product with few output tiles and a long inner dimension (upstream's benchmark/bench_bmm.py multiplies
@@ -2827,8 +2898,6 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
       return TI_OK;
     }
   }
-  // 8-bit outputs take the orientation whose lanes own 16 consecutive columns.
-  constexpr bool SWAP = sizeof(Out) == 1;
   const long long t256 = (long long)((p.M + 255) / 256) * ((p.N + 255) / 256) * p.batch;
   const long long t128 = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
   if (p.K % PBK == 0 && p.K >= PBK) {
@@ -2857,6 +2926,14 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
           return launch_pipe16q<Pipe16QCfg<256, 192, 4, 2, KIND>>(p, stream);
         case WIDE_256x256:
           g_last_kernel = "pipe_256x256";
+          // 8-bit outputs from K = 2048 on: 16x16 blocks, 64x128 per wave, 1.50 us a step against 1.63 and 2 us more of fill
+          // and epilogue.  Bound by the power limit, as the 32x32 blocks are.  8192x20480x5120 700 -> 670 us, 1900x16384x4096
+          // 118 -> 113, 2112x5120x5120 64 -> 61; 4096x4096x768 18.5 against 19.2, so a short K and the attention products stay.
+          // 32-bit outputs stay as well: 64 rows of 512 bytes to a wave leave more slowly than 128 rows of 256, behind
+          // the next tile's first copies (8192x20480x5120 764 against 803 us).
+          if constexpr (SWAP) {
+            if (wide_step && p.K >= 2048) return launch_pipe16q<Pipe16QCfg<256, 256, 4, 2, KIND>>(p, stream);
+          }
           if (wide_step) return launch_pipe2<Pipe2Cfg<256, 256, 2, 4, KIND, SWAP>>(p, stream);  // whole cache lines per row
           return launch_pipe<PipeCfg<256, 256, 2, 4, 4, KIND, SWAP>>(p, stream);
         default:
@@ -2870,6 +2947,11 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
     }
     if (t128 >= 128) {
       g_last_kernel = "pipe_128x128";
+      // Tiles that are all resident with one workgroup per CU: 128-byte steps, five stages, eight waves of 32x64 (0.50 us a
+      // step against 0.70 for the same K in two 64-byte steps, 2048x2048x8192 50.4 -> 38.6 us, 2048x2048x2048 16.4 -> 13.6).
+      // More tiles share the CUs better with two workgroups each (8192x768x768 13.3 against 14.3 us).
+      if (p.batch == 1 && p.K % QBK == 0 && p.K >= 512 && t128 <= num_cus())
+        return launch_pipe16q<Pipe16QCfg<128, 128, 4, 2, KIND, false, 5>>(p, stream);
       return launch_pipe<PipeCfg<128, 128, 2, 2, 4, KIND, SWAP>>(p, stream);
     }
   }
