@@ -1,5 +1,6 @@
-"""The tiles whose copies read one operand panel each (8-bit 256x256 and the 128x128 of one round), at the edges of their rows,
-columns and K, and rows too far apart for 32-bit panel offsets.  Bit for bit against an exact fp64 product on the device."""
+"""The tilings of 1025 rows and more that are chosen by price (8-bit 256x256, the 128x128 of one round, 192x128, 192x256, 160x256),
+at the edges of their rows, columns and K, three of them in one launch, and rows too far apart for 32-bit panel offsets.
+Bit for bit against an exact fp64 product on the device."""
 import ctypes
 
 import pytest
@@ -33,8 +34,11 @@ def _run(M, N, K, out_dtype, seed):
 @pytest.mark.parametrize("out_dtype", [torch.int8, torch.int32])
 @pytest.mark.parametrize("M,N,K,family", [
     (1025, 2048, 512, "pipe_128x128"), (2048, 2048, 640, "pipe_128x128"), (2047, 2033, 2048, "pipe_128x128"),
-    (1921, 2064, 4224, "pipe_128x128"), (2048, 7168, 2048, "pipe_256x256"), (2047, 7151, 2176, "pipe_256x256"),
-    (1793, 7424, 4096, "pipe_256x256")])
+    (1921, 2041, 4224, "pipe_128x128"), (2048, 7168, 2048, "pipe_256x256"), (2047, 7151, 2176, "pipe_256x256"),
+    (1793, 7424, 4096, "pipe_256x256"),
+    (3000, 2048, 2048, "pipe16_192x128"), (2881, 2048, 768, "pipe16_192x128"), (2945, 2001, 1024, "pipe16_192x128"),
+    (2112, 5120, 5120, "pipe16_192x256"), (2113, 5120, 2048, "pipe16_192x256"), (2111, 5104, 1152, "pipe16_192x256"),
+    (2400, 4096, 4096, "pipe16_160x256"), (2241, 4096, 1280, "pipe16_160x256")])
 def test_panel_tiles(M, N, K, family, out_dtype):
     import torch_int._CUDA as C
     C._lib.ti_last_kernel.restype = ctypes.c_char_p
@@ -47,3 +51,20 @@ def test_panel_tiles(M, N, K, family, out_dtype):
 def test_rows_too_far_apart_for_panel_offsets():
     out, want = _run(20, 24, (1 << 23) + 128, torch.int32, 5)
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("B,T,H,d,K", [(8, 256, 32, 64, 2048), (1, 1905, 16, 128, 2048), (3, 683, 32, 64, 2176)])
+def test_three_projections_on_256x256_tiles(B, T, H, d, K):
+    import torch_int._CUDA as C
+    import torch_int._hip_ext as X
+    C._lib.ti_last_kernel.restype = ctypes.c_char_p
+    gen = torch.Generator(device=DEV).manual_seed(T)
+    M, N = B * T, H * d
+    x, ws, bs = _s8(gen, (M, K), 3.0), [_s8(gen, (N, K), 3.0) for _ in range(3)], [_s8(gen, (N,), 20.0) for _ in range(3)]
+    al, be = [2.0 ** -8, 2.0 ** -7, 2.0 ** -9], [0.5, 1.0, 0.25]
+    print(f"group {M}x{N}x{K}", flush=True)
+    out = X.linear_a8_w8_b8_o8_group_heads(x, ws, bs, al, be, B, T, H, d)
+    assert C._lib.ti_last_kernel().decode() == "pipe16_256x256_group"
+    for o, w, b, a, c in zip(out, ws, bs, al, be):
+        want = torch.clamp(torch.round((x.double() @ w.double().t()) * a + c * b.double()), -128, 127).to(torch.int8)
+        assert torch.equal(o, want.view(B, T, H, d).transpose(1, 2))

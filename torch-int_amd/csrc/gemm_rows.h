@@ -33,6 +33,7 @@ namespace ti {
 
 #define TI_ROWS_MAX_M 64
 
+
 template <int KIND_, int MX_, int KS_, int KP_, int RING_, int NW_, bool GROUPED_ = false>
 struct RowsCfg {
   static constexpr int KIND = KIND_, MX = MX_, KS = KS_, KP = KP_, RING = RING_, NW = NW_;

@@ -436,7 +436,7 @@ int launch_splitk_raw(int tile, const GemmParams& q, hipStream_t stream) {
 }
 
 // Tile width of the one persistent launch that runs a group of `count` [M,K] x [N,K] s8 linears at prefill sizes
-// (160, 288 or 128), or 0 when the problems run one after the other.
+// (160, 288, 256 or 128), or 0 when the problems run one after the other.
 static int group_prefill_tile(long long M, long long N, long long K, int count) {
   if (!(M > 128 && K % QBK == 0 && K >= QBK && K <= PANEL_MAX_LD && count > 1)) return 0;
   const long long cus = num_cus();
@@ -451,6 +451,22 @@ static int group_prefill_tile(long long M, long long N, long long K, int count) 
   double e128 = N % 128 == 0 ? 0.87 * fill(rows256 * (N / 128) * count) : 0.0;
   if (e128 < 0.5 || e128 <= e256_alone) e128 = 0.0;
   const double e = e160 > e288 ? (e160 > e128 ? e160 : e128) : (e288 > e128 ? e288 : e128);
+  // Beyond 1024 rows the grouped launch and the problems one after the other are priced as price_wide prices tilings, and
+  // 256x256 tiles are in the race too: three 2048x2048x2048 are 192 of them, one round (34.1 -> 30.8 us).
+  if (M > 1024 && wide_priced(M, N, K, 1)) {
+    int tile = 0;
+    double best = (double)count * (price_wide(M, N, K).us + 1.0);
+    for (const WideRate& r : kWideRates) {
+      if (r.tile != WIDE_256x160 && r.tile != WIDE_256x288 && r.tile != WIDE_256x128 && !(r.tile == WIDE_256x256 && K >= 2048)) continue;
+      if (N % r.bn != 0) continue;
+      const double us = wide_us(r, M, N, K, count, false);
+      if (us < best) {
+        best = us;
+        tile = r.bn;
+      }
+    }
+    return tile;
+  }
   if (e <= 0.0) return 0;
   // Up to 1024 rows a problem may have a one-round tiling of its own that needs no workspace (128x80, 128x192 or
   // 256x192 tiles over the whole of K): when the cost model prices the problems one after the other below the
@@ -527,7 +543,7 @@ int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStrea
     return deep ? launch(gemm_stream_kernel<KIND, 16, 3, true>, 3, 32, 1)
                 : launch(gemm_stream_kernel<KIND, 16, 2, true>, 2, 32, 2);
   }
-  // Prefill shapes whose width the 256x160, 256x288 or 256x128 tiles divide: the problems are the batches of one
+  // Prefill shapes whose width the 256x160, 256x288, 256x256 or 256x128 tiles divide: the problems are the batches of one
   // persistent launch, so the pipeline fill and the epilogue of one projection overlap the next one's work.
   if (ptr_ok && shape.lda == shape.K && shape.ldb == shape.K) {
     const int tile = group_prefill_tile(shape.M, shape.N, shape.K, grp.count);
@@ -541,6 +557,10 @@ int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStrea
       if (tile == 288) {
         g_last_kernel = "pipe16_256x288_group";
         return launch_pipe16q<Pipe16QCfg<256, 288, 4, 2, KIND, true>>(q, stream, grp);
+      }
+      if (tile == 256) {
+        g_last_kernel = "pipe16_256x256_group";
+        return launch_pipe16q<Pipe16QCfg<256, 256, 4, 2, KIND, true>>(q, stream, grp);
       }
       g_last_kernel = "pipe16_256x128_group";
       return launch_pipe16q<Pipe16QCfg<256, 128, 4, 2, KIND, true>>(q, stream, grp);

@@ -1001,7 +1001,8 @@ __device__ __forceinline__ void store_tile16(v4i (&acc)[Cfg::TM][Cfg::TN], const
   if constexpr (sizeof(Out) == 4 && !E::kAccumulate && TN % 2 == 0) {
     // 32-bit outputs of a wave tile that lies inside the matrix: two column blocks of a row are one 128-byte line.  Lanes
     // er and er ^ 8 swap one block each, so that a store instruction writes eight rows x 128 bytes instead of sixteen x 64
-    // (256x128 tiles, 2048x12288x12288: 281 -> 276 us).
+    // (256x128 tiles, 2048x12288x12288: 281 -> 276 us).  Not for odd numbers of blocks: with pairs that begin at the even
+    // blocks of a row, 256x160 tiles took 192 us instead of 160 (1552x5120x20480).
     const int nw = tile_n * BN + wave_n * Cfg::WTN;
     if (vec_ok && bias_al && nw + Cfg::WTN <= N) {
       const bool upper = er >= 8;
@@ -1339,7 +1340,9 @@ struct Pipe16QCfg {
   static constexpr int TAIL_ROWS = RPW % 8;
   static constexpr int COPIES = RPW / 8 + (TAIL_ROWS ? 1 : 0);
   static constexpr bool SINGLE_B = 4 * TM * TN + 8 * (TM + TN) >= 224;  // as in Pipe16Cfg
-  static constexpr bool PANEL_COPIES = RPW % 8 == 0 && BM % 8 == 0;
+  // copies of one panel each, with 32-bit offsets (see the kernel): where the registers are short.  192x256 tiles 3 to 4 %
+  // faster, 256x192 1 %, 256x128 level, and the small tiles, which have registers to spare, 1 to 3 % slower.
+  static constexpr bool PANEL_COPIES = RPW % 8 == 0 && BM % 8 == 0 && BM * BN >= 256 * 192;
   static_assert(WTM % 16 == 0 && WTN % 16 == 0, "wave tile must be made of 16x16 blocks");
   static_assert((BM + BN) % NWAVES == 0 && RPW % 2 == 0, "a wave must copy whole pairs of rows");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
@@ -2499,12 +2502,66 @@ static int launch_fused(const GemmParams& q_in, hipStream_t stream) {
 // count as waste; batched products count tiles only, they are bound by HBM, where padding costs no bytes).  The
 // 128x128 kernel (64-byte steps, two stages) runs at half that rate per CU, a little more with two workgroups on
 // every CU, and takes over where few tiles of 256 rows would leave most CUs idle.
-enum WideTile { WIDE_NONE = 0, WIDE_256x160, WIDE_256x288, WIDE_256x128, WIDE_256x256, WIDE_256x192 };
+enum WideTile { WIDE_NONE = 0, WIDE_256x160, WIDE_256x288, WIDE_256x128, WIDE_256x256, WIDE_256x192, WIDE_128x128,
+                WIDE_192x128, WIDE_192x256, WIDE_160x256 };
 struct WidePick {
   int tile;       // WideTile; WIDE_NONE = leave it to the 128x128 / small-tile kernels
-  double eff;     // efficiency of the choice relative to the 256x256 kernel on a full chip (0 for WIDE_NONE)
+  double us = 0;  // price_wide: what the choice is priced at
 };
-static WidePick pick_wide(long long M, long long N, long long K, long long batch) {
+
+// Prices in us of the tilings of a linear (or of `count` linears of one shape in one launch) with a K of six or more steps.
+// A tiling's time is rounds x steps x step, where a step is what the 128 bytes of K take a workgroup while all CUs multiply,
+// plus its fill and last epilogue, plus what each further round adds; a chip that is not full clocks higher, so a step of a
+// tiling that leaves half of it idle takes a seventh less.  Measured with 256 tiles at K = 2048 and 8192, weights from HBM, us:
+// 128x128 38.6 at K = 8192, 192x128 48.1, 256x128 59.5, 160x256 70.2, 256x160 70.9, 192x256 83.8, 256x256 108.  What bounds
+// a step is the power the operands' bits cost on their way through the LDS, which is why larger tiles have the better rates
+// (30 to 44 thousand outputs a us and CU); what the others are for is row counts that leave the larger ones idle: 2112 rows
+// are nine rows of 256 (288 tiles of 256x160, a second round for 32 of them) but eleven of 192 (220 tiles of 192x256, one
+// round).  Tilings that divide neither rows nor columns well lose by their padding and need no rule.
+struct WideRate {
+  int tile, bm, bn;
+  double step, fixed, again;
+  bool newer;  // replaces an older choice only where it is clearly cheaper
+};
+static constexpr WideRate kWideRates[] = {
+    {WIDE_256x128, 256, 128, 0.83, 7.0, 4.0, false}, {WIDE_256x160, 256, 160, 0.977, 8.3, 5.0, false},
+    {WIDE_256x256, 256, 256, 1.50, 11.0, 7.0, false}, {WIDE_256x288, 256, 288, 1.72, 11.0, 7.0, false},
+    {WIDE_256x192, 256, 192, 1.217, 9.1, 6.0, false}, {WIDE_128x128, 128, 128, 0.505, 6.3, 2.7, false},
+    {WIDE_192x128, 192, 128, 0.67, 6.8, 3.5, true}, {WIDE_160x256, 160, 256, 1.02, 8.3, 5.0, true},
+    {WIDE_192x256, 192, 256, 1.19, 9.8, 6.0, true}};
+
+static bool wide_priced(long long M, long long N, long long K, long long batch) {
+  return batch == 1 && M > 128 && N > 128 && K % QBK == 0 && K >= 768 && ((M + 127) / 128) * ((N + 127) / 128) >= 128;
+}
+static double wide_us(const WideRate& r, long long M, long long N, long long K, long long count, bool out32) {
+  const double cus = num_cus(), steps = (double)(K / QBK);
+  const double tiles = (double)((M + r.bm - 1) / r.bm) * (double)((N + r.bn - 1) / r.bn) * (double)count;
+  auto time = [&](double slots, double step, double fixed, double again) {
+    const double rounds = (double)(long long)((tiles + slots - 1) / slots);
+    // What 32-bit outputs of a tile take longer to leave: up to twice that where the rows lie many KiB apart, but for the
+    // 32x32 blocks (8192x20480x5120: 764 us on those, 855 on 256x160; 3932x10240x2560: 123 against 116).
+    const double apart = r.tile == WIDE_256x256 || N <= 10240 ? 1.0 : N >= 20480 ? 2.0 : N / 10240.0;
+    const double store = out32 ? r.bm * r.bn * 1e-4 * apart : 0.0;
+    return rounds * steps * step * (0.7 + 0.3 * tiles / (rounds * slots)) + fixed + store + (rounds - 1) * (again + store);
+  };
+  if (r.tile == WIDE_128x128 && (tiles > cus || K < 1536))  // the 64-byte steps, two workgroups per CU
+    return tiles > cus ? time(2 * cus, 1.4, 5.6, out32 ? 5.0 : 1.5) : time(cus, 0.68, 5.6, 1.5);
+  if (r.tile == WIDE_256x256 && (K < 2048 || out32)) return time(cus, out32 && N > 12288 ? 1.72 : 1.63, 8.9, 6.0);  // the 32x32 blocks
+  return time(cus, r.step, r.fixed, r.again);
+}
+static WidePick price_wide(long long M, long long N, long long K, bool out32 = false) {
+  WidePick best{WIDE_NONE, 1e30};
+  for (const WideRate& r : kWideRates) {
+    // 256x160 and 256x288 have no narrow last column; 256x192 is for widths that neither divides, in one round
+    if ((r.bn == 160 || r.bn == 288) && N % r.bn != 0) continue;
+    if (r.bn == 192 && (N % 192 != 0 || N % 160 == 0 || N % 288 == 0)) continue;
+    const double us = wide_us(r, M, N, K, 1, out32);
+    if (us < (r.newer ? 0.95 : 1.0) * best.us) best = WidePick{r.tile, us};
+  }
+  return best;
+}
+static WidePick pick_wide(long long M, long long N, long long K, long long batch, bool out32) {
+  if (wide_priced(M, N, K, batch)) return price_wide(M, N, K, out32);
   const long long cus = num_cus();
   const long long t256 = ((M + 255) / 256) * ((N + 255) / 256) * batch;
   const long long t128 = ((M + 127) / 128) * ((N + 127) / 128) * batch;
@@ -2535,12 +2592,12 @@ static WidePick pick_wide(long long M, long long N, long long K, long long batch
   const double best_other = e256 > e160 ? (e256 > e288 ? (e256 > e128w ? e256 : e128w) : (e288 > e128w ? e288 : e128w))
                                   : (e160 > e288 ? (e160 > e128w ? e160 : e128w) : (e288 > e128w ? e288 : e128w));
   const double best = best_other > e192 ? best_other : e192;
-  if (!(t256 >= 160 || (priced && best > e128))) return WidePick{WIDE_NONE, 0.0};
-  if (e192 > best_other * 1.03) return WidePick{WIDE_256x192, e192};
-  if (e160 > e256 && e160 >= e288 && e160 >= e128w) return WidePick{WIDE_256x160, e160};
-  if (e288 > e256 && e288 >= e128w) return WidePick{WIDE_256x288, e288};
-  if (e128w > e256) return WidePick{WIDE_256x128, e128w};
-  return WidePick{WIDE_256x256, e256};
+  if (!(t256 >= 160 || (priced && best > e128))) return WidePick{WIDE_NONE};
+  if (e192 > best_other * 1.03) return WidePick{WIDE_256x192};
+  if (e160 > e256 && e160 >= e288 && e160 >= e128w) return WidePick{WIDE_256x160};
+  if (e288 > e256 && e288 >= e128w) return WidePick{WIDE_256x288};
+  if (e128w > e256) return WidePick{WIDE_256x128};
+  return WidePick{WIDE_256x256};
 }
 
 // K slices for a batched product (1 = none): only where the problems together have too few 128x128 tiles to fill
@@ -2554,14 +2611,17 @@ static int batched_splits(long long batch, long long M, long long N, long long K
   return choose_splits(M, N, K, tile_kind, nullptr, batch);
 }
 
+}  // namespace ti
+#include "gemm_rows.h"
+namespace ti {
+
 // Rows to cut off the end of a linear with many rows and run as a second, small problem (0 = none).
 // A tiled GEMM pays for whole tiles and whole rounds of 256 CUs: 2112 rows (a 4 x 528-token prefill; prefill lengths
 // are padded to 16, not to 256) are nine row tiles where 2048 rows are eight, 288 tiles of 256x160 instead of 256 - a
 // second round for 64 rows.  When the rows beyond the last multiple of 256 are few, the first M - r rows run on the
 // tiling that suits them and the r rows left over as a problem of their own through the split-K forms, if the cost
-// model prices the pair clearly below the whole.  Times in us: a tiling of efficiency e takes M N K / e at the 256x256
-// kernel's rate (0.85 us per 64-byte step and 256 tiles) plus 8 us of fill and epilogue; the small problem is priced
-// by choose_splits (its workspace must have been given), rows <= 16 as weight streaming at 4.5 TB/s.
+// model prices the pair clearly below the whole: the tilings by price_wide, the small problem by choose_splits (its
+// workspace must have been given), rows <= 16 as weight streaming at 4.5 TB/s.
 static int row_split_rows(long long M, long long N, long long K, long long* rest_ws_bytes = nullptr) {
   if (rest_ws_bytes) *rest_ws_bytes = 0;
   static const bool enabled = [] {  // TORCH_INT_ROW_SPLIT=0 keeps every linear in one piece
@@ -2571,11 +2631,7 @@ static int row_split_rows(long long M, long long N, long long K, long long* rest
   if (!enabled) return 0;
   const long long r = M % 256;
   if (M <= 1024 || r == 0 || r > 128 || N <= 128 || K % QBK != 0 || K < 1024) return 0;
-  const WidePick whole = pick_wide(M, N, K, 1), main = pick_wide(M - r, N, K, 1);
-  if (whole.tile == WIDE_NONE || main.tile == WIDE_NONE) return 0;
-  auto tiled_us = [&](long long rows, double eff) {
-    return (double)rows * (double)N * (double)(K / 64) * 0.85 / (65536.0 * (double)num_cus() * eff) + 8.0;
-  };
+  if (!wide_priced(M, N, K, 1) || !wide_priced(M - r, N, K, 1)) return 0;
   double rest_us = 0.0;
   long long need = 0;
   if (r <= 16) {
@@ -2585,15 +2641,14 @@ static int row_split_rows(long long M, long long N, long long K, long long* rest
     const int splits = choose_splits(r, N, K, &tile, &rest_us);
     if (rest_us < 0.0) return 0;
     need = splits > 1 ? (long long)splits * r * N * 4 : 0;
+    const double streamed = (double)N * (double)K / 5.4e6 + 3.0;
+    if (r <= TI_ROWS_MAX_M && rest_us > streamed && rows_pick(r, N, K).tiling != ROWS_NONE) rest_us = streamed;
   }
-  if (tiled_us(M - r, main.eff) + rest_us + 3.0 >= 0.95 * tiled_us(M, whole.eff)) return 0;
+  for (const bool out32 : {false, true})  // the answer depends on the shape alone
+    if (price_wide(M - r, N, K, out32).us + rest_us + 2.0 >= 0.99 * price_wide(M, N, K, out32).us) return 0;
   if (rest_ws_bytes) *rest_ws_bytes = need;
   return (int)r;
 }
-
-}  // namespace ti
-#include "gemm_rows.h"
-namespace ti {
 
 template <int KIND, bool GROUPED>
 static int launch_gemv(const GemmParams& p, const GemmGroup& grp, int problems, hipStream_t stream) {
@@ -2909,7 +2964,7 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
       // 76 -> 47, 2048x4096x4096 48 -> 35, 2048x4096x16384 170 -> 118, 2048x2560x2560 25 -> 20, 2048x12288x12288
       // 285 -> 253.
       const bool wide_step = p.K % QBK == 0;
-      switch (pick_wide(p.M, p.N, p.K, p.batch).tile) {
+      switch (pick_wide(p.M, p.N, p.K, p.batch, !SWAP).tile) {
         case WIDE_256x160:
           g_last_kernel = "pipe16_256x160";
           if (wide_step) return launch_pipe16q<Pipe16QCfg<256, 160, 4, 2, KIND>>(p, stream);
@@ -2924,6 +2979,15 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
         case WIDE_256x192:
           g_last_kernel = "pipe16_256x192";
           return launch_pipe16q<Pipe16QCfg<256, 192, 4, 2, KIND>>(p, stream);
+        case WIDE_192x128:
+          g_last_kernel = "pipe16_192x128";
+          return launch_pipe16q<Pipe16QCfg<192, 128, 4, 2, KIND>>(p, stream);
+        case WIDE_192x256:
+          g_last_kernel = "pipe16_192x256";
+          return launch_pipe16q<Pipe16QCfg<192, 256, 4, 2, KIND>>(p, stream);
+        case WIDE_160x256:
+          g_last_kernel = "pipe16_160x256";
+          return launch_pipe16q<Pipe16QCfg<160, 256, 2, 4, KIND>>(p, stream);
         case WIDE_256x256:
           g_last_kernel = "pipe_256x256";
           // 8-bit outputs from K = 2048 on: 16x16 blocks, 64x128 per wave, 1.50 us a step against 1.63 and 2 us more of fill
@@ -2949,8 +3013,9 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
       g_last_kernel = "pipe_128x128";
       // Tiles that are all resident with one workgroup per CU: 128-byte steps, five stages, eight waves of 32x64 (0.50 us a
       // step against 0.70 for the same K in two 64-byte steps, 2048x2048x8192 50.4 -> 38.6 us, 2048x2048x2048 16.4 -> 13.6).
-      // More tiles share the CUs better with two workgroups each (8192x768x768 13.3 against 14.3 us).
-      if (p.batch == 1 && p.K % QBK == 0 && p.K >= 512 && t128 <= num_cus())
+      // More tiles share the CUs better with two workgroups each (8192x768x768 13.3 against 14.3 us), and a short K does
+      // not pay for the longer fill (3146x768x768 fp32 9.6 against 10.0, 2271x1024x1024 8.7 against 9.0).
+      if (p.batch == 1 && p.K % QBK == 0 && p.K >= 1536 && t128 <= num_cus())
         return launch_pipe16q<Pipe16QCfg<128, 128, 4, 2, KIND, false, 5>>(p, stream);
       return launch_pipe<PipeCfg<128, 128, 2, 2, 4, KIND, SWAP>>(p, stream);
     }
