@@ -392,9 +392,9 @@ int ti_kv_append_s8(const int8_t* k_new, const int8_t* v_new, int8_t* k_buf, int
  * same bits, without the score and probability tensors.  vt is V transposed, [BH, D, S] packed (what
  * ti_transpose_last2_s8 makes, as upstream's `value_states.transpose(1,2).contiguous()`); ctx is [BH/heads, T,
  * heads*D] packed.  Limits (ti_attn_prefill_supported): S a multiple of 16 in [16, 4096] and D a multiple of 16 up to
- * 128 (OPT-2.7B: 80; rows keep their own length in memory).  Up to 576 keys all keys
- * of a head sit in the LDS and are swept once; other shapes sweep the keys three times in tiles of 256 (row maximum, row
- * sum, probabilities): the same bits either way. */
+ * 128 (OPT-2.7B: 80; rows keep their own length in memory).  Up to 576 keys all keys of a head sit in the LDS, or, as beyond
+ * that up to 2048, the scores of a row stay in registers; longer ones sweep the keys three times in tiles of 256 (row
+ * maximum, row sum, probabilities): the same bits either way. */
 int ti_attn_prefill_supported(int64_t T, int64_t S, int64_t D);
 int ti_attn_prefill_s8(const int8_t* q, const int8_t* k, const int8_t* vt, const float* mask, int8_t* ctx, int64_t BH,
                        int64_t T, int64_t S, int64_t D, int64_t stride_q, int64_t stride_k, int64_t heads,
@@ -436,8 +436,8 @@ int ti_attn_qk_softmax_q(const int8_t* q, const int8_t* k, const float* mask, in
 /* Classes of an additive attention mask, an optional accelerator for the two prefill entry points above (no
  * counterpart in the reference).  classes[b][i][j] describes the mask values of batch b, query rows 64 i .. 64 i + 63,
  * keys 256 j .. 256 j + 255: 1 = all of them are +-0 (the kernels then do not read them), 2 = all of them are one
- * and the same value, -1e30 or below (the row-maximum sweep of the long-prefill kernel then takes that value instead
- * of loading keys and multiplying), 0 = anything else.  ti_attn_mask_classes fills the array (one read of the mask;
+ * and the same value, -1e30 or below (whose keys are then not multiplied, but for rows that are masked throughout), 0 =
+ * anything else.  ti_attn_mask_classes fills the array (one read of the mask;
  * ti_attn_mask_classes_bytes = its size, 0 when the shape takes none), once per mask: every head and every layer that
  * adds the same mask shares it.  The _mc entry points are ti_attn_qk_softmax_q / ti_attn_prefill_s8 with that
  * array (NULL = none); the bits of the results do not depend on it.  Under a causal mask only the tiles on the

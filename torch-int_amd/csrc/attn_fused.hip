@@ -300,6 +300,12 @@ int launch_attn_long(const int8_t* q, const int8_t* k, const float* mask, int8_t
                      long long S, long long D, long long stride_q, long long stride_k, long long heads, float alpha,
                      const int8_t* vt, int8_t* ctx, float alpha_pv, hipStream_t stream, const unsigned char* cls);
 
+// attn_rows.hip: up to 2048 keys, the scores of a row in the registers of four waves; with V^T
+bool attn_rows_supported(long long T, long long S, long long D);
+int launch_attn_rows(const int8_t* q, const int8_t* k, const float* mask, const unsigned char* cls, const int8_t* vt,
+                     int8_t* ctx, long long BH, long long T, long long S, long long D, long long stride_q, long long stride_k,
+                     long long heads, float alpha, float alpha_pv, hipStream_t stream);
+
 // shapes the single-sweep kernel of this file takes (all keys of a head in the LDS at once)
 static bool single_sweep_ok(long long T, long long S, long long D, bool pv) {
   (void)pv;  // with or without the product with V
@@ -313,6 +319,19 @@ bool attn_qk_softmax_q_supported(long long T, long long S, long long D) {
 // the form that multiplies on with V^T
 bool attn_prefill_supported(long long T, long long S, long long D) {
   return single_sweep_ok(T, S, D, true) || attn_long_supported(T, S, D);
+}
+
+// Whether attn_rows_kernel is ahead.  Beyond 576 keys always: the other form sweeps the keys three times (us, with the mask's
+// classes: 64 heads x 640 x 128 46.9 -> 25.9, 1024 94.7 -> 47.0, 32 heads x 1904 131 -> 91, 64 heads x 1280 x 64 120 -> 51).  Up
+// to 576 the single sweep shares its keys among 64 query rows and this one among none, but a quarter of the rows to a workgroup
+// fill the chip four times as well: from 65 keys on where 16-row workgroups are few (12 heads x 256 x 64 9.3 -> 5.1, 80 heads x
+// 128 x 128 7.9 -> 7.5, 160 heads 8.9 against 11.3), and with many of them from 353 keys on, if no mask has to be read for
+// every tile of keys (160 heads x 512 x 128 56.8 -> 42.5, without the classes 58.2 -> 52.2 but 160 x 528 57.9 against 68.3; 256
+// heads x 320 x 128, a second tile of 64 keys that one wave of four multiplies, 30.7 against 36.5).
+static bool rows_form_ahead(long long BH, long long T, long long S, long long D, bool no_mask_or_classes) {
+  if (!attn_rows_supported(T, S, D) || S <= 64) return false;
+  if (S > AF_MAX_S || BH * ((T + 15) / 16) <= (S > 128 ? 1024 : 640)) return true;
+  return S > 352 && no_mask_or_classes;
 }
 
 template <int NB, bool PV, int SPEC, int D, bool PAD>
@@ -340,6 +359,8 @@ int launch_attn_qk_softmax_q(const int8_t* q, const int8_t* k, const float* mask
                              long long heads, float alpha, const int8_t* vt, int8_t* ctx, float alpha_pv,
                              hipStream_t stream, const unsigned char* mask_classes) {
   if (BH == 0 || T == 0) return TI_OK;
+  if (vt != nullptr && rows_form_ahead(BH, T, S, D, mask == nullptr || mask_classes != nullptr))
+    return launch_attn_rows(q, k, mask, mask_classes, vt, ctx, BH, T, S, D, stride_q, stride_k, heads, alpha, alpha_pv, stream);
   if (!single_sweep_ok(T, S, D, vt != nullptr))
     return launch_attn_long(q, k, mask, probs, BH, T, S, D, stride_q, stride_k, heads, alpha, vt, ctx, alpha_pv, stream,
                             mask_classes);

@@ -1,4 +1,5 @@
-// Prefill attention for any number of keys and head sizes 64 / 128, without the fp32 score tensor in memory:
+// Prefill attention for any number of keys (it runs beyond 2048 with the product with V, beyond 576 without) and head
+// sizes 64 / 128, without the fp32 score tensor in memory:
 // probs = round(127 softmax(max(alpha q.k^T + mask, lowest))) and, on request, context = s8(alpha_pv probs . V).
 // The bits are those of bmm_s8t_s8n_f32t -> attn_softmax_q -> bmm_s8t_s8n_s8t: the row maximum is taken over all
 // keys before any exponential, and the row sum adds the exponentials in the reference order (chunk c of four

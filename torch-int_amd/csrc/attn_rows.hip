@@ -1,0 +1,445 @@
+// Prefill attention with the scores of a whole row in registers: context = s8(alpha_pv round(127 softmax(max(alpha q.k^T +
+// mask, lowest))) . V), up to 2048 keys (any multiple of 16) and head sizes up to 128 (any multiple of 16).  The bits are
+// those of bmm_s8t_s8n_f32t -> attn_softmax_q -> bmm_s8t_s8n_s8t.
+//
+// One workgroup of four waves per (batch * head, 16 query rows).  The keys are cut so that a wave owns whole partial sums of
+// the reference order (chunk c of four keys belongs to partial sum c % 64, which takes its chunks in ascending order): of
+// every 256 keys, wave w has keys 64 w .. 64 w + 63 as four blocks of 16, and its partial sums are 16 w .. 16 w + 15.  Each
+// score is computed once and stays in its accumulator register (128 of them at 2048 keys) until the row maximum and then
+// the row sum are known; the waves meet twice in between, over a few KiB of LDS, and once more to add their integer
+// contexts.  The three-sweep form this replaces up to 2048 keys computed scores three and exponentials up to two times, with a
+// barrier and an exposed copy per tile of 256 keys and sweep.
+//
+// Bound by the vector ALUs (some 24 instructions a live score: at 32 heads x 2048 x 128 without a mask 82 us of 126) and, under
+// a causal mask, by the few tiles of most rows.  What it measures against the other forms is at the rule that chooses
+// (attn_fused.hip).
+//
+// Keys, mask values and V^T reach a wave through an LDS ring of its own, without barriers: no two waves of a workgroup use the same key, but
+// a fragment load straight from global memory asks for 16 rows x 64 bytes with neighbouring lanes on different rows, a
+// quarter of the rate of the copies' (32 heads x 2048 x 2048 without a mask: 264 us).  The pieces (32 keys, the mask values of 64,
+// half of V^T's rows for 64 keys) follow one another in one sequence, V^T last, so that it lands under the last scores
+// and the exponentials.  For P.V the four dwords of probabilities that a lane holds of 64 keys are transposed across the four
+// 16-lane rows, after which a lane holds 16 consecutive keys, as a 16-byte read of V^T does.
+#include <atomic>
+#include "ti_common.h"
+#include "softmax_math.h"
+
+namespace ti {
+
+#define TI_GLOBAL_AS __attribute__((address_space(1)))
+#define TI_LDS_AS __attribute__((address_space(3)))
+
+constexpr int AR_TILE = 256;  // keys per round of the 64 partial sums
+constexpr int AR_MAX_TILES = 8;
+constexpr int AR_BUFFER_FLAGS = 0x00020000;  // raw buffer, 32-bit data: offsets from the descriptor's size on read as zeros
+constexpr int AR_MC_ROWS = 64;  // rows to a mask class (attn_long.hip)
+constexpr int AR_MC_ZERO = 1, AR_MC_UNIFORM = 2;
+
+// 16-byte chunk c of row `row` of a piece whose rows hold B bytes sits at this chunk position
+template <int B>
+__device__ __forceinline__ int ar_swz(int row, int c) {
+  return B == 128 ? (c ^ ((row >> 1) & 7)) : (c ^ ((row >> 2) & 3));
+}
+
+// chunk c of mask row `row` of a piece whose rows hold MC chunks (16 or 8)
+template <int MC>
+__device__ __forceinline__ int ar_mask_swz(int row, int c) {
+  return MC == 16 ? c ^ row : c ^ (row >> 1);
+}
+
+template <int NT, int D>
+struct AttnRows {
+  static constexpr int PIECE = 32 * D;            // bytes: 32 keys, or D / 2 rows of 64 bytes of V^T, or MKEYS keys' mask
+  static constexpr int COPIES = PIECE / 1024;     // copy instructions per piece
+  static constexpr int MKEYS = PIECE / 64;        // 16 rows of mask values
+  static constexpr int RING = 2;                  // pieces per wave (three or four: no faster, and fewer workgroups fit)
+  static constexpr int WAVES = NT <= 4 ? 3 : 2;   // waves per SIMD the registers are sized for
+  static constexpr int PART = 4 * RING * PIECE;   // [16][64] floats behind the rings, then [4][16]
+  static constexpr int LDS = PART + 16 * 64 * 4 + 4 * 16 * 4;
+  static_assert(RING * PIECE >= D / 16 * 1024, "a wave's context goes over its ring");
+  static_assert(WAVES * LDS <= 160 * 1024, "resident workgroups");
+};
+
+// The ring of one wave.  A tile of `keys` puts two pieces of keys into it and, if it is one of `masked`, its mask values;
+// after the last of them every tile of `vals` puts in two pieces of V^T.  The addresses are bounds-checked by the buffer
+// descriptors: rows past the last key, the last query row or the head size read as zeros (and count for nothing).
+template <int NT, int D>
+struct AttnRing {
+  using L = AttnRows<NT, D>;
+  static constexpr int CP = L::COPIES, STAGES = 2 + 64 / L::MKEYS;
+  char* ring;
+  __amdgpu_buffer_rsrc_t kres, vres, mres;
+  int S, dr, w;
+  unsigned keys, masked, vals;
+  unsigned key_off[2], v_off, m_row, m_chunk;  // a lane's offsets (keys: of even and odd copies)
+  int stage = 0;                      // of the tile that comes next: 0, 1 keys or V^T, from 2 mask
+  int head = 0, tail = 0, ahead = 0;  // next slot to fill, next to read, pieces between them
+
+  __device__ __forceinline__ const char* at_tail() const { return ring + tail * L::PIECE; }
+  __device__ __forceinline__ void issue() {
+    if ((keys | vals) == 0) return;
+    TI_LDS_AS char* dst = (TI_LDS_AS char*)ring + head * L::PIECE;
+    const int tile = __builtin_ctz(keys != 0 ? keys : vals);
+    const int at = tile * AR_TILE + 64 * w;
+    ++stage;
+    if (keys != 0) {
+      if (stage <= 2) {
+        const unsigned base = (unsigned)((at + 32 * (stage - 1)) * dr);
+#pragma unroll
+        for (int i = 0; i < CP; ++i)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(kres, (TI_LDS_AS void*)(dst + i * 1024), 16,
+                                                   key_off[i & 1] + (base + (unsigned)(i * (1024 / D) * dr)), 0, 0, 0);
+      } else {
+        const unsigned base = (unsigned)(at + L::MKEYS * (stage - 3)) * 4u;
+#pragma unroll
+        for (int i = 0; i < CP; ++i)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(
+              mres, (TI_LDS_AS void*)(dst + i * 1024), 16,
+              (m_chunk ^ (unsigned)(64 * i)) + (m_row + base + (unsigned)(i * (16 / CP) * S * 4)), 0, 0, 0);
+      }
+      if (stage == (masked >> tile & 1 ? STAGES : 2)) {
+        stage = 0;
+        keys &= keys - 1;
+      }
+    } else {
+      const unsigned base = (unsigned)((stage - 1) * (D / 2) * S + at);
+#pragma unroll
+      for (int i = 0; i < CP; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(vres, (TI_LDS_AS void*)(dst + i * 1024), 16, v_off + (base + (unsigned)(i * 16 * S)),
+                                                 0, 0, 0);
+      if (stage == 2) {
+        stage = 0;
+        vals &= vals - 1;
+      }
+    }
+    head = head + 1 == L::RING ? 0 : head + 1;
+    ++ahead;
+  }
+  // waits for the piece at the tail: loads complete in order, so at most the copies of the pieces behind it may be outstanding
+  __device__ __forceinline__ void wait() const {
+    if (L::RING > 3 && ahead == 4) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * CP) : "memory");
+    else if (L::RING > 2 && ahead == 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * CP) : "memory");
+    else if (ahead == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CP) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+  // the piece has been read: its slot is free for the next
+  __device__ __forceinline__ void release() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    tail = tail + 1 == L::RING ? 0 : tail + 1;
+    --ahead;
+    issue();
+  }
+};
+
+// NT = tiles of 256 keys (only the last one may be cut short); D = 64 or 128, the head size in memory (dr) rounded up:
+// the chunks of a query row beyond dr are zeros, so whatever the keys' copies put there adds nothing, and context columns
+// beyond dr are computed and not stored.
+template <int NT, int D, bool MASKED>
+__global__ __launch_bounds__(256, (AttnRows<NT, D>::WAVES)) void attn_rows_kernel(
+    const int8_t* __restrict__ q, const int8_t* __restrict__ k, const float* __restrict__ mask,
+    const unsigned char* __restrict__ cls, const int8_t* __restrict__ vt, int8_t* __restrict__ ctx, int T, int S,
+    long long stride_q, long long stride_k, int heads, int row_blocks, float alpha, float alpha_pv, int dr) {
+  using L = AttnRows<NT, D>;
+  constexpr int KS = D / 64;  // 64-byte slices of the head dimension
+  constexpr int CH = D / 16;  // blocks of 16 context columns
+  constexpr int RING = L::RING, PIECE = L::PIECE;
+  constexpr unsigned ALL = (1u << NT) - 1;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  char* ring = smem + w * RING * PIECE;
+  float(*s_part)[64] = reinterpret_cast<float(*)[64]>(smem + L::PART);
+  float(*s_max)[16] = reinterpret_cast<float(*)[16]>(smem + L::PART + 16 * 64 * 4);
+  const int n_bh = gridDim.x / row_blocks;
+  const long long bh = blockIdx.x % n_bh;
+  const int t0 = (row_blocks - 1 - (int)(blockIdx.x / n_bh)) * 16;  // heaviest rows of a causal mask first
+  const int rows = T - t0 < 16 ? T - t0 : 16;                       // rows past the end repeat the last one; never stored
+  const float lowest = -3.402823466e+38f;
+
+  v4i qf[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const int c = 64 * s + 16 * g;
+    qf[s] = *reinterpret_cast<const v4i*>(q + bh * stride_q + (long long)(t0 + (r < rows ? r : rows - 1)) * dr + (c < dr ? c : 0));
+  }
+  // mask classes of this row block's tiles.  `todo`: the tiles whose keys are multiplied, all but those whose mask is one
+  // value of -1e30 or below; `zero`: those whose mask adds nothing
+  unsigned todo = ALL, zero = MASKED ? 0u : ALL;
+  if (MASKED && cls != nullptr) {
+    const unsigned char* c = cls + ((bh / heads) * ((T + AR_MC_ROWS - 1) / AR_MC_ROWS) + t0 / AR_MC_ROWS) * NT;
+    const int v = c[lane < NT ? lane : 0];
+    zero = (unsigned)__builtin_amdgcn_ballot_w64(v == AR_MC_ZERO && lane < NT);
+    todo &= ~(unsigned)__builtin_amdgcn_ballot_w64(v == AR_MC_UNIFORM && lane < NT);
+  }
+  AttnRing<NT, D> pieces;
+  pieces.ring = ring;
+  pieces.S = S;
+  pieces.dr = dr;
+  pieces.w = w;
+  pieces.kres = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(k + bh * stride_k), 0, S * dr, AR_BUFFER_FLAGS);
+  pieces.vres = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(vt + bh * (long long)dr * S), 0, S * dr, AR_BUFFER_FLAGS);
+  pieces.mres = pieces.kres;
+  if (MASKED)
+    pieces.mres = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(mask + ((bh / heads) * T + t0) * (long long)S), 0,
+                                                    rows * S * 4, AR_BUFFER_FLAGS);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = lane / (D / 16), c = ar_swz<D>(i * (1024 / D) + row, lane % (D / 16)) * 16;
+    pieces.key_off[i] = (unsigned)(row * dr + (c < dr ? c : 0));
+  }
+  pieces.v_off = (unsigned)((lane >> 2) * S + ar_swz<64>(lane >> 2, lane & 3) * 16);
+  {
+    constexpr int MC = L::MKEYS / 4;  // 16-byte chunks to a mask row
+    const int row = lane / MC;
+    pieces.m_row = (unsigned)(row * S * 4);
+    pieces.m_chunk = (unsigned)(ar_mask_swz<MC>(row, lane % MC) * 16);
+  }
+  // a block past the last key (last tile only) is replaced by -infinity
+  auto exists = [&](int t, int j) { return t < NT - 1 || t * AR_TILE + 64 * w + 16 * j < S; };
+
+  v4i acc[NT][4];
+  float m;
+  for (;;) {  // once; a second time, without the classes, where a row is masked throughout
+    pieces.keys = pieces.vals = todo;
+    pieces.masked = ~zero;
+#pragma unroll
+    for (int i = 0; i < RING; ++i) pieces.issue();
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) qf[s][e] = 64 * s + 16 * g < dr ? qf[s][e] : 0;
+
+    // ---- scores
+    m = lowest;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (MASKED && !(todo >> t & 1)) continue;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        pieces.wait();
+        const char* src = pieces.at_tail();
+        v4i kf[2][KS];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int s = 0; s < KS; ++s)
+            kf[j][s] = *reinterpret_cast<const v4i*>(src + (16 * j + r) * D + (ar_swz<D>(16 * j + r, 4 * s + g) << 4));
+        pieces.release();
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          v4i a = {0, 0, 0, 0};
+#pragma unroll
+          for (int s = 0; s < KS; ++s) a = __builtin_amdgcn_mfma_i32_16x16x64_i8(kf[j][s], qf[s], a, 0, 0, 0);
+          acc[t][2 * h + j] = a;
+        }
+      }
+      auto finish = [&](auto masked_, int j, v4f mk) __attribute__((always_inline)) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          float x = Epi<EPI_F32_SCALE>::apply(acc[t][j][v], 0.0f, alpha);
+          if constexpr (decltype(masked_)::value) x = x + mk[v];
+          x = __builtin_fmaxf(x, lowest);  // NaN included
+          if (t == NT - 1) x = exists(t, j) ? x : -__builtin_inff();
+          m = __builtin_fmaxf(m, x);
+          acc[t][j][v] = __float_as_int(x);
+        }
+      };
+      if (MASKED && !(zero >> t & 1)) {
+        constexpr int MC = L::MKEYS / 4, JP = L::MKEYS / 16;  // blocks per piece of mask
+#pragma unroll
+        for (int i = 0; i < 4 / JP; ++i) {
+          pieces.wait();
+          const char* src = pieces.at_tail();
+          v4f mk[JP];
+#pragma unroll
+          for (int j = 0; j < JP; ++j)
+            mk[j] = *reinterpret_cast<const v4f*>(src + r * (MC * 16) + ar_mask_swz<MC>(r, 4 * j + g) * 16);
+          pieces.release();
+#pragma unroll
+          for (int j = 0; j < JP; ++j) finish(std::integral_constant<bool, true>{}, JP * i + j, mk[j]);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) finish(std::integral_constant<bool, false>{}, j, v4f{0.f, 0.f, 0.f, 0.f});
+      }
+    }
+    float o = __shfl_xor(m, 16, 64);
+    m = m > o ? m : o;
+    o = __shfl_xor(m, 32, 64);
+    m = m > o ? m : o;
+    if (g == 0) s_max[w][r] = m;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (not for the copies of V^T)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      o = s_max[i][r];
+      m = m > o ? m : o;
+    }
+    // Tiles that were passed over hold one mask value of -1e30 or below: beside a row maximum above -1e29 they add exact
+    // zeros.  A row without such a maximum needs them.  (The same rows, and the same answer, in all four waves.)
+    if (!MASKED || todo == ALL || __builtin_amdgcn_ballot_w64(!(m > -1e29f)) == 0) break;
+    todo = ALL;
+    zero = 0;
+    pieces.stage = pieces.head = pieces.tail = pieces.ahead = 0;
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // s_max has been read, no copy is on its way
+  }
+
+  // ---- exponentials and partial sums; a block in which nothing is above exp's cut-off adds exact zeros
+  unsigned live = 0;  // bit 4 t + j
+  float part[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    if (MASKED && !(todo >> t & 1)) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float top = __builtin_fmaxf(__builtin_fmaxf(__int_as_float(acc[t][j][0]), __int_as_float(acc[t][j][1])),
+                                        __builtin_fmaxf(__int_as_float(acc[t][j][2]), __int_as_float(acc[t][j][3])));
+      if (__builtin_amdgcn_ballot_w64(top - m > -87.0f) != 0) {
+        live |= 1u << (4 * t + j);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float e = exp_nonpos(__int_as_float(acc[t][j][v]) - m);
+          acc[t][j][v] = __float_as_int(e);
+          part[j] = part[j] + e;
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) s_part[4 * w + j][lane] = part[j];
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  float all[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) all[j] = s_part[j][lane];
+#pragma unroll
+  for (int h = 8; h >= 1; h >>= 1)
+#pragma unroll
+    for (int j = 0; j < h; ++j) all[j] = all[j] + all[j + h];
+  float sum = all[0];
+  sum = sum + __shfl_xor(sum, 32, 64);
+  sum = sum + __shfl_xor(sum, 16, 64);
+  const float scale = 127.0f / sum;
+
+  // ---- probabilities and their product with V
+  v4i o[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) o[c] = v4i{0, 0, 0, 0};
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    if (MASKED && !(todo >> t & 1)) continue;
+    int pw[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      unsigned p = 0;
+      if (live >> (4 * t + j) & 1) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)  // in [0, 127], whole numbers
+          p = __builtin_amdgcn_cvt_pk_u8_f32(__builtin_rintf(__int_as_float(acc[t][j][v]) * scale), v, p);
+      }
+      pw[j] = (int)p;
+    }
+    row_transpose4(pw);  // keys 16 j + 4 g .. +3 -> keys 16 g + 4 j .. +3
+    const v4i pa = {pw[0], pw[1], pw[2], pw[3]};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      pieces.wait();
+      const char* src = pieces.at_tail();
+      v4i vf[CH / 2];
+#pragma unroll
+      for (int c = 0; c < CH / 2; ++c)
+        vf[c] = *reinterpret_cast<const v4i*>(src + (16 * c + r) * 64 + (ar_swz<64>(16 * c + r, g) << 4));
+      pieces.release();
+#pragma unroll
+      for (int c = 0; c < CH / 2; ++c)
+        o[h * (CH / 2) + c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(vf[c], pa, o[h * (CH / 2) + c], 0, 0, 0);
+    }
+  }
+
+  // ---- the four waves' contexts, over the rings (every copy of this wave has landed and been read)
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int c = 0; c < CH; ++c) *reinterpret_cast<v4i*>(ring + (c * 64 + lane) * 16) = o[c];
+  __syncthreads();
+  if (r < rows) {
+    const long long batch = bh / heads, h = bh - batch * heads;
+    int8_t* crow = ctx + ((batch * T + t0 + r) * heads + h) * (long long)dr + 4 * g;
+#pragma unroll
+    for (int i = 0; i < CH / 4; ++i) {
+      const int c = w * (CH / 4) + i;
+      if (16 * c >= dr) continue;
+      v4i a = {0, 0, 0, 0};
+#pragma unroll
+      for (int u = 0; u < 4; ++u) a += *reinterpret_cast<const v4i*>(smem + u * RING * PIECE + (c * 64 + lane) * 16);
+      unsigned out = 0;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) out |= (unsigned)(unsigned char)Epi<EPI_S8_SCALE>::apply(a[v], 0.0f, alpha_pv) << (8 * v);
+      *reinterpret_cast<unsigned*>(crow + 16 * c) = out;
+    }
+  }
+}
+
+bool attn_rows_supported(long long T, long long S, long long D) {
+  return T >= 1 && D >= 16 && D <= 128 && D % 16 == 0 && S >= 16 && S % 16 == 0 && S <= (long long)AR_TILE * AR_MAX_TILES;
+}
+
+template <int NT, int D, bool MASKED, class... Args>
+static int launch_ar(dim3 grid, hipStream_t stream, Args... args) {
+  auto kern = attn_rows_kernel<NT, D, MASKED>;
+  constexpr int lds = AttnRows<NT, D>::LDS;
+  static std::atomic<unsigned long long> lds_ok{0};  // bit per device: the large dynamic LDS size has been allowed
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return fail(TI_ERR_LAUNCH, "attn_rows: no current device");
+  const unsigned long long bit = 1ull << (dev & 63);
+  if (lds > 64 * 1024 && !(lds_ok.load(std::memory_order_relaxed) & bit)) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "attn_rows: LDS limit: %s", hipGetErrorString(e));
+    lds_ok.fetch_or(bit, std::memory_order_relaxed);
+  }
+  hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream, args...);
+  return TI_OK;
+}
+
+int launch_attn_rows(const int8_t* q, const int8_t* k, const float* mask, const unsigned char* cls, const int8_t* vt,
+                     int8_t* ctx, long long BH, long long T, long long S, long long D, long long stride_q, long long stride_k,
+                     long long heads, float alpha, float alpha_pv, hipStream_t stream) {
+  if (BH == 0 || T == 0) return TI_OK;
+  if (mask == nullptr || !(alpha >= -1e12f && alpha <= 1e12f)) cls = nullptr;  // as in attn_long.hip
+  if (!attn_rows_supported(T, S, D))
+    return fail(TI_ERR_INVALID_ARG, "attn_rows: unsupported shape (T=%lld S=%lld head_dim=%lld)", T, S, D);
+  const int nt = (int)((S + AR_TILE - 1) / AR_TILE);
+  const long long row_blocks = (T + 15) / 16;
+  if (BH * row_blocks > 0x7fffffffLL || T > 0x7fffffffLL)
+    return fail(TI_ERR_INVALID_ARG, "attn_rows: too many row blocks (%lld)", BH * row_blocks);
+  const dim3 grid((unsigned)(BH * row_blocks));
+  int rc = TI_OK;
+#define TI_AR(NT, DD, MASKED)                                                                                   \
+  rc = launch_ar<NT, DD, MASKED>(grid, stream, q, k, mask, cls, vt, ctx, (int)T, (int)S, stride_q, stride_k, (int)heads, \
+                                 (int)row_blocks, alpha, alpha_pv, (int)D)
+#define TI_AR_NT(NT)                                 \
+  case NT:                                           \
+    if (D > 64) {                                    \
+      if (mask != nullptr) TI_AR(NT, 128, true);     \
+      else TI_AR(NT, 128, false);                    \
+    } else {                                         \
+      if (mask != nullptr) TI_AR(NT, 64, true);      \
+      else TI_AR(NT, 64, false);                     \
+    }                                                \
+    break
+  switch (nt) {
+    TI_AR_NT(1);
+    TI_AR_NT(2);
+    TI_AR_NT(3);
+    TI_AR_NT(4);
+    TI_AR_NT(5);
+    TI_AR_NT(6);
+    TI_AR_NT(7);
+    TI_AR_NT(8);
+  }
+#undef TI_AR_NT
+#undef TI_AR
+  if (rc) return rc;
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "attn_rows launch: %s", hipGetErrorString(e));
+  return TI_OK;
+}
+
+}  // namespace ti

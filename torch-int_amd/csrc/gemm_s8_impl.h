@@ -914,20 +914,6 @@ struct Pipe16Cfg {
   static_assert(LDS_BYTES <= 160 * 1024 && STAGES >= 3, "LDS budget");
 };
 
-// 4x4 transpose of dwords across the four 16-lane rows of a wave: lane (r, g) = r + 16 g enters with x[k] and
-// leaves with x[k] = what lane (r, k) held in x[g].  Two v_permlane32_swap and two v_permlane16_swap; every lane
-// of the wave must take part.
-__device__ __forceinline__ void row_transpose4(int (&x)[4]) {
-  auto a = __builtin_amdgcn_permlane32_swap((unsigned)x[0], (unsigned)x[2], false, false);  // rows 2,3 of x0 <-> rows 0,1 of x2
-  auto b = __builtin_amdgcn_permlane32_swap((unsigned)x[1], (unsigned)x[3], false, false);
-  auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);  // odd rows of the first <-> even rows of the second
-  auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
-  x[0] = (int)c[0];
-  x[1] = (int)c[1];
-  x[2] = (int)d[0];
-  x[3] = (int)d[1];
-}
-
 // Epilogue of the 16x16-block kernels: the lane holds row (lane & 15) and four consecutive columns
 // 4 * (lane >> 4) .. +3 of every block.
 template <class Cfg>

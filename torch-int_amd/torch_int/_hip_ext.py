@@ -409,14 +409,17 @@ _mask_classes_cache = {}  # id(mask) -> (weak reference, version counter, classe
 
 
 def mask_classes(mask):
-    """The class array of an additive fp32 mask [bsz, 1, T, S] for the long-prefill attention kernel (which tiles of
+    """The class array of an additive fp32 mask [bsz, 1, T, S] for the prefill attention kernels (which tiles of
     64 rows x 256 keys are all zero / all one masked value / mixed), or None when the shape takes none.  Made once per
-    mask tensor and version: every head and every layer of a forward pass adds the same mask."""
+    mask tensor and version: every head and every layer of a forward pass adds the same mask.  Made anew at each call
+    while a graph is recorded (its replays read the mask as it is then) and for a tensor without a version."""
     import weakref
+    keep = not (mask.is_inference() or torch.cuda.is_current_stream_capturing())
     key = id(mask)
-    hit = _mask_classes_cache.get(key)
-    if hit is not None and hit[0]() is mask and hit[1] == mask._version:
-        return hit[2]
+    if keep:
+        hit = _mask_classes_cache.get(key)
+        if hit is not None and hit[0]() is mask and hit[1] == mask._version:
+            return hit[2]
     bsz, _, T, S = mask.shape
     n = _lib.ti_attn_mask_classes_bytes(bsz, T, S)
     if n <= 0:
@@ -426,18 +429,24 @@ def mask_classes(mask):
         rc = _lib.ti_attn_mask_classes(mask.data_ptr(), cls.data_ptr(), bsz, T, S, _raw_stream(mask.device.index) or None)
     if rc:
         raise RuntimeError(f"torch_int._hip_ext.mask_classes: {_lib.ti_last_error().decode()} (status {rc})")
-    if len(_mask_classes_cache) >= 64:
-        _mask_classes_cache.clear()
-    _mask_classes_cache[key] = (weakref.ref(mask, lambda _r, k=key: _mask_classes_cache.pop(k, None)), mask._version, cls)
+    if keep:
+        if len(_mask_classes_cache) >= 64:
+            _mask_classes_cache.clear()
+        _mask_classes_cache[key] = (weakref.ref(mask, lambda _r, k=key: _mask_classes_cache.pop(k, None)), mask._version, cls)
     return cls
 
 
-def _classes_ptr(mask, S):
-    """Pointer to the mask's class array where the kernel that will run reads one (more than 576 keys), else None."""
-    if mask is None or S <= 576:
+def _classes(mask, BH, T, S, pv):
+    """The mask's class array where the kernel that will run reads one, else None: more than 576 keys, or, with the product
+    with V (``pv``), more than 352 for so many heads and rows that the kernel with a row's scores in registers wants them.
+    To be held until the kernel has been launched."""
+    if mask is None or not (S > 576 or (pv and S > 352 and BH * ((T + 15) // 16) > 1024)):
         return None
-    cls = mask_classes(mask)
-    return cls.data_ptr() if cls is not None else None
+    return mask_classes(mask)
+
+
+def _ptr(tensor):
+    return tensor.data_ptr() if tensor is not None else None
 
 
 def attn_qk_softmax_q(q, k, mask, alpha, heads, checked=False):
@@ -451,8 +460,9 @@ def attn_qk_softmax_q(q, k, mask, alpha, heads, checked=False):
     dev = q.device
     probs = torch.empty((BH, T, S), dtype=torch.int8, device=dev)
     with _on(dev):
+        cls = _classes(mask, BH, T, S, False)
         rc = _lib.ti_attn_qk_softmax_q_mc(q.data_ptr(), k.data_ptr(), mask.data_ptr() if mask is not None else None,
-                                          _classes_ptr(mask, S), probs.data_ptr(), BH, T, S, d, T * d, k.stride(0), heads,
+                                          _ptr(cls), probs.data_ptr(), BH, T, S, d, T * d, k.stride(0), heads,
                                           alpha, _raw_stream(dev.index) or None)
     if rc:
         raise RuntimeError(f"torch_int._hip_ext.attn_qk_softmax_q: {_lib.ti_last_error().decode()} (status {rc})")
@@ -484,8 +494,9 @@ def attn_prefill(q, k, vt, mask, alpha_qk, alpha_pv, heads, checked=False):
     dev = q.device
     ctx = torch.empty((BH // heads, T, heads * d), dtype=torch.int8, device=dev)
     with _on(dev):
+        cls = _classes(mask, BH, T, S, True)
         rc = _lib.ti_attn_prefill_s8_mc(q.data_ptr(), k.data_ptr(), vt.data_ptr(),
-                                        mask.data_ptr() if mask is not None else None, _classes_ptr(mask, S),
+                                        mask.data_ptr() if mask is not None else None, _ptr(cls),
                                         ctx.data_ptr(), BH, T, S, d, T * d, k.stride(0), heads, alpha_qk, alpha_pv,
                                         _raw_stream(dev.index) or None)
     if rc:
@@ -670,8 +681,8 @@ def opt_layer_prefill(plan, hidden, mask, k_out, v_out, chain=0, carry=None, mem
     B, T = hidden.shape[0], hidden.shape[1]
     with _on(dev):
         scratch, ws, ws_ptr, ws_bytes = memory if memory is not None else opt_prefill_scratch((plan,), hidden)
-        cls = _classes_ptr(mask, T) if mask is not None else None
-        rc = _opt_layer_prefill(plan.addr, hidden.data_ptr(), mask.data_ptr() if mask is not None else 0, cls or 0,
+        cls = _classes(mask, B * k_out.shape[1], T, T, True)
+        rc = _opt_layer_prefill(plan.addr, hidden.data_ptr(), mask.data_ptr() if mask is not None else 0, _ptr(cls) or 0,
                                 k_out.data_ptr(), v_out.data_ptr(), B, T, chain, carry.data_ptr() if chain else 0, scratch.data_ptr(),
                                 scratch.numel(), ws_ptr, ws_bytes, _raw_stream(dev.index))
     if rc:
