@@ -13,8 +13,12 @@ def _mask(kind, B, T, S, gen):
     if kind == "none":
         return None
     m = torch.zeros(B, 1, T, S, device=DEV)
-    if kind in ("causal", "padded", "infinite"):
-        m.masked_fill_(torch.ones(T, S, dtype=torch.bool, device=DEV).triu(1 + S - T), LOW if kind != "infinite" else float("-inf"))
+    if kind in ("causal", "padded", "infinite", "half"):
+        low = {"infinite": float("-inf"), "half": -65504.0}.get(kind, LOW)
+        m.masked_fill_(torch.ones(T, S, dtype=torch.bool, device=DEV).triu(1 + S - T), low)
+    if kind == "half":            # as an fp16 model's, with padding in front of some rows and rows masked throughout
+        m[:, :, T // 3:T // 3 + 17] = -65504.0
+        m[-1, ..., :S // 3] = -65504.0
     if kind == "padded":          # the last keys of every sequence, and every key of the last sequence's
         for b in range(B):
             m[b, ..., max(1, S - (b + 1) * S // (B + 1)):] = LOW
@@ -46,7 +50,7 @@ def _check(B, H, T, S, d, kind, alpha=None):
         assert rc == 0 and torch.equal(ctx, want), (kind, classes is not None)
 
 
-@pytest.mark.parametrize("kind", ["none", "causal", "padded", "random", "rows", "infinite"])
+@pytest.mark.parametrize("kind", ["none", "causal", "padded", "random", "rows", "infinite", "half"])
 @pytest.mark.parametrize("B,H,T,S,d", [(1, 3, 80, 80, 64), (2, 2, 256, 256, 128), (1, 2, 257, 272, 16), (1, 3, 500, 512, 80),
                                        (2, 1, 528, 528, 128), (1, 2, 592, 592, 64), (1, 1, 33, 768, 112), (2, 1, 1024, 1024, 128),
                                        (1, 2, 1025, 1040, 48), (1, 1, 1, 1280, 128), (1, 2, 700, 1296, 64), (1, 1, 1792, 1792, 96),
@@ -60,9 +64,11 @@ def test_many_heads_at_the_edge_of_the_rule(S):
     _check(8, 32, S, S, 64, "causal")
 
 
-@pytest.mark.parametrize("alpha", [float("inf"), float("nan"), 1e13, -0.01])
-def test_odd_scales(alpha):
-    _check(1, 2, 300, 304, 64, "causal", alpha)
+@pytest.mark.parametrize("kind", ["causal", "half"])
+@pytest.mark.parametrize("alpha", [float("inf"), float("nan"), 1e13, -0.01, 0.02, 0.05])
+def test_odd_scales(alpha, kind):
+    _check(1, 2, 300, 304, 64, kind, alpha)      # 0.02 and 0.05: products of a few thousand, on both sides of the room there is
+    _check(1, 1, 600, 608, 128, kind, alpha)
 
 
 def test_recorded_prefill_reads_the_mask_as_it_is():

@@ -44,6 +44,7 @@ __device__ __forceinline__ int al_swz(int row, int c) {
 // 3e22: the first sweep takes its maximum from one mask value and neither loads the keys nor multiplies).  Under a
 // causal mask only the tiles on the diagonal are MIXED.
 constexpr int MC_MIXED = 0, MC_ZERO = 1, MC_UNIFORM = 2;
+constexpr int MC_HALF_UNIFORM = 3;  // one number from -1e6 to -6e4, such as the lowest of 16 bits: for attn_rows_kernel; MIXED here
 
 __global__ __launch_bounds__(256) void mask_classes_kernel(const float* __restrict__ mask, unsigned char* __restrict__ cls,
                                                            int T, int S, int row_blocks, int ntiles) {
@@ -67,7 +68,11 @@ __global__ __launch_bounds__(256) void mask_classes_kernel(const float* __restri
   }
   const int all_zero = __syncthreads_and(zero), all_same = __syncthreads_and(same);
   if (threadIdx.x == 0)
-    cls[blockIdx.x] = all_zero ? MC_ZERO : (all_same && __int_as_float(first) <= -1e30f) ? MC_UNIFORM : MC_MIXED;
+    cls[blockIdx.x] = all_zero ? MC_ZERO
+                      : !all_same ? MC_MIXED
+                      : __int_as_float(first) <= -1e30f ? MC_UNIFORM
+                      : __int_as_float(first) >= -1e6f && __int_as_float(first) <= -6e4f ? MC_HALF_UNIFORM
+                                                                                         : MC_MIXED;
 }
 
 // PART: the head size in memory (dr) is smaller than the LDS row size D; the forms for dr == D carry none of its tests.

@@ -33,7 +33,7 @@ constexpr int AR_TILE = 256;  // keys per round of the 64 partial sums
 constexpr int AR_MAX_TILES = 8;
 constexpr int AR_BUFFER_FLAGS = 0x00020000;  // raw buffer, 32-bit data: offsets from the descriptor's size on read as zeros
 constexpr int AR_MC_ROWS = 64;  // rows to a mask class (attn_long.hip)
-constexpr int AR_MC_ZERO = 1, AR_MC_UNIFORM = 2;
+constexpr int AR_MC_ZERO = 1, AR_MC_UNIFORM = 2, AR_MC_HALF_UNIFORM = 3;
 
 // 16-byte chunk c of row `row` of a piece whose rows hold B bytes sits at this chunk position
 template <int B>
@@ -162,14 +162,20 @@ __global__ __launch_bounds__(256, (AttnRows<NT, D>::WAVES)) void attn_rows_kerne
     const int c = 64 * s + 16 * g;
     qf[s] = *reinterpret_cast<const v4i*>(q + bh * stride_q + (long long)(t0 + (r < rows ? r : rows - 1)) * dr + (c < dr ? c : 0));
   }
-  // mask classes of this row block's tiles.  `todo`: the tiles whose keys are multiplied, all but those whose mask is one
-  // value of -1e30 or below; `zero`: those whose mask adds nothing
+  // Mask classes of this row block's tiles.  `todo`: the tiles whose keys are multiplied, all but those whose mask is one low
+  // value throughout; `zero`: those whose mask adds nothing.  A score of a tile that is passed over is below `passed`: -1e30
+  // takes no notice of any product (the launcher looks at alpha), and -6e4, the mask of an fp16 model, is raised by the largest
+  // product there can be (such tiles are multiplied like others where that is not far below it).
   unsigned todo = ALL, zero = MASKED ? 0u : ALL;
+  float passed = -1e29f;
   if (MASKED && cls != nullptr) {
     const unsigned char* c = cls + ((bh / heads) * ((T + AR_MC_ROWS - 1) / AR_MC_ROWS) + t0 / AR_MC_ROWS) * NT;
     const int v = c[lane < NT ? lane : 0];
     zero = (unsigned)__builtin_amdgcn_ballot_w64(v == AR_MC_ZERO && lane < NT);
-    todo &= ~(unsigned)__builtin_amdgcn_ballot_w64(v == AR_MC_UNIFORM && lane < NT);
+    const float product = __builtin_fabsf(alpha) * (float)(dr * 16384);
+    const unsigned half = product < 3e4f ? (unsigned)__builtin_amdgcn_ballot_w64(v == AR_MC_HALF_UNIFORM && lane < NT) : 0u;
+    if (half != 0) passed = product - 5.9e4f;
+    todo &= ~(half | (unsigned)__builtin_amdgcn_ballot_w64(v == AR_MC_UNIFORM && lane < NT));
   }
   AttnRing<NT, D> pieces;
   pieces.ring = ring;
@@ -199,7 +205,7 @@ __global__ __launch_bounds__(256, (AttnRows<NT, D>::WAVES)) void attn_rows_kerne
 
   v4i acc[NT][4];
   float m;
-  for (;;) {  // once; a second time, without the classes, where a row is masked throughout
+  for (;;) {  // once; a second time, without the classes, where a row needs the tiles that were passed over
     pieces.keys = pieces.vals = todo;
     pieces.masked = ~zero;
 #pragma unroll
@@ -274,9 +280,9 @@ __global__ __launch_bounds__(256, (AttnRows<NT, D>::WAVES)) void attn_rows_kerne
       o = s_max[i][r];
       m = m > o ? m : o;
     }
-    // Tiles that were passed over hold one mask value of -1e30 or below: beside a row maximum above -1e29 they add exact
-    // zeros.  A row without such a maximum needs them.  (The same rows, and the same answer, in all four waves.)
-    if (!MASKED || todo == ALL || __builtin_amdgcn_ballot_w64(!(m > -1e29f)) == 0) break;
+    // Beside a row maximum that is 100 above them, the scores of the tiles that were passed over add exact zeros.  A row
+    // without such a maximum needs them.  (The same rows, and the same answer, in all four waves.)
+    if (!MASKED || todo == ALL || __builtin_amdgcn_ballot_w64(!(m > passed + 100.0f)) == 0) break;
     todo = ALL;
     zero = 0;
     pieces.stage = pieces.head = pieces.tail = pieces.ahead = 0;
