@@ -749,6 +749,15 @@ def _additive_decoder_mask(attention_mask, tgt_len, past_len, dtype, device):
     return pad + causal[None, None]
 
 
+def _causal_mask(bsz, tgt_len, dtype, device):
+    """``_additive_decoder_mask`` of tokens that are all attended and have no past, as the layers read it: fp32 with the lowest
+    value of ``dtype``."""
+    return torch.full((bsz, 1, tgt_len, tgt_len), torch.finfo(dtype).min, dtype=torch.float32, device=device).triu_(1)
+
+
+_STOCK_POSITIONS_FORWARD = OPTLearnedPositionalEmbedding.forward
+
+
 class Int8OPTDecoder(nn.Module):
     """Stack of ``Int8OPTDecoderLayer`` with fp embeddings and final LayerNorm
     (upstream ``torch_int/models/opt.py:302-398``).  Without a KV cache the token dimension
@@ -844,6 +853,23 @@ class Int8OPTDecoder(nn.Module):
                     cache.append((key, value))
         return tuple(cache)
 
+    def _positions_in_order(self, past_len, count):
+        """The position embeddings [1, count, width] of tokens past_len, past_len + 1, ..., as a view of the table, or None where
+        the table's module is not the stock one or is shorter (its lookup then says so)."""
+        m = self.embed_positions
+        if (type(m) is not OPTLearnedPositionalEmbedding or m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__
+                or OPTLearnedPositionalEmbedding.forward is not _STOCK_POSITIONS_FORWARD or m.max_norm is not None
+                or _GLOBAL_FORWARD_HOOKS or _GLOBAL_FORWARD_PRE_HOOKS or past_len + count + m.offset > m.weight.shape[0]):
+            return None
+        return m.weight[past_len + m.offset:past_len + m.offset + count].unsqueeze(0)
+
+    @staticmethod
+    def _layer_mask(attention_mask, tgt_len, past_len, inputs_embeds):
+        mask = _additive_decoder_mask(attention_mask, tgt_len, past_len, inputs_embeds.dtype, inputs_embeds.device)
+        if mask.is_cuda and mask.dtype in (torch.float16, torch.bfloat16):
+            mask = mask.float()  # once here instead of once per layer (see Int8OPTAttention.forward)
+        return mask
+
     @torch.no_grad()
     def forward(self, input_ids: torch.LongTensor = None, attention_mask: Optional[torch.Tensor] = None,
                 head_mask: Optional[torch.Tensor] = None,
@@ -865,13 +891,17 @@ class Int8OPTDecoder(nn.Module):
         if inputs_embeds is None:
             inputs_embeds = self.embed_tokens(input_ids)
         bsz, tgt_len = inputs_embeds.shape[:2]
-        if attention_mask is None:
-            attention_mask = torch.ones((bsz, past_len + tgt_len), dtype=torch.bool, device=inputs_embeds.device)
-        pos = self.embed_positions(attention_mask, past_len)
-        mask = _additive_decoder_mask(attention_mask, tgt_len, past_len, inputs_embeds.dtype,
-                                      inputs_embeds.device)
-        if mask.is_cuda and mask.dtype in (torch.float16, torch.bfloat16):
-            mask = mask.float()  # once here instead of once per layer (see Int8OPTAttention.forward)
+        # Without an attention mask every key up to a token is attended and positions follow the past: a slice of the
+        # position table and, in a prefill, one triangle take the place of some fifteen kernels.
+        pos = self._positions_in_order(past_len, tgt_len) if attention_mask is None and inputs_embeds.is_cuda else None
+        in_order = pos is not None and inputs_embeds.dtype in (torch.float16, torch.bfloat16, torch.float32)
+        if in_order and (tgt_len == 1 or past_len == 0):
+            mask = None if tgt_len == 1 else _causal_mask(bsz, tgt_len, inputs_embeds.dtype, inputs_embeds.device)
+        else:
+            if attention_mask is None:
+                attention_mask = torch.ones((bsz, past_len + tgt_len), dtype=torch.bool, device=inputs_embeds.device)
+            pos = self.embed_positions(attention_mask, past_len)
+            mask = self._layer_mask(attention_mask, tgt_len, past_len, inputs_embeds)
         if self.project_in is not None:
             inputs_embeds = self.project_in(inputs_embeds)
         hidden = inputs_embeds + pos  # a fresh tensor: the layers update it in place
@@ -884,6 +914,9 @@ class Int8OPTDecoder(nn.Module):
             chained = self._chain_layers(hidden, mask, past_key_values, use_cache)
         if chained is not None:
             cache = chained if use_cache else None
+        elif mask is None:   # layers called by themselves are handed the mask of zeros
+            attention_mask = torch.ones((bsz, past_len + tgt_len), dtype=torch.bool, device=hidden.device)
+            mask = self._layer_mask(attention_mask, tgt_len, past_len, inputs_embeds)
         for i, layer in enumerate(self.layers if chained is None else ()):
             if output_hidden_states:
                 all_hidden += (hidden.clone(),)
