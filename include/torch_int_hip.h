@@ -413,6 +413,14 @@ int ti_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_new,
                       const float* mask, int8_t* ctx, int8_t* probs_out, int64_t BH, int64_t T, int64_t D, int64_t cap,
                       int64_t S, int64_t heads, float alpha_qk, float alpha_pv, void* stream);
 
+/* ti_decode_attn_s8 for a cache that has no room behind it: the S - T positions before this step are read from k_past /
+ * v_past ([BH, past_cap, D], past_cap >= S - T >= 1, 16-byte aligned, not overlapping the buffers) and written to k_buf / v_buf
+ * on the way, the new ones behind them.  k_past and v_past NULL: ti_decode_attn_s8.  Same arithmetic and bits. */
+int ti_decode_attn_s8_from(const int8_t* q, const int8_t* k_new, const int8_t* v_new, const int8_t* k_past,
+                           const int8_t* v_past, int64_t past_cap, int8_t* k_buf, int8_t* v_buf, const float* mask,
+                           int8_t* ctx, int64_t BH, int64_t T, int64_t D, int64_t cap, int64_t S, int64_t heads,
+                           float alpha_qk, float alpha_pv, void* stream);
+
 /* ti_decode_attn_s8 for a launch that is recorded once (HIP graph capture) and replayed while the cache grows: the
  * number of positions after the append is read from device memory (*s_dev, T <= *s_dev <= S_max) when the kernel
  * runs, S_max is the largest value it will ever hold (the launch is sized for it; S_max <= cap).  No mask, no
@@ -514,6 +522,12 @@ int64_t ti_opt_decoder_layer_prefill_chained_scratch_bytes(int64_t rows, int64_t
 int ti_opt_decoder_layer_decode_chained(const TiOptDecodeLayer* layer, void* hidden, const float* mask, int8_t* k_buf,
                                         int8_t* v_buf, int64_t B, int64_t cap, int64_t S, int chain, float* carry,
                                         void* scratch, int64_t scratch_bytes, void* stream);
+/* ti_opt_decoder_layer_decode_chained with the S - 1 positions before this step in other buffers (ti_decode_attn_s8_from):
+ * k_past / v_past [B, heads, past_cap, head_dim], or NULL. */
+int ti_opt_decoder_layer_decode_from(const TiOptDecodeLayer* layer, void* hidden, const float* mask, const int8_t* k_past,
+                                     const int8_t* v_past, int64_t past_cap, int8_t* k_buf, int8_t* v_buf, int64_t B,
+                                     int64_t cap, int64_t S, int chain, float* carry, void* scratch,
+                                     int64_t scratch_bytes, void* stream);
 int ti_opt_decoder_layer_prefill_chained(const TiOptDecodeLayer* layer, void* hidden, const float* mask,
                                          const uint8_t* mask_classes, int8_t* k_out, int8_t* v_out, int64_t B, int64_t T,
                                          int chain, float* carry, void* scratch, int64_t scratch_bytes, void* workspace,

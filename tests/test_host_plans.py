@@ -64,3 +64,23 @@ def test_two_continuations_of_one_past_get_rooms_of_their_own():
     assert both[0] is not both[1]
     opt._kv_give_back(first)
     assert opt._kv_rooms(past)[0] is first[0]
+
+
+def test_a_cache_without_room_is_left_to_the_kernel_only_where_it_lies_as_the_kernel_reads_it():
+    """Bare buffers only for both halves of a cache and for one pitch from row to row, head to head and sequence to sequence; any other
+    cache is copied first."""
+    from torch_int.models import opt
+    flat = torch.arange(2 * 3 * 10 * 16, dtype=torch.int32).to(torch.int8)
+    plain = flat.view(2, 3, 10, 16)
+    long = torch.cat([plain, plain], 2)[:, :, :10]
+    others = [torch.cat([plain, plain], 1)[:, :3], plain.transpose(0, 1).contiguous().transpose(0, 1), plain[:, :1].expand(2, 3, 10, 16),
+              plain.transpose(2, 3).contiguous().transpose(2, 3), torch.cat([flat[:3], flat])[3:].view(2, 3, 10, 16), plain[:, :, :0]]
+    for past, bare in ([((plain, plain), True), ((long, long), True), ((plain, long), False)]
+                       + [(pair, False) for o in others for pair in ((o, o), (plain[:, :, :o.shape[2]], o))]):
+        kk, vv = opt._kv_rooms(past)
+        S = past[0].shape[2]
+        assert kk.bare is vv.bare is bare and kk.filled == vv.filled == S + 1 and kk.buf.shape[2] > S
+        if not bare:
+            assert torch.equal(kk.buf[:, :, :S], past[0]) and torch.equal(vv.buf[:, :, :S], past[1])
+    kept = opt._kv_view(opt._KVBuffer(torch.zeros(2, 3, 80, 16, dtype=torch.int8), 10), 10)
+    assert [kv.bare for kv in opt._kv_rooms((kept, plain))] == [False, False]

@@ -657,11 +657,13 @@ int ti_attn_prefill_s8_mc(const int8_t* q, const int8_t* k, const int8_t* vt, co
 
 int ti_decode_attn_supported(int64_t T, int64_t S, int64_t D) { return decode_attn_supported(T, S, D) ? 1 : 0; }
 
-int ti_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_new, int8_t* k_buf, int8_t* v_buf,
-                      const float* mask, int8_t* ctx, int8_t* probs_out, int64_t BH, int64_t T, int64_t D, int64_t cap,
-                      int64_t S, int64_t heads, float alpha_qk, float alpha_pv, void* stream) {
+namespace {
+// k_past / v_past: the cache before this step where it lies in other buffers ([BH, past_cap, D]), else NULL
+int decode_attn(const char* op, const int8_t* q, const int8_t* k_new, const int8_t* v_new, const int8_t* k_past,
+                const int8_t* v_past, int64_t past_cap, int8_t* k_buf, int8_t* v_buf, const float* mask, int8_t* ctx,
+                int8_t* probs_out, int64_t BH, int64_t T, int64_t D, int64_t cap, int64_t S, int64_t heads, float alpha_qk,
+                float alpha_pv, void* stream) {
   g_err[0] = 0;
-  const char* op = "decode_attn_s8";
   const int64_t lim = 0x7fffffffLL;
   if (BH < 0 || T < 0 || D < 0 || cap < 0 || S < 0 || heads < 1 || BH > lim || cap > lim || heads > lim)
     return fail(TI_ERR_INVALID_ARG, "%s: sizes must be in [0, 2^31) and heads >= 1", op);
@@ -673,6 +675,11 @@ int ti_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_new,
                            (long long)cap);
   if (k_new != nullptr && S < T)
     return fail(TI_ERR_INVALID_ARG, "%s: S = %lld counts the %lld appended positions", op, (long long)S, (long long)T);
+  if ((k_past == nullptr) != (v_past == nullptr))
+    return fail(TI_ERR_INVALID_ARG, "%s: k_past and v_past must both be given or both be NULL", op);
+  if (k_past != nullptr && (k_new == nullptr || S <= T || past_cap < S - T || past_cap > lim))
+    return fail(TI_ERR_INVALID_ARG, "%s: a cache of %lld positions in buffers of %lld cannot be continued by %lld", op,
+                (long long)(S - T), (long long)past_cap, (long long)T);
   if (BH == 0) return TI_OK;
   if (!decode_attn_supported(T, S, D))
     return fail(TI_ERR_INVALID_ARG, "%s: unsupported shape T=%lld S=%lld head_dim=%lld (needs 1 <= T <= 4, head_dim a multiple of 16 up "
@@ -684,8 +691,26 @@ int ti_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_new,
   if (int rc = check_ptr(op, "v_buf", v_buf, 16, true)) return rc;
   if (int rc = check_ptr(op, "mask", mask, 4, mask != nullptr)) return rc;
   if (int rc = check_ptr(op, "ctx", ctx, 1, true)) return rc;
+  if (int rc = check_ptr(op, "k_past", k_past, 16, k_past != nullptr)) return rc;
+  if (int rc = check_ptr(op, "v_past", v_past, 16, v_past != nullptr)) return rc;
   return launch_decode_attn_s8(q, k_new, v_new, k_buf, v_buf, mask, ctx, probs_out, BH, T, D, cap, S, heads, alpha_qk,
-                               alpha_pv, static_cast<hipStream_t>(stream));
+                               alpha_pv, static_cast<hipStream_t>(stream), nullptr, k_past, v_past, past_cap);
+}
+}  // namespace
+
+int ti_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_new, int8_t* k_buf, int8_t* v_buf,
+                      const float* mask, int8_t* ctx, int8_t* probs_out, int64_t BH, int64_t T, int64_t D, int64_t cap,
+                      int64_t S, int64_t heads, float alpha_qk, float alpha_pv, void* stream) {
+  return decode_attn("decode_attn_s8", q, k_new, v_new, nullptr, nullptr, 0, k_buf, v_buf, mask, ctx, probs_out, BH, T, D,
+                     cap, S, heads, alpha_qk, alpha_pv, stream);
+}
+
+int ti_decode_attn_s8_from(const int8_t* q, const int8_t* k_new, const int8_t* v_new, const int8_t* k_past,
+                           const int8_t* v_past, int64_t past_cap, int8_t* k_buf, int8_t* v_buf, const float* mask,
+                           int8_t* ctx, int64_t BH, int64_t T, int64_t D, int64_t cap, int64_t S, int64_t heads,
+                           float alpha_qk, float alpha_pv, void* stream) {
+  return decode_attn("decode_attn_s8_from", q, k_new, v_new, k_past, v_past, past_cap, k_buf, v_buf, mask, ctx, nullptr, BH,
+                     T, D, cap, S, heads, alpha_qk, alpha_pv, stream);
 }
 
 int ti_decode_attn_s8_devlen(const int8_t* q, const int8_t* k_new, const int8_t* v_new, int8_t* k_buf, int8_t* v_buf,
@@ -805,8 +830,8 @@ int64_t decode_workspace_bytes(int64_t B, int64_t embed, int64_t ffn) {
   return most;
 }
 
-int decode_layer(const char* op, const TiOptDecodeLayer* L, void* hidden, const float* mask, int8_t* k_buf, int8_t* v_buf,
-                 int64_t B, int64_t cap, int64_t S, int chain, float* carry, void* scratch, int64_t scratch_bytes,
+int decode_layer(const char* op, const TiOptDecodeLayer* L, void* hidden, const float* mask, const int8_t* k_past,
+                 const int8_t* v_past, int64_t past_cap, int8_t* k_buf, int8_t* v_buf, int64_t B, int64_t cap, int64_t S, int chain, float* carry, void* scratch, int64_t scratch_bytes,
                  void* stream, int64_t most) {
   if (int rc = check_layer(op, L)) return rc;
   const int64_t E = L->embed, H = L->heads, d = L->head_dim, F = L->ffn;
@@ -839,8 +864,8 @@ int decode_layer(const char* op, const TiOptDecodeLayer* L, void* hidden, const 
   const float be3[3] = {L->beta_q, L->beta_k, L->beta_v};
   if ((rc = linear_group(op, x, w3, b3, o3, a3, be3, 3, B, E, E, 0, 0, stream, ws, ws_bytes))) return rc;
   // cache append + attention; [B, 1, E] rows are [B * heads, 1, head_dim] as they lie
-  if ((rc = ti_decode_attn_s8(q, k, v, k_buf, v_buf, mask, ctx, nullptr, B * H, 1, d, cap, S, H, L->alpha_qk, L->alpha_pv,
-                              stream)))
+  if ((rc = ti_decode_attn_s8_from(q, k, v, k_past, v_past, past_cap, k_buf, v_buf, mask, ctx, B * H, 1, d, cap, S, H,
+                                   L->alpha_qk, L->alpha_pv, stream)))
     return rc;
   return after_attention(L, ctx, f32, x, h, hidden, B, chain, carry, ws, ws_bytes, stream);
 }
@@ -914,15 +939,25 @@ int64_t ti_opt_decoder_layer_decode_scratch_bytes(int64_t B, int64_t embed, int6
 int ti_opt_decoder_layer_decode(const TiOptDecodeLayer* L, void* hidden, const float* mask, int8_t* k_buf, int8_t* v_buf,
                                 int64_t B, int64_t cap, int64_t S, void* scratch, int64_t scratch_bytes, void* stream) {
   g_err[0] = 0;
-  return decode_layer("opt_decoder_layer_decode", L, hidden, mask, k_buf, v_buf, B, cap, S, 0, nullptr, scratch, scratch_bytes, stream, 16);
+  return decode_layer("opt_decoder_layer_decode", L, hidden, mask, nullptr, nullptr, 0, k_buf, v_buf, B, cap, S, 0, nullptr, scratch,
+                      scratch_bytes, stream, 16);
 }
 
 int ti_opt_decoder_layer_decode_chained(const TiOptDecodeLayer* L, void* hidden, const float* mask, int8_t* k_buf,
                                         int8_t* v_buf, int64_t B, int64_t cap, int64_t S, int chain, float* carry,
                                         void* scratch, int64_t scratch_bytes, void* stream) {
   g_err[0] = 0;
-  return decode_layer("opt_decoder_layer_decode_chained", L, hidden, mask, k_buf, v_buf, B, cap, S, chain, carry, scratch,
-                      scratch_bytes, stream, 64);
+  return decode_layer("opt_decoder_layer_decode_chained", L, hidden, mask, nullptr, nullptr, 0, k_buf, v_buf, B, cap, S, chain,
+                      carry, scratch, scratch_bytes, stream, 64);
+}
+
+int ti_opt_decoder_layer_decode_from(const TiOptDecodeLayer* L, void* hidden, const float* mask, const int8_t* k_past,
+                                     const int8_t* v_past, int64_t past_cap, int8_t* k_buf, int8_t* v_buf, int64_t B,
+                                     int64_t cap, int64_t S, int chain, float* carry, void* scratch,
+                                     int64_t scratch_bytes, void* stream) {
+  g_err[0] = 0;
+  return decode_layer("opt_decoder_layer_decode_from", L, hidden, mask, k_past, v_past, past_cap, k_buf, v_buf, B, cap, S,
+                      chain, carry, scratch, scratch_bytes, stream, 64);
 }
 
 int64_t ti_opt_decoder_layer_prefill_scratch_bytes(int64_t rows, int64_t embed, int64_t ffn) {

@@ -50,11 +50,16 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // 7.8 -> 3.8, 128 x 904 21.5 -> 10.3, 768 x 250 20.0 -> 10.9, 768 x 904 36.5 -> 32.1 (5.5 TB/s), 128 x 2000 40.4 -> 18.3; head size
 // 64, 12 x 108 7.7 -> 3.6, 576 x 500 20.0 -> 10.8.
 // LDS: exponentials [Sp], maxima [NW], scale, probabilities as bytes [NW][RPW][NIP], partial outputs [NW][D].
-template <int D, int NW, int NI, bool PART>
+// MOVE: the rows before the new one are read from k_past / v_past and written into the buffers on the way, which saves a pass of
+// its own over the cache where it has to go to a buffer with room (the first step after a prefill, a full buffer): two strided
+// copies of 54 us a layer at 768 heads x 900 positions, eight tokens of 24 sequences on 16 layers of OPT-6.7B's width 14.50 ->
+// 13.50 ms.  A form of its own, so that the stores do not stand between the products of the other steps.
+template <int D, int NW, int NI, bool PART, bool MOVE>
 __global__ __launch_bounds__(NW * 64, 4) void decode_attn_one_kernel(
     const int8_t* __restrict__ q, const int8_t* __restrict__ k_new, const int8_t* __restrict__ v_new, int8_t* k_buf,
     int8_t* v_buf, const float* __restrict__ mask, int8_t* __restrict__ ctx, int8_t* __restrict__ probs_out, int S_arg,
-    long long cap, int heads, float alpha_qk, float alpha_pv, const int* __restrict__ s_dev, int dr_arg) {
+    long long cap, int heads, float alpha_qk, float alpha_pv, const int* __restrict__ s_dev, int dr_arg,
+    const int8_t* k_past, const int8_t* v_past, long long past_cap) {
   constexpr int LPR = D / 16;                // lanes per cache row
   constexpr int RPW = 64 / LPR;              // rows per wave per load
   constexpr int STEP = NW * RPW;             // rows per group
@@ -82,6 +87,8 @@ __global__ __launch_bounds__(NW * 64, 4) void decode_attn_one_kernel(
   const int S_old = grow ? S - 1 : S;
   int8_t* kb = k_buf + bh * cap * dr;
   int8_t* vb = v_buf + bh * cap * dr;
+  const int8_t* ko = MOVE ? k_past + bh * past_cap * dr : kb;  // the rows before the new one
+  const int8_t* vo = MOVE ? v_past + bh * past_cap * dr : vb;
   const v4i zero = {0, 0, 0, 0};
   const int col = in_row ? cs * 16 : 0;
 
@@ -105,8 +112,12 @@ __global__ __launch_bounds__(NW * 64, 4) void decode_attn_one_kernel(
       }
     }
   };
+  auto move_row = [&](int8_t* buf, int u, v4i row) {  // group u of the old rows goes into the buffer
+    const int s = base + u * STEP + rs;
+    if (s < S_old && in_row) *reinterpret_cast<v4i*>(buf + (unsigned)(s * dr + col)) = row;
+  };
   v4i kv[NI], vv[NI];
-  load_rows(kv, kb);
+  load_rows(kv, ko);
   // the additive mask of the scores this lane keeps, fetched together with the cache rows
   float mk[NJ];
   const float* msk = mask != nullptr ? mask + (bh / heads) * (long long)S : nullptr;
@@ -124,11 +135,12 @@ __global__ __launch_bounds__(NW * 64, 4) void decode_attn_one_kernel(
 #pragma unroll
   for (int u = 0; u < NI; ++u) {
     if (base + u * STEP >= S) break;  // the same for every lane of the wave
+    if (MOVE) move_row(kb, u, kv[u]);
     if (base + u * STEP <= S_old && S_old < base + u * STEP + RPW && rs == S_old - base - u * STEP) kv[u] = fresh_k;
     const int a = row_sum<LPR>(in_row ? dot16(kv[u], qr, 0) : 0);
     if (cs == u % LPR) own[u / LPR] = a;
   }
-  load_rows(vv, vb);  // on their way during the softmax; together with the keys they only cost registers
+  load_rows(vv, vo);  // on their way during the softmax; together with the keys they only cost registers
   float x[NJ], m = lowest;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
@@ -192,6 +204,7 @@ __global__ __launch_bounds__(NW * 64, 4) void decode_attn_one_kernel(
     for (int i = 0; i < 4; ++i) {
       const int u = u0 + i;
       r[i] = u < NI ? vv[u < NI ? u : 0] : zero;
+      if (MOVE && u < NI) move_row(vb, u, r[i]);
       if (u < NI && base + u * STEP <= S_old && S_old < base + u * STEP + RPW && rs == S_old - base - u * STEP)
         r[i] = fresh_v;
     }
@@ -257,7 +270,8 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(const int8_t* __restri
                                                           int8_t* v_buf, const float* __restrict__ mask,
                                                           int8_t* __restrict__ ctx, int8_t* __restrict__ probs_out,
                                                           int T, int S_arg, long long cap, int heads, float alpha_qk,
-                                                          float alpha_pv, const int* __restrict__ s_dev, int dr_arg) {
+                                                          float alpha_pv, const int* __restrict__ s_dev, int dr_arg,
+                                                          const int8_t* k_past, const int8_t* v_past, long long past_cap) {
   const int dr = PART ? dr_arg : D;
   // dr = the head size in memory, a multiple of 16 up to D (64 or 128, the lanes a cache row is spread over):
   // rows of q, the caches and ctx are dr bytes long; the lanes beyond a row hold zeros and store nothing
@@ -286,6 +300,10 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(const int8_t* __restri
   const int S_old = k_new != nullptr ? S - T : S;  // rows below come from the cache, the rest from k_new / v_new
   int8_t* kb = k_buf + bh * cap * dr;
   int8_t* vb = v_buf + bh * cap * dr;
+  // k_past != nullptr: the rows before the new ones come from there and go into the buffers as well
+  const bool move = k_past != nullptr;
+  const int8_t* ko = move ? k_past + bh * past_cap * dr : kb;
+  const int8_t* vo = move ? v_past + bh * past_cap * dr : vb;
   const int8_t* kn = k_new != nullptr ? k_new + bh * T * dr : nullptr;
   const int8_t* vn = v_new != nullptr ? v_new + bh * T * dr : nullptr;
 
@@ -296,20 +314,20 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(const int8_t* __restri
     qr[t] = t < T && in_row ? *reinterpret_cast<const v4i*>(q + (bh * T + t) * dr + cs * 16) : v4i{0, 0, 0, 0};
   constexpr int U = NI > 0 ? NI : 4;  // row groups in flight per wave
   // Rows past the end re-read the last row (their products are never used), so the loads need no branches;
-  // rows that come from k_new / v_new are also written into the cache.
-  auto load_rows = [&](int base, v4i (&dst)[U], int8_t* buf, const int8_t* fresh) {
+  // rows that come from k_new / v_new (or from another cache) are also written into the cache.
+  auto load_rows = [&](int base, v4i (&dst)[U], int8_t* buf, const int8_t* old, const int8_t* fresh) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       int s = base + u * 4 * RPW + rs;
       s = s < S ? s : S - 1;
-      const int8_t* src = s < S_old ? buf + (long long)s * dr : fresh + (long long)(s - S_old) * dr;
+      const int8_t* src = s < S_old ? old + (long long)s * dr : fresh + (long long)(s - S_old) * dr;
       dst[u] = in_row ? *reinterpret_cast<const v4i*>(src + cs * 16) : v4i{0, 0, 0, 0};
     }
     if (S_old < S) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int s = base + u * 4 * RPW + rs;
-        if (s >= S_old && s < S && in_row) *reinterpret_cast<v4i*>(buf + (long long)s * dr + cs * 16) = dst[u];
+        if ((move || s >= S_old) && s < S && in_row) *reinterpret_cast<v4i*>(buf + (long long)s * dr + cs * 16) = dst[u];
       }
     }
   };
@@ -345,15 +363,15 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(const int8_t* __restri
   if constexpr (NI > 0) {
     v4i kv[U];
     float mk[U][TQ];
-    load_rows(wave * RPW, kv, kb, kn);
+    load_rows(wave * RPW, kv, kb, ko, kn);
     load_mask(wave * RPW, mk);
-    load_rows(wave * RPW, vv, vb, vn);
+    load_rows(wave * RPW, vv, vb, vo, vn);
     score_rows(wave * RPW, kv, mk);
   } else {
     for (int base = wave * RPW; base < S; base += 4 * RPW * U) {
       v4i kv[U];
       float mk[U][TQ];
-      load_rows(base, kv, kb, kn);
+      load_rows(base, kv, kb, ko, kn);
       load_mask(base, mk);
       score_rows(base, kv, mk);
     }
@@ -433,7 +451,7 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(const int8_t* __restri
     weigh_rows(wave * RPW);
   } else {
     for (int base = wave * RPW; base < S; base += 4 * RPW * U) {
-      load_rows(base, vv, vb, vn);
+      load_rows(base, vv, vb, vo, vn);
       weigh_rows(base);
     }
   }
@@ -475,7 +493,8 @@ bool decode_attn_supported(long long T, long long S, long long D) {
 int launch_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_new, int8_t* k_buf, int8_t* v_buf,
                           const float* mask, int8_t* ctx, int8_t* probs_out, long long BH, long long T, long long D,
                           long long cap, long long S, long long heads, float alpha_qk, float alpha_pv,
-                          hipStream_t stream, const int* s_dev) {
+                          hipStream_t stream, const int* s_dev, const int8_t* k_past, const int8_t* v_past,
+                          long long past_cap) {
   // with s_dev the kernel reads the length from device memory; S is the largest value it may find there (the LDS
   // and the kernel variant are sized for it)
   if (BH == 0) return TI_OK;
@@ -495,14 +514,16 @@ int launch_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_
   // only its bound: 320 heads, bound 2048, length 20 / 512 / 1024 / 2048 9.1 / 13.7 / 25.4 / 44.9 us, streaming 5.6 / 13.0 /
   // 25.0 / 44.4 (a length the host knows, 300 heads x 2040: 40.3, streaming 44.0; head size 80 keeps it, 18.0 against 25.9 at 1024).
   const long long groups = (S + 64 / (lanes_d / 16) - 1) / (64 / (lanes_d / 16));
-#define TI_DA1(DD, NW, NI)                                                                                             \
-  do {                                                                                                                 \
-    if (D == DD)                                                                                                       \
-      hipLaunchKernelGGL((decode_attn_one_kernel<DD, NW, NI, false>), grid, dim3(NW * 64), 0, stream, q, k_new, v_new, \
-                         k_buf, v_buf, mask, ctx, probs_out, (int)S, cap, (int)heads, alpha_qk, alpha_pv, s_dev, (int)D); \
-    else                                                                                                               \
-      hipLaunchKernelGGL((decode_attn_one_kernel<DD, NW, NI, true>), grid, dim3(NW * 64), 0, stream, q, k_new, v_new,  \
-                         k_buf, v_buf, mask, ctx, probs_out, (int)S, cap, (int)heads, alpha_qk, alpha_pv, s_dev, (int)D); \
+#define TI_DA1_LAUNCH(DD, NW, NI, PART, MOVE)                                                                          \
+  hipLaunchKernelGGL((decode_attn_one_kernel<DD, NW, NI, PART, MOVE>), grid, dim3(NW * 64), 0, stream, q, k_new, v_new, \
+                     k_buf, v_buf, mask, ctx, probs_out, (int)S, cap, (int)heads, alpha_qk, alpha_pv, s_dev, (int)D,    \
+                     k_past, v_past, past_cap)
+#define TI_DA1(DD, NW, NI)                                          \
+  do {                                                              \
+    if (D == DD && k_past == nullptr) TI_DA1_LAUNCH(DD, NW, NI, false, false); \
+    else if (D == DD) TI_DA1_LAUNCH(DD, NW, NI, false, true);       \
+    else if (k_past == nullptr) TI_DA1_LAUNCH(DD, NW, NI, true, false); \
+    else TI_DA1_LAUNCH(DD, NW, NI, true, true);                     \
   } while (0)
 #define TI_DA1_FORMS(DD)                                            \
   do {                                                              \
@@ -520,10 +541,12 @@ int launch_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_
   do {                                                                                                                 \
     if (D == DD)                                                                                                       \
       hipLaunchKernelGGL((decode_attn_kernel<TQ, DD, NI, false>), grid, block, lds, stream, q, k_new, v_new, k_buf,    \
-                         v_buf, mask, ctx, probs_out, (int)T, (int)S, cap, (int)heads, alpha_qk, alpha_pv, s_dev, (int)D); \
+                         v_buf, mask, ctx, probs_out, (int)T, (int)S, cap, (int)heads, alpha_qk, alpha_pv, s_dev, (int)D,  \
+                         k_past, v_past, past_cap); \
     else                                                                                                               \
       hipLaunchKernelGGL((decode_attn_kernel<TQ, DD, NI, true>), grid, block, lds, stream, q, k_new, v_new, k_buf,     \
-                         v_buf, mask, ctx, probs_out, (int)T, (int)S, cap, (int)heads, alpha_qk, alpha_pv, s_dev, (int)D); \
+                         v_buf, mask, ctx, probs_out, (int)T, (int)S, cap, (int)heads, alpha_qk, alpha_pv, s_dev, (int)D,  \
+                         k_past, v_past, past_cap); \
   } while (0)
   const bool one = T == 1 && (groups <= 128 || (groups <= 256 && BH <= (s_dev != nullptr && D > 96 ? 256 : 512)));
   // caches of at most 20 row groups per lane (640 positions at head size 128) with two query rows take
@@ -542,6 +565,7 @@ int launch_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_
   }
 #undef TI_DA1_FORMS
 #undef TI_DA1
+#undef TI_DA1_LAUNCH
 #undef TI_DA
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "decode_attn launch: %s", hipGetErrorString(e));

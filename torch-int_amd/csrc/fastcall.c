@@ -196,22 +196,24 @@ static PyObject* fc_decode_attn(PyObject* self, PyObject* const* a, Py_ssize_t n
                                            (float)apv, st));
 }
 
-/* opt_layer_decode(layer, hidden, mask, k_buf, v_buf, B, cap, S, chain, carry, scratch, scratch_bytes, stream) -> status;
+/* opt_layer_decode(layer, hidden, mask, k_past, v_past, past_cap, k_buf, v_buf, B, cap, S, chain, carry, scratch, scratch_bytes, stream) -> status;
  * layer = address of a TiOptDecodeLayer that the caller keeps alive */
 static PyObject* fc_opt_layer_decode(PyObject* self, PyObject* const* a, Py_ssize_t n) {
   (void)self;
-  if (n != 13) {
-    PyErr_SetString(PyExc_TypeError, "opt_layer_decode expects 13 arguments");
+  if (n != 16) {
+    PyErr_SetString(PyExc_TypeError, "opt_layer_decode expects 16 arguments");
     return NULL;
   }
-  void *layer = as_ptr(a[0]), *hidden = as_ptr(a[1]), *mask = as_ptr(a[2]), *kb = as_ptr(a[3]), *vb = as_ptr(a[4]);
-  int64_t B = as_i64(a[5]), cap = as_i64(a[6]), S = as_i64(a[7]), chain = as_i64(a[8]);
-  void *carry = as_ptr(a[9]), *scratch = as_ptr(a[10]);
-  int64_t sb = as_i64(a[11]);
-  void* st = as_ptr(a[12]);
+  void *layer = as_ptr(a[0]), *hidden = as_ptr(a[1]), *mask = as_ptr(a[2]), *kp = as_ptr(a[3]), *vp = as_ptr(a[4]);
+  int64_t past_cap = as_i64(a[5]);
+  void *kb = as_ptr(a[6]), *vb = as_ptr(a[7]);
+  int64_t B = as_i64(a[8]), cap = as_i64(a[9]), S = as_i64(a[10]), chain = as_i64(a[11]);
+  void *carry = as_ptr(a[12]), *scratch = as_ptr(a[13]);
+  int64_t sb = as_i64(a[14]);
+  void* st = as_ptr(a[15]);
   if (PyErr_Occurred()) return NULL;
-  return PyLong_FromLong(ti_opt_decoder_layer_decode_chained((const TiOptDecodeLayer*)layer, hidden, (const float*)mask, kb,
-                                                             vb, B, cap, S, (int)chain, carry, scratch, sb, st));
+  return PyLong_FromLong(ti_opt_decoder_layer_decode_from((const TiOptDecodeLayer*)layer, hidden, (const float*)mask, kp, vp,
+                                                          past_cap, kb, vb, B, cap, S, (int)chain, carry, scratch, sb, st));
 }
 
 /* opt_layer_prefill(layer, hidden, mask, classes, k_out, v_out, B, T, chain, carry, scratch, scratch_bytes, ws, ws_bytes, stream) -> status */
@@ -316,7 +318,7 @@ static PyMethodDef methods[] = {
     {"linear_group3", (PyCFunction)(void (*)(void))fc_linear_group3, METH_FASTCALL, "forward to ti_linear_a8_w8_b8_o8_group"},
     {"kv_append", (PyCFunction)(void (*)(void))fc_kv_append, METH_FASTCALL, "forward to ti_kv_append_s8"},
     {"decode_attn", (PyCFunction)(void (*)(void))fc_decode_attn, METH_FASTCALL, "forward to ti_decode_attn_s8"},
-    {"opt_layer_decode", (PyCFunction)(void (*)(void))fc_opt_layer_decode, METH_FASTCALL, "forward to ti_opt_decoder_layer_decode_chained"},
+    {"opt_layer_decode", (PyCFunction)(void (*)(void))fc_opt_layer_decode, METH_FASTCALL, "forward to ti_opt_decoder_layer_decode_from"},
     {"opt_layer_prefill", (PyCFunction)(void (*)(void))fc_opt_layer_prefill, METH_FASTCALL, "forward to ti_opt_decoder_layer_prefill_chained"},
     {"plan_current", (PyCFunction)(void (*)(void))fc_plan_current, METH_FASTCALL, "tensors and hooks as a plan found them"},
     {"last_error", fc_last_error, METH_NOARGS, "ti_last_error()"},

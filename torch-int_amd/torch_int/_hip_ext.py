@@ -118,11 +118,14 @@ _lib.ti_opt_decoder_layer_prefill.restype = ctypes.c_int
 _lib.ti_opt_decoder_layer_decode_chained.argtypes = [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, ctypes.c_int, _vp, _vp, _i64,
                                                      _vp]
 _lib.ti_opt_decoder_layer_decode_chained.restype = ctypes.c_int
+_lib.ti_opt_decoder_layer_decode_from.argtypes = [_vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _i64, _i64, _i64, ctypes.c_int,
+                                                  _vp, _vp, _i64, _vp]
+_lib.ti_opt_decoder_layer_decode_from.restype = ctypes.c_int
 _lib.ti_opt_decoder_layer_prefill_chained.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, ctypes.c_int, _vp, _vp, _i64,
                                                       _vp, _i64, _vp]
 _lib.ti_opt_decoder_layer_prefill_chained.restype = ctypes.c_int
 _raw_stream = torch._C._cuda_getCurrentRawStream
-_opt_layer_decode = getattr(_CUDA._fast, "opt_layer_decode", None) or _lib.ti_opt_decoder_layer_decode_chained
+_opt_layer_decode = getattr(_CUDA._fast, "opt_layer_decode", None) or _lib.ti_opt_decoder_layer_decode_from
 _opt_layer_prefill = getattr(_CUDA._fast, "opt_layer_prefill", None) or _lib.ti_opt_decoder_layer_prefill_chained
 _fast = _CUDA._fast if getattr(_CUDA._fast, "kv_append", None) is not None else None
 _fast_decode_attn = getattr(_CUDA._fast, "decode_attn", None)
@@ -624,10 +627,11 @@ def opt_decode_scratch(plans, hidden):
         return _scratch_for(dev, _raw_stream(dev.index), need)
 
 
-def opt_layer_decode(plan, hidden, mask, k_buf, v_buf, S, chain=0, carry=None, scratch=None):
-    """One decode step of one decoder layer from one C call (``ti_opt_decoder_layer_decode_chained``): ``hidden`` [B, 1, embed]
+def opt_layer_decode(plan, hidden, mask, k_buf, v_buf, S, chain=0, carry=None, scratch=None, past=None):
+    """One decode step of one decoder layer from one C call (``ti_opt_decoder_layer_decode_from``): ``hidden`` [B, 1, embed]
     (fp32, or fp16 when the plan says half; up to 64 sequences) is updated in place, the new key and value rows are appended
-    to the cache buffers, which hold S - 1 positions before the call.  ``plan`` carries ``addr`` (the address of an
+    to the cache buffers, which hold S - 1 positions before the call (or are given them: ``past``, the key and value cache elsewhere, as
+    ``cache_rows_movable`` accepts them).  ``plan`` carries ``addr`` (the address of an
     ``OptDecodeLayer`` that the caller filled from tensors it keeps alive), ``embed`` and ``ffn``; the caller has checked
     shapes, dtypes, devices and contiguity (the decoder layer does).  ``chain`` and ``carry`` (fp32 [B, embed], of this pass)
     tie the layers of one forward pass together, which share ``scratch`` (``opt_decode_scratch``)."""
@@ -637,12 +641,24 @@ def opt_layer_decode(plan, hidden, mask, k_buf, v_buf, S, chain=0, carry=None, s
         stream = _raw_stream(dev.index)
         if scratch is None:
             scratch = opt_decode_scratch((plan,), hidden)
-        rc = _opt_layer_decode(plan.addr, hidden.data_ptr(), mask.data_ptr() if mask is not None else 0, k_buf.data_ptr(),
-                               v_buf.data_ptr(), B, k_buf.shape[2], S, chain, carry.data_ptr() if chain else 0, scratch.data_ptr(),
+        k_past, v_past, past_cap = (0, 0, 0) if past is None else (past[0].data_ptr(), past[1].data_ptr(),
+                                                                   past[0].stride(1) // past[0].stride(2))
+        rc = _opt_layer_decode(plan.addr, hidden.data_ptr(), mask.data_ptr() if mask is not None else 0, k_past, v_past,
+                               past_cap, k_buf.data_ptr(), v_buf.data_ptr(), B, k_buf.shape[2], S, chain, carry.data_ptr() if chain else 0, scratch.data_ptr(),
                                scratch.numel(), stream)
     if rc:
         raise RuntimeError(f"torch_int._hip_ext.opt_layer_decode: {_lib.ti_last_error().decode()} (status {rc})")
     return hidden
+
+
+def cache_rows_movable(past):
+    """Whether the decode step can read the key and value cache ``past`` ([bsz, heads, length, head_dim], int8) where it lies:
+    rows of head_dim bytes one after the other, one pitch from head to head and from sequence to sequence, for both."""
+    k, v = past
+    b, h, n, d = k.shape
+    sb, sh, sn, sd = strides = k.stride()
+    return (n > 0 and sd == 1 and sn == d and sh % d == 0 and sh >= n * d and sb == h * sh and v.stride() == strides
+            and k.data_ptr() % 16 == 0 and v.data_ptr() % 16 == 0)
 
 
 def opt_prefill_scratch(plans, hidden):

@@ -26,11 +26,12 @@ from ..nn.linear import W8A8B8O8Linear, W8A8B8O8LinearReLU, W8A8BFP32OFP32Linear
 class _KVBuffer:
     """Backing store of one growing K or V cache tensor: ``buf`` is [bsz, heads, capacity, head_dim] and the
     first ``filled`` positions hold tokens.  The tensors handed out as ``past_key_value`` are views
-    ``buf[:, :, :n]`` that carry a reference to this object."""
-    __slots__ = ("buf", "filled")
+    ``buf[:, :, :n]`` that carry a reference to this object.  ``bare``: the tokens are still elsewhere, and the kernel that
+    appends the next one moves them here."""
+    __slots__ = ("buf", "filled", "bare")
 
-    def __init__(self, buf, filled):
-        self.buf, self.filled = buf, filled
+    def __init__(self, buf, filled, bare=False):
+        self.buf, self.filled, self.bare = buf, filled, bare
 
 
 def _kv_room(past, new):
@@ -54,35 +55,47 @@ def _kv_room_for(past, T):
     return None
 
 
-def _kv_fresh(past, T):
-    """A new buffer holding ``past`` with room for T + max(64, a quarter of the length) further positions."""
+def _kv_empty(past, T):
+    """A bare buffer for ``past`` with room for T + max(64, a quarter of the length) further positions."""
     S = past.shape[2]
     cap = -(-(S + T + max(64, (S + T) // 4)) // 16) * 16
     buf = torch.empty((past.shape[0], past.shape[1], cap, past.shape[3]), dtype=past.dtype, device=past.device)
-    buf[:, :, :S].copy_(past)
-    return _KVBuffer(buf, S)
+    return _KVBuffer(buf, S, bare=True)
+
+
+def _kv_fresh(past, T):
+    """A new buffer holding ``past`` with room behind it."""
+    kv = _kv_empty(past, T)
+    kv.buf[:, :, :past.shape[2]].copy_(past)
+    kv.bare = False
+    return kv
 
 
 _kv_lock = threading.Lock()
 
 
 def _kv_claim(past):
-    """A buffer with room for one more position behind ``past``, taken: it counts as filled from here on, so that nobody else
-    who continues the same past (another thread, while this one's layers are on their way) is given the same position."""
-    S = past.shape[2]
+    """The buffer with room for one more position behind ``past``, taken, or None: it counts as filled from here on, so that nobody
+    else who continues the same past (another thread, while this one's layers are on their way) is given the same position."""
     with _kv_lock:
         kv = _kv_room_for(past, 1)
         if kv is not None:
-            kv.filled = S + 1
-            return kv
-    kv = _kv_fresh(past, 1)
-    kv.filled = S + 1
-    return kv
+            kv.filled = past.shape[2] + 1
+        return kv
 
 
 def _kv_rooms(past):
-    """``_kv_claim`` for a layer's (key, value) cache, or None when a kernel cannot write there."""
+    """Buffers for one more position behind a layer's (key, value) cache, taken (``_kv_claim``), both of them bare where there is no
+    room and the kernel that appends can read the cache as it lies; None when a kernel cannot write there."""
     kk, vv = _kv_claim(past[0]), _kv_claim(past[1])
+    if kk is None or vv is None:
+        new = _kv_empty if kk is None and vv is None and _hip_ext.cache_rows_movable(past) else _kv_fresh
+        if kk is None:
+            kk = new(past[0], 1)
+            kk.filled += 1
+        if vv is None:
+            vv = new(past[1], 1)
+            vv.filled += 1
     kb, vb = kk.buf, vv.buf
     if kb.data_ptr() % 16 or vb.data_ptr() % 16 or not (kb.is_contiguous() and vb.is_contiguous() and kb.shape == vb.shape):
         _kv_give_back((kk, vv))
@@ -93,6 +106,14 @@ def _kv_rooms(past):
 def _kv_give_back(rooms):
     for kv in rooms:
         kv.filled -= 1
+
+
+def _kv_append_in_layer(plan, hidden, mask, rooms, past, S, **chain):
+    """One layer's decode step, which appends to ``rooms`` (``_kv_rooms(past)``) and moves the past there if they are bare."""
+    kk, vv = rooms
+    _hip_ext.opt_layer_decode(plan, hidden, mask, kk.buf, vv.buf, S, past=past if kk.bare else None, **chain)
+    kk.bare = vv.bare = False
+    return _kv_view(kk, S), _kv_view(vv, S)
 
 
 def _kv_view(kv, n):
@@ -590,10 +611,10 @@ class Int8OPTDecoderLayer(nn.Module):
         rooms = found and _kv_rooms(past_key_value)
         if not rooms:
             return None
-        (plan, S), (kk, vv) = found, rooms
-        _hip_ext.opt_layer_decode(plan, hidden_states, mask, kk.buf, vv.buf, S)
+        plan, S = found
+        present = _kv_append_in_layer(plan, hidden_states, mask, rooms, past_key_value, S)
         if use_cache:
-            return hidden_states, (_kv_view(kk, S), _kv_view(vv, S))
+            return hidden_states, present
         return (hidden_states,)
 
     #: a prefill (more than 16 tokens per sequence, a multiple of 16) likewise: up to 4096 tokens a layer's kernels take less
@@ -840,10 +861,10 @@ class Int8OPTDecoder(nn.Module):
                 _kv_give_back(kv for pair in rooms if pair for kv in pair)
                 return None
             scratch = _hip_ext.opt_decode_scratch([plan for plan, _ in found], hidden)
-            for (plan, S), (kk, vv), chain in zip(found, rooms, links):
-                _hip_ext.opt_layer_decode(plan, hidden, mask, kk.buf, vv.buf, S, chain=chain, carry=carry, scratch=scratch)
+            for (plan, S), room, past, chain in zip(found, rooms, past_key_values, links):
+                present = _kv_append_in_layer(plan, hidden, mask, room, past, S, chain=chain, carry=carry, scratch=scratch)
                 if use_cache:
-                    cache.append((_kv_view(kk, S), _kv_view(vv, S)))
+                    cache.append(present)
         else:
             memory = _hip_ext.opt_prefill_scratch(found, hidden)
             for plan, chain in zip(found, links):
