@@ -14,13 +14,16 @@ long long gemm_workspace_bytes(long long M, long long N, long long K, bool least
     const int r = row_split_rows(M, N, K, &need);
     if (r <= 0) return 0;
     // the first rows are a problem of their own too: at exactly 1024 of them they may split K themselves
-    const long long head = M - r <= 1024 ? gemm_workspace_bytes(M - r, N, K, least) : 0;
-    return head > need ? head : need;
+    const long long head = M - r <= 1024 ? gemm_workspace_bytes(M - r, N, K, least) : 0, rest = gemm_workspace_bytes(r, N, K, least);
+    return head > need ? (head > rest ? head : rest) : need > rest ? need : rest;
   }
   const RowsPick rows = least ? RowsPick{ROWS_NONE, 1} : rows_pick(M, N, K);
   if (M > 16 && rows.tiling != ROWS_NONE && (N % 16 == 0 || K % SBK == 0)) return rows.slices > 1 ? (long long)rows.slices * M * N * 4 : 0;
-  const int s = choose_splits(M, N, K, nullptr, nullptr, 1, !least);
-  return s > 1 ? (long long)s * M * N * 4 : 0;
+  int tile = SPLIT_128;
+  const int s = choose_splits(M, N, K, &tile, nullptr, 1, !least);
+  if (s <= 1) return 0;
+  long long one_launch = 0;
+  return !least && one_launch_split(tile, s, M, N, K, &one_launch) ? one_launch : (long long)s * M * N * 4;
 }
 
 // one per epilogue kind (EpiKind value n), each in its own translation unit
@@ -423,6 +426,8 @@ int warm_fused_split(void* stream) {
 }
 
 int launch_splitk_raw(int tile, const GemmParams& q, hipStream_t stream) {
+  if (tile == SPLIT_128 && split_128_deep((long long)((q.M + 127) / 128) * ((q.N + 127) / 128) * q.batch, q.K, false, num_cus()))
+    return launch_pipe16q<Pipe16QCfg<128, 128, 4, 2, EPI_S32_RAW, false, 5>>(q, stream);
   if (tile == SPLIT_128) return launch_pipe<PipeCfg<128, 128, 2, 2, 4, EPI_S32_RAW, false>>(q, stream);
   if (tile == SPLIT_256x160) return launch_pipe16q<Pipe16QCfg<256, 160, 4, 2, EPI_S32_RAW>>(q, stream);
   if (tile == SPLIT_160x160) return launch_pipe16q<Pipe16QCfg<160, 160, 2, 2, EPI_S32_RAW>>(q, stream);

@@ -1308,6 +1308,7 @@ struct Pipe16QCfg {
   static constexpr int BM = BM_, BN = BN_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, KIND = KIND_;
   static constexpr bool FUSED = FUSED_;
   static_assert(!(FUSED_ && GROUPED_), "the fused split takes one problem");
+  static constexpr bool RAGGED = FUSED_ && (BN_ == 128 || BN_ == 192);  // FUSED for any M, see one_launch_split
   // GROUPED: the "batches" are the problems of a GemmGroup (same activations and shape; weight, bias,
   // output and scales per problem), so that q/k/v projections run as one persistent launch
   static constexpr bool GROUPED = GROUPED_;
@@ -1559,7 +1560,9 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_pipe16q_kernel(GemmParams p, 
     tile_of_workgroup(tile_id, tiles_m, tiles_n, tile_m, tile_n, p.band);
     int lane_here = lane;  // opaque copy: keeps the epilogue's address arithmetic out of the mainloop
     asm volatile("" : "+v"(lane_here));
-    if constexpr (Cfg::FUSED) {
+    // A wave whose rows all lie beyond M has nothing to park or to store, in any slice (wave 0 of a tile always has).
+    if (Cfg::RAGGED && tile_m * BM + wave_m * Cfg::WTM >= M) {
+    } else if constexpr (Cfg::FUSED) {
       constexpr long long PER_WAVE = (long long)TM * TN * 64;  // v4i elements a wave parks per (tile, slice)
       const int splits = p.splits;
       v4i* parts = reinterpret_cast<v4i*>(p.parts);
@@ -2336,8 +2339,19 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmParams p, const 
 // they would, while without it 800x2560x10240 took 44.4 us instead of 39.8 and 770x6400x5120 55.3 instead of 36.5.  One row of
 // tiles in two slices (129 to 160 rows) is priced evenly against the 256-row tiles it replaces: 130x20480x5120 0.82 times
 // their time, 160x20480x5120 0.95; with more slices 160x7680x20480 lost 13 %.
+//
+// 128x128 tiles with a CU to themselves step 128 bytes at a time through five stages (split_128_deep): 0.25 us per 64 bytes and
+// 5 TB/s, against 0.35 us and 3.5 TB/s, which is what two workgroups that share a CU still run at.  At that price they replace
+// 256x256 tiles (257x4096x16384 47.7 -> 36.8 us, 90x16384x4096 30.5 -> 20.1), 128x160 and 256x160 ones (384x5120x5120 26.0 ->
+// 23.3, 700x2560x10240 37.3 -> 30.8, 350x5120x20480 58.8 -> 56.9) and unsplit products (see the pairs at one_launch_split).
 enum SplitTile { SPLIT_128 = 0, SPLIT_256 = 1, SPLIT_256x160 = 2, SPLIT_256x288 = 3, SPLIT_128x160 = 4, SPLIT_128x288 = 5,
                  SPLIT_128x80 = 6, SPLIT_128x192 = 7, SPLIT_256x192 = 8, SPLIT_160x160 = 9 };
+// Slices on 128x128 tiles whose workgroups all have a CU to themselves run on the kernel with 128-byte steps, where a slice is long
+// enough for its five stages, or the slices meet in one launch, which only that kernel can.  (Sixteen slices of 512, two
+// launches: 100x2048x8192 19.1 us with 64-byte steps, 19.4 with 128; 256x2048x8192, eight of 1024, 19.0 / 18.6.)
+static inline bool split_128_deep(long long workgroups, long long slice, bool one_launch, long long cus) {
+  return slice % QBK == 0 && workgroups <= cus && (one_launch || slice >= 1024);
+}
 // `batch` > 1: a batched product (A and B per batch); every tile count, byte count and the streaming floor scale with
 // it, the one-launch form is not available, and the tile shapes are those that exist for every epilogue of the
 // raw-int32 kernels.
@@ -2387,7 +2401,21 @@ static int choose_splits(long long M, long long N, long long K, int* tile_kind =
       if (s == 1 && (wide192 || tall192) && tiles > cus) continue;  // more than a round: left to the ordinary dispatch
       const double wgs = tiles * s;
       double rounds, step_us, fixed_us = 8.0;
-      if (kind == SPLIT_128) {
+      // (not against the tiles of widths that 192 or 160 divide, but for 160 where those pad the rows as 128 does and more than one
+      // row of tiles shares the weights: 100x5120x20480 31.2 us in eight slices of 128x160, 37.4 so)
+      // (nor where a K of 2048 or less and more than 32 tiles leave the product to the 64x64 tiles, unsplit: 800x2048x2048 12.7 us,
+      // in two slices 13.8; 256x2048x2048 in four 12.0)
+      // (and where slices leave half of the CUs idle, twice as many in two launches: 256x2048x8192 in four slices 19.3 us, in eight
+      // 18.6)
+      const bool deep = kind == SPLIT_128 && batch == 1 && s > 1 && N % 192 != 0 && (K > 2048 || tiles <= 32.0) &&
+                        (N % 160 != 0 || (M > 128 && (M + 159) / 160 * 160 >= (M + 127) / 128 * 128)) &&
+                        split_128_deep((long long)wgs, K / s, s <= 4 && N % 128 == 0, (long long)cus) &&
+                        !(wgs * 2 <= cus && K % (2 * s * QBK) == 0 && K / (2 * s) >= 1024);
+      if (deep) {
+        rounds = 1.0;
+        step_us = 0.25;
+        fixed_us = 7.5;
+      } else if (kind == SPLIT_128) {
         rounds = (double)(long long)((wgs + 2 * cus - 1) / (2 * cus));
         step_us = wgs <= cus ? 0.35 : 0.70;
       } else if (small) {  // two fit a CU and then share it
@@ -2406,19 +2434,20 @@ static int choose_splits(long long M, long long N, long long K, int* tile_kind =
       // all resident workgroups have in flight over a 2 us round trip bounds the streaming rate (5 TB/s at most).
       const double ahead = kind == SPLIT_128 ? 4.0 : kind == SPLIT_256x160 || half || small || wide192 || square ? 2.5 : 1.5;
       const double step_bytes = (double)bn * (kind == SPLIT_128 ? 64.0 : 128.0);
-      const double resident = wgs < cus * (kind == SPLIT_128 ? 2 : 1) ? wgs : cus * (kind == SPLIT_128 ? 2 : 1);
+      const double resident = wgs < cus * (kind == SPLIT_128 && !deep ? 2 : 1) ? wgs : cus * (kind == SPLIT_128 && !deep ? 2 : 1);
       double rate = resident * ahead * step_bytes / 2.0;  // bytes per us
       // 5 TB/s at most; 3.5 TB/s for the 64-byte steps of the 128x128 tiles, which ask for every line twice
       // (128x9216x36864: 110 us against 83 us with 128x288 tiles)
       // (128x80 tiles ask for 80 scattered lines per step: 3.8 TB/s, 2.4 TB/s when two workgroups share a CU:
       // 128x20480x5120 30 us, 256x20480x5120 48 us)
-      const double cap = kind == SPLIT_128 ? 3.5e6 : small ? (wgs <= cus ? 3.8e6 : 2.4e6) : 5.0e6;
+      const double cap = kind == SPLIT_128 && !deep ? 3.5e6 : small ? (wgs <= cus ? 3.8e6 : 2.4e6) : 5.0e6;
       if (rate > cap) rate = cap;
       const double t_stream = (double)batch * (double)N * (double)K / rate + (small ? 4.0 : 8.0);
       if (t < t_stream) t = t_stream;
       // the slices' partial tiles: written once and read once (they mostly stay in the last-level cache) plus the
       // second launch; in the one-launch form they stay in the XCD's L2 and the reading is the last workgroup's tail
-      const bool one_launch = batch == 1 && kind >= SPLIT_256x160 && !square && M % bm == 0 && s <= (kind == SPLIT_256x288 ? 2 : 4);
+      const bool one_launch = batch == 1 && ((kind >= SPLIT_256x160 && !square && M % bm == 0 && s <= (kind == SPLIT_256x288 ? 2 : 4)) ||
+                                             (deep && s <= 4 && N % 128 == 0));
       if (s > 1 && one_launch) t += (double)(2 * s - 1) * M * N * 4.0 / 8.0e6 + 1.0;
       else if (s > 1) t += (double)batch * (double)(2 * s + 1) * M * N * 4.0 / 5.5e6 + 3.0;  // at 5.5 TB/s, in us
       if (square) {  // weighed against the best of the others below
@@ -2458,6 +2487,38 @@ int launch_splitk_raw(int tile, const GemmParams& q, hipStream_t stream);
 // TI_ERR_* code when an earlier fused launch reported a misplaced workgroup.
 int fused_split_prepare(hipStream_t stream, long long counters, GemmParams& q);
 
+// Rows and columns of the split tilings.
+static inline int split_bm(int tile) { return tile == SPLIT_256 || tile == SPLIT_256x160 || tile == SPLIT_256x288 || tile == SPLIT_256x192 ? 256 : tile == SPLIT_160x160 ? 160 : 128; }
+static inline int split_bn(int tile) {
+  return tile == SPLIT_128x80 ? 80 : tile == SPLIT_128 ? 128 : tile == SPLIT_256 ? 256 : tile == SPLIT_128x192 || tile == SPLIT_256x192 ? 192
+         : tile == SPLIT_256x288 || tile == SPLIT_128x288 ? 288 : 160;
+}
+
+// Whether a split product can be one launch (gemm_pipe16q_kernel, FUSED), but for the epilogue, the stream and the workspace, and
+// the workspace it needs then: the tiles are parked whole, rows beyond M included.  (Parked row by row, in the room of the outputs,
+// the adding wave's loads came one by one: 400x4096x4096 24.6 us instead of 17.7.)
+static inline bool one_launch_split(int tile, int splits, long long M, long long N, long long K, long long* bytes) {
+  const int bm = split_bm(tile), bn = split_bn(tile);
+  const long long tiles_m = (M + bm - 1) / bm;
+  *bytes = tiles_m * bm * N * 4 * splits;
+  // Rows that end inside a tile: 128x128 tiles (72 to 1000 rows of widths 2048 to 16384, cold, 44 shapes against two launches and
+  // 64-byte steps: 0.69 to 1.01 times the time, 0.83 in the mean; 400x4096x4096 23.3 -> 17.7 us, 1000x2048x8192 37.0 -> 27.8), and
+  // 128x192 ones from three row tiles on (800x768x3072 18.4 -> 16.1, 350 rows 15.0 / 14.7, but 200 rows 13.9 / 14.4).  The others
+  // gained nothing: 128x80 0.99 times the two launches, 128x160 0.98, 256x160 1.01, and 160x160 tiles, 25 blocks a wave, spill.
+  if (tile == SPLIT_160x160 || (M % bm != 0 && tile != SPLIT_128 && !(tile == SPLIT_128x192 && M > 320))) return false;
+  // up to four slices: the wave that arrives last reads the others' accumulators one slice after the other,
+  // and beyond four that tail costs more than the reduction launch it saves (measured: 2 slices -3 to -12 %,
+  // 4 slices -3 to -8 %, 7 and 8 slices +3 to +6 %)
+  // (256x288 tiles, which spill registers, with two slices only: 512x9216x36864 in four slices 181 against 179 us)
+  if (tile == SPLIT_256 || tile == SPLIT_256x192 || splits < 2 || splits > (tile == SPLIT_256x288 ? 2 : 4)) return false;
+  if (N % bn != 0 || (K / splits) % QBK != 0) return false;
+  const long long tiles = tiles_m * (N / bn), cus = num_cus();
+  if (tile == SPLIT_128 && !split_128_deep(tiles * splits, K / splits, true, cus)) return false;
+  // An XCD has the slices of its own tiles only: not where the fullest one then needs a round more than the chip would.
+  if (((tiles + 7) / 8 * splits + cus / 8 - 1) / (cus / 8) > (tiles * splits + cus - 1) / cus) return false;
+  return true;
+}
+
 // One launch of the FUSED form of the 16x16-block kernel: q.K is the slice length, q.splits the slice count.
 template <class Cfg>
 static int launch_fused(const GemmParams& q_in, hipStream_t stream) {
@@ -2465,7 +2526,7 @@ static int launch_fused(const GemmParams& q_in, hipStream_t stream) {
   q.band = 3 * Cfg::BN <= 2 * Cfg::BM ? 4 : 8;
   static std::atomic<unsigned long long> lds_ok{0};
   if (int rc = allow_lds(gemm_pipe16q_kernel<Cfg>, Cfg::LDS_BYTES, lds_ok)) return rc;
-  const int tiles_m = q.M / Cfg::BM, tiles_n = q.N / Cfg::BN;  // whole tiles only (the caller checked)
+  const int tiles_m = (q.M + Cfg::BM - 1) / Cfg::BM, tiles_n = q.N / Cfg::BN;  // whole columns (the caller checked)
   const long long tiles = (long long)tiles_m * tiles_n;
   // every XCD gets the same number of workgroups: enough for its tiles x slices, at most what is resident
   const long long slots = (long long)num_cus() * ((160 * 1024) / Cfg::LDS_BYTES) / 8 * 8;
@@ -2872,21 +2933,12 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
       // by the whole chip in the reduction kernel, cost more than the launch saved (512x9216x36864: 288 against
       // 178 us, 256x5120x5120: 29 against 22 us)
       if constexpr (KIND != EPI_S32_RAW && KIND != EPI_F32_BIAS_ACC) {
-        // one launch when the tile is one of the 16x16-block kernel's and covers M in whole tiles
-        const int bm = tile == SPLIT_256x160 || tile == SPLIT_256x288 ? 256 : 128;
-        const int bn = tile == SPLIT_128x80 ? 80 : tile == SPLIT_128x192 ? 192
-                       : tile == SPLIT_256x160 || tile == SPLIT_128x160 ? 160 : 288;
-        const bool tall = tile == SPLIT_128x80 || tile == SPLIT_128x160 || tile == SPLIT_128x288 ||
-                          tile == SPLIT_256x160 || tile == SPLIT_256x288 || tile == SPLIT_128x192;
-        // up to four slices: the wave that arrives last reads the others' accumulators one slice after the other,
-        // and beyond four that tail costs more than the reduction launch it saves (measured: 2 slices -3 to -12 %,
-        // 4 slices -3 to -8 %, 7 and 8 slices +3 to +6 %)
-        // (256x288 tiles, which spill registers, with two slices only: 512x9216x36864 in four slices 181 against 179 us)
         // (a workspace on a 256-byte boundary only: the 1 KiB regions the waves park and read back must not share a
         // 128-byte line with a neighbour's, or a line fetched for one region could be reused, stale, for the next)
-        if (tall && splits <= (tile == SPLIT_256x288 ? 2 : 4) && p.M % bm == 0 && p.N % bn == 0 &&
+        long long need_one = 0;
+        if (one_launch_split(tile, splits, p.M, p.N, p.K, &need_one) && workspace_bytes >= need_one &&
             (reinterpret_cast<uintptr_t>(workspace) & 255) == 0) {
-          const long long tiles = (long long)(p.M / bm) * (p.N / bn);
+          const long long tiles = (long long)((p.M + split_bm(tile) - 1) / split_bm(tile)) * (p.N / split_bn(tile));
           GemmParams f = p;
           f.K = p.K / splits;
           f.strideA = f.K;
@@ -2901,6 +2953,9 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
               case SPLIT_128x80:
                 g_last_kernel = "fusedk_128x80";
                 return launch_fused<Pipe16QCfg<128, 80, 4, 1, KIND, false, 3, true>>(f, stream);
+              case SPLIT_128:
+                g_last_kernel = "fusedk_128x128";
+                return launch_fused<Pipe16QCfg<128, 128, 4, 2, KIND, false, 5, true>>(f, stream);
               case SPLIT_128x160:
                 g_last_kernel = "fusedk_128x160";
                 return launch_fused<Pipe16QCfg<128, 160, 4, 2, KIND, false, 3, true>>(f, stream);
