@@ -408,31 +408,40 @@ def can_attn_qk_softmax_q(q, k, mask, bsz, heads):
                             and mask.data_ptr() % 16 == 0)
 
 
-_mask_classes_cache = {}  # id(mask) -> (weak reference, version counter, classes tensor)
-
-
-def mask_classes(mask):
+def make_mask_classes(mask):
     """The class array of an additive fp32 mask [bsz, 1, T, S] for the prefill attention kernels (which tiles of
-    64 rows x 256 keys are all zero / all one masked value / mixed), or None when the shape takes none.  Made once per
-    mask tensor and version: every head and every layer of a forward pass adds the same mask.  Made anew at each call
-    while a graph is recorded (its replays read the mask as it is then) and for a tensor without a version."""
-    import weakref
-    keep = not (mask.is_inference() or torch.cuda.is_current_stream_capturing())
-    key = id(mask)
-    if keep:
-        hit = _mask_classes_cache.get(key)
-        if hit is not None and hit[0]() is mask and hit[1] == mask._version:
-            return hit[2]
+    64 rows x 256 keys are all zero / all one masked value / mixed), or None when the shape takes none: one read of the mask as it is
+    now, on the current stream.  The kernels leave out keys and mask values on its word, so it belongs to the pass whose mask it
+    describes: a later write to the mask need not show in its version (a graph's replay), and another stream does not wait
+    for it."""
     bsz, _, T, S = mask.shape
     n = _lib.ti_attn_mask_classes_bytes(bsz, T, S)
     if n <= 0:
         return None
-    cls = torch.empty(n, dtype=torch.uint8, device=mask.device)
     with _on(mask.device):
+        cls = torch.empty(n, dtype=torch.uint8, device=mask.device)
         rc = _lib.ti_attn_mask_classes(mask.data_ptr(), cls.data_ptr(), bsz, T, S, _raw_stream(mask.device.index) or None)
     if rc:
         raise RuntimeError(f"torch_int._hip_ext.mask_classes: {_lib.ti_last_error().decode()} (status {rc})")
-    if keep:
+    return cls
+
+
+_mask_classes_cache = {}  # (id(mask), stream) -> (weak reference, version counter, classes tensor)
+
+
+def mask_classes(mask):
+    """``make_mask_classes`` kept per mask tensor, version and stream, for a caller of the C entry points who holds a mask that nothing
+    writes to meanwhile but torch's own operators; the operators and layers of this package make their own.  Not kept while a
+    graph is recorded (its replays read the mask as it is then) and for a tensor without a version."""
+    import weakref
+    if mask.is_inference() or torch.cuda.is_current_stream_capturing():
+        return make_mask_classes(mask)
+    key = (id(mask), _raw_stream(mask.device.index))
+    hit = _mask_classes_cache.get(key)
+    if hit is not None and hit[0]() is mask and hit[1] == mask._version:
+        return hit[2]
+    cls = make_mask_classes(mask)
+    if cls is not None:
         if len(_mask_classes_cache) >= 64:
             _mask_classes_cache.clear()
         _mask_classes_cache[key] = (weakref.ref(mask, lambda _r, k=key: _mask_classes_cache.pop(k, None)), mask._version, cls)
@@ -445,7 +454,14 @@ def _classes(mask, BH, T, S, pv):
     To be held until the kernel has been launched."""
     if mask is None or not (S > 576 or (pv and S > 352 and BH * ((T + 15) // 16) > 1024)):
         return None
-    return mask_classes(mask)
+    return make_mask_classes(mask)
+
+
+def prefill_mask_classes(hidden, mask, heads):
+    """The class array that the layers of a prefill of ``hidden`` share, whose additive mask is ``mask``, or None (``_classes``)."""
+    B, T = hidden.shape[0], hidden.shape[1]
+    with _on(hidden.device):
+        return _classes(mask, B * heads, T, T, True)
 
 
 def _ptr(tensor):
@@ -688,17 +704,16 @@ def opt_prefill_scratch(plans, hidden):
         return (scratch,) + _CUDA._workspace(dev.index, stream, need_ws)
 
 
-def opt_layer_prefill(plan, hidden, mask, k_out, v_out, chain=0, carry=None, memory=None):
+def opt_layer_prefill(plan, hidden, mask, k_out, v_out, chain=0, carry=None, memory=None, classes=None):
     """A prefill through one decoder layer from one C call (``ti_opt_decoder_layer_prefill_chained``): ``hidden`` [B, T, embed]
     is updated in place, ``k_out`` / ``v_out`` (int8 [B, heads, T, head_dim], contiguous) receive the layer's key and
     value rows.  ``plan``, ``chain`` and ``carry`` as for ``opt_layer_decode``; the caller has checked shapes, dtypes, devices and
-    contiguity.  Layers of one chain share ``memory`` (``opt_prefill_scratch``)."""
+    contiguity.  Layers of one chain share ``memory`` (``opt_prefill_scratch``) and the mask's ``classes`` (``prefill_mask_classes``)."""
     dev = hidden.device
     B, T = hidden.shape[0], hidden.shape[1]
     with _on(dev):
         scratch, ws, ws_ptr, ws_bytes = memory if memory is not None else opt_prefill_scratch((plan,), hidden)
-        cls = _classes(mask, B * k_out.shape[1], T, T, True)
-        rc = _opt_layer_prefill(plan.addr, hidden.data_ptr(), mask.data_ptr() if mask is not None else 0, _ptr(cls) or 0,
+        rc = _opt_layer_prefill(plan.addr, hidden.data_ptr(), mask.data_ptr() if mask is not None else 0, _ptr(classes) or 0,
                                 k_out.data_ptr(), v_out.data_ptr(), B, T, chain, carry.data_ptr() if chain else 0, scratch.data_ptr(),
                                 scratch.numel(), ws_ptr, ws_bytes, _raw_stream(dev.index))
     if rc:
