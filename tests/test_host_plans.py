@@ -84,3 +84,26 @@ def test_a_cache_without_room_is_left_to_the_kernel_only_where_it_lies_as_the_ke
             assert torch.equal(kk.buf[:, :, :S], past[0]) and torch.equal(vv.buf[:, :, :S], past[1])
     kept = opt._kv_view(opt._KVBuffer(torch.zeros(2, 3, 80, 16, dtype=torch.int8), 10), 10)
     assert [kv.bare for kv in opt._kv_rooms((kept, plain))] == [False, False]
+
+
+def test_a_16_bit_mask_is_converted_by_every_call():
+    """A layer's fp32 copy of an fp16 mask is not kept on the mask: another stream would not wait for it, a graph that is recorded
+    would not make it, a replay that rewrites the mask does not show in its version, and a tensor of inference mode has none."""
+    from torch_int.models import opt
+
+    class Mask:
+        is_cuda, dtype = True, torch.float16
+        value = 1.0
+
+        def float(self):
+            return torch.full((1,), self.value)
+
+        @property
+        def _version(self):
+            raise RuntimeError("Inference tensors do not track version counter.")
+
+    mask = Mask()
+    first = opt._mask_as_fp32(mask)
+    mask.value = 2.0
+    second = opt._mask_as_fp32(mask)
+    assert first is not second and first.item() == 1.0 and second.item() == 2.0

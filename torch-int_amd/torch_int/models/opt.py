@@ -509,19 +509,14 @@ def _no_plan():
 
 def _mask_as_fp32(mask):
     """The additive mask as the fused kernels read it: fp32 on the device (None when it is neither that nor an fp16 /
-    bf16 HIP tensor).  The mask of an fp16 model is only ever added to fp32 scores (see ``Int8OPTAttention.forward``);
-    it is converted once per mask tensor and version, not once per layer."""
+    bf16 HIP tensor).  The mask of an fp16 model is only ever added to fp32 scores (see ``Int8OPTAttention.forward``).
+    A copy is this call's own, on its stream and of the values there are now; a decoder makes one for all of its layers
+    (``Int8OPTDecoder._layer_mask``)."""
     if not mask.is_cuda:
         return None
     if mask.dtype is torch.float32:
         return mask
-    if mask.dtype is torch.float16 or mask.dtype is torch.bfloat16:
-        m32 = getattr(mask, "_ti_f32", None)
-        if m32 is None or m32[0] != mask._version:
-            m32 = (mask._version, mask.float())
-            mask._ti_f32 = m32
-        return m32[1]
-    return None
+    return mask.float() if mask.dtype is torch.float16 or mask.dtype is torch.bfloat16 else None
 
 
 _GLOBAL_FORWARD_HOOKS = torch.nn.modules.module._global_forward_hooks
