@@ -1,0 +1,28 @@
+"""The tilings that linears and groups of them are given where a neighbouring choice measured slower, as far as the host
+can tell: by the workspace of their slices and by the launches of a group."""
+import ctypes
+
+import pytest
+
+import torch_int._CUDA as C
+
+C._lib.ti_linear_workspace_bytes.restype = ctypes.c_int64
+C._lib.ti_linear_workspace_bytes.argtypes = [ctypes.c_int64] * 3
+
+
+def _slices(M, N, K):
+    """Slices of a product on 128x128 tiles, whose workspace holds whole tiles when they meet in one launch (0: unsplit)."""
+    rows = {M, (M + 127) // 128 * 128}
+    need = C._lib.ti_linear_workspace_bytes(M, N, K)
+    return {need / (r * N * 4) for r in rows}
+
+
+@pytest.mark.parametrize("M,N,K", [(130, 1024, 1024), (256, 1024, 1024), (512, 1024, 1024), (384, 512, 1024), (1000, 512, 1280),
+                                   (256, 2048, 1024), (240, 1408, 1280)])
+def test_a_short_k_is_left_to_the_small_tiles(M, N, K):
+    assert _slices(M, N, K) == {0}
+
+
+@pytest.mark.parametrize("M,N", [(256, 1024), (512, 1024), (130, 2048), (384, 512)])
+def test_from_1536_on_few_tiles_are_split(M, N):
+    assert _slices(M, N, 1536) & {2, 3, 4}

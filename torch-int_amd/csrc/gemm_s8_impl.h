@@ -2403,11 +2403,12 @@ static int choose_splits(long long M, long long N, long long K, int* tile_kind =
       double rounds, step_us, fixed_us = 8.0;
       // (not against the tiles of widths that 192 or 160 divide, but for 160 where those pad the rows as 128 does and more than one
       // row of tiles shares the weights: 100x5120x20480 31.2 us in eight slices of 128x160, 37.4 so)
-      // (nor where a K of 2048 or less and more than 32 tiles leave the product to the 64x64 tiles, unsplit: 800x2048x2048 12.7 us,
-      // in two slices 13.8; 256x2048x2048 in four 12.0)
+      // (nor where a K below 1536, or one of up to 2048 with more than 32 tiles, leaves the product to the 64x64 tiles, unsplit:
+      // 256x1024x1024 9.1 us, split 10.5 to 11.1; 1000x512x1280 10.3 / 10.6 to 11.4, but 256x1024x1536 12.2 / 10.8 to 11.4;
+      // 800x2048x2048 12.7, in two slices 13.8; 256x2048x2048 in four 12.0)
       // (and where slices leave half of the CUs idle, twice as many in two launches: 256x2048x8192 in four slices 19.3 us, in eight
       // 18.6)
-      const bool deep = kind == SPLIT_128 && batch == 1 && s > 1 && N % 192 != 0 && (K > 2048 || tiles <= 32.0) &&
+      const bool deep = kind == SPLIT_128 && batch == 1 && s > 1 && N % 192 != 0 && K >= 1536 && (K > 2048 || tiles <= 32.0) &&
                         (N % 160 != 0 || (M > 128 && (M + 159) / 160 * 160 >= (M + 127) / 128 * 128)) &&
                         split_128_deep((long long)wgs, K / s, s <= 4 && N % 128 == 0, (long long)cus) &&
                         !(wgs * 2 <= cus && K % (2 * s * QBK) == 0 && K / (2 * s) >= 1024);
@@ -2513,7 +2514,8 @@ static inline bool one_launch_split(int tile, int splits, long long M, long long
   if (tile == SPLIT_256 || tile == SPLIT_256x192 || splits < 2 || splits > (tile == SPLIT_256x288 ? 2 : 4)) return false;
   if (N % bn != 0 || (K / splits) % QBK != 0) return false;
   const long long tiles = tiles_m * (N / bn), cus = num_cus();
-  if (tile == SPLIT_128 && !split_128_deep(tiles * splits, K / splits, true, cus)) return false;
+  // (128x128 tiles below K = 1536: 130x512x1024 in four slices 10.5 us, with 64-byte steps and two launches 9.6)
+  if (tile == SPLIT_128 && (K < 1536 || !split_128_deep(tiles * splits, K / splits, true, cus))) return false;
   // An XCD has the slices of its own tiles only: not where the fullest one then needs a round more than the chip would.
   if (((tiles + 7) / 8 * splits + cus / 8 - 1) / (cus / 8) > (tiles * splits + cus - 1) / cus) return false;
   return true;
