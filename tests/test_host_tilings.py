@@ -26,3 +26,10 @@ def test_a_short_k_is_left_to_the_small_tiles(M, N, K):
 @pytest.mark.parametrize("M,N", [(256, 1024), (512, 1024), (130, 2048), (384, 512)])
 def test_from_1536_on_few_tiles_are_split(M, N):
     assert _slices(M, N, 1536) & {2, 3, 4}
+
+
+@pytest.mark.parametrize("M,N,K,slices", [(130, 2048, 8192, 4), (256, 2048, 8192, 4), (256, 1024, 8192, 8), (256, 2048, 16384, 8),
+                                          (900, 1024, 4096, 2), (1024, 1024, 4096, 2), (700, 1024, 4096, 4), (1000, 1024, 16384, 4)])
+def test_slices_of_products_on_128x128_tiles(M, N, K, slices):
+    """Four that meet in one launch rather than eight short ones on a full chip; two rather than four short ones on a full chip."""
+    assert slices in _slices(M, N, K)

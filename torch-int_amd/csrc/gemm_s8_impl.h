@@ -2346,11 +2346,13 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmParams p, const 
 // 23.3, 700x2560x10240 37.3 -> 30.8, 350x5120x20480 58.8 -> 56.9) and unsplit products (see the pairs at one_launch_split).
 enum SplitTile { SPLIT_128 = 0, SPLIT_256 = 1, SPLIT_256x160 = 2, SPLIT_256x288 = 3, SPLIT_128x160 = 4, SPLIT_128x288 = 5,
                  SPLIT_128x80 = 6, SPLIT_128x192 = 7, SPLIT_256x192 = 8, SPLIT_160x160 = 9 };
-// Slices on 128x128 tiles whose workgroups all have a CU to themselves run on the kernel with 128-byte steps, where a slice is long
-// enough for its five stages, or the slices meet in one launch, which only that kernel can.  (Sixteen slices of 512, two
-// launches: 100x2048x8192 19.1 us with 64-byte steps, 19.4 with 128; 256x2048x8192, eight of 1024, 19.0 / 18.6.)
+// Slices on 128x128 tiles run on the kernel with 128-byte steps where they meet in one launch, which only that kernel can, and each
+// workgroup has a CU to itself.  In two launches: where a slice is long enough for its five stages and a quarter of the CUs is
+// free, else 64-byte steps (150 shapes with eight or sixteen slices, 128-byte steps against those: slices of 512 0.98 to 1.08
+// times the time, of 1024 0.93 to 1.01, of 2048 0.84 to 0.93, but 1.02 to 1.20 and 0.95 to 1.13 on a full chip: 256x2048x8192
+// in eight slices 23.0 us against 19.0).
 static inline bool split_128_deep(long long workgroups, long long slice, bool one_launch, long long cus) {
-  return slice % QBK == 0 && workgroups <= cus && (one_launch || slice >= 1024);
+  return slice % QBK == 0 && workgroups <= cus && (one_launch || (slice >= 1024 && 4 * workgroups <= 3 * cus));
 }
 // `batch` > 1: a batched product (A and B per batch); every tile count, byte count and the streaming floor scale with
 // it, the one-launch form is not available, and the tile shapes are those that exist for every epilogue of the
@@ -2406,12 +2408,15 @@ static int choose_splits(long long M, long long N, long long K, int* tile_kind =
       // (nor where a K below 1536, or one of up to 2048 with more than 32 tiles, leaves the product to the 64x64 tiles, unsplit:
       // 256x1024x1024 9.1 us, split 10.5 to 11.1; 1000x512x1280 10.3 / 10.6 to 11.4, but 256x1024x1536 12.2 / 10.8 to 11.4;
       // 800x2048x2048 12.7, in two slices 13.8; 256x2048x2048 in four 12.0)
-      // (and where slices leave half of the CUs idle, twice as many in two launches: 256x2048x8192 in four slices 19.3 us, in eight
-      // 18.6)
+      // (and where slices leave half of the CUs idle, twice as many in two launches, if those are still long: K = 16384 on up to
+      // half of the CUs, eight slices 0.70 to 0.95 times the time of four in one launch; K = 8192 on up to three eighths 0.91 to 1.07,
+      // on half 0.98 to 1.12)
+      // (nor four short slices on a full chip, where two are ahead: 900x1024x4096 18.1 us, in two 16.8, with 64-byte steps 17.7)
       const bool deep = kind == SPLIT_128 && batch == 1 && s > 1 && N % 192 != 0 && K >= 1536 && (K > 2048 || tiles <= 32.0) &&
                         (N % 160 != 0 || (M > 128 && (M + 159) / 160 * 160 >= (M + 127) / 128 * 128)) &&
                         split_128_deep((long long)wgs, K / s, s <= 4 && N % 128 == 0, (long long)cus) &&
-                        !(wgs * 2 <= cus && K % (2 * s * QBK) == 0 && K / (2 * s) >= 1024);
+                        !(wgs * 2 <= cus && K % (2 * s * QBK) == 0 && K / (2 * s) >= (wgs * 8 <= 3 * cus ? 1024 : 2048)) &&
+                        !(s > 2 && K <= 4096 && wgs * 8 > 7 * cus);
       if (deep) {
         rounds = 1.0;
         step_us = 0.25;
