@@ -1,0 +1,33 @@
+"""The kernels that linears and groups of them run on where a neighbouring choice measured slower (the rules by themselves,
+as far as the host can tell: test_host_tilings.py), bit for bit against an exact fp64 product on the device."""
+import ctypes
+
+import pytest
+import torch
+
+from test_gpu_panel_tiles import _run, _s8
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _family():
+    import torch_int._CUDA as C
+    C._lib.ti_last_kernel.restype = ctypes.c_char_p
+    return C._lib.ti_last_kernel().decode()
+
+
+@pytest.mark.parametrize("T,H,family", [(4096, 40, "pipe16_256x160_group"), (2560, 56, "pipe16_256x128_group"),
+                                        (3700, 20, "pipe16_256x160_group"), (2112, 40, "pipe16_256x160_group")])
+def test_three_projections(T, H, family):
+    import torch_int._hip_ext as X
+    gen = torch.Generator(device=DEV).manual_seed(T)
+    N = H * 128
+    x, ws, bs = _s8(gen, (T, N), 3.0), [_s8(gen, (N, N), 3.0) for _ in range(3)], [_s8(gen, (N,), 20.0) for _ in range(3)]
+    al, be = [2.0 ** -8, 2.0 ** -7, 2.0 ** -9], [0.5, 1.0, 0.25]
+    print(f"group {T}x{N}x{N}", flush=True)
+    out = X.linear_a8_w8_b8_o8_group_heads(x, ws, bs, al, be, 1, T, H, 128)
+    assert _family() == family
+    for o, w, b, a, c in zip(out, ws, bs, al, be):
+        want = torch.clamp(torch.round((x.double() @ w.double().t()) * a + c * b.double()), -128, 127).to(torch.int8)
+        assert torch.equal(o, want.view(1, T, H, 128).transpose(1, 2))

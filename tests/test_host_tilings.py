@@ -33,3 +33,8 @@ def test_from_1536_on_few_tiles_are_split(M, N):
 def test_slices_of_products_on_128x128_tiles(M, N, K, slices):
     """Four that meet in one launch rather than eight short ones on a full chip; two rather than four short ones on a full chip."""
     assert slices in _slices(M, N, K)
+
+
+@pytest.mark.parametrize("M,N,one_launch", [(2112, 5120, 1), (2064, 5120, 1), (2048, 2048, 1), (5696, 7168, 0)])
+def test_groups_that_are_one_launch(M, N, one_launch):
+    assert C._lib.ti_linear_group_is_one_launch(ctypes.c_int64(M), ctypes.c_int64(N), ctypes.c_int64(N), 3) == one_launch

@@ -457,14 +457,21 @@ static int group_prefill_tile(long long M, long long N, long long K, int count) 
   if (e128 < 0.5 || e128 <= e256_alone) e128 = 0.0;
   const double e = e160 > e288 ? (e160 > e128 ? e160 : e128) : (e288 > e128 ? e288 : e128);
   // Beyond 1024 rows the grouped launch and the problems one after the other are priced as price_wide prices tilings, and
-  // 256x256 tiles are in the race too: three 2048x2048x2048 are 192 of them, one round (34.1 -> 30.8 us).
+  // 256x256 tiles are in the race too.  Grouped, 256x128 and 256x160 tiles take 0.96 and 0.98 times their price and 256x256 ones
+  // 1.05 times, which have to be clearly ahead but in one round of a short K, where what a second round adds weighs most (three
+  // 2048x2048x2048, 192 tiles: 34.6 us with weights from HBM, 34.5 on 384 of 256x128; 30.8 and 34.1 with weights that the
+  // last-level cache holds).  1060 groups of three, widths 768 to 7168, 1025 to 8192 rows, weights from HBM, against the choice
+  // without 256x256 tiles: 0.99 times the time, worst 1.03; at the plain price 97 of them lost more than 5 % (4096x5120x5120 266
+  // -> 290 us).
   if (M > 1024 && wide_priced(M, N, K, 1)) {
     int tile = 0;
     double best = (double)count * (price_wide(M, N, K).us + 1.0);
     for (const WideRate& r : kWideRates) {
-      if (r.tile != WIDE_256x160 && r.tile != WIDE_256x288 && r.tile != WIDE_256x128 && !(r.tile == WIDE_256x256 && K >= 2048)) continue;
-      if (N % r.bn != 0) continue;
-      const double us = wide_us(r, M, N, K, count, false);
+      const bool one_round = rows256 * (N / 256) * count <= cus;
+      const double grouped = r.tile == WIDE_256x160 ? 0.98 : r.tile == WIDE_256x128 ? 0.97 : r.tile == WIDE_256x288 ? 1.0
+                             : r.tile == WIDE_256x256 && K >= 2048 ? (one_round && K <= 2304 ? 1.03 : 1.08) : 0.0;  // 0: no such form
+      if (grouped == 0.0 || N % r.bn != 0) continue;
+      const double us = grouped * wide_us(r, M, N, K, count, false);
       if (us < best) {
         best = us;
         tile = r.bn;
