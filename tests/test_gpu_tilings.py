@@ -31,3 +31,12 @@ def test_three_projections(T, H, family):
     for o, w, b, a, c in zip(out, ws, bs, al, be):
         want = torch.clamp(torch.round((x.double() @ w.double().t()) * a + c * b.double()), -128, 127).to(torch.int8)
         assert torch.equal(o, want.view(1, T, H, 128).transpose(1, 2))
+
+
+@pytest.mark.parametrize("out_dtype", [torch.int8, torch.int32])
+@pytest.mark.parametrize("M,N,K,family", [(1029, 16384, 4096, "pipe_256x256+stream"), (2064, 8192, 2048, "pipe_256x256+stream"),
+                                          (1538, 20480, 5120, "pipe16_256x160+stream")])
+def test_a_few_rows_beyond_a_multiple_of_256(M, N, K, family, out_dtype):
+    print(f"rows cut off {M}x{N}x{K} {out_dtype}", flush=True)
+    out, want = _run(M, N, K, out_dtype, M)
+    assert _family() == family and torch.equal(out, want)

@@ -38,3 +38,10 @@ def test_slices_of_products_on_128x128_tiles(M, N, K, slices):
 @pytest.mark.parametrize("M,N,one_launch", [(2112, 5120, 1), (2064, 5120, 1), (2048, 2048, 1), (5696, 7168, 0)])
 def test_groups_that_are_one_launch(M, N, one_launch):
     assert C._lib.ti_linear_group_is_one_launch(ctypes.c_int64(M), ctypes.c_int64(N), ctypes.c_int64(N), 3) == one_launch
+
+
+@pytest.mark.parametrize("M,N,K,cut", [(1538, 20480, 5120, 2), (2060, 5120, 20480, 12), (1029, 16384, 4096, 5), (2064, 8192, 2048, 16),
+                                       (2112, 5120, 20480, 64), (2368, 5120, 5120, 0), (2112, 5120, 5120, 0)])
+def test_rows_that_are_cut_off_the_end(M, N, K, cut):
+    """A few rows stream the weights in less time than a further round of tiles takes; 64 on small weights do not."""
+    assert C._lib.ti_linear_row_split(ctypes.c_int64(M), ctypes.c_int64(N), ctypes.c_int64(K)) == cut
