@@ -40,3 +40,13 @@ def test_a_few_rows_beyond_a_multiple_of_256(M, N, K, family, out_dtype):
     print(f"rows cut off {M}x{N}x{K} {out_dtype}", flush=True)
     out, want = _run(M, N, K, out_dtype, M)
     assert _family() == family and torch.equal(out, want)
+
+
+@pytest.mark.parametrize("out_dtype", [torch.int8, torch.int32])
+@pytest.mark.parametrize("M,N,K,family", [(300, 20480, 5120, "pipe16_256x160"), (320, 20480, 5120, "pipe16_256x160"),
+                                          (569, 16384, 4096, "pipe16_160x256"), (528, 8192, 2048, "pipe16_192x128")])
+def test_two_rows_of_tiles(M, N, K, family, out_dtype):
+    """Two rows of tiles keep every CU busy where they can, three and more go by their price."""
+    print(f"rows of tiles {M}x{N}x{K} {out_dtype}", flush=True)
+    out, want = _run(M, N, K, out_dtype, M)
+    assert _family() == family and torch.equal(out, want)

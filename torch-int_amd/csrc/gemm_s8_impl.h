@@ -2566,7 +2566,9 @@ struct WidePick {
 // Prices in us of the tilings of a linear (or of `count` linears of one shape in one launch) with a K of six or more steps.
 // A tiling's time is rounds x steps x step, where a step is what the 128 bytes of K take a workgroup while all CUs multiply,
 // plus its fill and last epilogue, plus what each further round adds; a chip that is not full clocks higher, so a step of a
-// tiling that leaves half of it idle takes a seventh less.  Measured with 256 tiles at K = 2048 and 8192, weights from HBM, us:
+// tiling that leaves half of it idle takes a seventh less, but not where at most two rows of tiles share the weights: those come
+// from HBM at the pace of the workgroups that ask for them (257 to 320 x 20480 x 5120, 160 tiles of 160x256: 53 us, 256 of 256x160:
+// 49).  Measured with 256 tiles at K = 2048 and 8192, weights from HBM, us:
 // 128x128 38.6 at K = 8192, 192x128 48.1, 256x128 59.5, 160x256 70.2, 256x160 70.9, 192x256 83.8, 256x256 108.  What bounds
 // a step is the power the operands' bits cost on their way through the LDS, which is why larger tiles have the better rates
 // (30 to 44 thousand outputs a us and CU); what the others are for is row counts that leave the larger ones idle: 2112 rows
@@ -2596,7 +2598,8 @@ static double wide_us(const WideRate& r, long long M, long long N, long long K, 
     // 32x32 blocks (8192x20480x5120: 764 us on those, 855 on 256x160; 3932x10240x2560: 123 against 116).
     const double apart = r.tile == WIDE_256x256 || N <= 10240 ? 1.0 : N >= 20480 ? 2.0 : N / 10240.0;
     const double store = out32 ? r.bm * r.bn * 1e-4 * apart : 0.0;
-    return rounds * steps * step * (0.7 + 0.3 * tiles / (rounds * slots)) + fixed + store + (rounds - 1) * (again + store);
+    const double clock = (M + r.bm - 1) / r.bm <= 2 ? 1.0 : 0.7 + 0.3 * tiles / (rounds * slots);
+    return rounds * steps * step * clock + fixed + store + (rounds - 1) * (again + store);
   };
   if (r.tile == WIDE_128x128 && (tiles > cus || K < 1536))  // the 64-byte steps, two workgroups per CU
     return tiles > cus ? time(2 * cus, 1.4, 5.6, out32 ? 5.0 : 1.5) : time(cus, 0.68, 5.6, 1.5);
