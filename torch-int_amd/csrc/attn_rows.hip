@@ -138,7 +138,7 @@ template <int NT, int D, bool MASKED>
 __global__ __launch_bounds__(256, (AttnRows<NT, D>::WAVES)) void attn_rows_kernel(
     const int8_t* __restrict__ q, const int8_t* __restrict__ k, const float* __restrict__ mask,
     const unsigned char* __restrict__ cls, const int8_t* __restrict__ vt, int8_t* __restrict__ ctx, int T, int S,
-    long long stride_q, long long stride_k, int heads, int row_blocks, float alpha, float alpha_pv, int dr) {
+    long long stride_q, long long stride_k, int heads, int row_blocks, int n_bh, int abreast, float alpha, float alpha_pv, int dr) {
   using L = AttnRows<NT, D>;
   constexpr int KS = D / 64;  // 64-byte slices of the head dimension
   constexpr int CH = D / 16;  // blocks of 16 context columns
@@ -150,9 +150,11 @@ __global__ __launch_bounds__(256, (AttnRows<NT, D>::WAVES)) void attn_rows_kerne
   char* ring = smem + w * RING * PIECE;
   float(*s_part)[64] = reinterpret_cast<float(*)[64]>(smem + L::PART);
   float(*s_max)[16] = reinterpret_cast<float(*)[16]>(smem + L::PART + 16 * 64 * 4);
-  const int n_bh = gridDim.x / row_blocks;
-  const long long bh = blockIdx.x % n_bh;
-  const int t0 = (row_blocks - 1 - (int)(blockIdx.x / n_bh)) * 16;  // heaviest rows of a causal mask first
+  // `abreast` heads at a time (all but the last ones), and of those the heaviest rows of a causal mask first
+  const int group = blockIdx.x / (abreast * row_blocks), in_group = blockIdx.x - group * (abreast * row_blocks);
+  const int heads_here = n_bh - group * abreast < abreast ? n_bh - group * abreast : abreast;
+  const long long bh = group * abreast + in_group % heads_here;
+  const int t0 = (row_blocks - 1 - in_group / heads_here) * 16;
   const int rows = T - t0 < 16 ? T - t0 : 16;                       // rows past the end repeat the last one; never stored
   const float lowest = -3.402823466e+38f;
 
@@ -416,10 +418,16 @@ int launch_attn_rows(const int8_t* q, const int8_t* k, const float* mask, const 
   if (BH * row_blocks > 0x7fffffffLL || T > 0x7fffffffLL)
     return fail(TI_ERR_INVALID_ARG, "attn_rows: too many row blocks (%lld)", BH * row_blocks);
   const dim3 grid((unsigned)(BH * row_blocks));
+  // The workgroups of a head read all of its keys and values, 16 rows at a time, so those have to stay in the L2 of the XCD that
+  // the head's workgroups are dealt to (one of eight, where a multiple of eight heads is abreast): 2 MiB of them to an XCD.  Us
+  // with all heads abreast / so: 256 heads x 512 x 128 without a mask 133 / 73, 256 heads x 1024 x 128 523 / 230, causal 272 / 169,
+  // 320 heads x 2048 x 128 2763 / 1237, causal 1565 / 979 (3 MiB to an XCD: 512 keys 87; 4 MiB: 134).
+  const long long fit = 16ll * 1024 * 1024 / (2 * S * D) / 8 * 8;
+  const long long abreast = fit < 8 ? 8 : fit < BH ? fit : BH;
   int rc = TI_OK;
 #define TI_AR(NT, DD, MASKED)                                                                                   \
   rc = launch_ar<NT, DD, MASKED>(grid, stream, q, k, mask, cls, vt, ctx, (int)T, (int)S, stride_q, stride_k, (int)heads, \
-                                 (int)row_blocks, alpha, alpha_pv, (int)D)
+                                 (int)row_blocks, (int)BH, (int)abreast, alpha, alpha_pv, (int)D)
 #define TI_AR_NT(NT)                                 \
   case NT:                                           \
     if (D > 64) {                                    \
