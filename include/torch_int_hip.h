@@ -396,6 +396,9 @@ int ti_kv_append_s8(const int8_t* k_new, const int8_t* v_new, int8_t* k_buf, int
  * that up to 2048, the scores of a row stay in registers; longer ones sweep the keys three times in tiles of 256 (row
  * maximum, row sum, probabilities): the same bits either way. */
 int ti_attn_prefill_supported(int64_t T, int64_t S, int64_t D);
+/* Diagnostics: the form ti_attn_prefill_s8_mc launches for a shape, with or without a mask and its classes: 0 none, 1 all keys in the
+ * LDS and swept once, 2 a row's scores in registers, 3 three sweeps. */
+int ti_attn_prefill_form(int64_t BH, int64_t T, int64_t S, int64_t D, int mask, int classes);
 int ti_attn_prefill_s8(const int8_t* q, const int8_t* k, const int8_t* vt, const float* mask, int8_t* ctx, int64_t BH,
                        int64_t T, int64_t S, int64_t D, int64_t stride_q, int64_t stride_k, int64_t heads,
                        float alpha_qk, float alpha_pv, void* stream);
@@ -451,6 +454,8 @@ int ti_attn_qk_softmax_q(const int8_t* q, const int8_t* k, const float* mask, in
  * array (NULL = none); the bits of the results do not depend on it.  Under a causal mask only the tiles on the
  * diagonal are class 0, which removes most of the mask traffic and half of the first sweep. */
 int64_t ti_attn_mask_classes_bytes(int64_t batch, int64_t T, int64_t S);
+/* Whether making them pays before one such call of that shape (with_v: ti_attn_prefill_s8_mc, else ti_attn_qk_softmax_q_mc). */
+int ti_attn_wants_mask_classes(int64_t BH, int64_t T, int64_t S, int64_t D, int with_v);
 int ti_attn_mask_classes(const float* mask, uint8_t* classes, int64_t batch, int64_t T, int64_t S, void* stream);
 int ti_attn_qk_softmax_q_mc(const int8_t* q, const int8_t* k, const float* mask, const uint8_t* mask_classes,
                             int8_t* probs, int64_t BH, int64_t T, int64_t S, int64_t D, int64_t stride_q,

@@ -577,6 +577,13 @@ int ti_attn_qk_softmax_q_supported(int64_t T, int64_t S, int64_t D) {
 }
 int ti_attn_prefill_supported(int64_t T, int64_t S, int64_t D) { return attn_prefill_supported(T, S, D) ? 1 : 0; }
 
+int ti_attn_prefill_form(int64_t BH, int64_t T, int64_t S, int64_t D, int mask, int classes) {
+  return BH < 0 ? 0 : attn_prefill_form(BH, T, S, D, mask != 0, classes != 0);
+}
+int ti_attn_wants_mask_classes(int64_t BH, int64_t T, int64_t S, int64_t D, int with_v) {
+  return BH >= 0 && attn_wants_classes(BH, T, S, D, with_v != 0) ? 1 : 0;
+}
+
 int64_t ti_attn_mask_classes_bytes(int64_t batch, int64_t T, int64_t S) { return attn_mask_classes_bytes(batch, T, S); }
 
 int ti_attn_mask_classes(const float* mask, uint8_t* classes, int64_t batch, int64_t T, int64_t S, void* stream) {

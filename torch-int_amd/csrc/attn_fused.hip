@@ -322,16 +322,37 @@ bool attn_prefill_supported(long long T, long long S, long long D) {
 }
 
 // Whether attn_rows_kernel is ahead.  Beyond 576 keys always: the other form sweeps the keys three times (us, with the mask's
-// classes: 64 heads x 640 x 128 46.9 -> 25.9, 1024 94.7 -> 47.0, 32 heads x 1904 131 -> 91, 64 heads x 1280 x 64 120 -> 51).  Up
-// to 576 the single sweep shares its keys among 64 query rows and this one among none, but a quarter of the rows to a workgroup
-// fill the chip four times as well: from 65 keys on where 16-row workgroups are few (12 heads x 256 x 64 9.3 -> 5.1, 80 heads x
-// 128 x 128 7.9 -> 7.5, 160 heads 8.9 against 11.3), and with many of them from 353 keys on, if no mask has to be read for
-// every tile of keys (160 heads x 512 x 128 56.8 -> 42.5, without the classes 58.2 -> 52.2 but 160 x 528 57.9 against 68.3; 256
-// heads x 320 x 128, a second tile of 64 keys that one wave of four multiplies, 30.7 against 36.5).
-static bool rows_form_ahead(long long BH, long long T, long long S, long long D, bool no_mask_or_classes) {
+// classes: 64 heads x 640 x 128 46.9 -> 25.9, 1024 94.7 -> 47.0, 64 heads x 1280 x 64 120 -> 51, 160 heads x 2048 x 128 747 -> 472).
+// Up to 576 the single sweep shares its keys among 64 query rows and this one among none, but a quarter of the rows to a workgroup
+// fill the chip four times as well: from 65 keys on where 16-row workgroups are few (12 heads x 256 x 64 9.3 -> 5.1; 80 heads x
+// 128 x 128 7.9 -> 7.5, 160 heads 8.9 against 11.3; 128 heads x 80 x 64 5.5 against 6.0), and with many of them from 400 keys on,
+// or 384 where a causal mask of a prefill leaves half of the tiles out, if no mask has to be read for every tile of keys (160
+// heads x 512 x 128 56.8 -> 42.5, without the classes 58.2 -> 52.2 but 160 x 528 57.9 against 68.3; 256 heads x 122 rows x 368 keys
+// x 128 18.3 against 23.7; 256 heads x 320 x 128, a second tile of 64 keys that one wave of four multiplies, 30.7 against 36.5), nor
+// the single sweep's workgroups are one round of two to a CU, in which it multiplies unmasked tiles at its best (160 heads x 192
+// rows x 576 keys x 128 22.4 against 26.3).  5616 shapes of 80 to 576 keys, 8 to 320 heads and three masks: 0.79 times the single
+// sweep's time in the mean, 0.4 % more than the better of the two.
+static bool rows_form_ahead(long long BH, long long T, long long S, long long D, bool mask, bool classes) {
   if (!attn_rows_supported(T, S, D) || S <= 64) return false;
-  if (S > AF_MAX_S || BH * ((T + 15) / 16) <= (S > 128 ? 1024 : 640)) return true;
-  return S > 352 && no_mask_or_classes;
+  if (S > AF_MAX_S || BH * ((T + 15) / 16) <= (S > 128 ? 1024 : S == 128 ? 640 : 256)) return true;
+  if (S < (mask && T == S ? 384 : 400) || (mask && !classes)) return false;
+  const long long single = BH * ((T + AF_ROWS - 1) / AF_ROWS);
+  return mask || single < 448 || single > 512;
+}
+
+int attn_prefill_form(long long BH, long long T, long long S, long long D, bool mask, bool classes) {
+  return !attn_prefill_supported(T, S, D)                  ? ATTN_NONE
+         : rows_form_ahead(BH, T, S, D, mask, classes)     ? ATTN_ROWS
+         : single_sweep_ok(T, S, D, true)                  ? ATTN_SINGLE_SWEEP
+                                                           : ATTN_THREE_SWEEPS;
+}
+
+// Whether making the classes of a mask pays before one of these launches: where the single sweep, which reads none, is not the
+// form, but for the few workgroups that attn_rows_kernel takes either way up to 576 keys.
+bool attn_wants_classes(long long BH, long long T, long long S, long long D, bool with_v) {
+  if (!(with_v ? attn_prefill_supported(T, S, D) : attn_qk_softmax_q_supported(T, S, D))) return false;
+  if (!single_sweep_ok(T, S, D, with_v)) return true;
+  return with_v && rows_form_ahead(BH, T, S, D, true, true) && !rows_form_ahead(BH, T, S, D, true, false);
 }
 
 template <int NB, bool PV, int SPEC, int D, bool PAD>
@@ -359,7 +380,7 @@ int launch_attn_qk_softmax_q(const int8_t* q, const int8_t* k, const float* mask
                              long long heads, float alpha, const int8_t* vt, int8_t* ctx, float alpha_pv,
                              hipStream_t stream, const unsigned char* mask_classes) {
   if (BH == 0 || T == 0) return TI_OK;
-  if (vt != nullptr && rows_form_ahead(BH, T, S, D, mask == nullptr || mask_classes != nullptr))
+  if (vt != nullptr && rows_form_ahead(BH, T, S, D, mask != nullptr, mask_classes != nullptr))
     return launch_attn_rows(q, k, mask, mask_classes, vt, ctx, BH, T, S, D, stride_q, stride_k, heads, alpha, alpha_pv, stream);
   if (!single_sweep_ok(T, S, D, vt != nullptr))
     return launch_attn_long(q, k, mask, probs, BH, T, S, D, stride_q, stride_k, heads, alpha, vt, ctx, alpha_pv, stream,

@@ -301,6 +301,9 @@ int launch_transpose_last2_s8(const int8_t* src, int8_t* dst, long long B, long 
                               hipStream_t stream);
 bool attn_qk_softmax_q_supported(long long T, long long S, long long D);
 bool attn_prefill_supported(long long T, long long S, long long D);
+enum AttnForm { ATTN_NONE = 0, ATTN_SINGLE_SWEEP = 1, ATTN_ROWS = 2, ATTN_THREE_SWEEPS = 3 };
+int attn_prefill_form(long long BH, long long T, long long S, long long D, bool mask, bool classes);
+bool attn_wants_classes(long long BH, long long T, long long S, long long D, bool with_v);
 int launch_attn_qk_softmax_q(const int8_t* q, const int8_t* k, const float* mask, int8_t* probs, long long BH,
                              long long T, long long S, long long D, long long stride_q, long long stride_k,
                              long long heads, float alpha, const int8_t* vt, int8_t* ctx, float alpha_pv,

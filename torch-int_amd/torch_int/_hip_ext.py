@@ -45,6 +45,8 @@ _lib.ti_attn_qk_softmax_q_supported.argtypes = [_i64, _i64, _i64]
 _lib.ti_attn_qk_softmax_q_supported.restype = ctypes.c_int
 _lib.ti_attn_prefill_supported.argtypes = [_i64, _i64, _i64]
 _lib.ti_attn_prefill_supported.restype = ctypes.c_int
+_lib.ti_attn_wants_mask_classes.argtypes = [_i64, _i64, _i64, _i64, ctypes.c_int]
+_lib.ti_attn_wants_mask_classes.restype = ctypes.c_int
 _lib.ti_attn_qk_softmax_q.argtypes = [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _vp]
 _lib.ti_attn_qk_softmax_q.restype = ctypes.c_int
 _lib.ti_attn_prefill_s8.argtypes = [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _f32, _vp]
@@ -448,20 +450,19 @@ def mask_classes(mask):
     return cls
 
 
-def _classes(mask, BH, T, S, pv):
-    """The mask's class array where the kernel that will run reads one, else None: more than 576 keys, or, with the product
-    with V (``pv``), more than 352 for so many heads and rows that the kernel with a row's scores in registers wants them.
-    To be held until the kernel has been launched."""
-    if mask is None or not (S > 576 or (pv and S > 352 and BH * ((T + 15) // 16) > 1024)):
+def _classes(mask, BH, T, S, d, pv):
+    """The mask's class array where the kernel that will run is ahead with one (``ti_attn_wants_mask_classes``; ``pv``: with the
+    product with V), else None.  To be held until the kernel has been launched."""
+    if mask is None or not _lib.ti_attn_wants_mask_classes(BH, T, S, d, pv):
         return None
     return make_mask_classes(mask)
 
 
-def prefill_mask_classes(hidden, mask, heads):
+def prefill_mask_classes(hidden, mask, heads, head_dim):
     """The class array that the layers of a prefill of ``hidden`` share, whose additive mask is ``mask``, or None (``_classes``)."""
     B, T = hidden.shape[0], hidden.shape[1]
     with _on(hidden.device):
-        return _classes(mask, B * heads, T, T, True)
+        return _classes(mask, B * heads, T, T, head_dim, True)
 
 
 def _ptr(tensor):
@@ -479,7 +480,7 @@ def attn_qk_softmax_q(q, k, mask, alpha, heads, checked=False):
     dev = q.device
     probs = torch.empty((BH, T, S), dtype=torch.int8, device=dev)
     with _on(dev):
-        cls = _classes(mask, BH, T, S, False)
+        cls = _classes(mask, BH, T, S, d, False)
         rc = _lib.ti_attn_qk_softmax_q_mc(q.data_ptr(), k.data_ptr(), mask.data_ptr() if mask is not None else None,
                                           _ptr(cls), probs.data_ptr(), BH, T, S, d, T * d, k.stride(0), heads,
                                           alpha, _raw_stream(dev.index) or None)
@@ -513,7 +514,7 @@ def attn_prefill(q, k, vt, mask, alpha_qk, alpha_pv, heads, checked=False):
     dev = q.device
     ctx = torch.empty((BH // heads, T, heads * d), dtype=torch.int8, device=dev)
     with _on(dev):
-        cls = _classes(mask, BH, T, S, True)
+        cls = _classes(mask, BH, T, S, d, True)
         rc = _lib.ti_attn_prefill_s8_mc(q.data_ptr(), k.data_ptr(), vt.data_ptr(),
                                         mask.data_ptr() if mask is not None else None, _ptr(cls),
                                         ctx.data_ptr(), BH, T, S, d, T * d, k.stride(0), heads, alpha_qk, alpha_pv,

@@ -636,7 +636,7 @@ class Int8OPTDecoderLayer(nn.Module):
             return None
         key, value = plan.new_cache(hidden_states)
         _hip_ext.opt_layer_prefill(plan, hidden_states, mask, key, value,
-                                   classes=_hip_ext.prefill_mask_classes(hidden_states, mask, plan.heads))
+                                   classes=_hip_ext.prefill_mask_classes(hidden_states, mask, plan.heads, plan.head_dim))
         if use_cache:
             return hidden_states, (key, value)
         return (hidden_states,)
@@ -863,7 +863,8 @@ class Int8OPTDecoder(nn.Module):
                     cache.append(present)
         else:
             memory = _hip_ext.opt_prefill_scratch(found, hidden)
-            classes = _hip_ext.prefill_mask_classes(hidden, mask, max(plan.heads for plan in found))
+            widest = max(found, key=lambda plan: plan.heads)
+            classes = _hip_ext.prefill_mask_classes(hidden, mask, widest.heads, widest.head_dim)
             for plan, chain in zip(found, links):
                 key, value = plan.new_cache(hidden)
                 _hip_ext.opt_layer_prefill(plan, hidden, mask, key, value, chain=chain, carry=carry, memory=memory, classes=classes)
