@@ -46,26 +46,33 @@ __device__ __forceinline__ int al_swz(int row, int c) {
 constexpr int MC_MIXED = 0, MC_ZERO = 1, MC_UNIFORM = 2;
 constexpr int MC_HALF_UNIFORM = 3;  // one number from -1e6 to -6e4, such as the lowest of 16 bits: for attn_rows_kernel; MIXED here
 
-__global__ __launch_bounds__(256) void mask_classes_kernel(const float* __restrict__ mask, unsigned char* __restrict__ cls,
-                                                           int T, int S, int row_blocks, int ntiles) {
+// A wave reads a row's KiB at a time and holds four rows: bound by the launch and one trip to memory (four of 1024 x 1024 8.1 -> 4.4 us
+// against 256 threads that tested each load before the next).
+__global__ __launch_bounds__(1024) void mask_classes_kernel(const float* __restrict__ mask, unsigned char* __restrict__ cls,
+                                                            int T, int S, int row_blocks, int ntiles) {
   const int tile = blockIdx.x % ntiles;
   const int rb = (blockIdx.x / ntiles) % row_blocks;
   const long long b = blockIdx.x / (ntiles * row_blocks);
   const int t0 = rb * AL_ROWS, k0 = tile * AL_TILE;
-  const int rows = T - t0 < AL_ROWS ? T - t0 : AL_ROWS;
-  const int quads = (S - k0 < AL_TILE ? S - k0 : AL_TILE) >> 2;  // S is a multiple of 16
+  const int last_row = (T - t0 < AL_ROWS ? T - t0 : AL_ROWS) - 1;
+  const int last_quad = ((S - k0 < AL_TILE ? S - k0 : AL_TILE) >> 2) - 1;  // S is a multiple of 16
   const float* base = mask + (b * T + t0) * (long long)S + k0;
+  const int qd = (int)(threadIdx.x & 63) < last_quad ? (int)(threadIdx.x & 63) : last_quad;  // lanes and rows past the end repeat the last
+  v4f v[AL_ROWS / 16];
+#pragma unroll
+  for (int i = 0; i < AL_ROWS / 16; ++i) {
+    const int row = (int)(threadIdx.x >> 6) + 16 * i;
+    v[i] = *reinterpret_cast<const v4f*>(base + (long long)(row < last_row ? row : last_row) * S + 4 * qd);
+  }
   const int first = __float_as_int(base[0]);
   bool zero = true, same = true;
-  for (int i = threadIdx.x; i < rows * quads; i += 256) {
-    const int row = i / quads, qd = i - row * quads;
-    const v4f v = *reinterpret_cast<const v4f*>(base + (long long)row * S + 4 * qd);
+#pragma unroll
+  for (int i = 0; i < AL_ROWS / 16; ++i)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      zero = zero && v[e] == 0.0f;
-      same = same && __float_as_int(v[e]) == first;
+      zero &= v[i][e] == 0.0f;
+      same &= __float_as_int(v[i][e]) == first;
     }
-  }
   const int all_zero = __syncthreads_and(zero), all_same = __syncthreads_and(same);
   if (threadIdx.x == 0)
     cls[blockIdx.x] = all_zero ? MC_ZERO
@@ -484,7 +491,7 @@ int launch_attn_mask_classes(const float* mask, unsigned char* cls, long long ba
   const long long n = attn_mask_classes_bytes(batch, T, S);
   if (n == 0) return fail(TI_ERR_INVALID_ARG, "attn_mask_classes: unsupported shape (batch=%lld T=%lld S=%lld)", batch, T, S);
   if (n > 0x7fffffffLL) return fail(TI_ERR_INVALID_ARG, "attn_mask_classes: too many blocks (%lld)", n);
-  hipLaunchKernelGGL(mask_classes_kernel, dim3((unsigned)n), dim3(256), 0, stream, mask, cls, (int)T, (int)S,
+  hipLaunchKernelGGL(mask_classes_kernel, dim3((unsigned)n), dim3(1024), 0, stream, mask, cls, (int)T, (int)S,
                      (int)((T + AL_ROWS - 1) / AL_ROWS), (int)((S + AL_TILE - 1) / AL_TILE));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "attn_mask_classes launch: %s", hipGetErrorString(e));
