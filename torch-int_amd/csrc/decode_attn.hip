@@ -265,7 +265,9 @@ __host__ __device__ inline long long decode_attn_lds(long long T, long long S, l
 // NI == 0: any length, four row groups in flight at a time.
 // PART: the head size in memory is smaller than D, the bytes of a cache row that the lanes cover; the forms for
 // head sizes 64 and 128 carry none of its tests.
-template <int TQ, int D, int NI, bool PART>
+// MOVE: as in decode_attn_one_kernel, a form of its own (tested at run time it cost the others up to 9 %: two tokens over 43 positions
+// 8.6 -> 9.7 us).
+template <int TQ, int D, int NI, bool PART, bool MOVE>
 __global__ __launch_bounds__(256) void decode_attn_kernel(const int8_t* __restrict__ q, const int8_t* __restrict__ k_new,
                                                           const int8_t* __restrict__ v_new, int8_t* k_buf,
                                                           int8_t* v_buf, const float* __restrict__ mask,
@@ -301,10 +303,8 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(const int8_t* __restri
   const int S_old = k_new != nullptr ? S - T : S;  // rows below come from the cache, the rest from k_new / v_new
   int8_t* kb = k_buf + bh * cap * dr;
   int8_t* vb = v_buf + bh * cap * dr;
-  // k_past != nullptr: the rows before the new ones come from there and go into the buffers as well
-  const bool move = k_past != nullptr;
-  const int8_t* ko = move ? k_past + bh * past_cap * dr : kb;
-  const int8_t* vo = move ? v_past + bh * past_cap * dr : vb;
+  const int8_t* ko = MOVE ? k_past + bh * past_cap * dr : kb;  // the rows before the new ones
+  const int8_t* vo = MOVE ? v_past + bh * past_cap * dr : vb;
   const int8_t* kn = k_new != nullptr ? k_new + bh * T * dr : nullptr;
   const int8_t* vn = v_new != nullptr ? v_new + bh * T * dr : nullptr;
 
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(256) void decode_attn_kernel(const int8_t* __restri
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int s = base + u * 4 * RPW + rs;
-        if ((move || s >= S_old) && s < S && in_row) *reinterpret_cast<v4i*>(buf + (long long)s * dr + cs * 16) = dst[u];
+        if ((MOVE || s >= S_old) && s < S && in_row) *reinterpret_cast<v4i*>(buf + (long long)s * dr + cs * 16) = dst[u];
       }
     }
   };
@@ -538,16 +538,16 @@ int launch_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_
     else if (groups <= 192) TI_DA1(DD, 16, 12);                     \
     else TI_DA1(DD, 16, 16);                                        \
   } while (0)
-#define TI_DA(TQ, DD, NI)                                                                                              \
-  do {                                                                                                                 \
-    if (D == DD)                                                                                                       \
-      hipLaunchKernelGGL((decode_attn_kernel<TQ, DD, NI, false>), grid, block, lds, stream, q, k_new, v_new, k_buf,    \
-                         v_buf, mask, ctx, probs_out, (int)T, (int)S, cap, (int)heads, alpha_qk, alpha_pv, s_dev, (int)D,  \
-                         k_past, v_past, past_cap); \
-    else                                                                                                               \
-      hipLaunchKernelGGL((decode_attn_kernel<TQ, DD, NI, true>), grid, block, lds, stream, q, k_new, v_new, k_buf,     \
-                         v_buf, mask, ctx, probs_out, (int)T, (int)S, cap, (int)heads, alpha_qk, alpha_pv, s_dev, (int)D,  \
-                         k_past, v_past, past_cap); \
+#define TI_DA_LAUNCH(TQ, DD, NI, PART, MOVE)                                                                            \
+  hipLaunchKernelGGL((decode_attn_kernel<TQ, DD, NI, PART, MOVE>), grid, block, lds, stream, q, k_new, v_new, k_buf, v_buf, \
+                     mask, ctx, probs_out, (int)T, (int)S, cap, (int)heads, alpha_qk, alpha_pv, s_dev, (int)D, k_past,  \
+                     v_past, past_cap)
+#define TI_DA(TQ, DD, NI)                                                \
+  do {                                                                   \
+    if (D == DD && k_past == nullptr) TI_DA_LAUNCH(TQ, DD, NI, false, false); \
+    else if (D == DD) TI_DA_LAUNCH(TQ, DD, NI, false, true);             \
+    else if (k_past == nullptr) TI_DA_LAUNCH(TQ, DD, NI, true, false);   \
+    else TI_DA_LAUNCH(TQ, DD, NI, true, true);                           \
   } while (0)
   const bool one = T == 1 && (groups <= 128 || (groups <= 256 && BH <= (s_dev != nullptr && D > 96 ? 256 : 512)));
   // caches of at most 20 row groups per lane (640 positions at head size 128) with two query rows take
@@ -567,6 +567,7 @@ int launch_decode_attn_s8(const int8_t* q, const int8_t* k_new, const int8_t* v_
 #undef TI_DA1_FORMS
 #undef TI_DA1
 #undef TI_DA1_LAUNCH
+#undef TI_DA_LAUNCH
 #undef TI_DA
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "decode_attn launch: %s", hipGetErrorString(e));
