@@ -57,6 +57,8 @@ int ti_init(void);
  * 0 when no split is worthwhile.  Passing a smaller or NULL workspace is always legal and
  * only selects another kernel, one that needs less or does not split. */
 int64_t ti_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
+/* The same for ti_linear_a8_w8_bfp32_ofp32_acc, which may want other slices; it does with the former as well. */
+int64_t ti_linear_acc_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
 /* Diagnostic: the number r of rows that a linear of this shape cuts off its end and runs as a second, small
  * problem (0 = none).  Tiled kernels pay for whole tiles of 256 rows and whole rounds of 256 CUs; when M > 1024 has

@@ -50,3 +50,22 @@ def test_two_rows_of_tiles(M, N, K, family, out_dtype):
     print(f"rows of tiles {M}x{N}x{K} {out_dtype}", flush=True)
     out, want = _run(M, N, K, out_dtype, M)
     assert _family() == family and torch.equal(out, want)
+
+
+@pytest.mark.parametrize("room", ["own", "the other epilogues'", "none"])
+@pytest.mark.parametrize("M,N,K,family", [(376, 5120, 20480, "splitk_256x160"), (406, 4096, 16384, "splitk_256x256"),
+                                          (588, 2560, 10240, "splitk_256x160")])
+def test_slices_of_the_accumulating_epilogue(M, N, K, family, room):
+    """They never meet in one launch, so they are not those that would; with less room than they want it takes what fits."""
+    import torch_int._CUDA as C
+    gen = torch.Generator(device=DEV).manual_seed(M)
+    x, w, bias = _s8(gen, (M, K), 3.0), _s8(gen, (N, K), 3.0), torch.randint(-99, 99, (N,), device=DEV, generator=gen).float()
+    before = torch.randint(-999, 999, (M, N), device=DEV, generator=gen).float()
+    out, want = before.clone(), (before.double() + x.double() @ w.double().t() + bias.double()).float()    # integers below 2^24
+    have = {"own": C._lib.ti_linear_acc_workspace_bytes(M, N, K), "none": 0}.get(room, C._lib.ti_linear_workspace_bytes(M, N, K))
+    ws = torch.full((have + 4096,), 77, dtype=torch.uint8, device=DEV)
+    print(f"accumulating {M}x{N}x{K} {room}", flush=True)
+    rc = C._lib.ti_linear_a8_w8_bfp32_ofp32_acc(x.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), M, N, K, 1.0, 1.0,
+                                                ws.data_ptr() if have else None, have, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and torch.equal(out, want) and bool((ws[have:] == 77).all())
+    assert room != "own" or _family() == family

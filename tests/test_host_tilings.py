@@ -45,3 +45,11 @@ def test_groups_that_are_one_launch(M, N, one_launch):
 def test_rows_that_are_cut_off_the_end(M, N, K, cut):
     """A few rows stream the weights in less time than a further round of tiles takes; 64 on small weights do not."""
     assert C._lib.ti_linear_row_split(ctypes.c_int64(M), ctypes.c_int64(N), ctypes.c_int64(K)) == cut
+
+
+@pytest.mark.parametrize("M,N,K,slices", [(376, 5120, 20480, 4), (368, 2560, 10240, 5), (406, 4096, 16384, 8)])
+def test_room_for_the_slices_of_the_accumulating_epilogue(M, N, K, slices):
+    need = C._lib.ti_linear_acc_workspace_bytes(M, N, K)
+    assert need >= C._lib.ti_linear_workspace_bytes(M, N, K) and need == slices * M * N * 4
+    for m in (1, 16, 40, 64, 512, 1024, 1030, 2112, 8192):     # never less than the others' room
+        assert C._lib.ti_linear_acc_workspace_bytes(m, N, K) >= C._lib.ti_linear_workspace_bytes(m, N, K)

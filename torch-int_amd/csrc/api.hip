@@ -145,6 +145,7 @@ int ti_init(void) {
 }
 
 int64_t ti_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) { return gemm_workspace_bytes(M, N, K); }
+int64_t ti_linear_acc_workspace_bytes(int64_t M, int64_t N, int64_t K) { return gemm_acc_workspace_bytes(M, N, K); }
 int ti_linear_row_split(int64_t M, int64_t N, int64_t K) { return gemm_row_split(M, N, K); }
 int ti_linear_group_is_one_launch(int64_t M, int64_t N, int64_t K, int count) {
   return M > 0 && N > 0 && K > 0 && count > 0 ? gemm_group_is_one_launch(M, N, K, count) : 0;

@@ -26,6 +26,22 @@ long long gemm_workspace_bytes(long long M, long long N, long long K, bool least
   return !least && one_launch_split(tile, s, M, N, K, &one_launch) ? one_launch : (long long)s * M * N * 4;
 }
 
+// The same for the accumulating epilogue, whose slices never meet in one launch and may be others.
+long long gemm_acc_workspace_bytes(long long M, long long N, long long K) {
+  long long most = gemm_workspace_bytes(M, N, K, false);
+  auto more = [&](long long rows) {
+    if (rows <= 16 || rows > 1024) return;
+    const RowsPick pick = rows_pick(rows, N, K);
+    if (pick.tiling != ROWS_NONE && (N % 16 == 0 || K % SBK == 0)) return;
+    const int s = choose_splits(rows, N, K, nullptr, nullptr, 1, true, false);
+    if (s > 1 && (long long)s * rows * N * 4 > most) most = (long long)s * rows * N * 4;
+  };
+  const int r = M > 1024 ? row_split_rows(M, N, K) : 0;
+  more(r > 0 ? r : M);
+  if (r > 0) more(M - r);
+  return most;
+}
+
 // one per epilogue kind (EpiKind value n), each in its own translation unit
 int launch_gemm_kind_0(const GemmParams& p, void* ws, long long ws_bytes, hipStream_t stream);
 int launch_gemm_kind_1(const GemmParams& p, void* ws, long long ws_bytes, hipStream_t stream);

@@ -2361,7 +2361,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmParams p, const 
 // 128x128 tiles with a CU to themselves step 128 bytes at a time through five stages (split_128_deep): 0.25 us per 64 bytes and
 // 5 TB/s, against 0.35 us and 3.5 TB/s, which is what two workgroups that share a CU still run at.  At that price they replace
 // 256x256 tiles (257x4096x16384 47.7 -> 36.8 us, 90x16384x4096 30.5 -> 20.1), 128x160 and 256x160 ones (384x5120x5120 26.0 ->
-// 23.3, 700x2560x10240 37.3 -> 30.8, 350x5120x20480 58.8 -> 56.9) and unsplit products (see the pairs at one_launch_split).
+// 23.3, 700x2560x10240 37.3 -> 30.8, 350x5120x20480 58.8 -> 56.9) and unsplit products (see the pairs at one_launch_split).  Not for the
+// accumulating epilogue, whose slices do not meet: 369x5120x20480 in two slices of 128x128 and two launches 87 us, of 256x160 60.
 enum SplitTile { SPLIT_128 = 0, SPLIT_256 = 1, SPLIT_256x160 = 2, SPLIT_256x288 = 3, SPLIT_128x160 = 4, SPLIT_128x288 = 5,
                  SPLIT_128x80 = 6, SPLIT_128x192 = 7, SPLIT_256x192 = 8, SPLIT_160x160 = 9 };
 // Slices on 128x128 tiles run on the kernel with 128-byte steps where they meet in one launch, which only that kernel can, and each
@@ -2375,8 +2376,10 @@ static inline bool split_128_deep(long long workgroups, long long slice, bool on
 // `batch` > 1: a batched product (A and B per batch); every tile count, byte count and the streaming floor scale with
 // it, the one-launch form is not available, and the tile shapes are those that exist for every epilogue of the
 // raw-int32 kernels.
+// `meet`: whether the epilogue lets slices meet in one launch (the accumulating one does not); `room`: bytes that the slices'
+// partial products may take.
 static int choose_splits(long long M, long long N, long long K, int* tile_kind = nullptr, double* time_us = nullptr,
-                         long long batch = 1, bool square_tiles = true) {
+                         long long batch = 1, bool square_tiles = true, bool meet = true, long long room = 1ll << 62) {
   if (tile_kind) *tile_kind = SPLIT_128;
   if (time_us) *time_us = -1.0;  // no estimate
   if (M <= 16 || M > 1024 || K % PBK != 0 || K < 1024) return 1;
@@ -2410,7 +2413,7 @@ static int choose_splits(long long M, long long N, long long K, int* tile_kind =
     if ((wide192 || tall192) && (N % 160 == 0 || N % 288 == 0)) continue;  // those widths keep their tuned tiles
     const double tiles = (double)((M + bm - 1) / bm) * (double)((N + bn - 1) / bn) * (double)batch;
     for (int s = 1; s <= 16; ++s) {
-      if (steps % s != 0 || steps / s < 4) continue;
+      if (steps % s != 0 || steps / s < 4 || (s > 1 && s * batch * M * N * 4 > room)) continue;
       if (kind >= SPLIT_256x160 && (K / s) % QBK != 0) continue;  // these tiles step 128 bytes at a time
       if ((half || square) && s == 1) continue;                    // exist as raw-int32 kernels only
       if (tall192 && s > 1) continue;
@@ -2430,7 +2433,7 @@ static int choose_splits(long long M, long long N, long long K, int* tile_kind =
       // half of the CUs, eight slices 0.70 to 0.95 times the time of four in one launch; K = 8192 on up to three eighths 0.91 to 1.07,
       // on half 0.98 to 1.12)
       // (nor four short slices on a full chip, where two are ahead: 900x1024x4096 18.1 us, in two 16.8, with 64-byte steps 17.7)
-      const bool deep = kind == SPLIT_128 && batch == 1 && s > 1 && N % 192 != 0 && K >= 1536 && (K > 2048 || tiles <= 32.0) &&
+      const bool deep = kind == SPLIT_128 && batch == 1 && s > (meet ? 1 : 4) && N % 192 != 0 && K >= 1536 && (K > 2048 || tiles <= 32.0) &&
                         (N % 160 != 0 || (M > 128 && (M + 159) / 160 * 160 >= (M + 127) / 128 * 128)) &&
                         split_128_deep((long long)wgs, K / s, s <= 4 && N % 128 == 0, (long long)cus) &&
                         !(wgs * 2 <= cus && K % (2 * s * QBK) == 0 && K / (2 * s) >= (wgs * 8 <= 3 * cus ? 1024 : 2048)) &&
@@ -2929,7 +2932,10 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
   }
   if (p.batch == 1 && p.lda == p.K && p.ldb == p.K) {
     int tile = SPLIT_128;
-    int splits = choose_splits(p.M, p.N, p.K, &tile);
+    // (the accumulating epilogue does with the workspace of the others, which may be less than its slices want)
+    int splits = KIND == EPI_F32_BIAS_ACC
+                     ? choose_splits(p.M, p.N, p.K, &tile, nullptr, 1, true, false, workspace != nullptr ? workspace_bytes : 0)
+                     : choose_splits(p.M, p.N, p.K, &tile);
     long long need = (long long)splits * p.M * p.N * 4;
     if (tile == SPLIT_160x160 && (workspace == nullptr || workspace_bytes < need)) {  // the best of the others, which may do with less
       splits = choose_splits(p.M, p.N, p.K, &tile, nullptr, 1, false);

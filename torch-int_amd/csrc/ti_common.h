@@ -257,6 +257,7 @@ int launch_gemm(int kind, const GemmParams& p, void* workspace, long long worksp
                 hipStream_t stream);
 // `least`: of the kernels that run where the workspace does not hold the slices of the weight-streaming kernel or of 160x160 tiles
 long long gemm_workspace_bytes(long long M, long long N, long long K, bool least = false);
+long long gemm_acc_workspace_bytes(long long M, long long N, long long K);
 int gemm_group_is_one_launch(long long M, long long N, long long K, int count);
 int gemm_row_split(long long M, long long N, long long K);
 long long bmm_workspace_bytes(long long batch, long long M, long long N, long long K);  // split-K scratch of a batched product  // rows a linear cuts off its end and runs as a second problem

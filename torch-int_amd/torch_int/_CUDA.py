@@ -67,6 +67,8 @@ def _load_library():
     lib.ti_init.restype = _int
     lib.ti_linear_workspace_bytes.argtypes = [_i64, _i64, _i64]
     lib.ti_linear_workspace_bytes.restype = _i64
+    lib.ti_linear_acc_workspace_bytes.argtypes = [_i64, _i64, _i64]
+    lib.ti_linear_acc_workspace_bytes.restype = _i64
     lib.ti_bmm_workspace_bytes.argtypes = [_i64, _i64, _i64, _i64]
     lib.ti_bmm_workspace_bytes.restype = _i64
     return lib
@@ -137,14 +139,14 @@ def _status(op, rc):
         _fail(op, f"{msg} (status {rc})")
 
 
-_ws_need = {}  # (M, N, K) -> bytes of workspace the library can use for that linear
+_ws_need = {}  # (M, N, K, accumulating) -> bytes of workspace the library can use for that linear
 
 
-def _ws_bytes(M, N, K):
-    key = (M, N, K)
+def _ws_bytes(M, N, K, acc=False):
+    key = (M, N, K, acc)
     n = _ws_need.get(key)
     if n is None:
-        n = _ws_need[key] = int(_lib.ti_linear_workspace_bytes(M, N, K))
+        n = _ws_need[key] = int((_lib.ti_linear_acc_workspace_bytes if acc else _lib.ti_linear_workspace_bytes)(M, N, K))
     return n
 
 
@@ -244,7 +246,7 @@ def _linear(op, kind, x, w, bias, bias_dtype, out_dtype, alpha, beta, inout=None
     try:
         stream = _raw_stream(idx)
         # split-K scratch is only ever wanted for mid-sized M (see choose_splits in csrc/gemm_s8.hip)
-        ws, ws_ptr, ws_bytes = _workspace(idx, stream, _ws_bytes(M, N, K)) if M > 16 else (None, 0, 0)
+        ws, ws_ptr, ws_bytes = _workspace(idx, stream, _ws_bytes(M, N, K, kind == _K_F32_ACC)) if M > 16 else (None, 0, 0)
         if _fast is not None:
             rc = _fast.linear(kind, x.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), M, N, K,
                               alpha, beta, ws_ptr, ws_bytes, stream)
