@@ -54,3 +54,4 @@ def test_a_step_waits_for_memory_once(tmp_path):
     odd = [(bm, bn, kind, waits) for bm, bn, kind, waits in loops if (bm, bn) not in SPILLS
            and (len(waits) > 1 or ("0" in waits and (bm, bn) not in TWO_STAGES))]
     assert len(loops) > 200 and odd == [], (len(loops), odd)
+    assert not [loop for loop in loops if loop[:3] == (256, 256, 6)]   # batched products without a bias: 3 to 12 % slower there

@@ -3071,7 +3071,9 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
           // 118 -> 113, 2112x5120x5120 64 -> 61; 4096x4096x768 18.5 against 19.2, so a short K and the attention products stay.
           // 32-bit outputs stay as well: 64 rows of 512 bytes to a wave leave more slowly than 128 rows of 256, behind
           // the next tile's first copies (8192x20480x5120 764 against 803 us).
-          if constexpr (SWAP) {
+          // And so do products of two activations, whose epilogue without a bias the compiler puts among the copies (94 of 289x160x4096
+          // 55 against 61 us, 7 of 1645x1648x4096 109 against 117).
+          if constexpr (SWAP && KIND != EPI_S8_SCALE) {
             if (wide_step && p.K >= 2048) return launch_pipe16q<Pipe16QCfg<256, 256, 4, 2, KIND>>(p, stream);
           }
           if (wide_step) return launch_pipe2<Pipe2Cfg<256, 256, 2, 4, KIND, SWAP>>(p, stream);  // whole cache lines per row
