@@ -78,6 +78,11 @@ int ti_linear_row_split(int64_t M, int64_t N, int64_t K);
  * "" before the first call).  Benchmarks use it to label their rows. */
 const char* ti_last_kernel(void);
 
+/* Diagnostics: which of the pipelined kernels that was, where one family has several ("pipe_128x128", "pipe_256x256" and
+ * "splitk_128x128"): "gemm_pipe" (64-byte steps), "gemm_pipe2" (128-byte steps, 32x32 blocks), "gemm_pipe16" and "gemm_pipe16q" (64-
+ * and 128-byte steps, 16x16 blocks); "" for the others.  Of two problems or launches, the last product's. */
+const char* ti_last_kernel_form(void);
+
 /* Diagnostic: what the calling thread's last linear or group did in the weight-streaming kernel of up to 64 rows: 0 = it
  * took another kernel, 1 = one slice of the inner dimension, 2 = several that met in one launch, 3 = several and a
  * reduction launch; *tiling = 1 .. 8 for the tilings A .. H of csrc/gemm_rows.h, *slices = their number. */

@@ -437,6 +437,7 @@ int ti_attn_softmax_q(const float* scores, const float* mask, int8_t* probs, int
 }
 
 const char* ti_last_kernel(void) { return last_gemm_kernel(); }
+const char* ti_last_kernel_form(void) { return last_gemm_form(); }
 int ti_last_rows(int* tiling, int* slices) { return last_rows(tiling, slices); }
 
 int ti_fused_splitk(int enable) { return set_fused_split(enable); }

@@ -20,7 +20,6 @@
 // half of V^T's rows for 64 keys) follow one another in one sequence, V^T last, so that it lands under the last scores
 // and the exponentials.  For P.V the four dwords of probabilities that a lane holds of 64 keys are transposed across the four
 // 16-lane rows, after which a lane holds 16 consecutive keys, as a 16-byte read of V^T does.
-#include <atomic>
 #include "ti_common.h"
 #include "softmax_math.h"
 
@@ -117,9 +116,8 @@ struct AttnRing {
   }
   // waits for the piece at the tail: loads complete in order, so at most the copies of the pieces behind it may be outstanding
   __device__ __forceinline__ void wait() const {
-    if (L::RING > 3 && ahead == 4) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * CP) : "memory");
-    else if (L::RING > 2 && ahead == 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * CP) : "memory");
-    else if (ahead == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CP) : "memory");
+    static_assert(L::RING == 2, "at most one piece behind it");
+    if (ahead == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CP) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
   // the piece has been read: its slot is free for the next
@@ -390,20 +388,10 @@ bool attn_rows_supported(long long T, long long S, long long D) {
 }
 
 template <int NT, int D, bool MASKED, class... Args>
-static int launch_ar(dim3 grid, hipStream_t stream, Args... args) {
-  auto kern = attn_rows_kernel<NT, D, MASKED>;
+static void launch_ar(dim3 grid, hipStream_t stream, Args... args) {
   constexpr int lds = AttnRows<NT, D>::LDS;
-  static std::atomic<unsigned long long> lds_ok{0};  // bit per device: the large dynamic LDS size has been allowed
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return fail(TI_ERR_LAUNCH, "attn_rows: no current device");
-  const unsigned long long bit = 1ull << (dev & 63);
-  if (lds > 64 * 1024 && !(lds_ok.load(std::memory_order_relaxed) & bit)) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "attn_rows: LDS limit: %s", hipGetErrorString(e));
-    lds_ok.fetch_or(bit, std::memory_order_relaxed);
-  }
-  hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream, args...);
-  return TI_OK;
+  static_assert(lds <= 64 * 1024, "no larger than a launch may ask for as it is");
+  hipLaunchKernelGGL((attn_rows_kernel<NT, D, MASKED>), grid, dim3(256), lds, stream, args...);
 }
 
 int launch_attn_rows(const int8_t* q, const int8_t* k, const float* mask, const unsigned char* cls, const int8_t* vt,
@@ -424,10 +412,9 @@ int launch_attn_rows(const int8_t* q, const int8_t* k, const float* mask, const 
   // 320 heads x 2048 x 128 2763 / 1237, causal 1565 / 979 (3 MiB to an XCD: 512 keys 87; 4 MiB: 134).
   const long long fit = 16ll * 1024 * 1024 / (2 * S * D) / 8 * 8;
   const long long abreast = fit < 8 ? 8 : fit < BH ? fit : BH;
-  int rc = TI_OK;
 #define TI_AR(NT, DD, MASKED)                                                                                   \
-  rc = launch_ar<NT, DD, MASKED>(grid, stream, q, k, mask, cls, vt, ctx, (int)T, (int)S, stride_q, stride_k, (int)heads, \
-                                 (int)row_blocks, (int)BH, (int)abreast, alpha, alpha_pv, (int)D)
+  launch_ar<NT, DD, MASKED>(grid, stream, q, k, mask, cls, vt, ctx, (int)T, (int)S, stride_q, stride_k, (int)heads, \
+                            (int)row_blocks, (int)BH, (int)abreast, alpha, alpha_pv, (int)D)
 #define TI_AR_NT(NT)                                 \
   case NT:                                           \
     if (D > 64) {                                    \
@@ -450,7 +437,6 @@ int launch_attn_rows(const int8_t* q, const int8_t* k, const float* mask, const 
   }
 #undef TI_AR_NT
 #undef TI_AR
-  if (rc) return rc;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "attn_rows launch: %s", hipGetErrorString(e));
   return TI_OK;

@@ -62,7 +62,9 @@ long long bmm_workspace_bytes(long long batch, long long M, long long N, long lo
 }
 
 thread_local const char* g_last_kernel = "";
+thread_local const char* g_last_form = "";
 const char* last_gemm_kernel() { return g_last_kernel; }
+const char* last_gemm_form() { return g_last_form; }
 thread_local RowsLast g_rows_last = {0, 0, 0};
 int last_rows(int* tiling, int* slices) {
   *tiling = g_rows_last.tiling;
@@ -499,7 +501,7 @@ static int group_prefill_tile(long long M, long long N, long long K, int count) 
   // Up to 1024 rows a problem may have a one-round tiling of its own that needs no workspace (128x80, 128x192 or
   // 256x192 tiles over the whole of K): when the cost model prices the problems one after the other below the
   // grouped launch, they run that way (three 512x12288x12288: 260 us grouped on 256x128 tiles, 250 us apart;
-  // three 512x5120x5120 stay grouped).  Times as row_split_rows prices a tiling.
+  // three 512x5120x5120 stay grouped).  The group at 0.85 us per 64 bytes of K and full round of 256x256 tiles, by its efficiency.
   if (M <= 1024) {
     int tile = 0;
     double t_one = -1.0;
@@ -533,6 +535,7 @@ int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStrea
   constexpr int KIND = EPI_S8_BIAS;
   if (shape.M == 0 || shape.N == 0 || grp.count == 0) return TI_OK;
   g_rows_last = {0, 0, 0};
+  g_last_form = "";
   bool ptr_ok = (reinterpret_cast<uintptr_t>(shape.A) & 15) == 0;
   for (int i = 0; i < grp.count; ++i) ptr_ok = ptr_ok && (reinterpret_cast<uintptr_t>(grp.B[i]) & 15) == 0;
   const bool aligned = ptr_ok && (shape.K % SBK == 0) && shape.K > 0;
@@ -609,6 +612,7 @@ int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStrea
 int launch_gemm(int kind, const GemmParams& p, void* ws, long long ws_bytes, hipStream_t stream) {
   if (p.M == 0 || p.N == 0 || p.batch == 0) return TI_OK;
   g_rows_last = {0, 0, 0};
+  g_last_form = "";
   if (int rc = fused_split_check()) return rc;
   switch (kind) {
     case EPI_S32_BIAS: return launch_gemm_kind_0(p, ws, ws_bytes, stream);

@@ -1348,6 +1348,7 @@ struct Pipe16QCfg {
   // copies of one panel each, with 32-bit offsets (see the kernel): where the registers are short.  192x256 tiles 3 to 4 %
   // faster, 256x192 1 %, 256x128 level, and the small tiles, which have registers to spare, 1 to 3 % slower.
   static constexpr bool PANEL_COPIES = RPW % 8 == 0 && BM % 8 == 0 && BM * BN >= 256 * 192;
+  static_assert(!PANEL_COPIES || (unsigned long long)(BM > BN ? BM : BN) * PANEL_MAX_LD <= 1ull << 32, "32-bit panel offsets");
   static_assert(WTM % 16 == 0 && WTN % 16 == 0, "wave tile must be made of 16x16 blocks");
   static_assert((BM + BN) % NWAVES == 0 && RPW % 2 == 0, "a wave must copy whole pairs of rows");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
@@ -2265,20 +2266,27 @@ static int launch_persistent(Kern kern, const GemmParams& p_in, hipStream_t stre
 // kernel (raw int32 output into a workspace [splits][M][N]); this kernel then
 // adds the slices and applies the epilogue.  Integer partial sums make the
 // result independent of the split.
+// kernel of the calling thread's last tiled launch (defined in gemm_s8.hip)
+extern thread_local const char* g_last_form;
+
 template <class Cfg>
 static int launch_pipe(const GemmParams& p, hipStream_t stream) {
+  g_last_form = "gemm_pipe";
   return launch_persistent<Cfg>(gemm_pipe_kernel<Cfg>, p, stream);
 }
 template <class Cfg>
 static int launch_pipe2(const GemmParams& p, hipStream_t stream) {
+  g_last_form = "gemm_pipe2";
   return launch_persistent<Cfg>(gemm_pipe2_kernel<Cfg>, p, stream);
 }
 template <class Cfg>
 static int launch_pipe16q(const GemmParams& p, hipStream_t stream, const GemmGroup& grp = GemmGroup{}) {
+  g_last_form = "gemm_pipe16q";
   return launch_persistent<Cfg>(gemm_pipe16q_kernel<Cfg>, p, stream, grp);
 }
 template <class Cfg>
 static int launch_pipe16(const GemmParams& p, hipStream_t stream) {
+  g_last_form = "gemm_pipe16";
   return launch_persistent<Cfg>(gemm_pipe16_kernel<Cfg>, p, stream);
 }
 
@@ -2531,7 +2539,8 @@ static inline bool one_launch_split(int tile, int splits, long long M, long long
   // Rows that end inside a tile: 128x128 tiles (72 to 1000 rows of widths 2048 to 16384, cold, 44 shapes against two launches and
   // 64-byte steps: 0.69 to 1.01 times the time, 0.83 in the mean; 400x4096x4096 23.3 -> 17.7 us, 1000x2048x8192 37.0 -> 27.8), and
   // 128x192 ones from three row tiles on (800x768x3072 18.4 -> 16.1, 350 rows 15.0 / 14.7, but 200 rows 13.9 / 14.4).  The others
-  // gained nothing: 128x80 0.99 times the two launches, 128x160 0.98, 256x160 1.01, and 160x160 tiles, 25 blocks a wave, spill.
+  // gained nothing: 128x80 0.99 times the two launches, 128x160 0.98, 256x160 1.01, and 160x160 1.22: with one wave to a SIMD
+  // and 253 registers the adding wave fetches five of its 25 blocks at a time.
   if (tile == SPLIT_160x160 || (M % bm != 0 && tile != SPLIT_128 && !(tile == SPLIT_128x192 && M > 320))) return false;
   // up to four slices: the wave that arrives last reads the others' accumulators one slice after the other,
   // and beyond four that tail costs more than the reduction launch it saves (measured: 2 slices -3 to -12 %,
@@ -2550,6 +2559,7 @@ static inline bool one_launch_split(int tile, int splits, long long M, long long
 // One launch of the FUSED form of the 16x16-block kernel: q.K is the slice length, q.splits the slice count.
 template <class Cfg>
 static int launch_fused(const GemmParams& q_in, hipStream_t stream) {
+  g_last_form = "gemm_pipe16q";
   GemmParams q = q_in;
   q.band = 3 * Cfg::BN <= 2 * Cfg::BM ? 4 : 8;
   static std::atomic<unsigned long long> lds_ok{0};
@@ -2567,7 +2577,7 @@ static int launch_fused(const GemmParams& q_in, hipStream_t stream) {
   return TI_OK;
 }
 
-// Tiles of 256 rows for a linear or batched product with M, N > 128: 256x256 (32x32 blocks), or 256x160 /
+// Tiles of 256 rows for a product with M, N > 128 that wide_priced leaves (batches, few tiles, a short or odd K): 256x256 (32x32 blocks), or 256x160 /
 // 256x288 / 256x128 (16x16 blocks) when the width divides and they fill the CUs more evenly (2048x5120: 160 tiles
 // of 256x256 but 256 of 256x160; 2048x9216: 288 tiles of 256x256 = two rounds, but exactly 256 of 256x288;
 // 2048x4096: 128 of 256x256 but 256 of 256x128).  Each candidate is priced as its rate relative to the 256x256
@@ -2598,14 +2608,16 @@ struct WidePick {
 struct WideRate {
   int tile, bm, bn;
   double step, fixed, again;
-  bool newer;  // replaces an older choice only where it is clearly cheaper
+  double edge;  // what has to be left of the price of the tilings before it: of these the prices miss most (up to 1024 rows 192x256
+                // takes 1.05 times its price, 1.11 where the chip is not full, and a tenth of the shapes 1.08 to 1.11 times on the
+                // other two; the rest 0.98 to 1.03 in the median)
 };
 static constexpr WideRate kWideRates[] = {
-    {WIDE_256x128, 256, 128, 0.83, 7.0, 4.0, false}, {WIDE_256x160, 256, 160, 0.977, 8.3, 5.0, false},
-    {WIDE_256x256, 256, 256, 1.50, 11.0, 7.0, false}, {WIDE_256x288, 256, 288, 1.72, 11.0, 7.0, false},
-    {WIDE_256x192, 256, 192, 1.217, 9.1, 6.0, false}, {WIDE_128x128, 128, 128, 0.505, 6.3, 2.7, false},
-    {WIDE_192x128, 192, 128, 0.67, 6.8, 3.5, true}, {WIDE_160x256, 160, 256, 1.02, 8.3, 5.0, true},
-    {WIDE_192x256, 192, 256, 1.19, 9.8, 6.0, true}};
+    {WIDE_256x128, 256, 128, 0.83, 7.0, 4.0, 1.0}, {WIDE_256x160, 256, 160, 0.977, 8.3, 5.0, 1.0},
+    {WIDE_256x256, 256, 256, 1.50, 11.0, 7.0, 1.0}, {WIDE_256x288, 256, 288, 1.72, 11.0, 7.0, 1.0},
+    {WIDE_256x192, 256, 192, 1.217, 9.1, 6.0, 1.0}, {WIDE_128x128, 128, 128, 0.505, 6.3, 2.7, 1.0},
+    {WIDE_192x128, 192, 128, 0.67, 6.8, 3.5, 0.95}, {WIDE_160x256, 160, 256, 1.02, 8.3, 5.0, 0.95},
+    {WIDE_192x256, 192, 256, 1.19, 9.8, 6.0, 0.95}};
 
 static bool wide_priced(long long M, long long N, long long K, long long batch) {
   return batch == 1 && M > 128 && N > 128 && K % QBK == 0 && K >= 768 && ((M + 127) / 128) * ((N + 127) / 128) >= 128;
@@ -2634,7 +2646,7 @@ static WidePick price_wide(long long M, long long N, long long K, bool out32 = f
     if ((r.bn == 160 || r.bn == 288) && N % r.bn != 0) continue;
     if (r.bn == 192 && (N % 192 != 0 || N % 160 == 0 || N % 288 == 0)) continue;
     const double us = wide_us(r, M, N, K, 1, out32);
-    if (us < (r.newer ? 0.95 : 1.0) * best.us) best = WidePick{r.tile, us};
+    if (us < r.edge * best.us) best = WidePick{r.tile, us};
   }
   return best;
 }
@@ -2655,11 +2667,11 @@ static WidePick pick_wide(long long M, long long N, long long K, long long batch
   const double e256 = fill(t256, 256);
   const double e160 = N % 160 == 0 ? f160 * fill(rows256 * (N / 160) * batch, 160) : 0.0;
   const double e288 = N % 288 == 0 ? f288 * fill(rows256 * (N / 288) * batch, 288) : 0.0;
-  // The 256x128 tiles and the comparison with the 128x128 kernel are for linears with a K of some length
-  // (the rates above were measured at K >= 4096; at K = 768 the 128x128 kernel's short prologue wins); batched
-  // products keep their tuned 256x256 / 128x128 choice, they are bound by HBM, not by the matrix pipe.
-  // (a batched product with an inner dimension that long is a stack of linears, not an attention product, and is
-  // priced like them: 8 x 1024 x 1024 x 12288 makes 256 tiles of 256x128 where it made 128 of 256x256)
+  // The 256x128 and 256x192 tiles and the comparison with the 128x128 kernel are for products with a K of some length (the rates
+  // above were measured at K >= 4096); attention products, whose K is a head size, keep their tuned 256x256 / 128x128 choice, they
+  // are bound by HBM, not by the matrix pipe.  (Linears of that size are priced in us, above.  A batched product with an inner
+  // dimension that long is a stack of linears: 8 x 1024 x 1024 x 12288 makes 256 tiles of 256x128 where it made 128 of
+  // 256x256.)
   const bool priced = K >= 2048 && t128 >= 128;
   const double e128w = priced && wide_step && N % 128 == 0 ? 0.93 * fill(rows256 * (N / 128) * batch, 128) : 0.0;
   const double e128 = t128 >= 2 * cus ? 0.6 : t128 >= cus ? 0.47 : 0.47 * (double)t128 / (double)cus;
@@ -2869,7 +2881,8 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
     return TI_OK;
   }
   constexpr bool SWAP = sizeof(Out) == 1;  // 8-bit outputs take the orientation whose lanes own 16 consecutive columns
-  // The kernels with 128-byte steps hold 32-bit offsets into a panel of at most 288 rows.
+  // Some of the tilings hold 32-bit offsets into their panels (Pipe16QCfg::PANEL_COPIES); rows that lie further apart than those
+  // reach go to the 64-byte steps, whose copies have whole addresses, before a tiling is chosen.
   if ((p.lda > PANEL_MAX_LD || p.ldb > PANEL_MAX_LD) && p.K % PBK == 0) {
     g_last_kernel = "pipe_128x128";
     return launch_pipe<PipeCfg<128, 128, 2, 2, 4, KIND, SWAP>>(p, stream);

@@ -271,7 +271,8 @@ int rows_pick_for_test(long long M, long long N, long long K, int cus, int* tili
 int rows_slot_for_test(long long* table, signed char* state, int cap, long long stream, int* fresh);
 int placement_of(const volatile int* words);
 int last_rows(int* tiling, int* slices);
-const char* last_gemm_kernel();  // kernel family of the calling thread's last launch_gemm ("" before the first)
+const char* last_gemm_kernel();
+const char* last_gemm_form();  // kernel family of the calling thread's last launch_gemm ("" before the first)
 
 // ln_q.hip
 int launch_dq_add_layernorm_q(const int32_t* in, float scale, const float* res, const float* gamma,
