@@ -475,7 +475,7 @@ static int group_prefill_tile(long long M, long long N, long long K, int count) 
   if (e128 < 0.5 || e128 <= e256_alone) e128 = 0.0;
   const double e = e160 > e288 ? (e160 > e128 ? e160 : e128) : (e288 > e128 ? e288 : e128);
   // Beyond 1024 rows the grouped launch and the problems one after the other are priced as price_wide prices tilings, and
-  // 256x256 tiles are in the race too.  Grouped, 256x128 and 256x160 tiles take 0.96 and 0.98 times their price and 256x256 ones
+  // 256x256 tiles are in the race too.  Grouped, 256x128 and 256x160 tiles take 0.97 and 0.98 times their price and 256x256 ones
   // 1.05 times, which have to be clearly ahead but in one round of a short K, where what a second round adds weighs most (three
   // 2048x2048x2048, 192 tiles: 34.6 us with weights from HBM, 34.5 on 384 of 256x128; 30.8 and 34.1 with weights that the
   // last-level cache holds).  1060 groups of three, widths 768 to 7168, 1025 to 8192 rows, weights from HBM, against the choice
