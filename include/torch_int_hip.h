@@ -516,7 +516,7 @@ int ti_opt_decoder_layer_decode(const TiOptDecodeLayer* layer, void* hidden, con
  * decode steps continue).  T a multiple of 16 that ti_attn_prefill_supported(T, T, head_dim) accepts, B * T <= 4096
  * (larger prefills are bound by their kernels, not by the host).  scratch:
  * ti_opt_decoder_layer_prefill_scratch_bytes(B * T, embed, ffn) bytes on a 256-byte boundary; workspace: the split-K
- * workspace of the linears (ti_linear_workspace_bytes of the largest of them, or NULL). */
+ * workspace of the linears (ti_linear_workspace_bytes of the largest of them, ti_linear_acc_workspace_bytes for fc2, or NULL). */
 int64_t ti_opt_decoder_layer_prefill_scratch_bytes(int64_t rows, int64_t embed, int64_t ffn);
 int ti_opt_decoder_layer_prefill(const TiOptDecodeLayer* layer, void* hidden, const float* mask,
                                  const uint8_t* mask_classes, int8_t* k_out, int8_t* v_out, int64_t B, int64_t T,

@@ -2260,13 +2260,7 @@ static int launch_persistent(Kern kern, const GemmParams& p_in, hipStream_t stre
   return TI_OK;
 }
 
-// ---------------------------------------------------------------------------
-// Split-K: when a problem has too few output tiles to fill the chip, K is cut
-// into `splits` slices that run as the batches of one launch of the pipelined
-// kernel (raw int32 output into a workspace [splits][M][N]); this kernel then
-// adds the slices and applies the epilogue.  Integer partial sums make the
-// result independent of the split.
-// kernel of the calling thread's last tiled launch (defined in gemm_s8.hip)
+// form of the calling thread's last tiled launch (defined in gemm_s8.hip)
 extern thread_local const char* g_last_form;
 
 template <class Cfg>
@@ -2290,6 +2284,12 @@ static int launch_pipe16(const GemmParams& p, hipStream_t stream) {
   return launch_persistent<Cfg>(gemm_pipe16_kernel<Cfg>, p, stream);
 }
 
+// ---------------------------------------------------------------------------
+// Split-K: when a problem has too few output tiles to fill the chip, K is cut
+// into `splits` slices that run as the batches of one launch of the pipelined
+// kernel (raw int32 output into a workspace [splits][M][N]); this kernel then
+// adds the slices and applies the epilogue.  Integer partial sums make the
+// result independent of the split.
 template <int KIND>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmParams p, const int* __restrict__ ws, int splits) {
   using E = Epi<KIND>;

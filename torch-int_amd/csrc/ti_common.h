@@ -259,8 +259,8 @@ int launch_gemm(int kind, const GemmParams& p, void* workspace, long long worksp
 long long gemm_workspace_bytes(long long M, long long N, long long K, bool least = false);
 long long gemm_acc_workspace_bytes(long long M, long long N, long long K);
 int gemm_group_is_one_launch(long long M, long long N, long long K, int count);
-int gemm_row_split(long long M, long long N, long long K);
-long long bmm_workspace_bytes(long long batch, long long M, long long N, long long K);  // split-K scratch of a batched product  // rows a linear cuts off its end and runs as a second problem
+int gemm_row_split(long long M, long long N, long long K);  // rows a linear cuts off its end and runs as a second problem
+long long bmm_workspace_bytes(long long batch, long long M, long long N, long long K);  // split-K scratch of a batched product
 void allow_fused_split_probe(bool allow);  // per thread: may a GEMM call run the one-time placement probe?
 int warm_fused_split(void* stream);        // run that probe now (1 = the one-launch split-K is usable on this device)
 int fused_split_faulted();                 // 1 = a one-launch split-K on the current device flagged a misplaced workgroup
@@ -271,8 +271,8 @@ int rows_pick_for_test(long long M, long long N, long long K, int cus, int* tili
 int rows_slot_for_test(long long* table, signed char* state, int cap, long long stream, int* fresh);
 int placement_of(const volatile int* words);
 int last_rows(int* tiling, int* slices);
-const char* last_gemm_kernel();
-const char* last_gemm_form();  // kernel family of the calling thread's last launch_gemm ("" before the first)
+const char* last_gemm_kernel();  // kernel family of the calling thread's last launch_gemm ("" before the first)
+const char* last_gemm_form();    // which of a family's pipelined kernels that was ("" for the others)
 
 // ln_q.hip
 int launch_dq_add_layernorm_q(const int32_t* in, float scale, const float* res, const float* gamma,
