@@ -455,7 +455,8 @@ int ti_attn_qk_softmax_q(const int8_t* q, const int8_t* k, const float* mask, in
  * counterpart in the reference).  classes[b][i][j] describes the mask values of batch b, query rows 64 i .. 64 i + 63,
  * keys 256 j .. 256 j + 255: 1 = all of them are +-0 (the kernels then do not read them), 2 = all of them are one
  * and the same value, -1e30 or below (whose keys are then not multiplied, but for rows that are masked throughout), 3 =
- * one value from -1e6 to -6e4 (the mask of an fp16 model: likewise, where alpha leaves it room), 0 = anything else.  ti_attn_mask_classes fills the array (one read of the mask;
+ * one value from -1e6 to -6e4 (the mask of an fp16 model), or -infinity among values of -6e4 or below (padding on top of a causal
+ * mask: likewise, where alpha leaves it room), 0 = anything else.  ti_attn_mask_classes fills the array (one read of the mask;
  * ti_attn_mask_classes_bytes = its size, 0 when the shape takes none), and whoever reads it on that stream,
  * after it, shares it: every head, every layer of a pass.  The _mc entry points are ti_attn_qk_softmax_q / ti_attn_prefill_s8 with that
  * array (NULL = none); the bits of the results do not depend on it.  Under a causal mask only the tiles on the

@@ -66,3 +66,44 @@ def test_one_class_array_to_a_pass(mode, monkeypatch):
         with mode():
             results.append(lm.model(ids).last_hidden_state)
     assert len(made) == 1 and torch.equal(*results)
+
+
+def _summed_mask(kind, B, T, S, gen):
+    """Causal part and padding of a 16-bit (or 32-bit) model as they add up: the lowest value, and -infinity where both say no."""
+    dtype = torch.float32 if kind.startswith("fp32") else torch.float16
+    low = torch.finfo(dtype).min
+    m = torch.zeros(B, 1, T, S, device=DEV, dtype=dtype)
+    causal = torch.zeros(T, S, device=DEV, dtype=dtype).masked_fill_(torch.ones(T, S, dtype=torch.bool, device=DEV).triu(1 + S - T), low)
+    for b in range(B):
+        cut = S - 13 - (b * S) // (2 * B)          # keys that are tokens
+        if kind.endswith("left"):
+            m[b, ..., :S - cut] = low              # queries in the padding are masked throughout
+        else:
+            m[b, ..., cut:] = low
+    m = (m + causal).float()
+    assert (m == low).any() and (torch.isinf(m).any() or kind.endswith("left"))
+    return m
+
+
+@pytest.mark.parametrize("kind", ["fp16 right", "fp16 left", "fp32 right", "fp32 left"])
+@pytest.mark.parametrize("B,H,T,S,d", [(2, 2, 384, 384, 80), (3, 1, 528, 528, 128), (2, 2, 1040, 1040, 64), (2, 1, 500, 768, 128),
+                                       (1, 2, 2048, 2048, 128), (2, 1, 2064, 2064, 64)])
+def test_padding_on_a_causal_mask(B, H, T, S, d, kind, monkeypatch):
+    import test_gpu_attn_rows as rows
+    monkeypatch.setattr(rows, "_mask", _summed_mask)
+    rows._check(B, H, T, S, d, kind)
+
+
+@pytest.mark.parametrize("kind", ["fp16 right", "fp32 right"])
+def test_masked_tiles_are_known_where_padding_meets_them(kind):
+    import torch_int._hip_ext as X
+    mask = _summed_mask(kind, 2, 512, 512, None)
+    classes = X.make_mask_classes(mask).view(2, 8, 2).cpu()
+    tiles = mask.view(2, 8, 64, 2, 256).cpu()
+    for b in range(2):
+        for i in range(8):
+            for j in range(2):
+                t = tiles[b, i, :, j]
+                want = 1 if (t == 0).all() else 0 if (t > -6e4).any() else 3 if (t != t[0, 0]).any() or t[0, 0] > -1e30 else 2
+                assert classes[b, i, j] == want, (b, i, j)
+    assert (classes[:, :4, 1] == 3).all()          # above the diagonal

@@ -32,7 +32,7 @@ constexpr int AR_TILE = 256;  // keys per round of the 64 partial sums
 constexpr int AR_MAX_TILES = 8;
 constexpr int AR_BUFFER_FLAGS = 0x00020000;  // raw buffer, 32-bit data: offsets from the descriptor's size on read as zeros
 constexpr int AR_MC_ROWS = 64;  // rows to a mask class (attn_long.hip)
-constexpr int AR_MC_ZERO = 1, AR_MC_UNIFORM = 2, AR_MC_HALF_UNIFORM = 3;
+constexpr int AR_MC_ZERO = 1, AR_MC_UNIFORM = 2, AR_MC_LOW = 3;
 
 // 16-byte chunk c of row `row` of a piece whose rows hold B bytes sits at this chunk position
 template <int B>
@@ -162,10 +162,10 @@ __global__ __launch_bounds__(256, (AttnRows<NT, D>::WAVES)) void attn_rows_kerne
     const int c = 64 * s + 16 * g;
     qf[s] = *reinterpret_cast<const v4i*>(q + bh * stride_q + (long long)(t0 + (r < rows ? r : rows - 1)) * dr + (c < dr ? c : 0));
   }
-  // Mask classes of this row block's tiles.  `todo`: the tiles whose keys are multiplied, all but those whose mask is one low
-  // value throughout; `zero`: those whose mask adds nothing.  A score of a tile that is passed over is below `passed`: -1e30
-  // takes no notice of any product (the launcher looks at alpha), and -6e4, the mask of an fp16 model, is raised by the largest
-  // product there can be (such tiles are multiplied like others where that is not far below it).
+  // Mask classes of this row block's tiles.  `todo`: the tiles whose keys are multiplied, all but those whose mask is low
+  // throughout; `zero`: those whose mask adds nothing.  A score of a tile that is passed over is below `passed`: -1e30
+  // takes no notice of any product (the launcher looks at alpha), and -6e4 or less, the mask of an fp16 model, is raised by at most the
+  // largest product there can be (such tiles are multiplied like others where that is not far below it).
   unsigned todo = ALL, zero = MASKED ? 0u : ALL;
   float passed = -1e29f;
   if (MASKED && cls != nullptr) {
@@ -173,9 +173,9 @@ __global__ __launch_bounds__(256, (AttnRows<NT, D>::WAVES)) void attn_rows_kerne
     const int v = c[lane < NT ? lane : 0];
     zero = (unsigned)__builtin_amdgcn_ballot_w64(v == AR_MC_ZERO && lane < NT);
     const float product = __builtin_fabsf(alpha) * (float)(dr * 16384);
-    const unsigned half = product < 3e4f ? (unsigned)__builtin_amdgcn_ballot_w64(v == AR_MC_HALF_UNIFORM && lane < NT) : 0u;
-    if (half != 0) passed = product - 5.9e4f;
-    todo &= ~(half | (unsigned)__builtin_amdgcn_ballot_w64(v == AR_MC_UNIFORM && lane < NT));
+    const unsigned low = product < 3e4f ? (unsigned)__builtin_amdgcn_ballot_w64(v == AR_MC_LOW && lane < NT) : 0u;
+    if (low != 0) passed = product - 5.9e4f;
+    todo &= ~(low | (unsigned)__builtin_amdgcn_ballot_w64(v == AR_MC_UNIFORM && lane < NT));
   }
   AttnRing<NT, D> pieces;
   pieces.ring = ring;
