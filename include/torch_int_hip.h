@@ -332,6 +332,21 @@ int ti_linear_a8_w8_bfp32_ofp32_acc(const int8_t* x, const int8_t* w, const floa
                                     int64_t M, int64_t N, int64_t K, float alpha, float beta,
                                     void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The same on an fp16 tensor: inout[m,n] = f16(inout[m,n] + f16(fmaf(alpha, acc, beta*bias[n]))), the result rounded to fp32,
+ * then to fp16, then added: `residual.add_(fc2(x).to(residual.dtype))` (torch_int/models/opt.py:287-289).  Up to 16 rows. */
+int ti_linear_a8_w8_bfp32_of16_acc(const int8_t* x, const int8_t* w, const float* bias, void* inout,
+                                   int64_t M, int64_t N, int64_t K, float alpha, float beta,
+                                   void* workspace, int64_t workspace_bytes, void* stream);
+
+/* LayerNormQ and the linears that read its result in one launch, for up to 4 rows of a decode step: q = the q_out of
+ * ti_add_layernorm_q (half: of ti_add_layernorm_q_f16) with x == NULL on hidden [M, K], then out[i] = ti_linear_a8_w8_b8_o8 (relu:
+ * ti_linear_relu_a8_w8_b8_o8) of q with w[i] [N, K], bias[i] [N], alpha[i], beta_s[i] for count = 1 to 3 problems; the values are
+ * theirs.  K a multiple of 16 up to 9216 (5120 for more than two rows); hidden, gamma and beta on a boundary of four elements, the weights of 16 bytes. */
+int ti_layernorm_q_linear_a8_w8_b8_o8(const void* hidden, int half, const void* gamma, const void* beta, float eps,
+                                      const int8_t* const* w, const int8_t* const* bias, int8_t* const* out,
+                                      const float* alpha, const float* beta_s, int64_t count, int relu,
+                                      int64_t M, int64_t N, int64_t K, void* stream);
+
 /* x != NULL: residual[row,i] += x[row,i] (in place), then
  *            q_out = s8(clamp(rint(LN(residual[row,:])[i] * gamma[i] + beta[i]), -128, 127));
  * x == NULL: the same without the add (residual is only read).
@@ -478,7 +493,8 @@ int ti_attn_prefill_s8_mc(const int8_t* q, const int8_t* k, const int8_t* vt, co
  * stream.  Each step is the entry point above that the modules call for it (ti_add_layernorm_q[_f16[_xf32]],
  * ti_linear_a8_w8_b8_o8_group, ti_decode_attn_s8, ti_linear_a8_w8_bfp32_ofp32[_acc], ti_linear_relu_a8_w8_b8_o8,
  * ti_add_f16_xf32), with the same arguments: the values are theirs; what the call saves is the host time of eight
- * trips through the caller's language.  hidden is the residual stream [B, 1, embed] (fp32, or fp16 with half = 1: then
+ * trips through the caller's language.  Up to 4 sequences the LayerNorms share a launch with the projections and with fc1
+ * (ti_layernorm_q_linear_a8_w8_b8_o8) and out_proj and fc2 add into the stream themselves: five launches, same values.  hidden is the residual stream [B, 1, embed] (fp32, or fp16 with half = 1: then
  * the LayerNorm parameters are fp16 too), updated in place; mask fp32 [B, 1, 1, S] or NULL; k_buf / v_buf the cache
  * buffers [B, heads, cap, head_dim] holding S - 1 positions, S after the call; scratch: device memory of
  * ti_opt_decoder_layer_decode_scratch_bytes(B, embed, ffn) bytes on a 256-byte boundary (the layers of a model can

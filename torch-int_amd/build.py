@@ -12,12 +12,12 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "torch_int", "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libtorch_int_hip.so")
-# (source, extra defines, object name).  The GEMM kernels are compiled once per epilogue kind (EpiKind 0..8 of
+# (source, extra defines, object name).  The GEMM kernels are compiled once per epilogue kind (EpiKind 0..9 of
 # csrc/ti_common.h), each kind in a translation unit of its own, so that they build in parallel.
 SOURCES = [(s, [], s[:-4] + ".o") for s in
-           ["api.hip", "gemm_s8.hip", "ln_q.hip", "softmax_q.hip", "permute.hip", "bmm_rowmajor.hip", "decode_attn.hip",
+           ["api.hip", "gemm_s8.hip", "ln_q.hip", "ln_linear.hip", "softmax_q.hip", "permute.hip", "bmm_rowmajor.hip", "decode_attn.hip",
             "attn_fused.hip", "attn_long.hip", "attn_rows.hip", "diag_mfma.hip"]]
-SOURCES += [("gemm_s8_kinds.hip", [f"-DTI_KIND={k}"], f"gemm_s8_kind{k}.o") for k in range(9)]
+SOURCES += [("gemm_s8_kinds.hip", [f"-DTI_KIND={k}"], f"gemm_s8_kind{k}.o") for k in range(10)]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

@@ -178,6 +178,13 @@ int ti_linear_a8_w8_bfp32_ofp32_acc(const int8_t* x, const int8_t* w, const floa
                   ws, ws_bytes, stream);
 }
 
+int ti_linear_a8_w8_bfp32_of16_acc(const int8_t* x, const int8_t* w, const float* bias, void* inout, int64_t M,
+                                   int64_t N, int64_t K, float alpha, float beta, void* ws, int64_t ws_bytes,
+                                   void* stream) {
+  return run_gemm("linear_a8_w8_bfp32_of16_acc", EPI_F16_BIAS_ACC, x, w, bias, 4, inout, 2, 1, M, N, K, alpha, beta,
+                  ws, ws_bytes, stream);
+}
+
 int ti_linear_a8_w8_b8_o8(const int8_t* x, const int8_t* w, const int8_t* bias, int8_t* out, int64_t M,
                           int64_t N, int64_t K, float alpha, float beta, void* ws, int64_t ws_bytes,
                           void* stream) {
@@ -420,6 +427,37 @@ int ti_add_layernorm_q_f16_xf32(const float* x, void* residual, const void* gamm
   if (int rc = check_ptr(op, "beta", beta, 2, nonempty)) return rc;
   if (int rc = check_ptr(op, "q_out", q_out, 1, nonempty)) return rc;
   return launch_add_layernorm_q_f16_xf32(x, residual, gamma, beta, eps, q_out, rows, H, static_cast<hipStream_t>(stream));
+}
+
+int ti_layernorm_q_linear_a8_w8_b8_o8(const void* hidden, int half, const void* gamma, const void* beta, float eps,
+                                      const int8_t* const* w, const int8_t* const* bias, int8_t* const* out,
+                                      const float* alpha, const float* beta_s, int64_t count, int relu, int64_t M, int64_t N,
+                                      int64_t K, void* stream) {
+  g_err[0] = 0;
+  const char* op = "layernorm_q_linear_a8_w8_b8_o8";
+  if (count < 1 || count > 3) return fail(TI_ERR_INVALID_ARG, "%s: 1 to 3 problems, got %lld", op, (long long)count);
+  if (int rc = check_dims(op, 1, M, N, K)) return rc;
+  if (M == 0 || N == 0) return TI_OK;
+  if (w == nullptr || bias == nullptr || out == nullptr || alpha == nullptr || beta_s == nullptr)
+    return fail(TI_ERR_INVALID_ARG, "%s: a per-problem array is NULL", op);
+  if (int rc = check_ptr(op, "hidden", hidden, half ? 2 : 4, true)) return rc;
+  if (int rc = check_ptr(op, "gamma", gamma, half ? 2 : 4, true)) return rc;
+  if (int rc = check_ptr(op, "beta", beta, half ? 2 : 4, true)) return rc;
+  LnLinear p{hidden, gamma, beta, eps, (int)M, (int)K, (int)N, (int)count, relu ? 0 : -128, {}, {}, {}, {}, {}};
+  for (int i = 0; i < count; ++i) {
+    if (int rc = check_ptr(op, "weight", w[i], 1, true)) return rc;
+    if (int rc = check_ptr(op, "bias", bias[i], 1, true)) return rc;
+    if (int rc = check_ptr(op, "output", out[i], 1, true)) return rc;
+    p.W[i] = w[i];
+    p.bias[i] = bias[i];
+    p.out[i] = out[i];
+    p.alpha[i] = alpha[i];
+    p.beta_s[i] = beta_s[i];
+  }
+  if (!ln_linear_takes(p, half != 0))
+    return fail(TI_ERR_INVALID_ARG, "%s: up to %d rows, K a multiple of 16 up to 9216, rows of hidden, gamma and beta on boundaries of "
+                "four elements, weights on 16 bytes (got M=%lld N=%lld K=%lld)", op, LN_LINEAR_ROWS, (long long)M, (long long)N, (long long)K);
+  return launch_ln_linear(p, half != 0, static_cast<hipStream_t>(stream));
 }
 
 int ti_attn_softmax_q(const float* scores, const float* mask, int8_t* probs, int64_t batch, int64_t heads, int64_t T,
@@ -802,6 +840,39 @@ int layernorm(const TiOptDecodeLayer* L, const float* pending, void* hidden, con
 // whether fc2's output is added by a later kernel rather than in the GEMM's epilogue
 bool adds_later(const TiOptDecodeLayer* L, int64_t rows) { return L->half || rows > 4096; }
 
+// Decode steps of a few rows: out_proj and fc2 add into the stream themselves, and the LayerNorm is part of the launch that
+// reads its result.  The layers of a chain agree on this (it looks at the rows alone): none leaves a carry.
+bool few_rows(int64_t rows) { return rows <= LN_LINEAR_ROWS; }
+
+// residual stream += x . w, as a linear with an fp32 bias and one addition of the stream's type
+int add_linear(const TiOptDecodeLayer* L, const int8_t* x, const int8_t* w, const float* bias, void* hidden, int64_t rows, int64_t K,
+               float alpha, void* stream) {
+  return L->half ? ti_linear_a8_w8_bfp32_of16_acc(x, w, bias, hidden, rows, L->embed, K, alpha, 1.0f, nullptr, 0, stream)
+                 : ti_linear_a8_w8_bfp32_ofp32_acc(x, w, bias, static_cast<float*>(hidden), rows, L->embed, K, alpha, 1.0f, nullptr,
+                                                   0, stream);
+}
+
+// q = LayerNormQ(hidden) and up to three linears that read it, in one launch where there is one; `x`: room for q where not
+int layernorm_linear(const char* op, const TiOptDecodeLayer* L, const void* hidden, const void* gamma, const void* beta, float eps,
+                     int8_t* x, const int8_t* const* w, const int8_t* const* bias, int8_t* const* out, const float* alpha,
+                     const float* beta_s, int count, bool relu, int64_t rows, int64_t N, void* stream) {
+  LnLinear p{hidden, gamma, beta, eps, (int)rows, (int)L->embed, (int)N, count, relu ? 0 : -128, {}, {}, {}, {}, {}};
+  for (int i = 0; i < count; ++i) {
+    p.W[i] = w[i];
+    p.bias[i] = bias[i];
+    p.out[i] = out[i];
+    p.alpha[i] = alpha[i];
+    p.beta_s[i] = beta_s[i];
+  }
+  if (ln_linear_takes(p, L->half != 0))
+    return ti_layernorm_q_linear_a8_w8_b8_o8(hidden, L->half, gamma, beta, eps, w, bias, out, alpha, beta_s, count, relu, rows, N,
+                                             L->embed, stream);
+  if (int rc = layernorm(L, nullptr, const_cast<void*>(hidden), gamma, beta, eps, x, rows, stream)) return rc;
+  if (count == 1 && relu)
+    return ti_linear_relu_a8_w8_b8_o8(x, w[0], bias[0], out[0], rows, N, L->embed, alpha[0], beta_s[0], nullptr, 0, stream);
+  return linear_group(op, x, w, bias, out, alpha, beta_s, count, rows, N, L->embed, 0, 0, stream);
+}
+
 // out_proj, the second LayerNorm, fc1 and fc2 of a layer
 int after_attention(const TiOptDecodeLayer* L, const int8_t* ctx, float* f32, int8_t* x, int8_t* h, void* hidden,
                     int64_t rows, int chain, float* carry, void* ws, int64_t ws_bytes, void* stream) {
@@ -863,14 +934,26 @@ int decode_layer(const char* op, const TiOptDecodeLayer* L, void* hidden, const 
   int8_t* h = carve.take<int8_t>(B * F);
   const int64_t ws_bytes = decode_workspace_bytes(B, E, F);
   void* ws = ws_bytes > 0 ? carve.take<void>(ws_bytes) : nullptr;
-  const float* pending = (chain & CHAIN_ADD) && adds_later(L, B) ? carry : nullptr;
   int rc;
-  if ((rc = layernorm(L, pending, hidden, L->ln1_gamma, L->ln1_beta, L->ln1_eps, x, B, stream))) return rc;
   const int8_t* w3[3] = {L->wq, L->wk, L->wv};
   const int8_t* b3[3] = {L->bq, L->bk, L->bv};
   int8_t* o3[3] = {q, k, v};
   const float a3[3] = {L->alpha_q, L->alpha_k, L->alpha_v};
   const float be3[3] = {L->beta_q, L->beta_k, L->beta_v};
+  if (few_rows(B)) {
+    if ((rc = layernorm_linear(op, L, hidden, L->ln1_gamma, L->ln1_beta, L->ln1_eps, x, w3, b3, o3, a3, be3, 3, false, B, E, stream)))
+      return rc;
+    if ((rc = ti_decode_attn_s8_from(q, k, v, k_past, v_past, past_cap, k_buf, v_buf, mask, ctx, B * H, 1, d, cap, S, H,
+                                     L->alpha_qk, L->alpha_pv, stream)))
+      return rc;
+    if ((rc = add_linear(L, ctx, L->wo, L->bo, hidden, B, E, L->alpha_o, stream))) return rc;
+    if ((rc = layernorm_linear(op, L, hidden, L->ln2_gamma, L->ln2_beta, L->ln2_eps, x, &L->w1, &L->b1, &h, &L->alpha_1, &L->beta_1,
+                               1, true, B, F, stream)))
+      return rc;
+    return add_linear(L, h, L->w2, L->b2, hidden, B, F, L->alpha_2, stream);
+  }
+  const float* pending = (chain & CHAIN_ADD) && adds_later(L, B) ? carry : nullptr;
+  if ((rc = layernorm(L, pending, hidden, L->ln1_gamma, L->ln1_beta, L->ln1_eps, x, B, stream))) return rc;
   if ((rc = linear_group(op, x, w3, b3, o3, a3, be3, 3, B, E, E, 0, 0, stream, ws, ws_bytes))) return rc;
   // cache append + attention; [B, 1, E] rows are [B * heads, 1, head_dim] as they lie
   if ((rc = ti_decode_attn_s8_from(q, k, v, k_past, v_past, past_cap, k_buf, v_buf, mask, ctx, B * H, 1, d, cap, S, H,

@@ -72,6 +72,12 @@ __device__ __forceinline__ void store_rows4(v4i acc, const GemmParams& p, int m,
       Out4 w4 = {o[0], o[1], o[2], o[3]};
       if constexpr (E::kAccumulate) w4 = *reinterpret_cast<const Out4*>(dst) + w4;
       *reinterpret_cast<Out4*>(dst) = w4;
+    } else if constexpr (sizeof(Out) == 2) {
+      typedef Out Out4 __attribute__((ext_vector_type(4)));
+      Out4 w4 = *reinterpret_cast<const Out4*>(dst);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) w4[v] = accumulated<Out>(w4[v], o[v]);
+      *reinterpret_cast<Out4*>(dst) = w4;
     } else {
       *reinterpret_cast<unsigned*>(dst) = (unsigned)(unsigned char)o[0] | ((unsigned)(unsigned char)o[1] << 8) |
                                           ((unsigned)(unsigned char)o[2] << 16) | ((unsigned)(unsigned char)o[3] << 24);

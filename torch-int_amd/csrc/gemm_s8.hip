@@ -52,6 +52,9 @@ int launch_gemm_kind_5(const GemmParams& p, void* ws, long long ws_bytes, hipStr
 int launch_gemm_kind_6(const GemmParams& p, void* ws, long long ws_bytes, hipStream_t stream);
 int launch_gemm_kind_7(const GemmParams& p, void* ws, long long ws_bytes, hipStream_t stream);
 int launch_gemm_kind_8(const GemmParams& p, void* ws, long long ws_bytes, hipStream_t stream);
+int launch_gemm_kind_9(const GemmParams& p, void* ws, long long ws_bytes, hipStream_t stream);
+
+int compute_units() { return num_cus(); }
 
 int gemm_row_split(long long M, long long N, long long K) { return row_split_rows(M, N, K); }
 
@@ -624,6 +627,7 @@ int launch_gemm(int kind, const GemmParams& p, void* ws, long long ws_bytes, hip
     case EPI_S8_SCALE: return launch_gemm_kind_6(p, ws, ws_bytes, stream);
     case EPI_S32_RAW: return launch_gemm_kind_7(p, ws, ws_bytes, stream);
     case EPI_F32_BIAS_ACC: return launch_gemm_kind_8(p, ws, ws_bytes, stream);
+    case EPI_F16_BIAS_ACC: return launch_gemm_kind_9(p, ws, ws_bytes, stream);
   }
   return fail(TI_ERR_INVALID_ARG, "unknown epilogue kind %d", kind);
 }

@@ -1686,7 +1686,7 @@ __device__ __forceinline__ void store_skinny_tile(v4i acc, const GemmParams& p, 
     v4i w4 = {__builtin_bit_cast(int, (W)o[0]), __builtin_bit_cast(int, (W)o[1]), __builtin_bit_cast(int, (W)o[2]),
               __builtin_bit_cast(int, (W)o[3])};
     *reinterpret_cast<v4i*>(dst) = w4;
-  } else if (whole) {
+  } else if (whole && sizeof(Out) == 1) {
     *reinterpret_cast<unsigned*>(dst) = (unsigned)(unsigned char)o[0] | ((unsigned)(unsigned char)o[1] << 8) |
                                         ((unsigned)(unsigned char)o[2] << 16) | ((unsigned)(unsigned char)o[3] << 24);
   } else {
@@ -1714,7 +1714,7 @@ __device__ __forceinline__ void store_skinny_tile_pre(v4i acc, const GemmParams&
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     o[v] = E::apply(acc[v], E::bias_term(bv[v], p.beta), p.alpha);
-    if constexpr (E::kAccumulate) o[v] = old[v] + o[v];
+    if constexpr (E::kAccumulate) o[v] = accumulated(old[v], o[v]);
   }
   if (!live) return;
   Out* dst = C + out_index(p, m, nb < N ? nb : 0);
@@ -1724,7 +1724,7 @@ __device__ __forceinline__ void store_skinny_tile_pre(v4i acc, const GemmParams&
     v4i w4 = {__builtin_bit_cast(int, (W)o[0]), __builtin_bit_cast(int, (W)o[1]), __builtin_bit_cast(int, (W)o[2]),
               __builtin_bit_cast(int, (W)o[3])};
     *reinterpret_cast<v4i*>(dst) = w4;
-  } else if (whole) {
+  } else if (whole && sizeof(Out) == 1) {
     *reinterpret_cast<unsigned*>(dst) = (unsigned)(unsigned char)o[0] | ((unsigned)(unsigned char)o[1] << 8) |
                                         ((unsigned)(unsigned char)o[2] << 16) | ((unsigned)(unsigned char)o[3] << 24);
   } else {
@@ -2053,7 +2053,7 @@ __global__ __launch_bounds__(256) void gemm_stream_kernel(GemmParams p, int stri
 #pragma unroll
           for (int v = 0; v < 4 / PARTS; ++v) {
             Out o = E::apply(d[v], E::bias_term(bias_pre[v], p.beta), p.alpha);
-            if constexpr (E::kAccumulate) o = old_pre[v] + o;
+            if constexpr (E::kAccumulate) o = accumulated(old_pre[v], o);
             if (f == 0 && m < m_real && n_first + v < n_real) C[(size_t)m * n_real + n_first + v] = o;
           }
           acc = v4i{0, 0, 0, 0};
@@ -2151,7 +2151,7 @@ __global__ __launch_bounds__(256) void gemm_gemv_kernel(GemmParams p, GemmGroup 
     const float alpha = GROUPED ? grp.alpha[prob] : p.alpha;
     const float beta = GROUPED ? grp.beta[prob] : p.beta;
     Out o = E::apply(acc, E::bias_term(bv, beta), alpha);
-    if constexpr (E::kAccumulate) o = old + o;
+    if constexpr (E::kAccumulate) o = accumulated(old, o);
     *dst = o;
   }
 }
@@ -2314,7 +2314,10 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmParams p, const 
       if (E::kHasBias) bv = bias[n + v];
       o[v] = merge_old<E>(E::apply(acc[v], E::bias_term(bv, p.beta), p.alpha), dst + v);
     }
-    if (sizeof(Out) == 4) {
+    if constexpr (sizeof(Out) == 2) {
+      typedef Out Out4 __attribute__((ext_vector_type(4)));
+      *reinterpret_cast<Out4*>(dst) = Out4{o[0], o[1], o[2], o[3]};
+    } else if (sizeof(Out) == 4) {
       using W = typename std::conditional<sizeof(Out) == 4, Out, int>::type;
       v4i w4 = {__builtin_bit_cast(int, (W)o[0]), __builtin_bit_cast(int, (W)o[1]), __builtin_bit_cast(int, (W)o[2]),
                 __builtin_bit_cast(int, (W)o[3])};
@@ -2880,6 +2883,8 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
     if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
     return TI_OK;
   }
+  if constexpr (sizeof(Out) == 2) return fail(TI_ERR_INVALID_ARG, "fp16 outputs: up to 16 rows (got %d)", p.M);
+  else {
   constexpr bool SWAP = sizeof(Out) == 1;  // 8-bit outputs take the orientation whose lanes own 16 consecutive columns
   // Some of the tilings hold 32-bit offsets into their panels (Pipe16QCfg::PANEL_COPIES); rows that lie further apart than those
   // reach go to the 64-byte steps, whose copies have whole addresses, before a tiling is chosen.
@@ -3121,6 +3126,7 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
   }
   g_last_kernel = "tile_64x64";
   return launch_tile<TileCfg<64, 64, 2, 2, KIND, SWAP>>(p, stream);
+  }
 }
 
 }  // namespace ti

@@ -17,59 +17,9 @@
 //   (offsets 32..1); the four wavefront sums are added left to right.
 #include <type_traits>
 
-#include "ti_common.h"
+#include "ln_math.h"
 
 namespace ti {
-
-__device__ __forceinline__ float wave_butterfly_sum(float s) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) s = s + __shfl_xor(s, off, 64);
-  return s;
-}
-
-// `red`: four floats that nothing else uses
-__device__ __forceinline__ float block_sum_256(float s, float* red) {
-  s = wave_butterfly_sum(s);
-  const int wave = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) red[wave] = s;
-  __syncthreads();
-  return ((red[0] + red[1]) + red[2]) + red[3];
-}
-
-typedef _Float16 v4h __attribute__((ext_vector_type(4)));
-
-// four consecutive elements as they lie in memory; chunk c of a row as fp32 / stored from fp32
-template <class T> struct Chunk;
-template <> struct Chunk<float> { typedef v4f type; };
-template <> struct Chunk<_Float16> { typedef v4h type; };
-__device__ __forceinline__ v4f to_f32(v4f v) { return v; }
-__device__ __forceinline__ v4f to_f32(v4h h) { return v4f{(float)h[0], (float)h[1], (float)h[2], (float)h[3]}; }
-__device__ __forceinline__ v4f load4(const float* row, int c) { return reinterpret_cast<const v4f*>(row)[c]; }
-__device__ __forceinline__ v4f load4(const _Float16* row, int c) {
-  const v4h h = reinterpret_cast<const v4h*>(row)[c];
-  return v4f{(float)h[0], (float)h[1], (float)h[2], (float)h[3]};
-}
-__device__ __forceinline__ void store4(float* row, int c, v4f v) { reinterpret_cast<v4f*>(row)[c] = v; }
-__device__ __forceinline__ void store4(_Float16* row, int c, v4f v) {
-  reinterpret_cast<v4h*>(row)[c] = v4h{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-}
-// The value a tensor of element type T holds after the fp32 value `x` is stored to it (round to nearest even
-// for fp16).  The empty asm keeps the fp32 result of the preceding operation a value of its own: without it the
-// compiler merges an fma and the conversion into one mixed-precision instruction that rounds the exact sum
-// straight to fp16, which differs from "fp32 operation, then conversion" when the fp32 result is a tie.
-template <class T>
-__device__ __forceinline__ float as_stored(float x) {
-  if constexpr (sizeof(T) == 2) asm volatile("" : "+v"(x));
-  return (float)(T)x;
-}
-
-__device__ __forceinline__ int pack_s8x4(float y0, float y1, float y2, float y3) {
-  unsigned b0 = (unsigned char)(int8_t)rne_s8(y0);
-  unsigned b1 = (unsigned char)(int8_t)rne_s8(y1);
-  unsigned b2 = (unsigned char)(int8_t)rne_s8(y2);
-  unsigned b3 = (unsigned char)(int8_t)rne_s8(y3);
-  return (int)(b0 | (b1 << 8) | (b2 << 16) | (b3 << 24));
-}
 
 // What is normalised: MODE_DQ_ADD  r = res + scale * float(in)   (int32 in; dq_add_layernorm_q)
 //                     MODE_ADD     r = res + x                   (fp32 x passed through `in`)

@@ -28,6 +28,7 @@ enum EpiKind : int {
   EPI_S8_SCALE = 6,    // out = s8(rint(clamp(a * acc)))
   EPI_S32_RAW = 7,     // out = acc
   EPI_F32_BIAS_ACC = 8,  // out = out + fma(a, acc, b*bias)   (fp32; adds into the tensor already there)
+  EPI_F16_BIAS_ACC = 9,  // out = f16(out + f16(fma(a, acc, b*bias)))   (fp16 tensor already there, fp32 bias)
 };
 
 // round-half-even then v_cvt_i32_f32, which saturates to int32 and maps NaN to 0
@@ -153,12 +154,33 @@ struct Epi<EPI_F32_BIAS_ACC> {
   }
 };
 
-// `fresh` for the ordinary kinds; `*where + fresh` (one fp32 add, the linear's own result rounded first)
-// for the accumulate-into-output kind.
+template <>
+struct Epi<EPI_F16_BIAS_ACC> {
+  using Out = _Float16;
+  using Bias = float;
+  static constexpr bool kHasBias = true;
+  static constexpr bool kAccumulate = true;
+  static __device__ __forceinline__ float bias_term(Bias b, float beta) { return beta * b; }
+  static __device__ __forceinline__ Out apply(int acc, float bt, float alpha) {
+    float t = __builtin_fmaf(alpha, (float)acc, bt);
+    asm("" : "+v"(t));  // rounded to fp32 first: not one instruction that rounds the exact sum to fp16
+    return (_Float16)t;
+  }
+};
+
+// What the accumulating kinds store: the old value plus the linear's own rounded result, one add of the output's type (for fp16 in
+// fp32 and then rounded, which is the same number: 24 bits are more than twice 11 and two).
+template <class Out>
+__device__ __forceinline__ Out accumulated(Out old, Out fresh) {
+  if constexpr (sizeof(Out) == 2) return (Out)((float)old + (float)fresh);
+  else return old + fresh;
+}
+
+// `fresh` for the ordinary kinds; `*where + fresh` for the accumulate-into-output ones.
 template <class E>
 __device__ __forceinline__ typename E::Out merge_old(typename E::Out fresh, const typename E::Out* where) {
   if constexpr (E::kAccumulate)
-    return *where + fresh;
+    return accumulated(*where, fresh);
   else
     return fresh;
 }
@@ -271,6 +293,7 @@ int rows_pick_for_test(long long M, long long N, long long K, int cus, int* tili
 int rows_slot_for_test(long long* table, signed char* state, int cap, long long stream, int* fresh);
 int placement_of(const volatile int* words);
 int last_rows(int* tiling, int* slices);
+int compute_units();  // of the current device
 const char* last_gemm_kernel();  // kernel family of the calling thread's last launch_gemm ("" before the first)
 const char* last_gemm_form();    // which of a family's pipelined kernels that was ("" for the others)
 
@@ -291,6 +314,21 @@ int launch_add_layernorm_q_f16_xf32(const float* x, void* residual, const void* 
                                     int8_t* q_out, long long rows, long long H, hipStream_t stream);
 int launch_add_layernorm_q_f16(const void* x, void* residual, const void* gamma, const void* beta, float eps,
                                int8_t* q_out, long long rows, long long H, hipStream_t stream);
+
+// ln_linear.hip: LayerNorm-quantise up to LN_LINEAR_ROWS rows and multiply them with up to three weight matrices in one launch
+constexpr int LN_LINEAR_ROWS = 4;
+struct LnLinear {
+  const void *hidden, *gamma, *beta;  // the stream (only read) and the LayerNorm's parameters: fp32, or all three fp16
+  float eps;
+  int M, K, N, problems;              // rows, width, outputs of one problem, problems
+  int lo;                             // lower bound of an output: -128, or 0 behind a ReLU
+  const int8_t* W[3];
+  const int8_t* bias[3];
+  int8_t* out[3];                     // [M, N] each
+  float alpha[3], beta_s[3];
+};
+bool ln_linear_takes(const LnLinear& p, bool half);
+int launch_ln_linear(const LnLinear& p, bool half, hipStream_t stream);
 
 // softmax_q.hip
 int launch_attn_softmax_q(const float* scores, const float* mask, int8_t* out, long long batch, long long heads,
