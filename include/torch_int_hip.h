@@ -333,7 +333,7 @@ int ti_linear_a8_w8_bfp32_ofp32_acc(const int8_t* x, const int8_t* w, const floa
                                     void* workspace, int64_t workspace_bytes, void* stream);
 
 /* The same on an fp16 tensor: inout[m,n] = f16(inout[m,n] + f16(fmaf(alpha, acc, beta*bias[n]))), the result rounded to fp32,
- * then to fp16, then added: `residual.add_(fc2(x).to(residual.dtype))` (torch_int/models/opt.py:287-289).  Up to 16 rows. */
+ * then to fp16, then added: `residual.add_(fc2(x).to(residual.dtype))` (torch_int/models/opt.py:287-289). */
 int ti_linear_a8_w8_bfp32_of16_acc(const int8_t* x, const int8_t* w, const float* bias, void* inout,
                                    int64_t M, int64_t N, int64_t K, float alpha, float beta,
                                    void* workspace, int64_t workspace_bytes, void* stream);
@@ -543,7 +543,7 @@ int ti_opt_decoder_layer_prefill(const TiOptDecodeLayer* layer, void* hidden, co
 /* The two calls above for the layers of a model one after the other on one residual stream (Int8OPTDecoder.forward's loop,
  * torch_int/models/opt.py:302-398): decode steps of up to 64 sequences, prefills of any number of tokens.  carry: fp32
  * [rows, embed] that belongs to this pass (16-byte aligned; unused with chain = 0).  chain & 2: where the output of fc2 would be
- * added to the stream by a kernel of its own (an fp16 stream, or more than 4096 rows), leave it in carry instead; chain & 1:
+ * added to the stream by a kernel of its own (an fp16 stream of 5 to 64 rows, an fp32 one of more than 4096), leave it in carry instead; chain & 1:
  * this call's first LayerNorm kernel adds what the call before left there.  Every layer but the last leaves, every layer but
  * the first adds; the additions and their order are those of the separate calls.  A prefill with chain != 0 keeps the output of
  * out_proj in carry too and does with less scratch: ti_opt_decoder_layer_prefill_chained_scratch_bytes(B * T, embed, ffn). */

@@ -806,8 +806,8 @@ int ti_transpose_last2_s8(const int8_t* src, int8_t* dst, int64_t B, int64_t R, 
 // ---------------------------------------------------------------- a decoder layer from one C call
 // A decoder layer, one new token per sequence or a prefill: the calls that Int8OPTDecoderLayer's modules make, each of them
 // the public entry point with the arguments the modules pass, so the values are theirs.  In a chain of layers (CHAIN_*, the
-// layers of a model one after the other) one thing is moved: on an fp16 residual stream, and on an fp32 one
-// beyond 4096 rows, where the GEMM's accumulating epilogue costs more than it saves, the output of fc2 is added by the NEXT
+// layers of a model one after the other) one thing is moved: on an fp16 residual stream of 5 to 64 rows, and on an fp32 one
+// beyond 4096 rows, where the GEMM's accumulating epilogue costs more than it saves (adds_later), the output of fc2 is added by the NEXT
 // layer's LayerNorm kernel, which reads the stream anyway, instead of by a kernel of its own (3 us of a decode layer, 6.3 us
 // at 2048 x 2048: a launch, and the stream read and written once more).  Same additions, same order.
 }  // extern "C"
@@ -837,8 +837,10 @@ int layernorm(const TiOptDecodeLayer* L, const float* pending, void* hidden, con
                             : ti_add_layernorm_q_f16_xf32(pending, hidden, gamma, beta, eps, out, rows, E, stream);
 }
 
-// whether fc2's output is added by a later kernel rather than in the GEMM's epilogue
-bool adds_later(const TiOptDecodeLayer* L, int64_t rows) { return L->half || rows > 4096; }
+// Whether fc2's output is added by a later kernel rather than in the GEMM's epilogue.  On an fp16 stream the epilogue of fc2, and of
+// out_proj with it, adds from 65 rows on: four bytes of an element read and written instead of four written, and a LayerNorm that reads
+// two instead of six and writes none of the stream (2048 x 2048 8.5 -> 5.3 us, 1904 x 4096 14.5 -> 7.6).  The kernels of fewer rows stream weights, and gain nothing.
+bool adds_later(const TiOptDecodeLayer* L, int64_t rows) { return L->half ? rows <= 64 : rows > 4096; }
 
 // Decode steps of a few rows: out_proj and fc2 add into the stream themselves, and the LayerNorm is part of the launch that
 // reads its result.  The layers of a chain agree on this (it looks at the rows alone): none leaves a carry.
@@ -878,6 +880,12 @@ int after_attention(const TiOptDecodeLayer* L, const int8_t* ctx, float* f32, in
                     int64_t rows, int chain, float* carry, void* ws, int64_t ws_bytes, void* stream) {
   const int64_t E = L->embed, F = L->ffn;
   int rc;
+  if (L->half && !adds_later(L, rows)) {
+    if ((rc = ti_linear_a8_w8_bfp32_of16_acc(ctx, L->wo, L->bo, hidden, rows, E, E, L->alpha_o, 1.0f, ws, ws_bytes, stream))) return rc;
+    if ((rc = layernorm(L, nullptr, hidden, L->ln2_gamma, L->ln2_beta, L->ln2_eps, x, rows, stream))) return rc;
+    if ((rc = ti_linear_relu_a8_w8_b8_o8(x, L->w1, L->b1, h, rows, F, E, L->alpha_1, L->beta_1, ws, ws_bytes, stream))) return rc;
+    return ti_linear_a8_w8_bfp32_of16_acc(h, L->w2, L->b2, hidden, rows, E, F, L->alpha_2, 1.0f, ws, ws_bytes, stream);
+  }
   if ((rc = ti_linear_a8_w8_bfp32_ofp32(ctx, L->wo, L->bo, f32, rows, E, E, L->alpha_o, 1.0f, ws, ws_bytes, stream))) return rc;
   if ((rc = layernorm(L, f32, hidden, L->ln2_gamma, L->ln2_beta, L->ln2_eps, x, rows, stream))) return rc;
   if ((rc = ti_linear_relu_a8_w8_b8_o8(x, L->w1, L->b1, h, rows, F, E, L->alpha_1, L->beta_1, ws, ws_bytes, stream))) return rc;

@@ -217,7 +217,7 @@ __device__ __forceinline__ void store_tile(v16i (&acc)[Cfg::TM][Cfg::TN], const 
               w[q] = (int)(b0 | (b1 << 8) | (b2 << 16) | (b3 << 24));
             }
             *reinterpret_cast<v4i*>(dst) = w;
-          } else {
+          } else if constexpr (sizeof(Out) == 4) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               Out o0 = merge_old<E>(E::apply(acc[i][j][4 * q + 0], bt[4 * q + 0], alpha), dst + 4 * q + 0);
@@ -279,6 +279,33 @@ __device__ __forceinline__ void store_tile(v16i (&acc)[Cfg::TM][Cfg::TN], const 
         continue;
        }
       }
+      if constexpr (sizeof(Out) == 2) {  // the same exchange: eight bytes of a row to a lane, for what is there and for the sum
+        if ((N & 3) == 0 && nq + 32 <= N && (reinterpret_cast<uintptr_t>(C) & 7) == 0) {
+          typedef Out Out4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+          for (int i = 0; i < TM; ++i) {
+            Out4 old[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const int m = m0 + wave_m * Cfg::WTM + i * 32 + 8 * q + 4 * half + (lane & 3);
+              old[q] = *reinterpret_cast<const Out4*>(C + ((long long)(m < M ? m : M - 1) * N + nq + (frow & ~3)));
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              int x[4];
+#pragma unroll
+              for (int k = 0; k < 4; ++k) x[k] = __builtin_bit_cast(unsigned short, E::apply(acc[i][j][4 * q + k], bt, alpha));
+              quad_transpose(x, lane);
+              const int m = m0 + wave_m * Cfg::WTM + i * 32 + 8 * q + 4 * half + (lane & 3);
+              const unsigned lo = (unsigned)x[0] | (unsigned)x[1] << 16, hi = (unsigned)x[2] | (unsigned)x[3] << 16;
+              const unsigned long long both = lo | (unsigned long long)hi << 32;
+              const Out4 sum = old[q] + __builtin_bit_cast(Out4, both);
+              if (m < M) *reinterpret_cast<Out4*>(C + ((long long)m * N + nq + (frow & ~3))) = sum;
+            }
+          }
+          continue;
+        }
+      }
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -288,7 +315,7 @@ __device__ __forceinline__ void store_tile(v16i (&acc)[Cfg::TM][Cfg::TN], const 
             Out fresh = E::apply(acc[i][j][v], bt, alpha);
             // plain row-major only: head-major output exists for 8-bit outputs, which take the branch above
             Out* at = C + ((long long)m * N + n);
-            if constexpr (E::kAccumulate) fresh = *at + fresh;
+            if constexpr (E::kAccumulate) fresh = accumulated(*at, fresh);
             *at = fresh;
           }
         }
@@ -1030,6 +1057,86 @@ __device__ __forceinline__ void store_tile16(v4i (&acc)[Cfg::TM][Cfg::TN], const
       }
       return;
     }
+  }
+  if constexpr (sizeof(Out) == 2) {
+    // fp16 outputs that are added to (launch_kind: whole groups of eight columns, on 16 bytes).  The lanes of a row swap halves of
+    // two column blocks, a result being two dwords a block, so that a lane ends with eight consecutive columns of one of them:
+    // sixteen bytes, 64 contiguous ones a row, for the loads of what is there and for the stores.  Bound as the 32-bit epilogue is by
+    // the stores of a CU, of which there are half as many, and by one round trip for what is there: 2048 x 2048 x 2048 and x 8192 28.7 us
+    // in the mean with fp32 outputs, 27.7 so; 1904 x 4096 x 4096 and x 16384 71.4 and 70.8; the LayerNorm behind reads 2 bytes for 6.
+    typedef Out Out4 __attribute__((ext_vector_type(4)));
+    typedef Out Out8 __attribute__((ext_vector_type(8)));
+    typedef unsigned U2 __attribute__((ext_vector_type(2)));
+    typedef unsigned U4 __attribute__((ext_vector_type(4)));
+    constexpr int PAIRS = (TN + 1) / 2;  // an odd last block is a pair by itself, four columns to a lane
+    // pairs whose values and bias are fetched ahead: all where the accumulators leave the registers
+    constexpr int AHEAD = TM * TN < 24 ? PAIRS : TM * TN == 24 ? 2 : 1;
+    // The rows of the tile that the matrix has, as a buffer: 32-bit offsets, and what lies beyond it loads zeros and stores nothing.
+    const int rows = M - tile_m * BM < BM ? M - tile_m * BM : BM;
+    const __amdgpu_buffer_rsrc_t tile =
+        __builtin_amdgcn_make_buffer_rsrc(C + (long long)tile_m * BM * N, 0, (int)((unsigned)rows * (unsigned)N * 2u), 0x00020000);
+    const __amdgpu_buffer_rsrc_t columns = __builtin_amdgcn_make_buffer_rsrc(const_cast<BiasT*>(bias), 0, (int)((unsigned)N * 4u), 0x00020000);
+    const int nw = tile_n * BN + wave_n * Cfg::WTN;
+    const unsigned row_at = (unsigned)(wave_m * Cfg::WTM + er) * (unsigned)N * 2u, down = 16u * (unsigned)N * 2u;
+    auto column_of = [&](int j) { return 2 * j + 1 == TN ? nw + j * 32 + 4 * eg : nw + j * 32 + (eg & 1) * 16 + (eg >> 1) * 8; };
+    auto at = [&](int j) { return column_of(j) < N ? row_at + (unsigned)column_of(j) * 2u : 0xfffff000u - (TM - 1) * down; };
+    Out8 held[AHEAD][TM];
+    v4f braw[AHEAD][2];
+    auto fetch_row = [&](int j, int i) {
+      if (2 * j + 1 == TN) {
+        const U2 w = __builtin_amdgcn_raw_buffer_load_b64(tile, at(j) + i * down, 0, 0);
+        held[j % AHEAD][i] = __builtin_bit_cast(Out8, U4{w[0], w[1], 0, 0});
+      } else {
+        held[j % AHEAD][i] = __builtin_bit_cast(Out8, __builtin_amdgcn_raw_buffer_load_b128(tile, at(j) + i * down, 0, 0));
+      }
+    };
+    auto fetch_bias = [&](int j) {
+      const unsigned b0 = (unsigned)(nw + j * 32 + 4 * eg) * 4u;
+      braw[j % AHEAD][0] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(columns, b0, 0, 0));
+      if (2 * j + 1 != TN) braw[j % AHEAD][1] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(columns, b0 + 64, 0, 0));
+    };
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+      fetch_bias(j);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) fetch_row(j, i);
+    }
+#pragma unroll
+    for (int j = 0; j < PAIRS; ++j) {
+      const bool odd = 2 * j + 1 == TN;
+      const unsigned to = at(j);
+      float bt[2][4];
+#pragma unroll
+      for (int q = 0; q < (odd ? 1 : 2); ++q)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) bt[q][v] = E::bias_term(braw[j % AHEAD][q][v], p.beta);
+      if (j + AHEAD < PAIRS) fetch_bias(j + AHEAD);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        auto block = [&](int q) {
+          const v4i& a = acc[i][2 * j + q];
+          return Out4{E::apply(a[0], bt[q][0], p.alpha), E::apply(a[1], bt[q][1], p.alpha), E::apply(a[2], bt[q][2], p.alpha),
+                      E::apply(a[3], bt[q][3], p.alpha)};
+        };
+        const Out8 old = held[j % AHEAD][i];
+        if (j + AHEAD < PAIRS) fetch_row(j + AHEAD, i);
+        if (odd) {
+          const Out4 sum = Out4{old[0], old[1], old[2], old[3]} + block(0);  // one rounding each, as `accumulated`
+          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, sum), tile, to + i * down, 0, 0);
+        } else {
+          const Out4 a = block(0), b2 = block(1);
+          unsigned x[2], y[2];
+          __builtin_memcpy(x, &a, 8);
+          __builtin_memcpy(y, &b2, 8);
+          auto s0 = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false);
+          auto s1 = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
+          const Out8 fresh = __builtin_bit_cast(Out8, U4{s0[0], s1[0], s0[1], s1[1]});
+          const Out8 sum = old + fresh;
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, sum), tile, to + i * down, 0, 0);
+        }
+      }
+    }
+    return;
   }
   // accumulate-into-output kind: fetch what the tile holds now, the loads in flight together before the
   // first use -- the whole wave tile when its TM*TN*4 registers fit, else one column block at a time
@@ -2883,8 +2990,13 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
     if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
     return TI_OK;
   }
-  if constexpr (sizeof(Out) == 2) return fail(TI_ERR_INVALID_ARG, "fp16 outputs: up to 16 rows (got %d)", p.M);
-  else {
+  if constexpr (sizeof(Out) == 2) {  // store_tile16 adds to whole groups of eight columns; anything else: tiles that add one by one
+    if (p.N % 8 != 0 || p.N > 1 << 22 || p.batch != 1 || p.out_d != 0 || (reinterpret_cast<uintptr_t>(p.C) & 15) != 0 ||
+        (reinterpret_cast<uintptr_t>(p.bias) & 3) != 0) {
+      g_last_kernel = "tile_64x64";
+      return launch_tile<TileCfg<64, 64, 2, 2, KIND, false>>(p, stream);
+    }
+  }
   constexpr bool SWAP = sizeof(Out) == 1;  // 8-bit outputs take the orientation whose lanes own 16 consecutive columns
   // Some of the tilings hold 32-bit offsets into their panels (Pipe16QCfg::PANEL_COPIES); rows that lie further apart than those
   // reach go to the 64-byte steps, whose copies have whole addresses, before a tiling is chosen.
@@ -2982,9 +3094,10 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
                       : tile == SPLIT_128x192 ? "splitk_128x192"
                       : tile == SPLIT_160x160 ? "splitk_160x160"
                                               : "splitk_256x288";
-      // not for the accumulating epilogue: its reads of the old outputs, done by one workgroup per tile instead of
+      // not for the fp32 accumulating epilogue: its reads of the old outputs, done by one workgroup per tile instead of
       // by the whole chip in the reduction kernel, cost more than the launch saved (512x9216x36864: 288 against
-      // 178 us, 256x5120x5120: 29 against 22 us)
+      // 178 us, 256x5120x5120: 29 against 22 us).  An fp16 tile, read and written, is as many bytes as an fp32 one written:
+      // passes of OPT-6.7B 1 x 500 fp16 3.06 ms in two launches, 2.66 so (2.83 with fp32 outputs added by the LayerNorm).
       if constexpr (KIND != EPI_S32_RAW && KIND != EPI_F32_BIAS_ACC) {
         // (a workspace on a 256-byte boundary only: the 1 KiB regions the waves park and read back must not share a
         // 128-byte line with a neighbour's, or a line fetched for one region could be reused, stale, for the next)
@@ -3058,7 +3171,7 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
       // 76 -> 47, 2048x4096x4096 48 -> 35, 2048x4096x16384 170 -> 118, 2048x2560x2560 25 -> 20, 2048x12288x12288
       // 285 -> 253.
       const bool wide_step = p.K % QBK == 0;
-      switch (pick_wide(p.M, p.N, p.K, p.batch, !SWAP).tile) {
+      switch (pick_wide(p.M, p.N, p.K, p.batch, sizeof(Out) == 4).tile) {
         case WIDE_256x160:
           g_last_kernel = "pipe16_256x160";
           if (wide_step) return launch_pipe16q<Pipe16QCfg<256, 160, 4, 2, KIND>>(p, stream);
@@ -3091,8 +3204,9 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
           // the next tile's first copies (8192x20480x5120 764 against 803 us).
           // And so do products of two activations, whose epilogue without a bias the compiler puts among the copies (94 of 289x160x4096
           // 55 against 61 us, 7 of 1645x1648x4096 109 against 117).
-          if constexpr (SWAP && KIND != EPI_S8_SCALE) {
-            if (wide_step && p.K >= 2048) return launch_pipe16q<Pipe16QCfg<256, 256, 4, 2, KIND>>(p, stream);
+          // (fp16 outputs leave from 16x16 blocks only.)
+          if constexpr ((SWAP && KIND != EPI_S8_SCALE) || sizeof(Out) == 2) {
+            if (wide_step && (p.K >= 2048 || sizeof(Out) == 2)) return launch_pipe16q<Pipe16QCfg<256, 256, 4, 2, KIND>>(p, stream);
           }
           if (wide_step) return launch_pipe2<Pipe2Cfg<256, 256, 2, 4, KIND, SWAP>>(p, stream);  // whole cache lines per row
           return launch_pipe<PipeCfg<256, 256, 2, 4, 4, KIND, SWAP>>(p, stream);
@@ -3126,7 +3240,6 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
   }
   g_last_kernel = "tile_64x64";
   return launch_tile<TileCfg<64, 64, 2, 2, KIND, SWAP>>(p, stream);
-  }
 }
 
 }  // namespace ti

@@ -697,7 +697,7 @@ def opt_prefill_scratch(plans, hidden):
                 _layer_scratch_need.clear()
             n = _layer_scratch_need[key] = (
                 scratch_bytes(M, E, F),
-                max(_CUDA._ws_bytes(M, E, E), _CUDA._ws_bytes(M, F, E), _CUDA._ws_bytes(M, E, F, True)))
+                max(_CUDA._ws_bytes(M, E, E, True), _CUDA._ws_bytes(M, F, E), _CUDA._ws_bytes(M, E, F, True)))
         need, need_ws = max(need, n[0]), max(need_ws, n[1])
     with _on(dev):
         stream = _raw_stream(dev.index)
