@@ -86,6 +86,13 @@ def test_every_epilogue_is_exact(M, N, K):
         assert torch.equal(X.linear_a8_w8_b8_o8_heads(xd, wd, b8d, al, be, 1, M, N // d, d).cpu(), want)
 
 
+@pytest.mark.parametrize("M,N,K,tiling", [(5, 768, 12288, "F3"), (17, 1024, 12288, "F3"), (24, 4096, 16384, "F4"), (64, 784, 16384, "F4"),
+                                          (49, 2048, 16384, "F4"), (16, 5120, 16384, "F4")])
+def test_slices_of_sixteen_waves(M, N, K, tiling, monkeypatch):
+    monkeypatch.setitem(SHAPES, (M, N, K), tiling)
+    test_every_epilogue_is_exact(M, N, K)
+
+
 @pytest.mark.parametrize("N,K,want", [(272, 768, "E1"), (272, 1024, "B1"), (272, 2048, "A1"), (272, 2560, "D1"), (272, 3072, "G1"),
                                       (272, 3584, "H1"), (272, 4096, "F1"), (272, 5120, "C1"), (272, 2304, "E3"),
                                       (272, 6144, "A3"), (272, 7168, "H2"), (272, 7680, "D3"), (272, 9216, "G3"),
