@@ -406,16 +406,13 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::NW == 16 ? 4 : 2) void gemm_rows_kern
 //   C  8 waves x 640 bytes, one workgroup per CU: K % 5120 == 0
 //   D  4 waves x 640 bytes, two per CU: K % 2560 == 0
 //   E  4 waves x 192 bytes, two per CU: K % 768 == 0
-//   F  16 waves x 256 bytes, one per CU: K = 4096, 12288 or 16384
+//   F  16 waves x 256 bytes, one per CU: K == 4096, and pairs of A's slices (rows_paired)
 //   G  8 waves x 384 bytes, one per CU: K % 3072 == 0
 //   H  8 waves x 448 bytes, one per CU: K % 3584 == 0
 // A divisor of K that is a whole slice comes first (C, F, H, then A, G, D, B, E): slices that meet cost 2 to 2.5 us a launch (park,
 // count, add), which only a long K repays.  Several slices take the first tiling in that order; the pairs that are measured
 // below compare one slice with several.  A K whose first divisor makes too many slices goes to the other kernels, also where
-// another tiling would fit (36864: 18 of A, 12 of G; 49152: 24 of A, 16 of G).  Three and four slices of F before twice as many of A:
-// half as many tiles to park, and to add at the end (24 x 4096 x 16384 17.5 us, 15.9 so; 64 x 7168 x 16384 35.7 / 28.9, 40 x 8192 x
-// 12288 32.3 / 23.2; 242 shapes of 768 to 12288 columns and 2 to 64 rows 0.92 times the time in the mean, worst 1.04).  Two are level with
-// four of A (8192: 16 and 48 x 2048 1.03 and 1.05, 17 to 48 x 8192 0.94 to 0.96), six and seven with twelve of A and eight of H.
+// another tiling would fit (36864: 18 of A, 12 of G; 49152: 24 of A, 16 of G).
 // us, cold weights, 16 / 32 / 64 rows: 5120 x 5120 C 8.9 / 10.5 / 13.3, B in five slices 9.5 / 11.7 / 15.4;
 // 4096 x 4096 F 6.3 / 7.8 / 9.7, A in two 7.2 / 8.7 / 10.5; 16384 x 4096 F 13.1 / 14.6 / 17.6, A in two 14.4 / 16.7 / 21.3 (F with 64
 // rows: 8 waves of 512 bytes, 16 waves have too few registers for the fragments and spill, 21.8); 768 x 3072 G
@@ -478,7 +475,7 @@ static inline bool few_rows_slices_ahead(RowsPick pick, long long M, long long N
 static inline RowsPick rows_pick(long long M, long long N, long long K, int cus = num_cus(), int problems = 1) {
   if (M < 1 || M > TI_ROWS_MAX_M || N < 1 || K < 768 || K > (1 << 20)) return {ROWS_NONE, 1};
   RowsPick pick{ROWS_NONE, 1};
-  if (K == 4096 || K == 12288 || K == 16384) pick = {ROWS_F, (int)(K / 4096)};
+  if (K == 4096) pick = {ROWS_F, 1};
   else if (K % 5120 == 0) pick = {ROWS_C, (int)(K / 5120)};
   else if (K % 3584 == 0) pick = {ROWS_H, (int)(K / 3584)};
   else if (K % 2048 == 0) pick = {ROWS_A, (int)(K / 2048)};
@@ -497,6 +494,14 @@ static inline RowsPick rows_pick(long long M, long long N, long long K, int cus 
                                    : rows_slices_ahead(pick, M, N, K, problems, cus)))
     return {ROWS_NONE, 1};
   return pick;
+}
+
+// Six and eight slices of A run as three and four of F: half as many tiles to park, and to add at the end.  24 x 4096 x 16384 17.5 us,
+// 15.9 so; 64 x 7168 x 16384 35.7 / 28.9, 5 x 2048 x 16384 10.9 / 9.8; 220 shapes of 768 to 12288 columns and 2 to 64 rows 0.92 times the time
+// in the mean, worst 1.04 (33 x 768 x 12288).  Four as two are level (8192: 16 and 48 x 2048 1.03 and 1.05, 17 to 48 x 8192 0.94 to 0.96),
+// twelve as six not everywhere ahead (768 columns 1.02).
+static inline RowsPick rows_paired(RowsPick pick, long long K) {
+  return pick.tiling == ROWS_A && (K == 12288 || K == 16384) ? RowsPick{ROWS_F, pick.slices / 2} : pick;
 }
 
 template <class Cfg>
@@ -550,7 +555,7 @@ template <int KIND, bool GROUPED>
 static int launch_rows(const GemmParams& p_in, const GemmGroup& grp, int problems, void* workspace,
                        long long workspace_bytes, hipStream_t stream) {
   if (p_in.batch != 1 || p_in.lda != p_in.K || p_in.ldb != p_in.K) return -1;
-  const RowsPick pick = rows_pick(p_in.M, p_in.N, p_in.K, num_cus(), problems);
+  const RowsPick pick = rows_paired(rows_pick(p_in.M, p_in.N, p_in.K, num_cus(), problems), p_in.K);
   if (pick.tiling == ROWS_NONE) return -1;
   GemmParams p = p_in;
   p.splits = pick.slices;
