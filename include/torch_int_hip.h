@@ -562,6 +562,13 @@ int ti_opt_decoder_layer_prefill_chained(const TiOptDecodeLayer* layer, void* hi
                                          int chain, float* carry, void* scratch, int64_t scratch_bytes, void* workspace,
                                          int64_t workspace_bytes, void* stream);
 
+/* The layers of one decode step one after the other from one call: ti_opt_decoder_layer_decode_chained for layers[0 .. count - 1],
+ * whose cache buffers are all [B, heads, cap, head_dim] of one cap; the first without chain & 1, the last without chain & 2, or
+ * with chain = 0 throughout where carry is NULL. */
+int ti_opt_decoder_layers_decode(const TiOptDecodeLayer* const* layers, int64_t count, void* hidden, const float* mask,
+                                 int8_t* const* k_bufs, int8_t* const* v_bufs, int64_t B, int64_t cap, int64_t S, float* carry,
+                                 void* scratch, int64_t scratch_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1060,6 +1060,22 @@ int ti_opt_decoder_layer_decode_from(const TiOptDecodeLayer* L, void* hidden, co
                       chain, carry, scratch, scratch_bytes, stream, 64);
 }
 
+int ti_opt_decoder_layers_decode(const TiOptDecodeLayer* const* layers, int64_t count, void* hidden, const float* mask,
+                                 int8_t* const* k_bufs, int8_t* const* v_bufs, int64_t B, int64_t cap, int64_t S, float* carry,
+                                 void* scratch, int64_t scratch_bytes, void* stream) {
+  g_err[0] = 0;
+  const char* op = "opt_decoder_layers_decode";
+  if (count < 0 || (count > 0 && (layers == nullptr || k_bufs == nullptr || v_bufs == nullptr)))
+    return fail(TI_ERR_INVALID_ARG, "%s: %lld layers, an array is NULL", op, (long long)count);
+  for (int64_t i = 0; i < count; ++i) {
+    const int chain = carry == nullptr ? 0 : (i > 0 ? CHAIN_ADD : 0) | (i + 1 < count ? CHAIN_LEAVE : 0);
+    if (int rc = decode_layer(op, layers[i], hidden, mask, nullptr, nullptr, 0, k_bufs[i], v_bufs[i], B, cap, S, chain, carry,
+                              scratch, scratch_bytes, stream, 64))
+      return rc;
+  }
+  return TI_OK;
+}
+
 int64_t ti_opt_decoder_layer_prefill_scratch_bytes(int64_t rows, int64_t embed, int64_t ffn) {
   if (rows <= 0 || embed <= 0 || ffn <= 0) return 0;
   return 4 * up256(rows * embed) + up256(4 * rows * embed) + up256(rows * ffn);

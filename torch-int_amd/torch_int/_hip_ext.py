@@ -126,6 +126,8 @@ _lib.ti_opt_decoder_layer_decode_from.restype = ctypes.c_int
 _lib.ti_opt_decoder_layer_prefill_chained.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, ctypes.c_int, _vp, _vp, _i64,
                                                       _vp, _i64, _vp]
 _lib.ti_opt_decoder_layer_prefill_chained.restype = ctypes.c_int
+_lib.ti_opt_decoder_layers_decode.argtypes = [_vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _i64, _vp]
+_lib.ti_opt_decoder_layers_decode.restype = ctypes.c_int
 _raw_stream = torch._C._cuda_getCurrentRawStream
 _opt_layer_decode = getattr(_CUDA._fast, "opt_layer_decode", None) or _lib.ti_opt_decoder_layer_decode_from
 _opt_layer_prefill = getattr(_CUDA._fast, "opt_layer_prefill", None) or _lib.ti_opt_decoder_layer_prefill_chained
@@ -720,6 +722,24 @@ def opt_layer_prefill(plan, hidden, mask, k_out, v_out, chain=0, carry=None, mem
     if rc:
         raise RuntimeError(f"torch_int._hip_ext.opt_layer_prefill: {_lib.ti_last_error().decode()} (status {rc})")
     return hidden
+
+
+def pointers(values):
+    """The addresses ``values`` as the array a C call reads."""
+    return (ctypes.c_void_p * len(values))(*values)
+
+
+def opt_layers_decode(plans, hidden, mask, k_bufs, v_bufs, cap, S, carry):
+    """``opt_layer_decode`` for the layers of one pass from one C call (``ti_opt_decoder_layers_decode``): ``k_bufs`` and ``v_bufs``
+    are ``pointers`` of cache buffers that all have room for ``cap`` positions and hold S - 1."""
+    dev = hidden.device
+    with _on(dev):
+        scratch = opt_decode_scratch(plans, hidden)
+        rc = _lib.ti_opt_decoder_layers_decode(pointers([plan.addr for plan in plans]), len(plans), hidden.data_ptr(), _ptr(mask), k_bufs,
+                                               v_bufs, hidden.shape[0], cap, S, _ptr(carry), scratch.data_ptr(), scratch.numel(),
+                                               _raw_stream(dev.index))
+    if rc:
+        raise RuntimeError(f"torch_int._hip_ext.opt_layers_decode: {_lib.ti_last_error().decode()} (status {rc})")
 
 
 def _plan_current(sources, modules):

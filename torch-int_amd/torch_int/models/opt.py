@@ -10,6 +10,7 @@ works as ``config``.
 """
 import ctypes
 import threading
+import weakref
 from dataclasses import dataclass
 from typing import List, Optional, Tuple
 
@@ -28,7 +29,7 @@ class _KVBuffer:
     first ``filled`` positions hold tokens.  The tensors handed out as ``past_key_value`` are views
     ``buf[:, :, :n]`` that carry a reference to this object.  ``bare``: the tokens are still elsewhere, and the kernel that
     appends the next one moves them here."""
-    __slots__ = ("buf", "filled", "bare")
+    __slots__ = ("buf", "filled", "bare", "__weakref__")
 
     def __init__(self, buf, filled, bare=False):
         self.buf, self.filled, self.bare = buf, filled, bare
@@ -106,6 +107,50 @@ def _kv_rooms(past):
 def _kv_give_back(rooms):
     for kv in rooms:
         kv.filled -= 1
+
+
+class _KVChain:
+    """The cache buffers of the layers of a model, as the pass that appended to them last left them: what the pass that
+    continues it compares the cache it is given with, instead of looking at every tensor of it anew.  Every buffer holds the same
+    positions of the same heads.  It keeps none of them alive: the tensors of a cache do, each its own."""
+    __slots__ = ("rooms", "keys", "values", "shape", "stride", "cap", "device")
+
+    def __reduce__(self):   # a copied or pickled cache has buffers of its own
+        return _no_plan, ()
+
+    @staticmethod
+    def of(rooms):
+        """The chain of ``rooms`` ((key buffer, value buffer) for every layer), or None where they differ in size."""
+        first = rooms[0][0].buf
+        if any(kv.buf.shape != first.shape or kv.buf.device != first.device or kv.bare for pair in rooms for kv in pair):
+            return None
+        chain = _KVChain()
+        chain.rooms = [(weakref.ref(kk), weakref.ref(vv)) for kk, vv in rooms]
+        chain.keys, chain.values = (_hip_ext.pointers([pair[i].buf.data_ptr() for pair in rooms]) for i in (0, 1))
+        chain.shape, chain.stride, chain.cap, chain.device = first.shape, first.stride(), first.shape[2], first.device
+        return chain
+
+    def claim(self, cache, S):
+        """The buffers with position S - 1 taken in each, as ``_kv_claim`` takes it, when ``cache`` is what they hold before it,
+        else None."""
+        held = (self.shape[0], self.shape[1], S - 1, self.shape[3])
+        if S > self.cap:
+            return None
+        rooms = []
+        for i, (kk, vv) in enumerate(self.rooms):
+            key, value = cache[i]
+            pair = getattr(key, "_ti_kv", None), getattr(value, "_ti_kv", None)
+            if not (pair[0] is not None and pair[1] is not None and kk() is pair[0] and vv() is pair[1] and key.shape == held
+                    and value.shape == held and key.stride() == self.stride and value.stride() == self.stride
+                    and key.data_ptr() == self.keys[i] and value.data_ptr() == self.values[i]):
+                return None
+            rooms.append(pair)
+        with _kv_lock:
+            if any(kk.filled != S - 1 or vv.filled != S - 1 for kk, vv in rooms):
+                return None
+            for kk, vv in rooms:
+                kk.filled = vv.filled = S
+        return rooms
 
 
 def _kv_append_in_layer(plan, hidden, mask, rooms, past, S, **chain):
@@ -830,6 +875,11 @@ class Int8OPTDecoder(nn.Module):
         ok, mask = Int8OPTDecoderLayer._one_call_tensors(hidden, attention_mask)
         if not ok or Int8OPTDecoderLayer.forward is not _STOCK_LAYER_FORWARD or (decode and len(past_key_values) != count):
             return None
+        chain = getattr(past_key_values[0][0], "_ti_chain", None) if decode else None
+        if chain is not None and len(chain.rooms) == count:
+            cache = self._continue_chain(layers, chain, hidden, mask, past_key_values)
+            if cache is not None:
+                return cache
         found = []
         for i, layer in enumerate(layers):
             if (type(layer) is not Int8OPTDecoderLayer or layer._forward_hooks or layer._forward_pre_hooks
@@ -846,9 +896,7 @@ class Int8OPTDecoder(nn.Module):
         # The carry: fc2's output on its way from one layer to the next, and in a prefill out_proj's too; memory of this pass, so
         # that passes of other threads on the same stream do not meet in it.  A decode step on an fp32 stream has none (fc2's
         # GEMM adds its output itself).
-        carry = None
-        if count > 1 and not (decode and hidden.dtype is torch.float32):
-            carry = torch.empty((hidden.shape[0] * hidden.shape[1], hidden.shape[2]), dtype=torch.float32, device=hidden.device)
+        carry = self._carry(hidden, count, decode)
         links = [0 if carry is None else (_hip_ext.CHAIN_ADD if i else 0) | (_hip_ext.CHAIN_LEAVE if i + 1 < count else 0)
                  for i in range(count)]
         cache = []
@@ -862,6 +910,8 @@ class Int8OPTDecoder(nn.Module):
                 present = _kv_append_in_layer(plan, hidden, mask, room, past, S, chain=chain, carry=carry, scratch=scratch)
                 if use_cache:
                     cache.append(present)
+            if use_cache:
+                cache[0][0]._ti_chain = _KVChain.of(rooms)
         else:
             memory = _hip_ext.opt_prefill_scratch(found, hidden)
             widest = max(found, key=lambda plan: plan.heads)
@@ -872,6 +922,43 @@ class Int8OPTDecoder(nn.Module):
                 if use_cache:
                     cache.append((key, value))
         return tuple(cache)
+
+    @staticmethod
+    def _carry(hidden, count, decode):
+        if count < 2 or (decode and hidden.dtype is torch.float32):
+            return None
+        return torch.empty((hidden.shape[0] * hidden.shape[1], hidden.shape[2]), dtype=torch.float32, device=hidden.device)
+
+    def _continue_chain(self, layers, chain, hidden, mask, past_key_values):
+        """``_chain_layers`` for a decode step whose cache is as the step before left it: the layers are looked at as there, their
+        caches together, and one C call issues them all.  (The loop there is some 12 us of Python a layer, what four of its five launches cost
+        the host, and a small model's step is bound by it.)"""
+        bsz, heads, _, d = chain.shape
+        S = past_key_values[0][0].shape[2] + 1
+        half, device = hidden.dtype is torch.float16, hidden.device
+        if (bsz != hidden.shape[0] or device != chain.device or not _hip_ext.decode_attention_shape_ok_cached(1, S, d)
+                or (mask is not None and mask.shape != (bsz, 1, 1, S))):
+            return None
+        plans = []
+        for layer in layers:
+            own = layer.__dict__
+            if (type(layer) is not Int8OPTDecoderLayer or own["_forward_hooks"] or own["_forward_pre_hooks"] or "forward" in own
+                    or not layer.decode_in_one_call):
+                return None
+            attn = own["_modules"]["self_attn"]
+            if type(attn) is not Int8OPTAttention or not attn.fused_softmax or not attn.kv_cache_in_place:
+                return None
+            plan = layer._decode_plan(half, device)
+            if plan is None or plan.heads != heads or plan.head_dim != d or plan.embed != hidden.shape[2]:
+                return None
+            plans.append(plan)
+        rooms = chain.claim(past_key_values, S)
+        if rooms is None:
+            return None
+        _hip_ext.opt_layers_decode(plans, hidden, mask, chain.keys, chain.values, chain.cap, S, self._carry(hidden, len(plans), True))
+        cache = tuple((_kv_view(kk, S), _kv_view(vv, S)) for kk, vv in rooms)
+        cache[0][0]._ti_chain = chain
+        return cache
 
     def _positions_in_order(self, past_len, count):
         """The position embeddings [1, count, width] of tokens past_len, past_len + 1, ..., as a view of the table, or None where
