@@ -486,6 +486,10 @@ int ti_attn_qk_softmax_q_mc(const int8_t* q, const int8_t* k, const float* mask,
 int ti_attn_prefill_s8_mc(const int8_t* q, const int8_t* k, const int8_t* vt, const float* mask,
                           const uint8_t* mask_classes, int8_t* ctx, int64_t BH, int64_t T, int64_t S, int64_t D,
                           int64_t stride_q, int64_t stride_k, int64_t heads, float alpha_qk, float alpha_pv, void* stream);
+/* ti_attn_prefill_s8_mc on V itself, [BH, S, D] packed as the cache holds it, up to 2048 keys: same values, no transpose. */
+int ti_attn_prefill_s8_v(const int8_t* q, const int8_t* k, const int8_t* v, const float* mask, const uint8_t* mask_classes,
+                         int8_t* ctx, int64_t BH, int64_t T, int64_t S, int64_t D, int64_t stride_q, int64_t stride_k,
+                         int64_t heads, float alpha_qk, float alpha_pv, void* stream);
 
 /* One decode step of one decoder layer (torch_int/models/opt.py:202-299, Int8OPTDecoderLayer.forward, with one new token
  * per sequence and a KV cache) from one call: LayerNormQ, the q/k/v projections, the cache append and the attention,
@@ -525,8 +529,8 @@ int ti_opt_decoder_layer_decode(const TiOptDecodeLayer* layer, void* hidden, con
 
 /* The same for a prefill (Int8OPTDecoderLayer.forward, torch_int/models/opt.py:202-299, on T > 16 tokens per sequence
  * without a cache): LayerNormQ, the q/k/v projections stored head-major (one grouped launch where
- * ti_linear_group_is_one_launch says so, else three calls with the workspace), V transposed, the one-launch prefill
- * attention with the head merge (ti_attn_prefill_s8_mc), out_proj, the residual update fused with the second
+ * ti_linear_group_is_one_launch says so, else three calls with the workspace), the one-launch prefill attention with the head merge
+ * (ti_attn_prefill_s8_v; beyond 2048 keys V transposed and ti_attn_prefill_s8_mc), out_proj, the residual update fused with the second
  * LayerNormQ, fc1 (ReLU), fc2 added into the residual stream -- the entry points and arguments of the module path, so
  * its values.  hidden [B, T, embed] is updated in place; mask fp32 [B, 1, T, T] or NULL, mask_classes its class array
  * (ti_attn_mask_classes) or NULL; k_out / v_out receive the key and value rows [B, heads, T, head_dim] (the cache the

@@ -675,11 +675,11 @@ int ti_attn_prefill_s8(const int8_t* q, const int8_t* k, const int8_t* vt, const
                                stream);
 }
 
-int ti_attn_prefill_s8_mc(const int8_t* q, const int8_t* k, const int8_t* vt, const float* mask,
-                          const uint8_t* mask_classes, int8_t* ctx, int64_t BH, int64_t T, int64_t S, int64_t D,
-                          int64_t stride_q, int64_t stride_k, int64_t heads, float alpha_qk, float alpha_pv, void* stream) {
+// v_rows: v is V [BH, S, D] as the cache holds it; else V^T [BH, D, S]
+static int attn_prefill(const char* op, const int8_t* q, const int8_t* k, const int8_t* v, bool v_rows, const float* mask,
+                        const uint8_t* mask_classes, int8_t* ctx, int64_t BH, int64_t T, int64_t S, int64_t D,
+                        int64_t stride_q, int64_t stride_k, int64_t heads, float alpha_qk, float alpha_pv, void* stream) {
   g_err[0] = 0;
-  const char* op = "attn_prefill_s8";
   const int64_t lim = 0x7fffffffLL;
   if (BH < 0 || T < 0 || S < 0 || D < 0 || heads < 1 || BH > lim || T > lim || heads > lim)
     return fail(TI_ERR_INVALID_ARG, "%s: sizes must be in [0, 2^31) and heads >= 1", op);
@@ -690,16 +690,33 @@ int ti_attn_prefill_s8_mc(const int8_t* q, const int8_t* k, const int8_t* vt, co
     return fail(TI_ERR_INVALID_ARG, "%s: unsupported shape T=%lld S=%lld head_dim=%lld (needs S a multiple of 16 in "
                 "[16, 4096] and head_dim a multiple of 16 up to 128)",
                 op, (long long)T, (long long)S, (long long)D);
+  const int form = attn_prefill_form(BH, T, S, D, mask != nullptr, mask_classes != nullptr);
+  if (v_rows && form != ATTN_SINGLE_SWEEP && form != ATTN_ROWS)
+    return fail(TI_ERR_INVALID_ARG, "%s: up to 2048 keys (got %lld)", op, (long long)S);
   if (stride_q < T * D || stride_k < S * D || stride_q % 16 != 0 || stride_k % 16 != 0)
     return fail(TI_ERR_INVALID_ARG, "%s: batch strides (%lld, %lld) must be multiples of 16 and cover one matrix", op,
                 (long long)stride_q, (long long)stride_k);
   if (int rc = check_ptr(op, "q", q, 16, true)) return rc;
   if (int rc = check_ptr(op, "k", k, 16, true)) return rc;
-  if (int rc = check_ptr(op, "vt", vt, 16, true)) return rc;
+  if (int rc = check_ptr(op, v_rows ? "v" : "vt", v, 16, true)) return rc;
   if (int rc = check_ptr(op, "mask", mask, 16, mask != nullptr)) return rc;
   if (int rc = check_ptr(op, "ctx", ctx, 4, true)) return rc;
-  return launch_attn_qk_softmax_q(q, k, mask, nullptr, BH, T, S, D, stride_q, stride_k, heads, alpha_qk, vt, ctx,
-                                  alpha_pv, static_cast<hipStream_t>(stream), mask_classes);
+  return launch_attn_qk_softmax_q(q, k, mask, nullptr, BH, T, S, D, stride_q, stride_k, heads, alpha_qk, v, ctx,
+                                  alpha_pv, static_cast<hipStream_t>(stream), mask_classes, v_rows);
+}
+
+int ti_attn_prefill_s8_mc(const int8_t* q, const int8_t* k, const int8_t* vt, const float* mask,
+                          const uint8_t* mask_classes, int8_t* ctx, int64_t BH, int64_t T, int64_t S, int64_t D,
+                          int64_t stride_q, int64_t stride_k, int64_t heads, float alpha_qk, float alpha_pv, void* stream) {
+  return attn_prefill("attn_prefill_s8", q, k, vt, false, mask, mask_classes, ctx, BH, T, S, D, stride_q, stride_k, heads, alpha_qk,
+                      alpha_pv, stream);
+}
+
+int ti_attn_prefill_s8_v(const int8_t* q, const int8_t* k, const int8_t* v, const float* mask, const uint8_t* mask_classes,
+                         int8_t* ctx, int64_t BH, int64_t T, int64_t S, int64_t D, int64_t stride_q, int64_t stride_k,
+                         int64_t heads, float alpha_qk, float alpha_pv, void* stream) {
+  return attn_prefill("attn_prefill_s8_v", q, k, v, true, mask, mask_classes, ctx, BH, T, S, D, stride_q, stride_k, heads, alpha_qk,
+                      alpha_pv, stream);
 }
 
 int ti_decode_attn_supported(int64_t T, int64_t S, int64_t D) { return decode_attn_supported(T, S, D) ? 1 : 0; }
@@ -1021,7 +1038,14 @@ int prefill_layer(const char* op, const TiOptDecodeLayer* L, void* hidden, const
                                              workspace_bytes, stream)))
         return rc;
   }
-  // V transposed, then the whole attention with the head merge
+  // the whole attention with the head merge: on V as it was just stored where a form reads that, else on its transpose
+  const int form = attn_prefill_form(B * H, T, T, d, mask != nullptr, mask_classes != nullptr);
+  if (form == ATTN_SINGLE_SWEEP || form == ATTN_ROWS) {
+    if ((rc = ti_attn_prefill_s8_v(q, k_out, v_out, mask, mask_classes, ctx, B * H, T, T, d, T * d, T * d, H, L->alpha_qk,
+                                   L->alpha_pv, stream)))
+      return rc;
+    return after_attention(L, ctx, f32, x, h, hidden, M, chain, carry, workspace, workspace_bytes, stream);
+  }
   if ((rc = ti_transpose_last2_s8(v_out, vt, B * H, T, d, stream))) return rc;
   if ((rc = ti_attn_prefill_s8_mc(q, k_out, vt, mask, mask_classes, ctx, B * H, T, T, d, T * d, T * d, H, L->alpha_qk,
                                   L->alpha_pv, stream)))

@@ -23,6 +23,8 @@ namespace ti {
 #define TI_GLOBAL_AS __attribute__((address_space(1)))
 #define TI_LDS_AS __attribute__((address_space(3)))
 
+typedef int v2i __attribute__((ext_vector_type(2)));
+
 constexpr int AF_ROWS = 64;   // query rows per workgroup
 constexpr int AF_D = 128;     // largest head size (sizes the LDS limit)
 constexpr int AF_MAX_S = 576;  // (64 + 576) rows of 128 bytes = 80 KiB: two workgroups per CU
@@ -44,7 +46,10 @@ constexpr int AF_MAX_S = 576;  // (64 + 576) rows of 128 bytes = 80 KiB: two wor
 // ctx is [batch, T, heads * 128].
 // SPEC: 1 / 2 = with / without a mask.  PAD = false: S == 16 * NB, the last three blocks exist like the others (the
 // forms for 128, 256, 512 ... keys are 2 to 4 % faster without the three tests).
-template <int NB, bool PV, int SPEC, int D = 128, bool PAD = true>
+// VR (with PV): v is V as the cache holds it, [batch*heads, S, head size]; its rows go into the K panel's place as the keys lay there, in a
+// swizzle of their own, and are read with the transposing LDS read, eight keys of sixteen columns to a row of lanes: half as many reads
+// as V^T's gathered dwords, and no transpose before (256 heads x 256 x 64 20.2 -> 15.5 us with it, 160 x 256 x 128 21.4 -> 15.8).
+template <int NB, bool PV, int SPEC, int D = 128, bool PAD = true, bool VR = false>
 __global__ __launch_bounds__(256, 2) void attn_qk_softmax_q_kernel(const int8_t* __restrict__ q,
                                                                    const int8_t* __restrict__ k,
                                                                    const float* __restrict__ mask,
@@ -173,7 +178,16 @@ __global__ __launch_bounds__(256, 2) void attn_qk_softmax_q_kernel(const int8_t*
   // V^T goes into the dead K panel now, after the last mask load: loads complete in issue order, so copies issued
   // before the mask rows would have to land before the first mask value could be used.  They run under the
   // exponentials and the quantisation and are waited for in front of P.V.
-  if constexpr (PV) {
+  auto v_chunk = [](int row, int c) { return D == 128 ? c ^ ((row >> 1) & 7) : c ^ ((row >> 2) & 3); };  // 16 rows: 16 bank groups
+  if constexpr (PV && VR) {
+    const int8_t* vb = vt + bh * (long long)dr * S;
+    for (int i = wave; i < S / RPS; i += 4) {
+      const int row = i * RPS + lane / CPR, chunk = v_chunk(row, lane % CPR);
+      if (chunk < nc)  // columns beyond the head size are multiplied as they are and not stored
+        __builtin_amdgcn_global_load_lds((const TI_GLOBAL_AS void*)(vb + (long long)row * dr + (chunk << 4)),
+                                         (TI_LDS_AS void*)((TI_LDS_AS char*)smem + AF_ROWS * D + i * 1024), 16, 0, 0);
+    }
+  } else if constexpr (PV) {
     const int8_t* vb = vt + bh * (long long)dr * S;
     const int instrs = (dr * pitch + 1023) >> 10;  // 1 KiB each; rows dr .. D-1 of the panel are never read
     for (int i = wave; i < instrs; i += 4) {
@@ -263,6 +277,8 @@ __global__ __launch_bounds__(256, 2) void attn_qk_softmax_q_kernel(const int8_t*
     v4i o[D / 16];
 #pragma unroll
     for (int c = 0; c < D / 16; ++c) o[c] = v4i{0, 0, 0, 0};
+    // VR: the keys whose columns lanes 2 i and 2 i + 1 of a row of sixteen read: of blocks 0 and 1 of a slice, then 2 and 3
+    const int vkey = (r < 8 ? 0 : 12) + 4 * g + (r >> 1);
     const char* vrow = vts + r * pitch + 4 * g;  // V^T row (= head-dim index) r of block c is 16c + r
 #pragma unroll
     for (int sl = 0; sl < NB / 4; ++sl) {
@@ -272,6 +288,19 @@ __global__ __launch_bounds__(256, 2) void attn_qk_softmax_q_kernel(const int8_t*
         // results are not stored.  A test on c here cost the 256-key forms their register allocation.)
 #pragma unroll
         for (int c = 0; c < D / 16; ++c) {
+          if constexpr (VR) {
+            v4i vf;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const int row = 64 * sl + 32 * h + vkey;
+              const char* src = smem + (AF_ROWS + row) * D + (v_chunk(row, c) << 4) + 8 * (r & 1);
+              const v2i got = __builtin_amdgcn_ds_read_tr8_b64_v2i32((TI_LDS_AS v2i*)src);
+              vf[2 * h] = got[0];
+              vf[2 * h + 1] = got[1];
+            }
+            o[c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(vf, pa, o[c], 0, 0, 0);
+            continue;
+          }
           const char* src = vrow + c * 16 * pitch + 64 * sl;
           const v4i vf = {*reinterpret_cast<const int*>(src), *reinterpret_cast<const int*>(src + 16),
                           *reinterpret_cast<const int*>(src + 32), *reinterpret_cast<const int*>(src + 48)};
@@ -300,11 +329,11 @@ int launch_attn_long(const int8_t* q, const int8_t* k, const float* mask, int8_t
                      long long S, long long D, long long stride_q, long long stride_k, long long heads, float alpha,
                      const int8_t* vt, int8_t* ctx, float alpha_pv, hipStream_t stream, const unsigned char* cls);
 
-// attn_rows.hip: up to 2048 keys, the scores of a row in the registers of four waves; with V^T
+// attn_rows.hip: up to 2048 keys, the scores of a row in the registers of four waves; with V or V^T
 bool attn_rows_supported(long long T, long long S, long long D);
-int launch_attn_rows(const int8_t* q, const int8_t* k, const float* mask, const unsigned char* cls, const int8_t* vt,
-                     int8_t* ctx, long long BH, long long T, long long S, long long D, long long stride_q, long long stride_k,
-                     long long heads, float alpha, float alpha_pv, hipStream_t stream);
+int launch_attn_rows(const int8_t* q, const int8_t* k, const float* mask, const unsigned char* cls, const int8_t* v,
+                     bool v_rows, int8_t* ctx, long long BH, long long T, long long S, long long D, long long stride_q,
+                     long long stride_k, long long heads, float alpha, float alpha_pv, hipStream_t stream);
 
 // shapes the single-sweep kernel of this file takes (all keys of a head in the LDS at once)
 static bool single_sweep_ok(long long T, long long S, long long D, bool pv) {
@@ -355,11 +384,11 @@ bool attn_wants_classes(long long BH, long long T, long long S, long long D, boo
   return with_v && rows_form_ahead(BH, T, S, D, true, true) && !rows_form_ahead(BH, T, S, D, true, false);
 }
 
-template <int NB, bool PV, int SPEC, int D, bool PAD>
+template <int NB, bool PV, int SPEC, int D, bool PAD, bool VR>
 static int launch_af(dim3 grid, size_t lds, hipStream_t stream, const int8_t* q, const int8_t* k, const float* mask,
                      int8_t* probs, int T, int S, long long stride_q, long long stride_k, int heads, int row_blocks,
                      float alpha, const int8_t* vt, int8_t* ctx, float alpha_pv, int dr) {
-  auto kern = attn_qk_softmax_q_kernel<NB, PV, SPEC, D, PAD>;
+  auto kern = attn_qk_softmax_q_kernel<NB, PV, SPEC, D, PAD, VR>;
   static unsigned long long lds_ok = 0;  // bit per device: the large dynamic LDS size has been allowed
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return fail(TI_ERR_LAUNCH, "attn_qk_softmax_q: no current device");
@@ -374,14 +403,17 @@ static int launch_af(dim3 grid, size_t lds, hipStream_t stream, const int8_t* q,
   return TI_OK;
 }
 
-// vt == nullptr: probabilities into probs.  Otherwise context into ctx ([batch, T, heads * head size]).
+// vt == nullptr: probabilities into probs.  Otherwise context into ctx ([batch, T, heads * head size]).  v_rows: vt is V itself (packed
+// [BH, S, head size]), for the forms of up to 2048 keys.
 int launch_attn_qk_softmax_q(const int8_t* q, const int8_t* k, const float* mask, int8_t* probs, long long BH,
                              long long T, long long S, long long D, long long stride_q, long long stride_k,
                              long long heads, float alpha, const int8_t* vt, int8_t* ctx, float alpha_pv,
-                             hipStream_t stream, const unsigned char* mask_classes) {
+                             hipStream_t stream, const unsigned char* mask_classes, bool v_rows) {
   if (BH == 0 || T == 0) return TI_OK;
   if (vt != nullptr && rows_form_ahead(BH, T, S, D, mask != nullptr, mask_classes != nullptr))
-    return launch_attn_rows(q, k, mask, mask_classes, vt, ctx, BH, T, S, D, stride_q, stride_k, heads, alpha, alpha_pv, stream);
+    return launch_attn_rows(q, k, mask, mask_classes, vt, v_rows, ctx, BH, T, S, D, stride_q, stride_k, heads, alpha, alpha_pv, stream);
+  if (!single_sweep_ok(T, S, D, vt != nullptr) && v_rows)
+    return fail(TI_ERR_INVALID_ARG, "attn_prefill: %lld keys want V transposed", S);
   if (!single_sweep_ok(T, S, D, vt != nullptr))
     return launch_attn_long(q, k, mask, probs, BH, T, S, D, stride_q, stride_k, heads, alpha, vt, ctx, alpha_pv, stream,
                             mask_classes);
@@ -396,19 +428,22 @@ int launch_attn_qk_softmax_q(const int8_t* q, const int8_t* k, const float* mask
 #define TI_AF_ARGS                                                                                                   \
   (grid, lds, stream, q, k, mask, probs, (int)T, (int)S, stride_q, stride_k, (int)heads, (int)row_blocks, alpha, vt, ctx, \
    alpha_pv, (int)D)
-#define TI_AF(NB, PV, SPEC)                                                                      \
-  rc = row_bytes == 128 ? (S == 16 * NB ? launch_af<NB, PV, SPEC, 128, false> TI_AF_ARGS         \
-                                        : launch_af<NB, PV, SPEC, 128, true> TI_AF_ARGS)         \
-                        : (S == 16 * NB ? launch_af<NB, PV, SPEC, 64, false> TI_AF_ARGS          \
-                                        : launch_af<NB, PV, SPEC, 64, true> TI_AF_ARGS)
+#define TI_AF(NB, PV, SPEC, VR)                                                                  \
+  rc = row_bytes == 128 ? (S == 16 * NB ? launch_af<NB, PV, SPEC, 128, false, VR> TI_AF_ARGS     \
+                                        : launch_af<NB, PV, SPEC, 128, true, VR> TI_AF_ARGS)     \
+                        : (S == 16 * NB ? launch_af<NB, PV, SPEC, 64, false, VR> TI_AF_ARGS      \
+                                        : launch_af<NB, PV, SPEC, 64, true, VR> TI_AF_ARGS)
 #define TI_AF_NB(NB)                                  \
   case NB / 4:                                        \
     if (vt == nullptr) {                              \
-      if (mask != nullptr) TI_AF(NB, false, 1);       \
-      else TI_AF(NB, false, 2);                       \
+      if (mask != nullptr) TI_AF(NB, false, 1, false); \
+      else TI_AF(NB, false, 2, false);                \
+    } else if (v_rows) {                              \
+      if (mask != nullptr) TI_AF(NB, true, 1, true);  \
+      else TI_AF(NB, true, 2, true);                  \
     } else {                                          \
-      if (mask != nullptr) TI_AF(NB, true, 1);        \
-      else TI_AF(NB, true, 2);                        \
+      if (mask != nullptr) TI_AF(NB, true, 1, false); \
+      else TI_AF(NB, true, 2, false);                 \
     }                                                 \
     break
   switch (nb4) {

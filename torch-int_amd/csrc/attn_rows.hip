@@ -20,6 +20,9 @@
 // half of V^T's rows for 64 keys) follow one another in one sequence, V^T last, so that it lands under the last scores
 // and the exponentials.  For P.V the four dwords of probabilities that a lane holds of 64 keys are transposed across the four
 // 16-lane rows, after which a lane holds 16 consecutive keys, as a 16-byte read of V^T does.
+// On V itself (VR), in pieces of 32 keys, a transposing LDS read (ds_read_b64_tr_b8) brings eight keys of a column to a lane, and any
+// eight: those whose probabilities the lane has.  The kernel takes as long either way (0.98 to 1.05 times); the transpose that went
+// before it is saved: 32 heads x 1904 x 128 101.6 -> 94.9 us, 160 x 528 x 128 53.5 -> 45.4, 12 x 128 x 64 7.0 -> 5.1 (2048 x 80 196 -> 198).
 #include "ti_common.h"
 #include "softmax_math.h"
 
@@ -33,6 +36,8 @@ constexpr int AR_MAX_TILES = 8;
 constexpr int AR_BUFFER_FLAGS = 0x00020000;  // raw buffer, 32-bit data: offsets from the descriptor's size on read as zeros
 constexpr int AR_MC_ROWS = 64;  // rows to a mask class (attn_long.hip)
 constexpr int AR_MC_ZERO = 1, AR_MC_UNIFORM = 2, AR_MC_LOW = 3;
+
+typedef int v2i __attribute__((ext_vector_type(2)));
 
 // 16-byte chunk c of row `row` of a piece whose rows hold B bytes sits at this chunk position
 template <int B>
@@ -62,7 +67,8 @@ struct AttnRows {
 // The ring of one wave.  A tile of `keys` puts two pieces of keys into it and, if it is one of `masked`, its mask values;
 // after the last of them every tile of `vals` puts in two pieces of V^T.  The addresses are bounds-checked by the buffer
 // descriptors: rows past the last key, the last query row or the head size read as zeros (and count for nothing).
-template <int NT, int D>
+// VR: V as the cache holds it, in rows of keys, whose pieces are then 32 keys as those of the keys are.
+template <int NT, int D, bool VR>
 struct AttnRing {
   using L = AttnRows<NT, D>;
   static constexpr int CP = L::COPIES, STAGES = 2 + 64 / L::MKEYS;
@@ -101,11 +107,15 @@ struct AttnRing {
         keys &= keys - 1;
       }
     } else {
-      const unsigned base = (unsigned)((stage - 1) * (D / 2) * S + at);
+      const unsigned base = VR ? (unsigned)((at + 32 * (stage - 1)) * dr) : (unsigned)((stage - 1) * (D / 2) * S + at);
 #pragma unroll
       for (int i = 0; i < CP; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(vres, (TI_LDS_AS void*)(dst + i * 1024), 16, v_off + (base + (unsigned)(i * 16 * S)),
-                                                 0, 0, 0);
+        if constexpr (VR)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(vres, (TI_LDS_AS void*)(dst + i * 1024), 16,
+                                                   key_off[i & 1] + (base + (unsigned)(i * (1024 / D) * dr)), 0, 0, 0);
+        else
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(vres, (TI_LDS_AS void*)(dst + i * 1024), 16, v_off + (base + (unsigned)(i * 16 * S)),
+                                                   0, 0, 0);
       if (stage == 2) {
         stage = 0;
         vals &= vals - 1;
@@ -132,10 +142,10 @@ struct AttnRing {
 // NT = tiles of 256 keys (only the last one may be cut short); D = 64 or 128, the head size in memory (dr) rounded up:
 // the chunks of a query row beyond dr are zeros, so whatever the keys' copies put there adds nothing, and context columns
 // beyond dr are computed and not stored.
-template <int NT, int D, bool MASKED>
+template <int NT, int D, bool MASKED, bool VR>
 __global__ __launch_bounds__(256, (AttnRows<NT, D>::WAVES)) void attn_rows_kernel(
     const int8_t* __restrict__ q, const int8_t* __restrict__ k, const float* __restrict__ mask,
-    const unsigned char* __restrict__ cls, const int8_t* __restrict__ vt, int8_t* __restrict__ ctx, int T, int S,
+    const unsigned char* __restrict__ cls, const int8_t* __restrict__ v, int8_t* __restrict__ ctx, int T, int S,
     long long stride_q, long long stride_k, int heads, int row_blocks, int n_bh, int abreast, float alpha, float alpha_pv, int dr) {
   using L = AttnRows<NT, D>;
   constexpr int KS = D / 64;  // 64-byte slices of the head dimension
@@ -177,13 +187,13 @@ __global__ __launch_bounds__(256, (AttnRows<NT, D>::WAVES)) void attn_rows_kerne
     if (low != 0) passed = product - 5.9e4f;
     todo &= ~(low | (unsigned)__builtin_amdgcn_ballot_w64(v == AR_MC_UNIFORM && lane < NT));
   }
-  AttnRing<NT, D> pieces;
+  AttnRing<NT, D, VR> pieces;
   pieces.ring = ring;
   pieces.S = S;
   pieces.dr = dr;
   pieces.w = w;
   pieces.kres = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(k + bh * stride_k), 0, S * dr, AR_BUFFER_FLAGS);
-  pieces.vres = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(vt + bh * (long long)dr * S), 0, S * dr, AR_BUFFER_FLAGS);
+  pieces.vres = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(v + bh * (long long)dr * S), 0, S * dr, AR_BUFFER_FLAGS);
   pieces.mres = pieces.kres;
   if (MASKED)
     pieces.mres = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(mask + ((bh / heads) * T + t0) * (long long)S), 0,
@@ -343,6 +353,28 @@ __global__ __launch_bounds__(256, (AttnRows<NT, D>::WAVES)) void attn_rows_kerne
       }
       pw[j] = (int)p;
     }
+    if constexpr (VR) {
+      // Two products of 32 keys: a lane's dwords of blocks 2 h and 2 h + 1 are the operand as they are, keys 16 j + 4 g .. +3, and the
+      // transposing read of eight rows of V gives lane (r, g) the same keys of column r
+      const int row = (r < 8 ? 0 : 12) + 4 * g + (r >> 1);  // the key whose 16 columns lanes 2 i and 2 i + 1 read
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        pieces.wait();
+        const char* src = pieces.at_tail() + row * D + 8 * (r & 1);
+        v2i vf[CH];
+#pragma unroll
+        for (int c = 0; c < CH; ++c)
+          vf[c] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((TI_LDS_AS v2i*)(src + (ar_swz<D>(row, c) << 4)));
+        pieces.release();
+        const long pa = (long)((unsigned long)(unsigned)pw[2 * h] | (unsigned long)(unsigned)pw[2 * h + 1] << 32);
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+          const long va = (long)((unsigned long)(unsigned)vf[c][0] | (unsigned long)(unsigned)vf[c][1] << 32);
+          o[c] = __builtin_amdgcn_mfma_i32_16x16x32_i8(va, pa, o[c], 0, 0, 0);
+        }
+      }
+      continue;
+    }
     row_transpose4(pw);  // keys 16 j + 4 g .. +3 -> keys 16 g + 4 j .. +3
     const v4i pa = {pw[0], pw[1], pw[2], pw[3]};
 #pragma unroll
@@ -387,16 +419,16 @@ bool attn_rows_supported(long long T, long long S, long long D) {
   return T >= 1 && D >= 16 && D <= 128 && D % 16 == 0 && S >= 16 && S % 16 == 0 && S <= (long long)AR_TILE * AR_MAX_TILES;
 }
 
-template <int NT, int D, bool MASKED, class... Args>
+template <int NT, int D, bool MASKED, bool VR, class... Args>
 static void launch_ar(dim3 grid, hipStream_t stream, Args... args) {
   constexpr int lds = AttnRows<NT, D>::LDS;
   static_assert(lds <= 64 * 1024, "no larger than a launch may ask for as it is");
-  hipLaunchKernelGGL((attn_rows_kernel<NT, D, MASKED>), grid, dim3(256), lds, stream, args...);
+  hipLaunchKernelGGL((attn_rows_kernel<NT, D, MASKED, VR>), grid, dim3(256), lds, stream, args...);
 }
 
-int launch_attn_rows(const int8_t* q, const int8_t* k, const float* mask, const unsigned char* cls, const int8_t* vt,
-                     int8_t* ctx, long long BH, long long T, long long S, long long D, long long stride_q, long long stride_k,
-                     long long heads, float alpha, float alpha_pv, hipStream_t stream) {
+int launch_attn_rows(const int8_t* q, const int8_t* k, const float* mask, const unsigned char* cls, const int8_t* v,
+                     bool v_rows, int8_t* ctx, long long BH, long long T, long long S, long long D, long long stride_q,
+                     long long stride_k, long long heads, float alpha, float alpha_pv, hipStream_t stream) {
   if (BH == 0 || T == 0) return TI_OK;
   if (mask == nullptr || !(alpha >= -1e12f && alpha <= 1e12f)) cls = nullptr;  // as in attn_long.hip
   if (!attn_rows_supported(T, S, D))
@@ -412,18 +444,25 @@ int launch_attn_rows(const int8_t* q, const int8_t* k, const float* mask, const 
   // 320 heads x 2048 x 128 2763 / 1237, causal 1565 / 979 (3 MiB to an XCD: 512 keys 87; 4 MiB: 134).
   const long long fit = 16ll * 1024 * 1024 / (2 * S * D) / 8 * 8;
   const long long abreast = fit < 8 ? 8 : fit < BH ? fit : BH;
-#define TI_AR(NT, DD, MASKED)                                                                                   \
-  launch_ar<NT, DD, MASKED>(grid, stream, q, k, mask, cls, vt, ctx, (int)T, (int)S, stride_q, stride_k, (int)heads, \
-                            (int)row_blocks, (int)BH, (int)abreast, alpha, alpha_pv, (int)D)
-#define TI_AR_NT(NT)                                 \
-  case NT:                                           \
-    if (D > 64) {                                    \
-      if (mask != nullptr) TI_AR(NT, 128, true);     \
-      else TI_AR(NT, 128, false);                    \
-    } else {                                         \
-      if (mask != nullptr) TI_AR(NT, 64, true);      \
-      else TI_AR(NT, 64, false);                     \
-    }                                                \
+#define TI_AR(NT, DD, MASKED, VR)                                                                                    \
+  launch_ar<NT, DD, MASKED, VR>(grid, stream, q, k, mask, cls, v, ctx, (int)T, (int)S, stride_q, stride_k, (int)heads, \
+                                (int)row_blocks, (int)BH, (int)abreast, alpha, alpha_pv, (int)D)
+#define TI_AR_V(NT, DD, MASKED)                \
+  if (v_rows) TI_AR(NT, DD, MASKED, true);     \
+  else TI_AR(NT, DD, MASKED, false)
+#define TI_AR_NT(NT)                           \
+  case NT:                                     \
+    if (D > 64) {                              \
+      if (mask != nullptr) {                   \
+        TI_AR_V(NT, 128, true);                \
+      } else {                                 \
+        TI_AR_V(NT, 128, false);               \
+      }                                        \
+    } else if (mask != nullptr) {              \
+      TI_AR_V(NT, 64, true);                   \
+    } else {                                   \
+      TI_AR_V(NT, 64, false);                  \
+    }                                          \
     break
   switch (nt) {
     TI_AR_NT(1);
@@ -436,6 +475,7 @@ int launch_attn_rows(const int8_t* q, const int8_t* k, const float* mask, const 
     TI_AR_NT(8);
   }
 #undef TI_AR_NT
+#undef TI_AR_V
 #undef TI_AR
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "attn_rows launch: %s", hipGetErrorString(e));

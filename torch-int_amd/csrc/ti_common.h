@@ -347,7 +347,7 @@ bool attn_wants_classes(long long BH, long long T, long long S, long long D, boo
 int launch_attn_qk_softmax_q(const int8_t* q, const int8_t* k, const float* mask, int8_t* probs, long long BH,
                              long long T, long long S, long long D, long long stride_q, long long stride_k,
                              long long heads, float alpha, const int8_t* vt, int8_t* ctx, float alpha_pv,
-                             hipStream_t stream, const unsigned char* mask_classes = nullptr);
+                             hipStream_t stream, const unsigned char* mask_classes = nullptr, bool v_rows = false);
 long long attn_mask_classes_bytes(long long batch, long long T, long long S);
 int launch_attn_mask_classes(const float* mask, unsigned char* cls, long long batch, long long T, long long S,
                              hipStream_t stream);
