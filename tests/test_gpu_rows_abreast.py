@@ -1,0 +1,62 @@
+"""Narrow outputs of 17 to 64 rows, whose 16-row blocks lie in several workgroups (csrc/gemm_rows.h, rows_blocks_each): one, two and
+three blocks to a workgroup, last groups that are cut off or hold fewer blocks, outputs at the lines of the rule, an fp16 and an fp32 stream
+that is added to, head-major stores and groups.  Integer sums: exact."""
+import pytest
+import torch
+
+from oracle import oracle as orc
+from test_gpu_rows import _last, _s8
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 63, 64])
+@pytest.mark.parametrize("N,K", [(16, 768), (50, 1024), (768, 3072), (1024, 5120), (1040, 2048), (2048, 4096), (2064, 2560)])
+def test_rows_in_several_workgroups(M, N, K):
+    import torch_int._CUDA as C
+    g = torch.Generator().manual_seed(M * 7 + N + K)
+    x, w, b8, bf = _s8(g, M, K), _s8(g, N, K), _s8(g, N), torch.randn(N, generator=g)
+    resid = torch.randn(M, N, generator=g) * 3
+    al, be = 3e-4, 0.02
+    acc = orc.gemm_acc_torch(x, w)
+    xd, wd, b8d, bfd = (t.to(DEV) for t in (x, w, b8, bf))
+    print("rows abreast", M, N, K, flush=True)
+    out = C.linear_a8_w8_b8_o8(xd, wd, b8d, al, be)
+    assert _last()[0] == 1
+    assert torch.equal(out.cpu(), orc.epi_b8_o8(acc, b8, al, be))
+    assert torch.equal(C.linear_a8_w8_bfp32_ofp32(xd, wd, bfd, al, 1.0).cpu(), orc.epi_bfp32_ofp32(acc, bf, al, 1.0))
+    assert torch.equal(C._linear_a8_w8_bfp32_ofp32_acc(xd, wd, bfd, al, 1.0, resid.to(DEV)).cpu(),
+                       orc.linear_a8_w8_bfp32_ofp32_acc(x, w, bf, al, 1.0, resid, acc_fn=lambda *_: acc))
+    if N % 16 == 0:
+        import torch_int._hip_ext as X
+        want = orc.epi_b8_o8(acc, b8, al, be).view(1, M, N // 16, 16).transpose(1, 2)
+        assert torch.equal(X.linear_a8_w8_b8_o8_heads(xd, wd, b8d, al, be, 1, M, N // 16, 16).cpu(), want)
+
+
+@pytest.mark.parametrize("M,N,K", [(48, 512, 1024), (33, 400, 768), (64, 272, 4096)])
+def test_groups_in_several_workgroups(M, N, K):
+    import torch_int._hip_ext as X
+    g = torch.Generator().manual_seed(M + N + K)
+    x, ws, bs = _s8(g, M, K), [_s8(g, N, K) for _ in range(3)], [_s8(g, N) for _ in range(3)]
+    al, be = [3e-4, 2e-4, 5e-4], [0.02, 0.1, 0.05]
+    print("rows abreast group", M, N, K, flush=True)
+    out = X.linear_a8_w8_b8_o8_group(x.to(DEV), [w.to(DEV) for w in ws], [b.to(DEV) for b in bs], al, be)
+    for o, w, b, a, c in zip(out, ws, bs, al, be):
+        assert torch.equal(o.cpu(), orc.linear_a8_w8_b8_o8(x, w, b, a, c, acc_fn=orc.gemm_acc_torch)), (M, N, K)
+
+
+@pytest.mark.parametrize("K,want", [(768, "E1"), (1024, "B1"), (2048, "A1"), (2560, "D1"), (3072, "G1"), (3584, "H1"), (4096, "F1"),
+                                    (5120, "C1")])
+def test_every_tiling_with_all_rows_in_a_workgroup(K, want):
+    """Outputs of more strips than there are CUs: one to four blocks of 16 rows to a workgroup, a kernel of its own each."""
+    import torch_int._CUDA as C
+    N = 4112
+    g = torch.Generator().manual_seed(K)
+    x, w, b = _s8(g, 64, K), _s8(g, N, K), _s8(g, N)
+    ref = orc.linear_a8_w8_b8_o8(x, w, b, 3e-4, 0.02, acc_fn=orc.gemm_acc_torch)
+    xd, wd, bd = x.to(DEV), w.to(DEV), b.to(DEV)
+    for M in (16, 17, 32, 33, 48, 49, 64):
+        print("rows whole", want, M, N, K, flush=True)
+        assert torch.equal(C.linear_a8_w8_b8_o8(xd[:M], wd, bd, 3e-4, 0.02).cpu(), ref[:M]), M
+        assert _last() == (1, want), M

@@ -14,7 +14,8 @@
 // Work: a workgroup of NW waves multiplies strips of 16 weight rows with one slice of the inner dimension, NW * KS * 64
 // bytes long; wave w owns KS * 64 of them.  Each wave has a ring of its own, so the copy pipeline has no barriers: a
 // wave waits for its own pieces with s_waitcnt.  The waves' 16 x (16 MX) partial tiles meet in the LDS (integer atomic
-// adds into one of two buffers, one barrier a strip); wave (strip * MX + m) mod NW finishes row block m.
+// adds into one of two buffers, one barrier a strip); wave (strip * MX + m) mod NW finishes row block m.  Narrow outputs
+// spread their row blocks over workgroups, too (grid.y, rows_blocks_each).
 //
 // S slices of the inner dimension (S > 1) are spread over workgroups of one XCD, which meet as the waves of the one-launch
 // split-K do (gemm_pipe16q_kernel, FUSED): partial tiles are parked in the XCD's L2, counted with an atomic that executes
@@ -101,6 +102,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::NW == 16 ? 4 : 2) void gemm_rows_kern
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int M = p.M, N = p.N, K = p.K, S = p.splits;
+  const int row0 = blockIdx.y * (16 * MX);  // rows_blocks_each; 0 where S > 1
 
   // Workgroup -> (XCD, slice, group of strips).  Workgroup ids congruent modulo 8 share an XCD (checked below); all slices
   // of a strip go to one XCD.  Strip number o of the launch order is taken by XCD o mod 8.
@@ -202,7 +204,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::NW == 16 ? 4 : 2) void gemm_rows_kern
     const char* base = reinterpret_cast<const char*>(p.A) + k_first + piece * (KP * 64);
 #pragma unroll
     for (int i = 0; i < KP; ++i) {
-      const int row = m * 16 + row_of[i];  // rows past M repeat the last one
+      const int row = row0 + m * 16 + row_of[i];  // rows past M repeat the last one
       const unsigned o = (unsigned)((row < M ? row : M - 1) * K + col_of[i]);
       __builtin_amdgcn_global_load_lds((const TI_GLOBAL_AS void*)(base + o), (TI_LDS_AS void*)(dst + i * 1024), 16, 0, 0);
     }
@@ -334,7 +336,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::NW == 16 ? 4 : 2) void gemm_rows_kern
             : "memory");
         sum = v4i{s0, s1, s2, s3};
       }
-      const int row = m * 16 + r;
+      const int row = row0 + m * 16 + r;
       if (S == 1) {
         finish(sum, si, strip, row);
       } else if (row < M) {
@@ -504,6 +506,21 @@ static inline RowsPick rows_paired(RowsPick pick, long long K) {
   return pick.tiling == ROWS_A && (K == 12288 || K == 16384) ? RowsPick{ROWS_F, pick.slices / 2} : pick;
 }
 
+// Blocks of 16 rows to a workgroup, one slice: as few as find a CU each.  A narrow output has fewer strips than there are CUs, and
+// what its launch takes is a chain: the rows' copies, then the weights', then one block's sums after the other.  Workgroups of
+// one strip share an XCD, whose L2 hands the weights to the later ones.  The line is one workgroup to a CU, also where two fit:
+// beyond it the strips' own workgroups share the copies' rate, or run one after the other.  Cold weights, us, all blocks in one workgroup /
+// so / a block less: 48 x 768 x 768 3.81 / 3.29, 48 x 768 x 3072 6.29 / 4.65, 64 x 1024 x 5120 8.83 / 5.97, 32 x 2048 x 2048 4.04 / 3.61,
+// 64 x 2048 x 2048 4.98 / 4.05 / 4.74, 64 x 2048 x 4096 7.42 / 6.56 / 9.59, 64 x 1536 x 3072 7.05 / 5.74 / 8.22; left whole: 32 x 2560 x 2560
+// 5.11, split 6.20, 32 x 3072 x 1024 3.56 / 3.95, 48 x 4096 x 4096 8.43 / 12.22.
+static inline int rows_blocks_each(long long M, long long strips, int cus) {
+  const int blocks = (int)((M + 15) / 16);
+  const long long grid = (strips + 7) / 8 * 8;
+  for (int each = 1; each < blocks; ++each)
+    if (grid * ((blocks + each - 1) / each) <= cus) return each;
+  return blocks;
+}
+
 template <class Cfg>
 static int launch_rows_cfg(const GemmParams& p, const GemmGroup& grp, int strips, int per_problem, hipStream_t stream) {
   const int slots = num_cus() * Cfg::PER_CU / 8 * 8;
@@ -514,7 +531,8 @@ static int launch_rows_cfg(const GemmParams& p, const GemmGroup& grp, int strips
   if (lds > 160 * 1024) return -1;  // so wide an output that the bias of a workgroup's strips leaves the ring no room
   static std::atomic<unsigned long long> lds_ok{0};
   if (int rc = allow_lds(gemm_rows_kernel<Cfg>, 160 * 1024, lds_ok)) return rc;
-  hipLaunchKernelGGL(gemm_rows_kernel<Cfg>, dim3((unsigned)grid), dim3(Cfg::NT), lds, stream, p, grp, strips, per_problem);
+  const unsigned abreast = (unsigned)((p.M + 16 * Cfg::MX - 1) / (16 * Cfg::MX));  // rows_blocks_each; slices hold all rows
+  hipLaunchKernelGGL(gemm_rows_kernel<Cfg>, dim3((unsigned)grid, abreast), dim3(Cfg::NT), lds, stream, p, grp, strips, per_problem);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
   return TI_OK;
@@ -562,7 +580,7 @@ static int launch_rows(const GemmParams& p_in, const GemmGroup& grp, int problem
   p.arrivals = nullptr;
   p.parts = nullptr;
   const int per_problem = (p.N + 15) / 16, strips = per_problem * problems;
-  const int mx = (p.M + 15) / 16;
+  const int mx = pick.slices > 1 ? (p.M + 15) / 16 : rows_blocks_each(p.M, strips, num_cus());
   const long long park = (long long)problems * pick.slices * p.M * p.N * 4;
   bool two_launches = false;
   if (pick.slices > 1) {
