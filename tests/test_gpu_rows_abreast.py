@@ -1,4 +1,4 @@
-"""Narrow outputs of 17 to 64 rows, whose 16-row blocks lie in several workgroups (csrc/gemm_rows.h, rows_blocks_each): one, two and
+"""Narrow outputs of 17 to 512 rows, whose 16-row blocks lie in several workgroups (csrc/gemm_rows.h, rows_blocks_each): one, two and
 three blocks to a workgroup, last groups that are cut off or hold fewer blocks, outputs at the lines of the rule, an fp16 and an fp32 stream
 that is added to, head-major stores and groups.  Integer sums: exact."""
 import pytest
@@ -60,3 +60,49 @@ def test_every_tiling_with_all_rows_in_a_workgroup(K, want):
         print("rows whole", want, M, N, K, flush=True)
         assert torch.equal(C.linear_a8_w8_b8_o8(xd[:M], wd, bd, 3e-4, 0.02).cpu(), ref[:M]), M
         assert _last() == (1, want), M
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 768, 768), (320, 768, 768), (512, 768, 768), (96, 3072, 768), (128, 2304, 768), (81, 768, 3072), (256, 768, 3072),
+                                   (511, 1024, 1024), (127, 4096, 1024), (65, 1000, 2048), (95, 2048, 2048), (256, 2048, 2048),
+                                   (179, 2560, 2560), (160, 784, 3584), (128, 1040, 5120)])
+def test_more_than_64_rows(M, N, K):
+    """From the first to the last row count of a rule's range, two workgroups to a CU among them."""
+    import torch_int._CUDA as C
+    import torch_int._hip_ext as X
+    g = torch.Generator().manual_seed(M + N + K)
+    x, w, b8, bf = _s8(g, M, K), _s8(g, N, K), _s8(g, N), torch.randn(N, generator=g)
+    resid = torch.randn(M, N, generator=g) * 3
+    al, be = 3e-4, 0.02
+    acc = orc.gemm_acc_torch(x, w)
+    xd, wd, b8d, bfd = (t.to(DEV) for t in (x, w, b8, bf))
+    print("rows beyond 64", M, N, K, flush=True)
+    want = orc.epi_b8_o8(acc, b8, al, be)
+    assert torch.equal(C.linear_a8_w8_b8_o8(xd, wd, b8d, al, be).cpu(), want)
+    assert _last()[0] == 1
+    assert torch.equal(C.linear_relu_a8_w8_b8_o8(xd, wd, b8d, al, be).cpu(), orc.epi_b8_o8(acc, b8, al, be, relu=True))
+    assert torch.equal(C.linear_a8_w8_bfp32_ofp32(xd, wd, bfd, al, 1.0).cpu(), orc.epi_bfp32_ofp32(acc, bf, al, 1.0))
+    assert torch.equal(C._linear_a8_w8_bfp32_ofp32_acc(xd, wd, bfd, al, 1.0, resid.to(DEV)).cpu(),
+                       orc.linear_a8_w8_bfp32_ofp32_acc(x, w, bf, al, 1.0, resid, acc_fn=lambda *_: acc))
+    if N % 16 == 0:
+        heads = want.view(1, M, N // 16, 16).transpose(1, 2)
+        assert torch.equal(X.linear_a8_w8_b8_o8_heads(xd, wd, b8d, al, be, 1, M, N // 16, 16).cpu(), heads)
+
+
+@pytest.mark.parametrize("M,N,K", [(192, 768, 768), (65, 768, 1024), (96, 1024, 2048), (80, 800, 2560)])
+def test_groups_of_more_than_64_rows(M, N, K):
+    import torch_int._hip_ext as X
+    test_groups_in_several_workgroups(M, N, K)
+    assert _last()[0] == 1 and X.linear_group_is_one_launch(M, N, K)
+
+
+def test_where_more_than_64_rows_end():
+    """One row further the tiled kernels have them, and the group says so before it is launched."""
+    import torch_int._CUDA as C
+    import torch_int._hip_ext as X
+    g = torch.Generator().manual_seed(1)
+    for M, N, K in ((513, 768, 768), (129, 3072, 768), (257, 768, 3072), (257, 2048, 2048), (193, 2560, 2560), (128, 752, 768)):
+        x, w, b = _s8(g, M, K), _s8(g, N, K), _s8(g, N)
+        print("rows end", M, N, K, flush=True)
+        out = C.linear_a8_w8_b8_o8(x.to(DEV), w.to(DEV), b.to(DEV), 3e-4, 0.02)
+        assert _last()[0] == 0 and torch.equal(out.cpu(), orc.linear_a8_w8_b8_o8(x, w, b, 3e-4, 0.02, acc_fn=orc.gemm_acc_torch))
+    assert X.linear_group_is_one_launch(192, 768, 768) and not X.linear_group_is_one_launch(208, 768, 768 + 64)

@@ -1,4 +1,4 @@
-// GEMM for a few rows of activations (2 to 64): decode steps of a served batch, short prompts.  Included by
+// GEMM for a few rows of activations (2 to 64, of narrow outputs to 512): decode steps of a served batch, short prompts.  Included by
 // gemm_s8_impl.h (it uses the epilogues of ti_common.h and the LDS-limit helper there).
 //
 // Bound by HBM: every weight byte is used once, for at most 64 rows of activations.  What the weights cost on this
@@ -32,7 +32,8 @@
 
 namespace ti {
 
-#define TI_ROWS_MAX_M 64
+#define TI_ROWS_MAX_M 64       // of any width
+#define TI_ROWS_ABREAST_M 512  // where the output is narrow (rows_blocks_each)
 
 
 template <int KIND_, int MX_, int KS_, int KP_, int RING_, int NW_, bool GROUPED_ = false>
@@ -474,8 +475,37 @@ static inline bool few_rows_slices_ahead(RowsPick pick, long long M, long long N
   return M > 8 || K > 7168 || strips > 512;
 }
 
+// Blocks of 16 rows to a workgroup, one slice; 0 = the rows are too many for the kernel.  As few as find a CU each: a narrow output has
+// fewer strips than there are CUs, and what its launch takes is a chain: the rows' copies, then the weights', then one block's sums
+// after the other.  Workgroups of one strip share an XCD, whose L2 hands the weights to the later ones.  The line is one workgroup to a CU, also
+// where two fit: beyond it they share the copies' rate, or run one after the other.  Cold weights, us, all blocks in one workgroup / so / a
+// block less: 48 x 768 x 768 3.81 / 3.29, 48 x 768 x 3072 6.29 / 4.65, 64 x 1024 x 5120 8.83 / 5.97, 32 x 2048 x 2048 4.04 / 3.61,
+// 64 x 2048 x 2048 4.98 / 4.05 / 4.74, 64 x 2048 x 4096 7.42 / 6.56 / 9.59, 64 x 1536 x 3072 7.05 / 5.74 / 8.22; left whole: 32 x 2560 x 2560
+// 5.11, split 6.20, 32 x 3072 x 1024 3.56 / 3.95, 48 x 4096 x 4096 8.43 / 12.22.
+// Beyond 64 rows the tiled kernels are the others, whose few tiles walk K one after the other or meet in slices: as long as every
+// workgroup is resident (two to a CU, three or four blocks each, where they fit) this is ahead of them, us before / so: 128 x 768 x 768 5.6 / 3.7,
+// 144 x 768 x 3072 13.9 / 5.9, 128 x 2048 x 2048 10.6 / 5.2, 256 x 2048 x 2048 14.2 / 7.4, 144 x 2560 x 2560 12.6 / 8.9, 192 x 2304 x 768 6.3 / 5.4; not so beyond that: 256 x 2304 x 768 6.3 / 7.5, 256 x 2560 x 2560 12.2 / 13.3.
+// `N`: columns of one problem; `strips`: of all of them.
+static inline int rows_blocks_each(int tiling, long long M, long long N, long long strips, int cus) {
+  const int blocks = (int)((M + 15) / 16);
+  const long long grid = (strips + 7) / 8 * 8;
+  auto fits = [&](int each, long long slots) { return grid * ((blocks + each - 1) / each) <= slots; };
+  if (blocks <= 4) {
+    for (int each = 1; each < blocks; ++each)
+      if (fits(each, cus)) return each;
+    return blocks;
+  }
+  // (given up, as the split products have these shapes to themselves, tests of their forms among them: 128 x 1024 x 4096 12.7 / 6.3,
+  // 320 x 768 x 3072 14.8 / 7.5, three 192 x 256 x 3072 49 / 7.3)
+  if (tiling == ROWS_F || N < 768 || (tiling == ROWS_G && M > 256)) return 0;
+  for (int each = 1; each <= 4; ++each)
+    if (fits(each, cus)) return each;
+  const bool pairs = tiling == ROWS_A || tiling == ROWS_B || tiling == ROWS_D || tiling == ROWS_E;
+  return !pairs ? 0 : fits(3, 2LL * cus) ? 3 : fits(4, 2LL * cus) ? 4 : 0;
+}
+
 static inline RowsPick rows_pick(long long M, long long N, long long K, int cus = num_cus(), int problems = 1) {
-  if (M < 1 || M > TI_ROWS_MAX_M || N < 1 || K < 768 || K > (1 << 20)) return {ROWS_NONE, 1};
+  if (M < 1 || M > TI_ROWS_ABREAST_M || N < 1 || K < 768 || K > (1 << 20)) return {ROWS_NONE, 1};
   RowsPick pick{ROWS_NONE, 1};
   if (K == 4096) pick = {ROWS_F, 1};
   else if (K % 5120 == 0) pick = {ROWS_C, (int)(K / 5120)};
@@ -486,6 +516,7 @@ static inline RowsPick rows_pick(long long M, long long N, long long K, int cus 
   else if (K % 1024 == 0) pick = {ROWS_B, (int)(K / 1024)};
   else if (K % 768 == 0) pick = {ROWS_E, (int)(K / 768)};
   else return {ROWS_NONE, 1};
+  if (M > TI_ROWS_MAX_M && (pick.slices > 1 || rows_blocks_each(pick.tiling, M, N, (N + 15) / 16 * problems, cus) == 0)) return {ROWS_NONE, 1};
   if (cus / 8 < pick.slices) return {ROWS_NONE, 1};  // an XCD has room for one workgroup of every slice
   // The parked tiles of all slices stay a fraction of the weights; the placement words of the groups, 64 bytes apart,
   // fit a stream's block of 4096; only whole strips are parked.
@@ -504,21 +535,6 @@ static inline RowsPick rows_pick(long long M, long long N, long long K, int cus 
 // twelve as six not everywhere ahead (768 columns 1.02).
 static inline RowsPick rows_paired(RowsPick pick, long long K) {
   return pick.tiling == ROWS_A && (K == 12288 || K == 16384) ? RowsPick{ROWS_F, pick.slices / 2} : pick;
-}
-
-// Blocks of 16 rows to a workgroup, one slice: as few as find a CU each.  A narrow output has fewer strips than there are CUs, and
-// what its launch takes is a chain: the rows' copies, then the weights', then one block's sums after the other.  Workgroups of
-// one strip share an XCD, whose L2 hands the weights to the later ones.  The line is one workgroup to a CU, also where two fit:
-// beyond it the strips' own workgroups share the copies' rate, or run one after the other.  Cold weights, us, all blocks in one workgroup /
-// so / a block less: 48 x 768 x 768 3.81 / 3.29, 48 x 768 x 3072 6.29 / 4.65, 64 x 1024 x 5120 8.83 / 5.97, 32 x 2048 x 2048 4.04 / 3.61,
-// 64 x 2048 x 2048 4.98 / 4.05 / 4.74, 64 x 2048 x 4096 7.42 / 6.56 / 9.59, 64 x 1536 x 3072 7.05 / 5.74 / 8.22; left whole: 32 x 2560 x 2560
-// 5.11, split 6.20, 32 x 3072 x 1024 3.56 / 3.95, 48 x 4096 x 4096 8.43 / 12.22.
-static inline int rows_blocks_each(long long M, long long strips, int cus) {
-  const int blocks = (int)((M + 15) / 16);
-  const long long grid = (strips + 7) / 8 * 8;
-  for (int each = 1; each < blocks; ++each)
-    if (grid * ((blocks + each - 1) / each) <= cus) return each;
-  return blocks;
 }
 
 template <class Cfg>
@@ -580,7 +596,7 @@ static int launch_rows(const GemmParams& p_in, const GemmGroup& grp, int problem
   p.arrivals = nullptr;
   p.parts = nullptr;
   const int per_problem = (p.N + 15) / 16, strips = per_problem * problems;
-  const int mx = pick.slices > 1 ? (p.M + 15) / 16 : rows_blocks_each(p.M, strips, num_cus());
+  const int mx = pick.slices > 1 ? (p.M + 15) / 16 : rows_blocks_each(pick.tiling, p.M, p.N, strips, num_cus());
   const long long park = (long long)problems * pick.slices * p.M * p.N * 4;
   bool two_launches = false;
   if (pick.slices > 1) {

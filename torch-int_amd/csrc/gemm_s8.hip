@@ -522,15 +522,15 @@ static int group_prefill_tile(long long M, long long N, long long K, int count) 
 // calls in the second case.
 int gemm_group_is_one_launch(long long M, long long N, long long K, int count) {
   if (M <= 16 && K % SBK == 0) return 1;
-  if (M <= TI_ROWS_MAX_M && N % 4 == 0) {
-    const RowsPick rows = rows_pick(M, N, K);
+  if (M <= TI_ROWS_ABREAST_M && N % 4 == 0) {
+    const RowsPick rows = rows_pick(M, N, K, num_cus(), count);
     if (rows.tiling != ROWS_NONE && rows.slices == 1) return 1;  // no workspace needed
   }
   if (M <= 16) return 0;
   return group_prefill_tile(M, N, K, count) != 0 ? 1 : 0;
 }
 
-// q/k/v-style group of s8 linears.  One launch over all the weights: one row on the dot-product kernel, up to 64 rows on the
+// q/k/v-style group of s8 linears.  One launch over all the weights: one row on the dot-product kernel, up to 64 rows (more where the outputs are narrow) on the
 // weight-streaming kernel of gemm_rows.h where its tilings divide K, else up to 16 rows on the streaming kernel (K % 1024 == 0),
 // and prefills whose tiles group_prefill_tile finds; anything else runs problem by problem.
 int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStream_t stream, void* workspace,
@@ -544,7 +544,7 @@ int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStrea
   const bool aligned = ptr_ok && (shape.K % SBK == 0) && shape.K > 0;
   const int spb = (shape.N + 15) / 16;
   const long long strips = (long long)spb * grp.count;
-  if (ptr_ok && shape.M <= TI_ROWS_MAX_M && shape.N % 4 == 0 && !(gemv_takes(shape) && strips >= 256)) {
+  if (ptr_ok && shape.M <= TI_ROWS_ABREAST_M && shape.N % 4 == 0 && !(gemv_takes(shape) && strips >= 256)) {
     const int rc = launch_rows<KIND, true>(shape, grp, grp.count, workspace, workspace_bytes, stream);
     if (rc >= 0) {
       if (rc == TI_OK) g_last_kernel = shape.M <= 16 ? "stream_group" : "mid_stream_group";

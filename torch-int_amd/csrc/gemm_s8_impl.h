@@ -2911,11 +2911,11 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
     if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
     return TI_OK;
   }
-  // Up to 64 rows: the weight-streaming kernel with the activations in registers.  Not for one row where the dot-product
+  // Up to 64 rows, more where the output is narrow: the weight-streaming kernel with the activations in registers.  Not for one row where the dot-product
   // kernel reads weight rows flat, one or two rows against the few, long weight rows of the view below, ragged widths of a
   // K that 1024 does not divide, nor up to four rows of a short K (2 x 768 x 768: 3.1 us against the skinny kernel's 2.9) or up
   // to eight on fewer than 128 strips (5 x 768 x 768 3.34 against 3.20, 8 x 1200 x 768 3.63 / 3.43; 6 x 2048 x 768 level).
-  if (p.M <= TI_ROWS_MAX_M && (p.N % 16 == 0 || p.K % SBK == 0) && stream_parts(p) == 1 && (p.M > 8 || p.K >= SBK || (p.M > 4 && p.N >= 2048)) &&
+  if (p.M <= TI_ROWS_ABREAST_M && (p.N % 16 == 0 || p.K % SBK == 0) && stream_parts(p) == 1 && (p.M > 8 || p.K >= SBK || (p.M > 4 && p.N >= 2048)) &&
       !(gemv_takes(p) && (p.N + 15) / 16 >= 256)) {
     const int rc = launch_rows<KIND, false>(p, GemmGroup{}, 1, workspace, workspace_bytes, stream);
     if (rc >= 0) {
