@@ -71,7 +71,7 @@ int ti_linear_row_split(int64_t M, int64_t N, int64_t K);
 /* Diagnostics: the kernel family the calling thread's last linear / bmm_s8t_s8n_* call launched
  * ("pipe_256x256", "pipe16_256x160", "pipe16_256x288", "pipe16_256x128", "pipe16_128x80", "pipe16_128x192", "pipe16_256x192", "pipe16_192x128",
  * "pipe16_192x256", "pipe16_160x256", "pipe_128x128",
- * "splitk_<tile>" and "fusedk_<tile>" for the two- and one-launch split-K forms, "stream", "mid_stream" (the weight-streaming kernel, up to 16 and 17 to 64 rows), "stream_parts" (the streaming
+ * "splitk_<tile>" and "fusedk_<tile>" for the two- and one-launch split-K forms, "stream", "mid_stream" (the weight-streaming kernel, up to 16 and 17 to 64 rows, of narrow outputs to 512), "stream_parts" (the streaming
  * kernel on the view with rows cut into parts), "gemv" (one row of activations), "skinny", "tile_*",
  * "scalar"; grouped launches add "_group": "stream_group", "mid_stream_group", "gemv_group", "pipe16_256x160_group", "pipe16_256x288_group",
  * "pipe16_256x256_group", "pipe16_256x128_group"; "<family>+<family>" when the last rows ran as a second problem, see ti_linear_row_split;
@@ -83,7 +83,7 @@ const char* ti_last_kernel(void);
  * and 128-byte steps, 16x16 blocks); "" for the others.  Of two problems or launches, the last product's. */
 const char* ti_last_kernel_form(void);
 
-/* Diagnostic: what the calling thread's last linear or group did in the weight-streaming kernel of up to 64 rows: 0 = it
+/* Diagnostic: what the calling thread's last linear or group did in the weight-streaming kernel of few rows: 0 = it
  * took another kernel, 1 = one slice of the inner dimension, 2 = several that met in one launch, 3 = several and a
  * reduction launch; *tiling = 1 .. 8 for the tilings A .. H of csrc/gemm_rows.h, *slices = their number. */
 int ti_last_rows(int* tiling, int* slices);
