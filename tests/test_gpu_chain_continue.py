@@ -1,6 +1,7 @@
 """Decode steps whose cache is as the step before left it: all layers from one C call.  Against the modules, logits and caches bit for
-bit: steps past the end of the buffers, one cache continued twice, copied, cut and re-ordered caches, hooks, a change of type."""
+bit: steps past the end of the buffers, one cache continued twice, copied, cut and re-ordered caches, hooks, two threads on one stream."""
 import copy
+import threading
 
 import pytest
 import torch
@@ -81,3 +82,33 @@ def test_steps_continue_each_other(bsz, half, monkeypatch):
     assert len(seen) == n
     with _Modules():
         _same(a, lm(ids[:, :1], past_key_values=past, use_cache=True))
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("half", [False, True])
+def test_two_threads_on_one_stream_do_not_meet(half):
+    """Two caches continued at once by two threads on the default stream, against the same steps one thread after the other."""
+    lm = _model(half)
+    prompts = [torch.randint(2, 64, (5, 32), device=DEV) for _ in range(2)]
+    tokens = [torch.randint(2, 64, (5, 60), device=DEV) for _ in range(2)]
+
+    @torch.no_grad()
+    def steps(i, out):
+        step = lm(prompts[i], use_cache=True)
+        for n in range(tokens[i].shape[1]):
+            step = lm(tokens[i][:, n:n + 1], past_key_values=step.past_key_values, use_cache=True)
+            out.append(step.logits)
+        out.append(step)
+
+    print("two threads", half, flush=True)
+    alone, together = [[], []], [[], []]
+    for i in range(2):
+        steps(i, alone[i])
+    threads = [threading.Thread(target=steps, args=(i, together[i])) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for a, b in zip(alone, together):
+        assert len(a) == len(b) == 61 and all(torch.equal(x, y) for x, y in zip(a[:-1], b[:-1]))
+        _same(a[-1], b[-1])

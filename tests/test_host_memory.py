@@ -1,5 +1,6 @@
 """Who holds the device memory whose address a launch is handed: scratch and workspaces of the Python layer, with the
 allocations done in host memory (no kernel runs)."""
+import threading
 import types
 import weakref
 
@@ -68,3 +69,29 @@ def test_memory_of_a_pass_fits_its_widest_layer(host_memory):
     assert ws_bytes >= _CUDA._ws_bytes(304, 5120, 20480) > 0
     one = types.SimpleNamespace(device=types.SimpleNamespace(index=0), shape=(40, 1, 5120))
     assert _hip_ext.opt_decode_scratch(plans, one).numel() >= _hip_ext._lib.ti_opt_decoder_layer_decode_scratch_bytes(40, 5120, 20480)
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_passes_of_two_threads_on_one_stream_have_memory_of_their_own(host_memory, monkeypatch, half):
+    # all layers of a decode step come from one C call that gives up the interpreter lock: two threads are inside at once, and
+    # what one layer hands to its next kernel must not lie where the other thread's layer does (the fp16 stream's carry neither)
+    both_inside, calls = threading.Barrier(2, timeout=20), []
+
+    def call(layers, count, hidden, mask, k_bufs, v_bufs, bsz, cap, S, carry, scratch, nbytes, stream):
+        calls.append((scratch, nbytes, carry))
+        both_inside.wait()
+        return 0
+    monkeypatch.setattr(_hip_ext, "_layers_decode", call)
+    plans = [types.SimpleNamespace(embed=64, ffn=256, addr=16, half=half)] * 3
+    hidden = types.SimpleNamespace(device=types.SimpleNamespace(index=0), shape=(5, 1, 64), data_ptr=lambda: 256)
+    threads = [threading.Thread(target=_hip_ext.opt_layers_decode, args=(plans, hidden, None, None, None, 64, 9)) for _ in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    need, carried = _hip_ext._lib.ti_opt_decoder_layer_decode_scratch_bytes(5, 64, 256), 4 * 5 * 64
+    ranges = sorted((at, at + n) for scratch, n, carry in calls for at, n in [(scratch, n)] + ([(carry, carried)] if half else []))
+    assert len(calls) == 2 and all(n >= need for _, n, _ in calls) and len(ranges) == (4 if half else 2)
+    assert all(carry is None or carry % 16 == 0 for *_, carry in calls) and all((carry is None) == (not half) for *_, carry in calls)
+    assert all(end <= start for (_, end), (start, _) in zip(ranges, ranges[1:])), ranges
+    assert not _hip_ext._layer_scratch

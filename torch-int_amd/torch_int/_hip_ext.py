@@ -128,6 +128,7 @@ _lib.ti_opt_decoder_layer_prefill_chained.argtypes = [_vp, _vp, _vp, _vp, _vp, _
 _lib.ti_opt_decoder_layer_prefill_chained.restype = ctypes.c_int
 _lib.ti_opt_decoder_layers_decode.argtypes = [_vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _i64, _vp]
 _lib.ti_opt_decoder_layers_decode.restype = ctypes.c_int
+_layers_decode = _lib.ti_opt_decoder_layers_decode
 _raw_stream = torch._C._cuda_getCurrentRawStream
 _opt_layer_decode = getattr(_CUDA._fast, "opt_layer_decode", None) or _lib.ti_opt_decoder_layer_decode_from
 _opt_layer_prefill = getattr(_CUDA._fast, "opt_layer_prefill", None) or _lib.ti_opt_decoder_layer_prefill_chained
@@ -632,9 +633,7 @@ _layer_scratch_need = {}
 CHAIN_ADD, CHAIN_LEAVE = 1, 2
 
 
-def opt_decode_scratch(plans, hidden):
-    """The scratch memory of the layers of one decode step, enough for each of ``plans``."""
-    dev, B = hidden.device, hidden.shape[0]
+def _decode_scratch_bytes(plans, B):
     need = 0
     for E, F in {(plan.embed, plan.ffn) for plan in plans}:
         key = (0, B, E, F)
@@ -642,8 +641,15 @@ def opt_decode_scratch(plans, hidden):
         if n is None:
             n = _layer_scratch_need[key] = _lib.ti_opt_decoder_layer_decode_scratch_bytes(B, E, F)
         need = max(need, n)
+    return need
+
+
+def opt_decode_scratch(plans, hidden):
+    """The scratch memory of the layers of one decode step that are issued one by one, enough for each of ``plans``: the stream's,
+    which a layer's call has to itself as it keeps the interpreter lock, and in which nothing stays from one layer to the next."""
+    dev = hidden.device
     with _on(dev):
-        return _scratch_for(dev, _raw_stream(dev.index), need)
+        return _scratch_for(dev, _raw_stream(dev.index), _decode_scratch_bytes(plans, hidden.shape[0]))
 
 
 def opt_layer_decode(plan, hidden, mask, k_buf, v_buf, S, chain=0, carry=None, scratch=None, past=None):
@@ -729,15 +735,19 @@ def pointers(values):
     return (ctypes.c_void_p * len(values))(*values)
 
 
-def opt_layers_decode(plans, hidden, mask, k_bufs, v_bufs, cap, S, carry):
+def opt_layers_decode(plans, hidden, mask, k_bufs, v_bufs, cap, S):
     """``opt_layer_decode`` for the layers of one pass from one C call (``ti_opt_decoder_layers_decode``): ``k_bufs`` and ``v_bufs``
-    are ``pointers`` of cache buffers that all have room for ``cap`` positions and hold S - 1."""
-    dev = hidden.device
+    are ``pointers`` of cache buffers that all have room for ``cap`` positions and hold S - 1.  Other threads run during the call and
+    may launch on this stream between any two of its kernels, so its scratch and carry (an fp16 stream's) are memory of this pass: the
+    allocator hands it to nobody before the last launch is on the stream, and to that stream alone afterwards."""
+    dev, B = hidden.device, hidden.shape[0]
+    scratch_bytes = _decode_scratch_bytes(plans, B)   # whole blocks of 256 bytes: the carry behind them is aligned
+    carry_bytes = 4 * B * hidden.shape[2] if plans[0].half and len(plans) > 1 else 0
     with _on(dev):
-        scratch = opt_decode_scratch(plans, hidden)
-        rc = _lib.ti_opt_decoder_layers_decode(pointers([plan.addr for plan in plans]), len(plans), hidden.data_ptr(), _ptr(mask), k_bufs,
-                                               v_bufs, hidden.shape[0], cap, S, _ptr(carry), scratch.data_ptr(), scratch.numel(),
-                                               _raw_stream(dev.index))
+        memory = torch.empty(scratch_bytes + carry_bytes, dtype=torch.uint8, device=dev)
+        scratch = memory.data_ptr()
+        rc = _layers_decode(pointers([plan.addr for plan in plans]), len(plans), hidden.data_ptr(), _ptr(mask), k_bufs, v_bufs, B, cap, S,
+                            scratch + scratch_bytes if carry_bytes else None, scratch, scratch_bytes, _raw_stream(dev.index))
     if rc:
         raise RuntimeError(f"torch_int._hip_ext.opt_layers_decode: {_lib.ti_last_error().decode()} (status {rc})")
 

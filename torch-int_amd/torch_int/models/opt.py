@@ -955,7 +955,7 @@ class Int8OPTDecoder(nn.Module):
         rooms = chain.claim(past_key_values, S)
         if rooms is None:
             return None
-        _hip_ext.opt_layers_decode(plans, hidden, mask, chain.keys, chain.values, chain.cap, S, self._carry(hidden, len(plans), True))
+        _hip_ext.opt_layers_decode(plans, hidden, mask, chain.keys, chain.values, chain.cap, S)
         cache = tuple((_kv_view(kk, S), _kv_view(vv, S)) for kk, vv in rooms)
         cache[0][0]._ti_chain = chain
         return cache
