@@ -1,5 +1,6 @@
 """Who holds the device memory whose address a launch is handed: scratch and workspaces of the Python layer, with the
 allocations done in host memory (no kernel runs)."""
+import ctypes
 import threading
 import types
 import weakref
@@ -95,3 +96,15 @@ def test_passes_of_two_threads_on_one_stream_have_memory_of_their_own(host_memor
     assert all(carry is None or carry % 16 == 0 for *_, carry in calls) and all((carry is None) == (not half) for *_, carry in calls)
     assert all(end <= start for (_, end), (start, _) in zip(ranges, ranges[1:])), ranges
     assert not _hip_ext._layer_scratch
+
+
+def test_calls_that_are_handed_memory_of_the_stream_keep_the_interpreter_lock():
+    # split-K products and layers issued one by one are several launches, which hand one another tiles in the stream's workspace or
+    # scratch: another thread must not launch between them.  (The forwarder in C keeps the lock as it is.)
+    kept = [*_CUDA._LINEAR_CTYPES.values(), *_CUDA._BMM_CTYPES.values(), *_CUDA._BMM_WS_CTYPES.values()]
+    kept += [getattr(_hip_ext._lib, name) for name in ("ti_linear_a8_w8_b8_o8_heads", "ti_opt_decoder_layer_decode_from",
+                                                       "ti_opt_decoder_layer_prefill_chained")]
+    flag = type(ctypes.pythonapi.Py_IncRef)._flags_ & ~ctypes.CDLL(None)._FuncPtr._flags_
+    assert flag and all(type(fn)._flags_ & flag for fn in kept)
+    # the call whose memory is its own lets other threads run
+    assert not type(_hip_ext._layers_decode)._flags_ & flag

@@ -57,7 +57,9 @@ def _load_library():
         raise ImportError(
             f"{LIB_PATH} is missing: build it with `python torch-int_amd/build.py` "
             "(hipcc, --offload-arch=gfx950). torch_int has no fallback implementation.")
-    lib = ctypes.CDLL(LIB_PATH)
+    # A handle that keeps the interpreter lock during a call, as the forwarder does: a product in slices, or a layer, is several
+    # launches that meet in memory which calls on one stream share, and no other thread may launch there between them.
+    lib = ctypes.PyDLL(LIB_PATH)
     for name, argtypes in _SIGNATURES.items():
         fn = getattr(lib, name)
         fn.argtypes = argtypes

@@ -126,9 +126,10 @@ _lib.ti_opt_decoder_layer_decode_from.restype = ctypes.c_int
 _lib.ti_opt_decoder_layer_prefill_chained.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, ctypes.c_int, _vp, _vp, _i64,
                                                       _vp, _i64, _vp]
 _lib.ti_opt_decoder_layer_prefill_chained.restype = ctypes.c_int
-_lib.ti_opt_decoder_layers_decode.argtypes = [_vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _i64, _vp]
-_lib.ti_opt_decoder_layers_decode.restype = ctypes.c_int
-_layers_decode = _lib.ti_opt_decoder_layers_decode
+# the one call that gives up the interpreter lock: some 200 launches, in memory of its own
+_layers_decode = ctypes.CDLL(_CUDA.LIB_PATH).ti_opt_decoder_layers_decode
+_layers_decode.argtypes = [_vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _i64, _vp]
+_layers_decode.restype = ctypes.c_int
 _raw_stream = torch._C._cuda_getCurrentRawStream
 _opt_layer_decode = getattr(_CUDA._fast, "opt_layer_decode", None) or _lib.ti_opt_decoder_layer_decode_from
 _opt_layer_prefill = getattr(_CUDA._fast, "opt_layer_prefill", None) or _lib.ti_opt_decoder_layer_prefill_chained
