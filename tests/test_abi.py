@@ -413,11 +413,11 @@ def test_square_split_tiles_only_where_they_are_ahead(M, N, K, slices):
 
 
 @pytest.mark.parametrize("M,N,K,slices", [(64, 20480, 13312, 0), (17, 9216, 13312, 0), (64, 20480, 1536, 0), (64, 5120, 11264, 0),
-                                          (24, 4096, 16384, 8), (64, 5120, 20480, 4), (48, 2560, 10240, 2), (40, 2048, 8192, 4),
+                                          (24, 4096, 16384, 4), (64, 5120, 20480, 4), (48, 2560, 10240, 2), (40, 2048, 8192, 4),
                                           (64, 4096, 4096, 1),
                                           (4, 7168, 7168, 0), (8, 7168, 7168, 0), (2, 36864, 9216, 0), (16, 5120, 11264, 0),
                                           (8, 7168, 16384, 0), (8, 4096, 1536, 0), (8, 768, 1536, 0),
-                                          (16, 7168, 7168, 2), (3, 7168, 20480, 4), (4, 5120, 16384, 8), (4, 2560, 10240, 2),
+                                          (16, 7168, 7168, 2), (3, 7168, 20480, 4), (4, 5120, 16384, 4), (4, 2560, 10240, 2),
                                           (8, 768, 2304, 3), (4, 20480, 5120, 1)])
 def test_rows_in_slices_only_where_they_are_ahead(M, N, K, slices):
     # the first four, and seven more of up to 16 rows, took up to 2.6 times as long in slices that meet as on the kernels they had
@@ -426,6 +426,17 @@ def test_rows_in_slices_only_where_they_are_ahead(M, N, K, slices):
     pick = C._lib.ti_selftest_rows_pick
     pick.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
     assert pick(M, N, K, 256, ctypes.byref(ctypes.c_int(0))) == slices
+
+
+@pytest.mark.parametrize("M,N,K,tiling,slices", [(24, 4096, 16384, 6, 4), (17, 1024, 12288, 6, 3), (64, 784, 16384, 6, 4), (40, 2048, 8192, 1, 4)])
+def test_the_workspace_is_of_the_slices_that_run(M, N, K, tiling, slices):
+    # slices of four waves that run as pairs are priced as those and launched, asked for and reported as pairs (tiling 6, F)
+    import torch_int._CUDA as C
+    pick = C._lib.ti_selftest_rows_pick
+    pick.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
+    told = ctypes.c_int(0)
+    assert (pick(M, N, K, 256, ctypes.byref(told)), told.value) == (slices, tiling)
+    assert C._lib.ti_linear_workspace_bytes(M, N, K) == slices * M * N * 4
 
 
 @pytest.mark.parametrize("M,N,K,refused", [(64, 50272, 11264, False), (19, 50272, 11264, False), (257, 11040, 16640, False), (300, 28800, 28672, False),

@@ -504,6 +504,15 @@ static inline int rows_blocks_each(int tiling, long long M, long long N, long lo
   return !pairs ? 0 : fits(3, 2LL * cus) ? 3 : fits(4, 2LL * cus) ? 4 : 0;
 }
 
+// Six and eight slices of A run as three and four of F: half as many tiles to park, and to add at the end.  24 x 4096 x 16384 17.5 us,
+// 15.9 so; 64 x 7168 x 16384 35.7 / 28.9, 5 x 2048 x 16384 10.9 / 9.8; 220 shapes of 768 to 12288 columns and 2 to 64 rows 0.92 times the time
+// in the mean, worst 1.04 (33 x 768 x 12288).  Four as two are level (8192: 16 and 48 x 2048 1.03 and 1.05, 17 to 48 x 8192 0.94 to 0.96),
+// twelve as six not everywhere ahead (768 columns 1.02).
+static inline RowsPick rows_paired(RowsPick pick, long long K) {
+  return pick.tiling == ROWS_A && (K == 12288 || K == 16384) ? RowsPick{ROWS_F, pick.slices / 2} : pick;
+}
+
+// What launches: the acceptance tests and prices are those of the slices before they are paired.
 static inline RowsPick rows_pick(long long M, long long N, long long K, int cus = num_cus(), int problems = 1) {
   if (M < 1 || M > TI_ROWS_ABREAST_M || N < 1 || K < 768 || K > (1 << 20)) return {ROWS_NONE, 1};
   RowsPick pick{ROWS_NONE, 1};
@@ -526,15 +535,7 @@ static inline RowsPick rows_pick(long long M, long long N, long long K, int cus 
   if (pick.slices > 1 && !(M <= 16 ? few_rows_slices_ahead(pick, M, N, K, problems)
                                    : rows_slices_ahead(pick, M, N, K, problems, cus)))
     return {ROWS_NONE, 1};
-  return pick;
-}
-
-// Six and eight slices of A run as three and four of F: half as many tiles to park, and to add at the end.  24 x 4096 x 16384 17.5 us,
-// 15.9 so; 64 x 7168 x 16384 35.7 / 28.9, 5 x 2048 x 16384 10.9 / 9.8; 220 shapes of 768 to 12288 columns and 2 to 64 rows 0.92 times the time
-// in the mean, worst 1.04 (33 x 768 x 12288).  Four as two are level (8192: 16 and 48 x 2048 1.03 and 1.05, 17 to 48 x 8192 0.94 to 0.96),
-// twelve as six not everywhere ahead (768 columns 1.02).
-static inline RowsPick rows_paired(RowsPick pick, long long K) {
-  return pick.tiling == ROWS_A && (K == 12288 || K == 16384) ? RowsPick{ROWS_F, pick.slices / 2} : pick;
+  return rows_paired(pick, K);
 }
 
 template <class Cfg>
@@ -589,7 +590,7 @@ template <int KIND, bool GROUPED>
 static int launch_rows(const GemmParams& p_in, const GemmGroup& grp, int problems, void* workspace,
                        long long workspace_bytes, hipStream_t stream) {
   if (p_in.batch != 1 || p_in.lda != p_in.K || p_in.ldb != p_in.K) return -1;
-  const RowsPick pick = rows_paired(rows_pick(p_in.M, p_in.N, p_in.K, num_cus(), problems), p_in.K);
+  const RowsPick pick = rows_pick(p_in.M, p_in.N, p_in.K, num_cus(), problems);
   if (pick.tiling == ROWS_NONE) return -1;
   GemmParams p = p_in;
   p.splits = pick.slices;

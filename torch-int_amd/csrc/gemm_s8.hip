@@ -102,7 +102,10 @@ static __device__ __align__(256) int g_fused_arrivals[kFusedStreams * (kFusedCou
 // it was recorded on.  33 blocks, as many as a program gets streams of from torch (the default one and a pool of 32);
 // further streams take the other forms.
 static constexpr int kRowsStreams = 33;
-static constexpr int kRowsCounters = 4096, kRowsWords = 4096;  // rows_pick: at most 256 groups x 8 waves, 256 words 64 bytes apart
+// rows_pick takes at most 256 groups of four or eight waves, of sixteen (half as many slices, half as many workgroups to a CU) too;
+// a placement word a group, 64 bytes apart
+static constexpr int kRowsCounters = 4096, kRowsWords = 4096;
+static_assert(kRowsCounters >= 256 * 16 && kRowsWords >= 256 * 16, "a counter to a wave, a placement word to a group");
 static __device__ __align__(256) int g_rows_arrivals[kRowsStreams * (kRowsCounters + kRowsWords)];
 static __device__ __align__(256) char g_rows_park[kRowsStreams * kRowsParkBytes];
 
