@@ -1,5 +1,6 @@
 """Decode steps whose cache is as the step before left it: all layers from one C call.  Against the modules, logits and caches bit for
-bit: steps past the end of the buffers, one cache continued twice, copied, cut and re-ordered caches, hooks, two threads on one stream."""
+bit: steps past the end of the buffers, one cache continued twice, copied, cut and re-ordered caches, hooks,
+padded batches, two threads on one stream."""
 import copy
 import threading
 
@@ -82,6 +83,27 @@ def test_steps_continue_each_other(bsz, half, monkeypatch):
     assert len(seen) == n
     with _Modules():
         _same(a, lm(ids[:, :1], past_key_values=past, use_cache=True))
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("bsz", [3, 9])
+def test_steps_of_a_padded_batch_continue_each_other(bsz, half, monkeypatch):
+    lm = _model(half)
+    masked = []
+    real = _hip_ext.opt_layers_decode
+    monkeypatch.setattr(_hip_ext, "opt_layers_decode", lambda *a: (masked.append(a[2] is not None), real(*a)) and None)
+    ids = torch.randint(2, 64, (bsz, 64), device=DEV)
+    keep = torch.arange(64, device=DEV) >= torch.arange(bsz, device=DEV)[:, None] * 7 % 31   # padding on the left, none to 30 tokens
+    print("continue padded", bsz, half, flush=True)
+    one = mod = lm(ids[:, :32], attention_mask=keep[:, :32], use_cache=True)
+    for step in range(32, 64):
+        mask = keep[:, :step + 1]
+        one = lm(ids[:, step:step + 1], attention_mask=mask, past_key_values=one.past_key_values, use_cache=True)
+        with _Modules():
+            mod = lm(ids[:, step:step + 1], attention_mask=mask, past_key_values=mod.past_key_values, use_cache=True)
+        _same(one, mod)
+    assert masked == [True] * 31   # all but the first step, which moves the cache
 
 
 @torch.no_grad()

@@ -1,14 +1,24 @@
 """Narrow outputs of 17 to 512 rows, whose 16-row blocks lie in several workgroups (csrc/gemm_rows.h, rows_blocks_each): one, two and
 three blocks to a workgroup, last groups that are cut off or hold fewer blocks, outputs at the lines of the rule, an fp16 and an fp32 stream
 that is added to, head-major stores and groups.  Integer sums: exact."""
+import ctypes
+
 import pytest
 import torch
 
 from oracle import oracle as orc
+from test_gpu_ln_linear import _add_f16
 from test_gpu_rows import _last, _s8
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
+
+
+def _adds_into_an_fp16_stream(x, w, bias, acc, resid, alpha):
+    fresh, old = orc.epi_bfp32_ofp32(acc, bias.cpu(), alpha, 1.0), resid.half()
+    got = old.to(DEV)
+    _add_f16(x, w, bias, got, alpha)
+    assert _last()[0] == 1 and torch.equal(got.cpu(), (old.float() + fresh.half().float()).half())
 
 
 @pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 63, 64])
@@ -28,6 +38,7 @@ def test_rows_in_several_workgroups(M, N, K):
     assert torch.equal(C.linear_a8_w8_bfp32_ofp32(xd, wd, bfd, al, 1.0).cpu(), orc.epi_bfp32_ofp32(acc, bf, al, 1.0))
     assert torch.equal(C._linear_a8_w8_bfp32_ofp32_acc(xd, wd, bfd, al, 1.0, resid.to(DEV)).cpu(),
                        orc.linear_a8_w8_bfp32_ofp32_acc(x, w, bf, al, 1.0, resid, acc_fn=lambda *_: acc))
+    _adds_into_an_fp16_stream(xd, wd, bfd, acc, resid, al)
     if N % 16 == 0:
         import torch_int._hip_ext as X
         want = orc.epi_b8_o8(acc, b8, al, be).view(1, M, N // 16, 16).transpose(1, 2)
@@ -83,6 +94,7 @@ def test_more_than_64_rows(M, N, K):
     assert torch.equal(C.linear_a8_w8_bfp32_ofp32(xd, wd, bfd, al, 1.0).cpu(), orc.epi_bfp32_ofp32(acc, bf, al, 1.0))
     assert torch.equal(C._linear_a8_w8_bfp32_ofp32_acc(xd, wd, bfd, al, 1.0, resid.to(DEV)).cpu(),
                        orc.linear_a8_w8_bfp32_ofp32_acc(x, w, bf, al, 1.0, resid, acc_fn=lambda *_: acc))
+    _adds_into_an_fp16_stream(xd, wd, bfd, acc, resid, al)
     if N % 16 == 0:
         heads = want.view(1, M, N // 16, 16).transpose(1, 2)
         assert torch.equal(X.linear_a8_w8_b8_o8_heads(xd, wd, b8d, al, be, 1, M, N // 16, 16).cpu(), heads)
@@ -105,4 +117,9 @@ def test_where_more_than_64_rows_end():
         print("rows end", M, N, K, flush=True)
         out = C.linear_a8_w8_b8_o8(x.to(DEV), w.to(DEV), b.to(DEV), 3e-4, 0.02)
         assert _last()[0] == 0 and torch.equal(out.cpu(), orc.linear_a8_w8_b8_o8(x, w, b, 3e-4, 0.02, acc_fn=orc.gemm_acc_torch))
-    assert X.linear_group_is_one_launch(192, 768, 768) and not X.linear_group_is_one_launch(208, 768, 768 + 64)
+    C._lib.ti_last_kernel.restype = ctypes.c_char_p
+    for M in (192, 193):   # three 768 x 768
+        test_groups_in_several_workgroups(M, 768, 768)
+        one = X.linear_group_is_one_launch(M, 768, 768)
+        assert one == (M == 192) == C._lib.ti_last_kernel().endswith(b"_group"), (M, C._lib.ti_last_kernel())
+        assert not one or _last()[0] == 1
