@@ -1,5 +1,6 @@
 """The layers of a model chained, one C call each with the last addition left to the next layer's first kernel, against the
 same model going through its modules: logits and key / value caches bit for bit."""
+import gc
 import pytest
 import torch
 
@@ -105,6 +106,7 @@ def test_a_chained_prefill_needs_hardly_more_memory_than_the_modules(bsz, T, hal
             print("memory", bsz, T, half, chained, flush=True)
             model(ids, use_cache=True)   # the stream's kept buffers are there
             torch.cuda.synchronize()
+            gc.collect()   # what earlier tests left in reference cycles would be freed during the pass, and hide as much of its peak
             torch.cuda.reset_peak_memory_stats()
             before = torch.cuda.memory_allocated()
             model(ids, use_cache=True)
