@@ -531,13 +531,14 @@ int ti_opt_decoder_layer_decode(const TiOptDecodeLayer* layer, void* hidden, con
  * without a cache): LayerNormQ, the q/k/v projections stored head-major (one grouped launch where
  * ti_linear_group_is_one_launch says so, else three calls with the workspace), the one-launch prefill attention with the head merge
  * (ti_attn_prefill_s8_v; beyond 2048 keys V transposed and ti_attn_prefill_s8_mc), out_proj, the residual update fused with the second
- * LayerNormQ, fc1 (ReLU), fc2 added into the residual stream -- the entry points and arguments of the module path, so
- * its values.  hidden [B, T, embed] is updated in place; mask fp32 [B, 1, T, T] or NULL, mask_classes its class array
+ * LayerNormQ (on an fp16 stream of more than 64 rows with out_proj: ti_linear_a8_w8_bfp32_of16_acc), fc1 (ReLU), fc2 added into the
+ * residual stream -- the values are those of the module path.  hidden [B, T, embed] is updated in place; mask fp32 [B, 1, T, T] or NULL, mask_classes its class array
  * (ti_attn_mask_classes) or NULL; k_out / v_out receive the key and value rows [B, heads, T, head_dim] (the cache the
  * decode steps continue).  T a multiple of 16 that ti_attn_prefill_supported(T, T, head_dim) accepts, B * T <= 4096
  * (larger prefills are bound by their kernels, not by the host).  scratch:
  * ti_opt_decoder_layer_prefill_scratch_bytes(B * T, embed, ffn) bytes on a 256-byte boundary; workspace: the split-K
- * workspace of the linears (ti_linear_workspace_bytes of the largest of them, ti_linear_acc_workspace_bytes for fc2, or NULL). */
+ * workspace of the linears (ti_linear_workspace_bytes of the largest of them, ti_linear_acc_workspace_bytes for fc2 and, on an fp16
+ * stream, for out_proj; or NULL). */
 int64_t ti_opt_decoder_layer_prefill_scratch_bytes(int64_t rows, int64_t embed, int64_t ffn);
 int ti_opt_decoder_layer_prefill(const TiOptDecodeLayer* layer, void* hidden, const float* mask,
                                  const uint8_t* mask_classes, int8_t* k_out, int8_t* v_out, int64_t B, int64_t T,
@@ -550,7 +551,9 @@ int ti_opt_decoder_layer_prefill(const TiOptDecodeLayer* layer, void* hidden, co
  * added to the stream by a kernel of its own (an fp16 stream of 5 to 64 rows, an fp32 one of more than 4096), leave it in carry instead; chain & 1:
  * this call's first LayerNorm kernel adds what the call before left there.  Every layer but the last leaves, every layer but
  * the first adds; the additions and their order are those of the separate calls.  A prefill with chain != 0 keeps the output of
- * out_proj in carry too and does with less scratch: ti_opt_decoder_layer_prefill_chained_scratch_bytes(B * T, embed, ffn). */
+ * out_proj in carry too, unless the stream is fp16 and has more than 64 rows (nothing is kept there then), and does with less scratch:
+ * ti_opt_decoder_layer_prefill_chained_scratch_bytes(B * T, embed, ffn).  What a layer's kernels hand one another lies in scratch and
+ * workspace: calls of several host threads on one stream may share them only if no other launch comes between those of a call. */
 int64_t ti_opt_decoder_layer_prefill_chained_scratch_bytes(int64_t rows, int64_t embed, int64_t ffn);
 int ti_opt_decoder_layer_decode_chained(const TiOptDecodeLayer* layer, void* hidden, const float* mask, int8_t* k_buf,
                                         int8_t* v_buf, int64_t B, int64_t cap, int64_t S, int chain, float* carry,
@@ -568,7 +571,7 @@ int ti_opt_decoder_layer_prefill_chained(const TiOptDecodeLayer* layer, void* hi
 
 /* The layers of one decode step one after the other from one call: ti_opt_decoder_layer_decode_chained for layers[0 .. count - 1],
  * whose cache buffers are all [B, heads, cap, head_dim] of one cap; the first without chain & 1, the last without chain & 2, or
- * with chain = 0 throughout where carry is NULL. */
+ * with chain = 0 throughout where carry is NULL.  scratch and carry must be this call's alone until its last kernel is on the stream. */
 int ti_opt_decoder_layers_decode(const TiOptDecodeLayer* const* layers, int64_t count, void* hidden, const float* mask,
                                  int8_t* const* k_bufs, int8_t* const* v_bufs, int64_t B, int64_t cap, int64_t S, float* carry,
                                  void* scratch, int64_t scratch_bytes, void* stream);

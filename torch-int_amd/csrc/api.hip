@@ -995,7 +995,7 @@ int prefill_layer(const char* op, const TiOptDecodeLayer* L, void* hidden, const
   if (B < 0 || T < 0 || B > 65535 || T > 4096) return fail(TI_ERR_INVALID_ARG, "%s: needs 0 <= B <= 65535, 0 <= T <= 4096", op);
   const int64_t M = B * T;
   if (M == 0) return TI_OK;
-  if (B * H > 65535)  // the transpose of the values; refused before anything is launched
+  if (B * H > 65535)  // the transpose of the values, which more than 2048 keys need; refused before anything is launched
     return fail(TI_ERR_INVALID_ARG, "%s: up to 65535 sequences x heads (got %lld x %lld)", op, (long long)B, (long long)H);
   if (M > most)
     return fail(TI_ERR_INVALID_ARG, "%s: up to %lld tokens in all (got %lld x %lld)", op, (long long)most, (long long)B, (long long)T);

@@ -10,9 +10,11 @@
 // contexts.  The three-sweep form this replaces up to 2048 keys computed scores three and exponentials up to two times, with a
 // barrier and an exposed copy per tile of 256 keys and sweep.
 //
-// Bound by the vector ALUs (some 24 instructions a live score: at 32 heads x 2048 x 128 without a mask 82 us of 126) and, under
-// a causal mask, by the few tiles of most rows.  What it measures against the other forms is at the rule that chooses
-// (attn_fused.hip).
+// Bound by the vector ALUs (some 24 instructions a score: at 32 heads x 2048 x 128 without a mask 82 us of 126) and by waits that
+// two waves to a SIMD, as many as the score registers allow, do not cover.  Causal, 32 heads x 1904 x 128, by the counters: the ALUs work in 53 % of
+// the SIMDs' cycles (37 instructions a live score: dead halves of the diagonal's tiles, meetings), the matrix pipes in 10 %, the LDS in 14 %; waves
+// wait for copies, LDS and one another during 37 % of their time and for an issue slot during 11 %.  What it measures against the other forms is at
+// the rule that chooses (attn_fused.hip).
 //
 // Keys, mask values and V^T reach a wave through an LDS ring of its own, without barriers: no two waves of a workgroup use the same key, but
 // a fragment load straight from global memory asks for 16 rows x 64 bytes with neighbouring lanes on different rows, a

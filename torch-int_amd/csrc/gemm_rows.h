@@ -1,7 +1,7 @@
 // GEMM for a few rows of activations (2 to 64, of narrow outputs to 512): decode steps of a served batch, short prompts.  Included by
 // gemm_s8_impl.h (it uses the epilogues of ti_common.h and the LDS-limit helper there).
 //
-// Bound by HBM: every weight byte is used once, for at most 64 rows of activations.  What the weights cost on this
+// Bound by HBM: every weight byte is read from there once, for up to 64 rows of activations by one workgroup, for more by workgroups of one XCD.  What the weights cost on this
 // chip is decided by two things, and the kernel is laid out for both of them:
 //   - bytes in flight.  A CU has to keep some 64 KiB of weight copies outstanding to cover the round trip to HBM.  The
 //     activations therefore do not share the LDS with the weights: a wave keeps the fragments of its slice of the

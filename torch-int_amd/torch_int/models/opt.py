@@ -668,7 +668,8 @@ class Int8OPTDecoderLayer(nn.Module):
         if T % 16 or bsz == 0 or bsz > 65535 or bsz * T > 1 << 20 or (mask is not None and mask.shape != (bsz, 1, T, T)):
             return None
         plan = self._decode_plan(hs.dtype is torch.float16, hs.device)
-        # one transpose of all values: up to 65535 matrices (beyond, ``_hip_ext.transpose_last2`` leaves them to torch)
+        # up to 65535 matrices, what one transpose of all values takes, which more than 2048 keys need (beyond, ``_hip_ext.transpose_last2``
+        # leaves them to torch)
         if (plan is None or hs.shape[2] != plan.embed or bsz * plan.heads > 65535
                 or not _hip_ext.attn_prefill_shape_ok_cached(T, T, plan.head_dim)):
             return None
@@ -895,7 +896,8 @@ class Int8OPTDecoder(nn.Module):
             found.append(hit)
         # The carry: fc2's output on its way from one layer to the next, and in a prefill out_proj's too; memory of this pass, so
         # that passes of other threads on the same stream do not meet in it.  A decode step on an fp32 stream has none (fc2's
-        # GEMM adds its output itself).
+        # GEMM adds its output itself).  On an fp16 stream of up to 4 or more than 64 rows nothing is left in it either: it is what
+        # lets a prefill's layers do with the smaller scratch.
         carry = self._carry(hidden, count, decode)
         links = [0 if carry is None else (_hip_ext.CHAIN_ADD if i else 0) | (_hip_ext.CHAIN_LEAVE if i + 1 < count else 0)
                  for i in range(count)]
