@@ -2275,7 +2275,7 @@ static int skinny_waves(const GemmParams& p) {
   return (int)nw;
 }
 
-// Any-shape fallback (K not a multiple of 16 or operands not 16-byte aligned):
+// Any-shape fallback of the linears (K not a multiple of 16 or operands not 16-byte aligned; batched products: bmm_any.h):
 // one thread per output element, scalar loop over K.
 template <int KIND>
 __global__ __launch_bounds__(256) void gemm_scalar_kernel(GemmParams p) {
@@ -2812,6 +2812,7 @@ static int batched_splits(long long batch, long long M, long long N, long long K
 }
 
 }  // namespace ti
+#include "bmm_any.h"
 #include "gemm_rows.h"
 namespace ti {
 
@@ -2903,13 +2904,17 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
                        ((reinterpret_cast<uintptr_t>(p.B) & 15) == 0) &&
                        (p.strideA % 16 == 0) && (p.strideB % 16 == 0);  // the stores check C themselves
   if (!aligned) {
-    g_last_kernel = "scalar";
-    const long long total = (long long)p.M * p.N;
-    dim3 grid((unsigned)((total + 255) / 256), 1, p.batch);
-    hipLaunchKernelGGL(gemm_scalar_kernel<KIND>, grid, dim3(256), 0, stream, p);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
-    return TI_OK;
+    if constexpr (KIND == EPI_F32_SCALE || KIND == EPI_S8_SCALE || KIND == EPI_S32_RAW) {  // products of two activations
+      return launch_any<KIND>(p, stream);
+    } else {
+      g_last_kernel = "scalar";
+      const long long total = (long long)p.M * p.N;
+      dim3 grid((unsigned)((total + 255) / 256), 1, p.batch);
+      hipLaunchKernelGGL(gemm_scalar_kernel<KIND>, grid, dim3(256), 0, stream, p);
+      hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
+      return TI_OK;
+    }
   }
   // Up to 64 rows, more where the output is narrow: the weight-streaming kernel with the activations in registers.  Not for one row where the dot-product
   // kernel reads weight rows flat, one or two rows against the few, long weight rows of the view below, ragged widths of a

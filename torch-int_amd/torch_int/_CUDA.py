@@ -180,15 +180,25 @@ def _workspace(dev_index, stream, nbytes):
     return ws, ws.data_ptr(), ws.numel()
 
 
-def _pad_inner(a, b, K, macs, weight=False):
-    """Operands whose inner dimension is not a multiple of 16 have no aligned rows for the tiled kernels, and the
-    library then runs a one-thread-per-output kernel (40 x 1500 x 128 x 1500: 32 ms).  From a size at which that
-    hurts, both operands are copied with K padded by zeros to a multiple of 64 first: the added products are zero,
-    the results the same (upstream rejects such shapes: "cutlass cannot implement")."""
-    if K % 16 == 0 or macs < (1 << 26):
+def _pad_inner(a, b, K):
+    """Operands of a linear whose inner dimension is not a multiple of 16 have no aligned rows for the tiled kernels, and the
+    library then runs a one-thread-per-output kernel.  From a size at which that hurts, both operands are copied with K
+    padded by zeros to a multiple of 64 first: the added products are zero, the results the same (upstream rejects such
+    shapes: "cutlass cannot implement")."""
+    if K % 16 == 0 or a.shape[0] * b.shape[0] * K < (1 << 26):
         return a, b, K
     pad = -K % 64
-    return torch.nn.functional.pad(a, (0, pad)), _padded_weight(b, pad) if weight else torch.nn.functional.pad(b, (0, pad)), K + pad
+    return torch.nn.functional.pad(a, (0, pad)), _padded_weight(b, pad), K + pad
+
+
+def _pad_products(a, b, batch, M, N, K):
+    """Batched products with such a K have kernels that read rows where they lie (csrc/bmm_any.h).  Copies padded as above
+    are ahead of those only where the products are many to a byte, or where K is long enough to be cut into slices."""
+    pad = -K % 64
+    if K % 16 == 0 or batch * M * N * K < (1 << 26) or not (
+            M * N >= 1024 * (M + N) or (K >= 2048 and M > 16 and _bmm_ws_bytes(batch, M, N, K + pad) > 0)):
+        return a, b, K
+    return torch.nn.functional.pad(a, (0, pad)), torch.nn.functional.pad(b, (0, pad)), K + pad
 
 
 _padded = {}  # id(weight) -> (weak reference, version counter, padded copy)
@@ -239,7 +249,7 @@ def _linear(op, kind, x, w, bias, bias_dtype, out_dtype, alpha, beta, inout=None
             _fail(op, f"the tensor to add into must be a contiguous {out_dtype} tensor of {M}x{N} elements on {dev}")
     if M == 0 or N == 0:
         return out
-    x, w, K = _pad_inner(x, w, K, M * N * K, weight=True)
+    x, w, K = _pad_inner(x, w, K)
     idx = dev.index
     switch = idx != _current_device()
     if switch:
@@ -308,7 +318,8 @@ def _bmm(op, kind, a, b, out_dtype, alpha):
     out = _empty((batch, M, N), dtype=out_dtype, device=dev)
     if out.numel() == 0:
         return out
-    a, b, K = _pad_inner(a, b, K, batch * M * N * K)
+    if K & 15:
+        a, b, K = _pad_products(a, b, batch, M, N, K)
     idx = dev.index
     switch = idx != _current_device()
     if switch:
