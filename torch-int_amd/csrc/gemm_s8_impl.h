@@ -2813,6 +2813,7 @@ static int batched_splits(long long batch, long long M, long long N, long long K
 
 }  // namespace ti
 #include "bmm_any.h"
+#include "bmm_scores.h"
 #include "gemm_rows.h"
 namespace ti {
 
@@ -2915,6 +2916,9 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
       if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
       return TI_OK;
     }
+  }
+  if constexpr (KIND == EPI_F32_SCALE || KIND == EPI_S32_RAW) {
+    if (scores_take(p)) return launch_scores<KIND>(p, stream);
   }
   // Up to 64 rows, more where the output is narrow: the weight-streaming kernel with the activations in registers.  Not for one row where the dot-product
   // kernel reads weight rows flat, one or two rows against the few, long weight rows of the view below, ragged widths of a
