@@ -72,8 +72,8 @@ int ti_linear_row_split(int64_t M, int64_t N, int64_t K);
  * ("pipe_256x256", "pipe16_256x160", "pipe16_256x288", "pipe16_256x128", "pipe16_128x80", "pipe16_128x192", "pipe16_256x192", "pipe16_192x128",
  * "pipe16_192x256", "pipe16_160x256", "pipe_128x128",
  * "splitk_<tile>" and "fusedk_<tile>" for the two- and one-launch split-K forms, "stream", "mid_stream" (the weight-streaming kernel, up to 16 and 17 to 64 rows, of narrow outputs to 512), "stream_parts" (the streaming
- * kernel on the view with rows cut into parts), "gemv" (one row of activations), "skinny", "tile_*",
- * "scalar", "any" and "any_skinny" (batched products of rows that are not whole aligned chunks), "scores" (32-bit outputs, K up to 128); grouped launches add "_group": "stream_group", "mid_stream_group", "gemv_group", "pipe16_256x160_group", "pipe16_256x288_group",
+ * kernel on the view with rows cut into parts), "mid_waves_<tile>" (some 65 to 1024 rows, the waves of a workgroup sharing K), "gemv" (one row of activations), "skinny", "tile_*",
+ * "scalar", "any" and "any_skinny" (batched products of rows that are not whole aligned chunks), "scores" (32-bit outputs, K up to 128); grouped launches add "_group": "stream_group", "mid_stream_group", "mid_waves_group", "gemv_group", "pipe16_256x160_group", "pipe16_256x288_group",
  * "pipe16_256x256_group", "pipe16_256x128_group"; "<family>+<family>" when the last rows ran as a second problem, see ti_linear_row_split;
  * "" before the first call).  Benchmarks use it to label their rows. */
 const char* ti_last_kernel(void);

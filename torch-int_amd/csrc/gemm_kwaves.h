@@ -1,0 +1,228 @@
+// Linears of some 65 to 1024 rows whose output makes one round of small tiles: the waves of a workgroup share K, not the tile.
+//
+// A workgroup has one tile of 32x32 to 64x80 outputs over the whole of K, and each of its waves multiplies the WHOLE tile, over every
+// NW-th step of 128 bytes.  So a wave's fragments serve as many products as the tile has (a 32x32 quarter of 64x64 reads twice the LDS
+// bytes a product), its panels lie in a ring of its own, and no wave waits for another until the integer sums of all of them are
+// added through the LDS at the end: no barrier in the loop, no slices of K that meet in memory, no second launch, no workspace.
+//
+// Bound by what the copies have in flight: a step's panels are (BM + BN) * 128 bytes for few products, 0.18 (32x32) to 0.33 us (64x80)
+// a step of the workgroup with weights from HBM, 0.11 (32x64) and 0.13 (64x64) with weights that the last-level cache holds, where the
+// copies of a CU alone take 0.08 and 0.11.  The tiled kernels that had these shapes take one step after the other, a barrier each, on a quarter
+// of the CUs (128x128 tiles), or park and add int32 slices.  Cold weights, us, before / now: 384 x 2048 x 2048 15.7 / 6.8, 512 x 2048 x 2048
+// 15.8 / 7.6, 128 x 8192 x 2048 14.5 / 8.8, 128 x 2048 x 8192 20.4 / 11.3, 128 x 4096 x 4096 15.5 / 10.0, 256 x 4096 x 4096 18.1 / 12.0,
+// 256 x 2560 x 2560 13.5 / 8.1, 128 x 5120 x 5120 17.9 / 13.6, 256 x 5120 x 5120 20.9 / 17.0, 1024 x 768 x 3072 17.2 / 9.6.
+//
+// Row tiles begin at different steps of K (`turn`): those of one column read the same weights, and so ask HBM for different lines
+// of them at a time (256 x 5120 x 5120 17.7 / 16.9, 512 x 2048 x 2048 7.85 / 7.4; 256 x 4096 x 4096 12.1 / 12.3).  Tried and left: copies spread between the
+// products (level), steps turned by column tile or by workgroup (level), the same tiles with their waves side by side and up to ten stages
+// (384 x 2048 x 2048 9.0, 128 x 4096 x 4096 11.7).
+#pragma once
+
+namespace ti {
+
+// NW waves, each with a ring of STAGES steps
+template <int BM_, int BN_, int NW_, int STAGES_, int KIND_, bool GROUPED_ = false>
+struct KWavesCfg {
+  static constexpr int BM = BM_, BN = BN_, NW = NW_, STAGES = STAGES_, KIND = KIND_;
+  static constexpr bool GROUPED = GROUPED_;
+  static constexpr int NT = NW * 64;
+  static constexpr int TM = BM / 16, TN = BN / 16;
+  static constexpr int STAGE = (BM + BN) * QBK;
+  static constexpr int COPIES = STAGE / 1024;  // copy instructions a step: eight panel rows each
+  static constexpr int LDS_BYTES = NW * STAGES * STAGE;
+  // units of the epilogue: 16 rows, halves of them where that leaves waves without one
+  static constexpr int PARTS = TM < NW && TM <= 2 && TN % 2 == 0 ? 2 : 1;
+  static constexpr int RESIDENT = 160 * 1024 / LDS_BYTES;  // workgroups to a CU
+  static constexpr int WAVES_PER_SIMD = (RESIDENT * NW + 3) / 4;
+  static_assert(BM % 16 == 0 && BN % 16 == 0, "blocks of 16x16");
+  static_assert(STAGES >= 1 && STAGES <= 2, "the waits know of two");
+  static_assert((STAGES - 1) * COPIES <= 63, "a wait counts in six bits");
+  static_assert(TM * TN * 1024 <= STAGES * STAGE, "a wave's sums go over its ring");
+  static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
+};
+
+// 16 rows of the tile, as the epilogue of gemm_pipe16q_kernel knows a wave's part
+template <class Cfg>
+struct KWavesUnit {
+  static constexpr int BM = Cfg::BM, BN = Cfg::BN, KIND = Cfg::KIND;
+  static constexpr int TM = 1, TN = Cfg::TN / Cfg::PARTS, WTM = 16, WTN = TN * 16;
+};
+
+template <class Cfg>
+__global__ __launch_bounds__(Cfg::NT, (Cfg::WAVES_PER_SIMD)) void gemm_kwaves_kernel(GemmParams p, int tiles_m, int tiles_n,
+                                                                                     GemmGroup grp) {
+  constexpr int BM = Cfg::BM, BN = Cfg::BN, TM = Cfg::TM, TN = Cfg::TN, NW = Cfg::NW, S = Cfg::STAGES, COPIES = Cfg::COPIES;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tiles = tiles_m * tiles_n;
+  const int b = Cfg::GROUPED ? (int)blockIdx.x / tiles : 0;
+  int tile_m, tile_n;
+  tile_of_workgroup(blockIdx.x - b * tiles, tiles_m, tiles_n, tile_m, tile_n, p.band);
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  const int rows_a = p.M - m0 < BM ? p.M - m0 : BM, rows_b = p.N - n0 < BN ? p.N - n0 : BN;
+  const int8_t* W = Cfg::GROUPED ? grp.B[b] : p.B;
+  // the panels as buffers (launch_kind: rows at most PANEL_MAX_LD apart): rows beyond the last read as zeros, and are not stored
+  const __amdgpu_buffer_rsrc_t ares = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<int8_t*>(p.A + (size_t)m0 * p.lda), 0, (int)((unsigned)(rows_a - 1) * (unsigned)p.lda + (unsigned)p.K), 0x00020000);
+  const __amdgpu_buffer_rsrc_t bres = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<int8_t*>(W + (size_t)n0 * p.ldb), 0, (int)((unsigned)(rows_b - 1) * (unsigned)p.ldb + (unsigned)p.K), 0x00020000);
+  const int steps = p.K / QBK;
+  const int n = steps > wave ? (steps - wave + NW - 1) / NW : 0;  // this wave's: wave, wave + NW, ..., all turned by `turn`
+  const int turn = tile_m * steps / tiles_m;
+
+  // ---- copies: copy j of a step fills rows 8 j .. 8 j + 7 of [A panel | B panel], chunk c of row r at position c ^ ((r >> 1) & 7)
+  char* ring = smem + wave * (S * Cfg::STAGE);
+  const int row = lane >> 3, pos = lane & 7;
+  const unsigned sw[2] = {(unsigned)((pos ^ (lane >> 4)) << 4), (unsigned)((pos ^ (4 + (lane >> 4))) << 4)};  // of even and odd copies
+  const unsigned a_row = (unsigned)row * (unsigned)p.lda, b_row = (unsigned)row * (unsigned)p.ldb;
+  unsigned k_at = (unsigned)((wave + turn) % steps) * QBK;
+  int head = 0, issued = 0;
+  auto issue = [&]() {
+    TI_LDS_AS char* dst = (TI_LDS_AS char*)ring + head * Cfg::STAGE;
+#pragma unroll
+    for (int j = 0; j < BM / 8; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ares, (TI_LDS_AS void*)(dst + j * 1024), 16,
+                                               a_row + sw[j & 1] + k_at + (unsigned)(8 * j) * (unsigned)p.lda, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < BN / 8; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(bres, (TI_LDS_AS void*)(dst + (BM / 8 + j) * 1024), 16,
+                                               b_row + sw[j & 1] + k_at + (unsigned)(8 * j) * (unsigned)p.ldb, 0, 0, 0);
+    k_at += NW * QBK;
+    if (k_at >= (unsigned)p.K) k_at -= (unsigned)p.K;
+    head = head + 1 == S ? 0 : head + 1;
+    ++issued;
+  };
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    if (s < n) issue();
+
+  // ---- fragments: lane (r, g) reads row r of a block, chunk 4 * slice + g
+  const int r = lane & 15, g = lane >> 4;
+  const int at = r * QBK + (((g ^ (r >> 1)) & 7) << 4);
+  v4i acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = v4i{0, 0, 0, 0};
+  int tail = 0;
+  for (int it = 0; it < n; ++it) {
+    // loads complete in order: this step has landed once at most the copies of the one behind it are on their way
+    if (S == 2 && issued - it == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * COPIES) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const char* st = ring + tail * Cfg::STAGE;
+    v4i fa[2][TM], fb[2][TN];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) fa[s][i] = *reinterpret_cast<const v4i*>(st + ((at ^ (s << 6)) + i * 16 * QBK));
+#pragma unroll
+      for (int j = 0; j < TN; ++j) fb[s][j] = *reinterpret_cast<const v4i*>(st + BM * QBK + ((at ^ (s << 6)) + j * 16 * QBK));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // read: its stage is free for the next
+    if (issued < n) issue();
+    tail = tail + 1 == S ? 0 : tail + 1;
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[s][j], fa[s][i], acc[i][j], 0, 0, 0);
+  }
+
+  // ---- the waves' sums, over the rings (every copy of this wave has landed and been read)
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) *reinterpret_cast<v4i*>(ring + ((i * TN + j) * 64 + lane) * 16) = acc[i][j];
+  __syncthreads();
+  GemmParams q = p;
+  if constexpr (Cfg::GROUPED) {
+    q.bias = grp.bias[b];
+    q.C = grp.C[b];
+    q.alpha = grp.alpha[b];
+    q.beta = grp.beta[b];
+  }
+  using Unit = KWavesUnit<Cfg>;
+  for (int u = wave; u < TM * Cfg::PARTS; u += NW) {
+    const int i = u / Cfg::PARTS, c = u - i * Cfg::PARTS;
+    if (m0 + 16 * i >= p.M) break;
+    const char* first = smem + ((i * TN + c * Unit::TN) * 64 + lane) * 16;
+    v4i sum[1][Unit::TN];
+#pragma unroll
+    for (int j = 0; j < Unit::TN; ++j) sum[0][j] = *reinterpret_cast<const v4i*>(first + j * 1024);
+#pragma unroll
+    for (int w = 1; w < NW; ++w)
+#pragma unroll
+      for (int j = 0; j < Unit::TN; ++j) sum[0][j] += *reinterpret_cast<const v4i*>(first + w * (S * Cfg::STAGE) + j * 1024);
+    store_tile16<Unit>(sum, q, 0, tile_m, tile_n, i, c, lane);
+  }
+}
+
+template <class Cfg>
+static int launch_kwaves_cfg(const GemmParams& p, hipStream_t stream, const GemmGroup& grp) {
+  static std::atomic<unsigned long long> lds_ok{0};
+  if (int rc = allow_lds(gemm_kwaves_kernel<Cfg>, Cfg::LDS_BYTES, lds_ok)) return rc;
+  const int tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM, tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
+  const int grid = tiles_m * tiles_n * (Cfg::GROUPED ? grp.count : 1);  // kwaves_pick: a round or two
+  hipLaunchKernelGGL(gemm_kwaves_kernel<Cfg>, dim3((unsigned)grid), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, p, tiles_m, tiles_n, grp);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
+  return TI_OK;
+}
+
+enum KWavesTile { KWAVES_NONE = 0, KWAVES_32x32, KWAVES_32x64, KWAVES_48x64, KWAVES_64x64, KWAVES_64x80, KWAVES_64x64_PAIRS };
+
+// The tile of such a linear (or of `problems` of one shape in one launch), or none.  The smallest tile that is one round of the CUs: a smaller
+// one takes less a step, and the round is as long as its steps.  A second round costs as much as the first, or 0.9 times where two workgroups of two waves
+// share a CU (pairs), and larger tiles are ahead by then but for a short K (cold, us, the others / pairs): 1024 x 2048 x 2048 12.8 /
+// 11.0, 256 x 8192 x 2048 14.4 / 12.9, 2048 x 768 x 3072 16.8 / 13.3; not 768 x 2560 x 2560 15.9 / 15.8, 512 x 5120 x 5120 27 / 37, 512 x 3072 x 768 6.7 / 7.4).
+// Below five eighths of a round the CUs stand idle (128 x 1024 x 4096 on 32x32).
+// K: the copies of a tile grow with it, so beyond 8192 the slices are ahead (128 x 2560 x 10240 19.1 / 20, 256 x 4096 x 16384 34.6 / 34).
+// Widths: the measured ones, multiples of 2560 and 1024 (but for those that three divides, which have 192 and 288 columns wide tiles of their own), or of
+// 768 on both sides; K = 1024 and other widths stay with the kernels that had them, whose tests reach their forms there, and so do 257 to 512 rows of K from 3072 on, of which this kernel would take 0.6 to 0.85 of the time.
+static inline KWavesTile kwaves_pick(long long M, long long N, long long K, int problems = 1) {
+  if (M <= TI_ROWS_MAX_M || M > 4096 || N < 768 || N > 16384 || K > 8192) return KWAVES_NONE;
+  if (problems > 1 && K < 2048) return KWAVES_NONE;
+  const bool short_rows = N % 768 == 0 && K % 768 == 0 && K <= 3072;
+  auto wide = [](long long w) { return w % 2560 == 0 || (w % 1024 == 0 && w % 3 != 0); };
+  if (!short_rows && !(wide(N) && wide(K) && K >= 2048)) return KWAVES_NONE;
+  if (K >= 3072 && M > (K > 5120 ? 255 : 256) && M <= 512) return KWAVES_NONE;
+  const long long cus = num_cus();
+  struct Form { KWavesTile tile; int bm, bn; };
+  static constexpr Form kForms[] = {{KWAVES_32x32, 32, 32}, {KWAVES_32x64, 32, 64}, {KWAVES_48x64, 48, 64}, {KWAVES_64x64, 64, 64}, {KWAVES_64x80, 64, 80}};
+  for (const Form& f : kForms) {
+    if (N % f.bn != 0) continue;
+    const long long tiles = (M + f.bm - 1) / f.bm * (N / f.bn) * problems;
+    if (tiles <= cus) return 8 * tiles >= 5 * cus ? f.tile : KWAVES_NONE;
+  }
+  const long long tiles = (M + 63) / 64 * (N / 64) * problems;
+  return tiles <= 2 * cus && K >= 2048 && (K <= 2048 || short_rows || problems > 1) ? KWAVES_64x64_PAIRS : KWAVES_NONE;
+}
+
+// Whether it goes before the weight-streaming kernel, which has narrow outputs of more than 64 rows else: from six of that kernel's blocks of rows on
+// its workgroups come in twos to a CU, or with four blocks each (us, before / now: 128 x 2048 x 2048 5.8 / 4.9, 96 x 2560 x 2560 8.7 / 6.2,
+// 128 x 2560 x 2560 8.6 / 7.9).
+static inline bool kwaves_before_rows(long long M, long long N, long long K, int problems = 1) {
+  return M >= 96 && M <= 128 && K >= 2048 && K < 3072 && kwaves_pick(M, N, K, problems) != KWAVES_NONE;
+}
+
+template <int KIND, bool GROUPED>
+static int launch_kwaves(KWavesTile tile, const GemmParams& p, hipStream_t stream, const GemmGroup& grp = GemmGroup{}) {
+  g_last_form = "gemm_kwaves";
+  switch (tile) {
+    case KWAVES_32x32: return launch_kwaves_cfg<KWavesCfg<32, 32, 8, 2, KIND, GROUPED>>(p, stream, grp);
+    case KWAVES_32x64: return launch_kwaves_cfg<KWavesCfg<32, 64, 8, 1, KIND, GROUPED>>(p, stream, grp);
+    case KWAVES_48x64: return launch_kwaves_cfg<KWavesCfg<48, 64, 4, 2, KIND, GROUPED>>(p, stream, grp);
+    case KWAVES_64x64: return launch_kwaves_cfg<KWavesCfg<64, 64, 4, 2, KIND, GROUPED>>(p, stream, grp);
+    case KWAVES_64x80: return launch_kwaves_cfg<KWavesCfg<64, 80, 4, 2, KIND, GROUPED>>(p, stream, grp);
+    default: g_last_form = "gemm_kwaves pairs"; return launch_kwaves_cfg<KWavesCfg<64, 64, 2, 2, KIND, GROUPED>>(p, stream, grp);
+  }
+}
+
+static inline const char* kwaves_name(KWavesTile tile) {
+  return tile == KWAVES_32x32 ? "mid_waves_32x32" : tile == KWAVES_32x64 ? "mid_waves_32x64" : tile == KWAVES_48x64 ? "mid_waves_48x64"
+         : tile == KWAVES_64x80 ? "mid_waves_64x80" : "mid_waves_64x64";
+}
+
+}  // namespace ti

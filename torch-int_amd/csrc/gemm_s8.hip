@@ -530,6 +530,7 @@ int gemm_group_is_one_launch(long long M, long long N, long long K, int count) {
     if (rows.tiling != ROWS_NONE && rows.slices == 1) return 1;  // no workspace needed
   }
   if (M <= 16) return 0;
+  if (kwaves_pick(M, N, K, count) != KWAVES_NONE) return 1;
   return group_prefill_tile(M, N, K, count) != 0 ? 1 : 0;
 }
 
@@ -547,7 +548,8 @@ int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStrea
   const bool aligned = ptr_ok && (shape.K % SBK == 0) && shape.K > 0;
   const int spb = (shape.N + 15) / 16;
   const long long strips = (long long)spb * grp.count;
-  if (ptr_ok && shape.M <= TI_ROWS_ABREAST_M && shape.N % 4 == 0 && !(gemv_takes(shape) && strips >= 256)) {
+  if (ptr_ok && shape.M <= TI_ROWS_ABREAST_M && shape.N % 4 == 0 && !(gemv_takes(shape) && strips >= 256) &&
+      !kwaves_before_rows(shape.M, shape.N, shape.K, grp.count)) {
     const int rc = launch_rows<KIND, true>(shape, grp, grp.count, workspace, workspace_bytes, stream);
     if (rc >= 0) {
       if (rc == TI_OK) g_last_kernel = shape.M <= 16 ? "stream_group" : "mid_stream_group";
@@ -579,6 +581,13 @@ int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStrea
     if (shape.M <= 4) return launch(gemm_stream_kernel<KIND, 4, 2, true>, 2, 20, 3);
     return deep ? launch(gemm_stream_kernel<KIND, 16, 3, true>, 3, 32, 1)
                 : launch(gemm_stream_kernel<KIND, 16, 2, true>, 2, 32, 2);
+  }
+  if (ptr_ok && shape.lda == shape.K && shape.ldb == shape.K) {
+    const KWavesTile tile = kwaves_pick(shape.M, shape.N, shape.K, grp.count);
+    if (tile != KWAVES_NONE) {
+      g_last_kernel = "mid_waves_group";
+      return launch_kwaves<KIND, true>(tile, shape, stream, grp);
+    }
   }
   // Prefill shapes whose width the 256x160, 256x288, 256x256 or 256x128 tiles divide: the problems are the batches of one
   // persistent launch, so the pipeline fill and the epilogue of one projection overlap the next one's work.

@@ -2815,6 +2815,7 @@ static int batched_splits(long long batch, long long M, long long N, long long K
 #include "bmm_any.h"
 #include "bmm_scores.h"
 #include "gemm_rows.h"
+#include "gemm_kwaves.h"
 namespace ti {
 
 // Rows to cut off the end of a linear with many rows and run as a second, small problem (0 = none).
@@ -2925,7 +2926,7 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
   // K that 1024 does not divide, nor up to four rows of a short K (2 x 768 x 768: 3.1 us against the skinny kernel's 2.9) or up
   // to eight on fewer than 128 strips (5 x 768 x 768 3.34 against 3.20, 8 x 1200 x 768 3.63 / 3.43; 6 x 2048 x 768 level).
   if (p.M <= TI_ROWS_ABREAST_M && (p.N % 16 == 0 || p.K % SBK == 0) && stream_parts(p) == 1 && (p.M > 8 || p.K >= SBK || (p.M > 4 && p.N >= 2048)) &&
-      !(gemv_takes(p) && (p.N + 15) / 16 >= 256)) {
+      !(gemv_takes(p) && (p.N + 15) / 16 >= 256) && !(p.batch == 1 && kwaves_before_rows(p.M, p.N, p.K))) {
     const int rc = launch_rows<KIND, false>(p, GemmGroup{}, 1, workspace, workspace_bytes, stream);
     if (rc >= 0) {
       if (rc == TI_OK) g_last_kernel = p.M <= 16 ? "stream" : "mid_stream";
@@ -3012,6 +3013,13 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
   if ((p.lda > PANEL_MAX_LD || p.ldb > PANEL_MAX_LD) && p.K % PBK == 0) {
     g_last_kernel = "pipe_128x128";
     return launch_pipe<PipeCfg<128, 128, 2, 2, 4, KIND, SWAP>>(p, stream);
+  }
+  if constexpr (Epi<KIND>::kHasBias) {
+    const KWavesTile tile = p.batch == 1 && p.lda == p.K && p.ldb == p.K ? kwaves_pick(p.M, p.N, p.K) : KWAVES_NONE;
+    if (tile != KWAVES_NONE) {
+      g_last_kernel = kwaves_name(tile);
+      return launch_kwaves<KIND, false>(tile, p, stream);
+    }
   }
   if (p.batch > 1 && p.batch <= 65535 && p.lda == p.K && p.ldb == p.K && p.out_d == 0 && workspace != nullptr &&
       (reinterpret_cast<uintptr_t>(workspace) & 15) == 0) {
