@@ -24,7 +24,9 @@ def _name():
     (129, 3072, 768, "32x64"), (513, 768, 768, "32x64"), (65, 4096, 4096, "32x64"), (257, 2048, 2048, "48x64"), (384, 2048, 2048, "48x64"),
     (768, 768, 768, "48x64"), (129, 5120, 5120, "48x64"), (385, 2048, 2048, "64x64"), (512, 2048, 2048, "64x64"), (1280, 768, 3072, "64x64"),
     (193, 4096, 4096, "64x64"), (97, 10240, 2560, "64x80"), (497, 2560, 2560, "64x80"), (256, 5120, 5120, "64x80"),
-    (513, 2048, 2048, "64x64 pairs"), (1024, 2048, 2048, "64x64 pairs"), (129, 8192, 2048, "64x64 pairs"), (2047, 768, 3072, "64x64 pairs")])
+    (513, 2048, 2048, "96x64"), (768, 2048, 2048, "96x64"), (384, 3072, 768, "96x64"), (65, 16384, 4096, "96x64"), (289, 5120, 5120, "80x80"),
+    (640, 2560, 2560, "80x80"), (321, 5120, 5120, "96x80"), (96, 20480, 5120, "96x80"), (769, 2048, 2048, "128x64"), (1024, 2048, 2048, "128x64"),
+    (2047, 768, 3072, "128x64"), (128, 16384, 4096, "128x64")])
 def test_every_tile_is_exact(M, N, K, tile):
     import torch_int._CUDA as C
     import torch_int._hip_ext as X
@@ -53,7 +55,25 @@ def test_every_tile_is_exact(M, N, K, tile):
     assert _name() == "mid_waves_" + tile and torch.equal(got.cpu(), (old.float() + fresh.half().float()).half())
 
 
-@pytest.mark.parametrize("M,N,K", [(65, 2048, 2048), (127, 2048, 2048), (129, 2048, 2048), (319, 2048, 2048), (128, 2560, 2560), (66, 5120, 5120)])
+@pytest.mark.parametrize("M,N,K", [(257, 4096, 4096), (512, 4096, 4096), (320, 2048, 8192), (512, 2048, 8192), (384, 5120, 5120), (512, 768, 3072)])
+def test_accumulating_epilogues_of_257_to_512_rows(M, N, K):
+    import torch_int._CUDA as C
+    g = torch.Generator().manual_seed(M * 7 + N + K)
+    x, w, bf, resid = _s8(g, M, K).to(DEV), _s8(g, N, K).to(DEV), torch.randn(N, generator=g), torch.randn(M, N, generator=g) * 3
+    acc = torch.mm(x.double(), w.double().t().contiguous()).to(torch.int32).cpu()
+    print("accumulating, waves that share K", M, N, K, flush=True)
+    got = C._linear_a8_w8_bfp32_ofp32_acc(x, w, bf.to(DEV), 3e-4, 1.0, resid.to(DEV)).cpu()
+    assert _name().startswith("mid_waves_")
+    assert torch.equal(got, orc.linear_a8_w8_bfp32_ofp32_acc(x.cpu(), w.cpu(), bf, 3e-4, 1.0, resid, acc_fn=lambda *_: acc))
+    old = resid.half()
+    got = old.to(DEV)
+    _add_f16(x, w, bf.to(DEV), got, 3e-4)
+    assert _name().startswith("mid_waves_")
+    assert torch.equal(got.cpu(), (old.float() + orc.epi_bfp32_ofp32(acc, bf, 3e-4, 1.0).half().float()).half())
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 2048, 2048), (128, 2048, 2048), (191, 2048, 2048), (256, 2048, 2048), (257, 2048, 2048), (319, 2048, 2048),
+                                   (128, 2560, 2560), (255, 2560, 2560), (66, 5120, 5120), (128, 5120, 5120), (97, 4096, 4096)])
 def test_groups(M, N, K):
     import torch_int._hip_ext as X
     g = torch.Generator().manual_seed(M + N)
@@ -67,8 +87,8 @@ def test_groups(M, N, K):
         assert torch.equal(o.cpu(), orc.epi_b8_o8(acc, b, a, c)), (M, N, K)
 
 
-@pytest.mark.parametrize("M,N,K", [(64, 4096, 4096), (95, 2048, 2048), (1025, 2048, 2048), (257, 4096, 4096), (256, 2048, 8192), (512, 2560, 1024),
-                                   (128, 1024, 4096), (384, 3072, 768), (257, 768, 3072)])
+@pytest.mark.parametrize("M,N,K", [(64, 4096, 4096), (96, 2048, 2048), (1025, 2048, 2048), (257, 4096, 4096), (256, 2048, 8192), (512, 2560, 1024),
+                                   (128, 1024, 4096), (481, 3072, 768), (257, 768, 3072)])
 def test_where_it_ends(M, N, K):
     import torch_int._CUDA as C
     g = torch.Generator().manual_seed(M)

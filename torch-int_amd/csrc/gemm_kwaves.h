@@ -1,11 +1,11 @@
 // Linears of some 65 to 1024 rows whose output makes one round of small tiles: the waves of a workgroup share K, not the tile.
 //
-// A workgroup has one tile of 32x32 to 64x80 outputs over the whole of K, and each of its waves multiplies the WHOLE tile, over every
+// A workgroup has one tile of 32x32 to 128x64 outputs over the whole of K, and each of its waves multiplies the WHOLE tile, over every
 // NW-th step of 128 bytes.  So a wave's fragments serve as many products as the tile has (a 32x32 quarter of 64x64 reads twice the LDS
 // bytes a product), its panels lie in a ring of its own, and no wave waits for another until the integer sums of all of them are
 // added through the LDS at the end: no barrier in the loop, no slices of K that meet in memory, no second launch, no workspace.
 //
-// Bound by what the copies have in flight: a step's panels are (BM + BN) * 128 bytes for few products, 0.18 (32x32) to 0.33 us (64x80)
+// Bound by what the copies have in flight: a step's panels are (BM + BN) * 128 bytes for few products, 0.18 (32x32) to 0.42 us (128x64)
 // a step of the workgroup with weights from HBM, 0.11 (32x64) and 0.13 (64x64) with weights that the last-level cache holds, where the
 // copies of a CU alone take 0.08 and 0.11.  The tiled kernels that had these shapes take one step after the other, a barrier each, on a quarter
 // of the CUs (128x128 tiles), or park and add int32 slices.  Cold weights, us, before / now: 384 x 2048 x 2048 15.7 / 6.8, 512 x 2048 x 2048
@@ -29,7 +29,8 @@ struct KWavesCfg {
   static constexpr int TM = BM / 16, TN = BN / 16;
   static constexpr int STAGE = (BM + BN) * QBK;
   static constexpr int COPIES = STAGE / 1024;  // copy instructions a step: eight panel rows each
-  static constexpr int LDS_BYTES = NW * STAGES * STAGE;
+  static constexpr int RING = STAGES * STAGE;
+  static constexpr int LDS_BYTES = NW * RING;
   // units of the epilogue: 16 rows, halves of them where that leaves waves without one
   static constexpr int PARTS = TM < NW && TM <= 2 && TN % 2 == 0 ? 2 : 1;
   static constexpr int RESIDENT = 160 * 1024 / LDS_BYTES;  // workgroups to a CU
@@ -37,7 +38,7 @@ struct KWavesCfg {
   static_assert(BM % 16 == 0 && BN % 16 == 0, "blocks of 16x16");
   static_assert(STAGES >= 1 && STAGES <= 2, "the waits know of two");
   static_assert((STAGES - 1) * COPIES <= 63, "a wait counts in six bits");
-  static_assert(TM * TN * 1024 <= STAGES * STAGE, "a wave's sums go over its ring");
+  static_assert(TM * TN * 1024 <= RING, "a wave's sums go over its ring");
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
 };
 
@@ -72,7 +73,7 @@ __global__ __launch_bounds__(Cfg::NT, (Cfg::WAVES_PER_SIMD)) void gemm_kwaves_ke
   const int turn = tile_m * steps / tiles_m;
 
   // ---- copies: copy j of a step fills rows 8 j .. 8 j + 7 of [A panel | B panel], chunk c of row r at position c ^ ((r >> 1) & 7)
-  char* ring = smem + wave * (S * Cfg::STAGE);
+  char* ring = smem + wave * Cfg::RING;
   const int row = lane >> 3, pos = lane & 7;
   const unsigned sw[2] = {(unsigned)((pos ^ (lane >> 4)) << 4), (unsigned)((pos ^ (4 + (lane >> 4))) << 4)};  // of even and odd copies
   const unsigned a_row = (unsigned)row * (unsigned)p.lda, b_row = (unsigned)row * (unsigned)p.ldb;
@@ -154,7 +155,7 @@ __global__ __launch_bounds__(Cfg::NT, (Cfg::WAVES_PER_SIMD)) void gemm_kwaves_ke
 #pragma unroll
     for (int w = 1; w < NW; ++w)
 #pragma unroll
-      for (int j = 0; j < Unit::TN; ++j) sum[0][j] += *reinterpret_cast<const v4i*>(first + w * (S * Cfg::STAGE) + j * 1024);
+      for (int j = 0; j < Unit::TN; ++j) sum[0][j] += *reinterpret_cast<const v4i*>(first + w * Cfg::RING + j * 1024);
     store_tile16<Unit>(sum, q, 0, tile_m, tile_n, i, c, lane);
   }
 }
@@ -171,40 +172,49 @@ static int launch_kwaves_cfg(const GemmParams& p, hipStream_t stream, const Gemm
   return TI_OK;
 }
 
-enum KWavesTile { KWAVES_NONE = 0, KWAVES_32x32, KWAVES_32x64, KWAVES_48x64, KWAVES_64x64, KWAVES_64x80, KWAVES_64x64_PAIRS };
+enum KWavesTile {
+  KWAVES_NONE = 0, KWAVES_32x32, KWAVES_32x64, KWAVES_48x64, KWAVES_64x64, KWAVES_64x80, KWAVES_96x64, KWAVES_80x80, KWAVES_96x80, KWAVES_128x64,
+  KWAVES_64x64_PAIRS
+};
 
-// The tile of such a linear (or of `problems` of one shape in one launch), or none.  The smallest tile that is one round of the CUs: a smaller
-// one takes less a step, and the round is as long as its steps.  A second round costs as much as the first, or 0.9 times where two workgroups of two waves
-// share a CU (pairs), and larger tiles are ahead by then but for a short K (cold, us, the others / pairs): 1024 x 2048 x 2048 12.8 /
-// 11.0, 256 x 8192 x 2048 14.4 / 12.9, 2048 x 768 x 3072 16.8 / 13.3; not 768 x 2560 x 2560 15.9 / 15.8, 512 x 5120 x 5120 27 / 37, 512 x 3072 x 768 6.7 / 7.4).
-// Below five eighths of a round the CUs stand idle (128 x 1024 x 4096 on 32x32).
-// K: the copies of a tile grow with it, so beyond 8192 the slices are ahead (128 x 2560 x 10240 19.1 / 20, 256 x 4096 x 16384 34.6 / 34).
+// The tile of such a linear (or of `problems` of one shape in one launch), or none.  The first of the list that is one round of the CUs: a
+// step takes as long as the panel rows of its tile, and the round as long as its steps (us, 0.0022 a panel row and step and some 3.5).  Below
+// five eighths of a round the CUs stand idle (128 x 1024 x 4096 on 32x32), and in a second round larger tiles of other kernels are ahead (cold, us: 768 x
+// 4096 x 4096 24.5, 26.2 here), but for groups, whose other choice are problems one after the other: there, two workgroups of two waves share a CU (pairs;
+// three 300 x 2048 x 2048 19.2 apart, 13.2 so).  The tallest tiles are where the others walk K on few CUs, too: not for a short K (512 x 3072 x 768 7.3, on
+// 128x64 7.8) nor for a long one (1024 x 2048 x 8192 27.8, on 128x64 28.1); 128x80 are level with those others (128 x 20480 x 5120 32.7 / 32.2, 1024 x 2560 x 2560
+// 16.2 / 16.9).
+// K beyond 8192: the slices are ahead, or level (128 x 2560 x 10240 19.1 / 20, 256 x 4096 x 16384 34.6 / 34).
 // Widths: the measured ones, multiples of 2560 and 1024 (but for those that three divides, which have 192 and 288 columns wide tiles of their own), or of
-// 768 on both sides; K = 1024 and other widths stay with the kernels that had them, whose tests reach their forms there, and so do 257 to 512 rows of K from 3072 on, of which this kernel would take 0.6 to 0.85 of the time.
-static inline KWavesTile kwaves_pick(long long M, long long N, long long K, int problems = 1) {
-  if (M <= TI_ROWS_MAX_M || M > 4096 || N < 768 || N > 16384 || K > 8192) return KWAVES_NONE;
+// 768 on both sides; K = 1024 and other widths stay with the kernels that had them, whose tests reach their forms there, and so do 257 to 512 rows of K
+// from 3072 on without an accumulating epilogue, of which this kernel would take 0.6 to 0.9 of the time (multiples of 2560 do not).
+static inline KWavesTile kwaves_pick(long long M, long long N, long long K, bool accumulates, int problems = 1) {
+  if (M <= TI_ROWS_MAX_M || M > 4096 || N < 768 || N > 20480 || K > 8192) return KWAVES_NONE;
   if (problems > 1 && K < 2048) return KWAVES_NONE;
   const bool short_rows = N % 768 == 0 && K % 768 == 0 && K <= 3072;
   auto wide = [](long long w) { return w % 2560 == 0 || (w % 1024 == 0 && w % 3 != 0); };
   if (!short_rows && !(wide(N) && wide(K) && K >= 2048)) return KWAVES_NONE;
-  if (K >= 3072 && M > (K > 5120 ? 255 : 256) && M <= 512) return KWAVES_NONE;
+  if (!accumulates && K >= 3072 && N % 2560 != 0 && M > (K > 5120 ? 255 : 256) && M <= 512) return KWAVES_NONE;
   const long long cus = num_cus();
-  struct Form { KWavesTile tile; int bm, bn; };
-  static constexpr Form kForms[] = {{KWAVES_32x32, 32, 32}, {KWAVES_32x64, 32, 64}, {KWAVES_48x64, 48, 64}, {KWAVES_64x64, 64, 64}, {KWAVES_64x80, 64, 80}};
+  struct Form { KWavesTile tile; int bm, bn, k_from, k_to; };
+  static constexpr Form kForms[] = {
+      {KWAVES_32x32, 32, 32, 0, 8192}, {KWAVES_32x64, 32, 64, 0, 8192}, {KWAVES_48x64, 48, 64, 0, 8192}, {KWAVES_64x64, 64, 64, 0, 8192},
+      {KWAVES_64x80, 64, 80, 0, 8192}, {KWAVES_96x64, 96, 64, 0, 8192}, {KWAVES_80x80, 80, 80, 2048, 5120}, {KWAVES_96x80, 96, 80, 2048, 5120},
+      {KWAVES_128x64, 128, 64, 2048, 5120}};
   for (const Form& f : kForms) {
     if (N % f.bn != 0) continue;
     const long long tiles = (M + f.bm - 1) / f.bm * (N / f.bn) * problems;
-    if (tiles <= cus) return 8 * tiles >= 5 * cus ? f.tile : KWAVES_NONE;
+    if (tiles > cus || K < f.k_from || K > f.k_to) continue;
+    return 8 * tiles >= 5 * cus ? f.tile : KWAVES_NONE;
   }
-  const long long tiles = (M + 63) / 64 * (N / 64) * problems;
-  return tiles <= 2 * cus && K >= 2048 && (K <= 2048 || short_rows || problems > 1) ? KWAVES_64x64_PAIRS : KWAVES_NONE;
+  return problems > 1 && (M + 63) / 64 * (N / 64) * problems <= 2 * cus ? KWAVES_64x64_PAIRS : KWAVES_NONE;
 }
 
 // Whether it goes before the weight-streaming kernel, which has narrow outputs of more than 64 rows else: from six of that kernel's blocks of rows on
-// its workgroups come in twos to a CU, or with four blocks each (us, before / now: 128 x 2048 x 2048 5.8 / 4.9, 96 x 2560 x 2560 8.7 / 6.2,
+// its workgroups come in twos to a CU, or with four blocks each (us, before / now: 128 x 2048 x 2048 5.1 / 4.8, 96 x 2048 x 2048 4.7 / 4.9, 96 x 2560 x 2560 8.7 / 6.2,
 // 128 x 2560 x 2560 8.6 / 7.9).
 static inline bool kwaves_before_rows(long long M, long long N, long long K, int problems = 1) {
-  return M >= 96 && M <= 128 && K >= 2048 && K < 3072 && kwaves_pick(M, N, K, problems) != KWAVES_NONE;
+  return M > (N > 2048 ? 95 : 96) && M <= 128 && K >= 2048 && K < 3072 && kwaves_pick(M, N, K, false, problems) != KWAVES_NONE;
 }
 
 template <int KIND, bool GROUPED>
@@ -216,13 +226,23 @@ static int launch_kwaves(KWavesTile tile, const GemmParams& p, hipStream_t strea
     case KWAVES_48x64: return launch_kwaves_cfg<KWavesCfg<48, 64, 4, 2, KIND, GROUPED>>(p, stream, grp);
     case KWAVES_64x64: return launch_kwaves_cfg<KWavesCfg<64, 64, 4, 2, KIND, GROUPED>>(p, stream, grp);
     case KWAVES_64x80: return launch_kwaves_cfg<KWavesCfg<64, 80, 4, 2, KIND, GROUPED>>(p, stream, grp);
-    default: g_last_form = "gemm_kwaves pairs"; return launch_kwaves_cfg<KWavesCfg<64, 64, 2, 2, KIND, GROUPED>>(p, stream, grp);
+    case KWAVES_96x64: return launch_kwaves_cfg<KWavesCfg<96, 64, 4, 2, KIND, GROUPED>>(p, stream, grp);
+    case KWAVES_80x80: return launch_kwaves_cfg<KWavesCfg<80, 80, 4, 2, KIND, GROUPED>>(p, stream, grp);
+    case KWAVES_96x80: return launch_kwaves_cfg<KWavesCfg<96, 80, 3, 2, KIND, GROUPED>>(p, stream, grp);
+    case KWAVES_128x64: return launch_kwaves_cfg<KWavesCfg<128, 64, 3, 2, KIND, GROUPED>>(p, stream, grp);
+    default:
+      if constexpr (GROUPED) {
+        g_last_form = "gemm_kwaves pairs";
+        return launch_kwaves_cfg<KWavesCfg<64, 64, 2, 2, KIND, GROUPED>>(p, stream, grp);
+      }
+      return fail(TI_ERR_INVALID_ARG, "no tile for waves that share K");
   }
 }
 
 static inline const char* kwaves_name(KWavesTile tile) {
-  return tile == KWAVES_32x32 ? "mid_waves_32x32" : tile == KWAVES_32x64 ? "mid_waves_32x64" : tile == KWAVES_48x64 ? "mid_waves_48x64"
-         : tile == KWAVES_64x80 ? "mid_waves_64x80" : "mid_waves_64x64";
+  static constexpr const char* kNames[] = {"", "mid_waves_32x32", "mid_waves_32x64", "mid_waves_48x64", "mid_waves_64x64", "mid_waves_64x80", "mid_waves_96x64",
+                                           "mid_waves_80x80", "mid_waves_96x80", "mid_waves_128x64", "mid_waves_64x64"};
+  return kNames[tile];
 }
 
 }  // namespace ti

@@ -476,9 +476,10 @@ static int group_prefill_tile(long long M, long long N, long long K, int count) 
   // widths that only 128 divides (OPT-6.7B: 4096): 256x128 tiles, unless one problem at a time fills the CUs
   // with 256x256 tiles as well (three 2048x4096x4096: 98 -> 93 us, at 512 rows 57 -> 28 us; 2048x7168x7168
   // stays with three launches, 277 against 283 us)
+  // (the line at 0.48: three 768x2048x2048 on 144 tiles 19.0 us, apart 27.4; 512 rows, 96 tiles, 20 apart)
   const double e256_alone = fill(rows256 * ((N + 255) / 256));
   double e128 = N % 128 == 0 ? 0.87 * fill(rows256 * (N / 128) * count) : 0.0;
-  if (e128 < 0.5 || e128 <= e256_alone) e128 = 0.0;
+  if (e128 < 0.48 || e128 <= e256_alone) e128 = 0.0;
   const double e = e160 > e288 ? (e160 > e128 ? e160 : e128) : (e288 > e128 ? e288 : e128);
   // Beyond 1024 rows the grouped launch and the problems one after the other are priced as price_wide prices tilings, and
   // 256x256 tiles are in the race too.  Grouped, 256x128 and 256x160 tiles take 0.97 and 0.98 times their price and 256x256 ones
@@ -530,7 +531,7 @@ int gemm_group_is_one_launch(long long M, long long N, long long K, int count) {
     if (rows.tiling != ROWS_NONE && rows.slices == 1) return 1;  // no workspace needed
   }
   if (M <= 16) return 0;
-  if (kwaves_pick(M, N, K, count) != KWAVES_NONE) return 1;
+  if (kwaves_pick(M, N, K, false, count) != KWAVES_NONE) return 1;
   return group_prefill_tile(M, N, K, count) != 0 ? 1 : 0;
 }
 
@@ -583,7 +584,7 @@ int launch_gemm_group_s8(const GemmParams& shape, const GemmGroup& grp, hipStrea
                 : launch(gemm_stream_kernel<KIND, 16, 2, true>, 2, 32, 2);
   }
   if (ptr_ok && shape.lda == shape.K && shape.ldb == shape.K) {
-    const KWavesTile tile = kwaves_pick(shape.M, shape.N, shape.K, grp.count);
+    const KWavesTile tile = kwaves_pick(shape.M, shape.N, shape.K, false, grp.count);
     if (tile != KWAVES_NONE) {
       g_last_kernel = "mid_waves_group";
       return launch_kwaves<KIND, true>(tile, shape, stream, grp);

@@ -3015,7 +3015,7 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
     return launch_pipe<PipeCfg<128, 128, 2, 2, 4, KIND, SWAP>>(p, stream);
   }
   if constexpr (Epi<KIND>::kHasBias) {
-    const KWavesTile tile = p.batch == 1 && p.lda == p.K && p.ldb == p.K ? kwaves_pick(p.M, p.N, p.K) : KWAVES_NONE;
+    const KWavesTile tile = p.batch == 1 && p.lda == p.K && p.ldb == p.K ? kwaves_pick(p.M, p.N, p.K, Epi<KIND>::kAccumulate) : KWAVES_NONE;
     if (tile != KWAVES_NONE) {
       g_last_kernel = kwaves_name(tile);
       return launch_kwaves<KIND, false>(tile, p, stream);
