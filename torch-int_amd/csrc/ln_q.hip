@@ -29,9 +29,8 @@ namespace ti {
 enum LnMode : int { MODE_DQ_ADD = 0, MODE_ADD = 1, MODE_PLAIN = 2, MODE_ADD_F32 = 3 };
 
 // H % 4 == 0, H <= NC * 1024, all row starts 16-byte aligned.
-// EARLY: gamma and beta are fetched together with the row instead of after the two reductions; with only
-// a few rows in flight (decode) the kernel is a chain of memory latencies and this removes one of them,
-// with many rows the extra registers would only cost occupancy.
+// EARLY: gamma and beta are fetched together with the row instead of after the two reductions: a row is a chain of memory
+// latencies, and this removes one of them (where: launch_rows).
 template <int NC, int MODE, bool EARLY, class T>
 __global__ __launch_bounds__(256) void ln_q_rows_kernel(const void* __restrict__ in, float scale,
                                                         const T* res,  // may alias r_out
@@ -190,7 +189,13 @@ template <int NC, class T>
 static void launch_rows(int mode, const void* in, float scale, const T* res, const T* gamma, const T* beta, float eps,
                         T* r_out, int8_t* q_out, long long rows, int H, hipStream_t stream) {
   const dim3 grid((unsigned)rows), block(256);
-  const bool early = rows <= 64;  // fewer rows than CUs: latency-bound
+  // Gamma and beta with the row, us after / with it.  Up to a row to a CU there is nothing else to do: 192 x 2048 fp16 read only 2.36 / 2.22,
+  // 192 x 5120 with the int32 addend 4.36 / 4.02.  Many rows hide a latency behind one another, but not the two of a row that starts late:
+  // 2048 x 2048 fp16 with an addend 7.63 / 7.06, 2048 x 5120 read only 9.46 / 8.74, 4096 x 5120 15.0 / 13.5, 2048 x 2048 fp32 read only 6.03 / 5.45; an fp32
+  // stream with an addend is bound by HBM and stays (2048 x 5120 24.4 / 24.7).  Between them two to four rows start together on a CU, and the loads for gamma and beta of all stand before some rows':
+  // 512 x 2048 fp32 read only 2.96 / 3.25, 320 x 5120 fp32 with an addend 6.04 / 6.39; rows of up to 1024, of which a CU holds more: 832 x 768 2.69 / 2.80,
+  // 2048 x 768 fp16 with the int32 addend 4.95 / 4.87.
+  const bool early = rows <= compute_units() || ((mode == MODE_PLAIN || sizeof(T) == 2) && rows >= (NC == 1 ? 2048 : 1024));
 #define TI_LN_LAUNCH(MODE)                                                                                        \
   if (early)                                                                                                      \
     hipLaunchKernelGGL((ln_q_rows_kernel<NC, MODE, true, T>), grid, block, 0, stream, in, scale, res, gamma, beta, eps, \
