@@ -4,7 +4,8 @@
 // A lane reads a run of consecutive bytes of its row as the dwords they lie in, and shifts them into place: 16-byte loads at byte
 // addresses work but take 1.7 times as long (200 heads, 1 x 2003 x 128: 25.6 us, at multiples of 4 bytes 15.1).  Those dwords hold a
 // byte of the run each, so a load never touches memory that the operand does not share a dword with.  What is left of a row behind
-// its last whole step comes from the 16 bytes that end with the row (byte by byte where it is shorter), zeros behind it.
+// its last whole step comes from the 16 bytes that end with the row, or from the dwords of a shorter one (byte by byte, 5 x 152 x 80 x 15 took
+// 11.5 us, so 4.4), zeros behind it.
 // Against a thread to an output (below 2^26 products) or copies with a padded K (four launches, the operands' bytes twice over), us:
 // 18 x 130 x 64 x 130 25.5 -> 4.9, 100 x 301 x 80 x 301 32.7 -> 10.9, 160 x 517 x 128 x 517 77.4 -> 31.4, 32 x 2045 x 128 x 2045 142 -> 54;
 // the copies are ahead from about M N = 1024 (M + N) on (4 x 2048 x 2048 x 4097 133 us against 142), and the callers make them there.
@@ -24,8 +25,17 @@ __device__ __forceinline__ v4i row_chunk(const int8_t* row, int k, int K) {
     const unsigned __int128 bits = __builtin_bit_cast(unsigned __int128, last) >> (8 * (k + 16 - K));
     return __builtin_bit_cast(v4i, bits);
   }
-  for (int i = k; i < K; ++i) out[(i - k) >> 2] |= (int)(unsigned char)row[i] << (8 * ((i - k) & 3));
-  return out;
+  // rows shorter than a chunk (k = 0): the dwords that hold a byte of it, the last one again in the place of those behind
+  const unsigned shift = (unsigned)(reinterpret_cast<uintptr_t>(row) & 3);
+  const int* at = reinterpret_cast<const int*>(row - shift);
+  const int last = (int)(shift + K - 1) >> 2;
+  int d[5];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) d[i] = at[i < last ? i : last];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) out[v] = (int)__builtin_amdgcn_alignbyte((unsigned)d[v + 1], (unsigned)d[v], shift);
+  const int cut = 8 * (16 - K);
+  return __builtin_bit_cast(v4i, __builtin_bit_cast(unsigned __int128, out) << cut >> cut);
 }
 
 // 4 n consecutive bytes of a row from p on: the aligned dwords that hold them, one more than n where p is not aligned.
@@ -229,9 +239,57 @@ static int launch_any_tiles(const GemmParams& p, hipStream_t stream) {
 }
 
 template <int KIND>
+static int launch_scalar(const GemmParams& p, hipStream_t stream) {
+  const long long total = (long long)p.M * p.N;
+  const dim3 grid((unsigned)((total + 255) / 256), 1, p.batch);
+  hipLaunchKernelGGL(gemm_scalar_kernel<KIND>, grid, dim3(256), 0, stream, p);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
+  return TI_OK;
+}
+
+// Forms of such a product (ti_last_kernel_form; the family is "any_skinny" up to 16 rows, else "any").
+enum AnyForm { ANY_THREADS = 0, ANY_SKINNY, ANY_64x64, ANY_64x128, ANY_128x128 };
+static constexpr const char* kAnyForms[] = {"a thread to an output", "strips of 16", "64x64", "64x128", "128x128"};
+
+// Tiles: bound by latency and by what the steps of the workgroups of a CU take from one another, us a step of 128 bytes: 64x64 0.5 a
+// workgroup and 0.9 at least, 64x128 0.84 and 1.1, 128x128 1.38 and 1.4 (1001 bytes of K: 4 x 2000 x 2000 64.6 / 54.1 / 44.2 us on the
+// three; 2 x 1000 x 1000 x 5001 37.1 / 45.9 / 56.3; 18 x 130 x 64 x 130 4.9 / 6.6 / 9.3; 64 x 777 x 80 x 777 32.1 / 33.2 / 27.1).
+//
+// A short K of few outputs is a chain of a few latencies, which a thread to an output has fewer of: us, so / on the tiles 13 x 18 x 80 x 15
+// 3.0 / 4.4, 5 x 40 x 128 x 24 3.5 / 4.1, 3 x 33 x 80 x 33 4.25 / 4.26; on the strips 64 x 1 x 128 x 7 2.5 / 3.1, 4 x 1 x 128 x 20 3.0 / 3.0.  Beyond
+// that its time grows with every byte of every output: 61 x 61 outputs of 36 heads, K = 32, 9.9 / 4.7.  Fitted to 5517 products with K below 48:
+// 0.80 times the time of a thread to an output everywhere, and 1.004 times the better of the two.
+static inline AnyForm any_form(long long batch, long long M, long long N, long long K, int out_bytes, long long cus) {
+  const long long strips = (N + 15) / 16 * batch;
+  auto price = [&](int bm, int bn, int resident, double each, double least) {
+    const long long tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch, slots = cus * resident;
+    const long long rest = (tiles % slots + cus - 1) / cus;
+    const double last = rest == 0 ? 0.0 : rest * each > least ? rest * each : least;
+    return (double)(tiles / slots) * resident * each + last;
+  };
+  const double small = price(64, 64, 5, 0.5, 0.9), wide = price(64, 128, 3, 0.84, 1.1), large = price(128, 128, 2, 1.38, 1.4);
+  if (K > 0 && K < 48) {
+    auto longer = [](double a, double b) { return a > b ? a : b; };
+    const double steps = small < wide ? (small < large ? small : large) : wide < large ? wide : large;
+    const double outputs = (double)M * N * batch, threads = (double)((M * N + 255) / 256 * 256) * batch;
+    const double by_threads = longer(2.0 + 0.064 * K, 2.1 + threads * (0.77 + 0.74 * K) * 1e-6);
+    const double others = M <= 16  ? longer(3.0, 3.1 + strips * 4e-4)
+                          : K < 16 ? longer(4.2, 2.1 + 2.6 * steps + 1.5e-7 * outputs * out_bytes) * (1.0 + 1.0 / K)
+                                   : longer(4.3, 2.7 + 2.0 * steps + 2.1e-7 * outputs * out_bytes);
+    if (by_threads < 0.97 * others) return ANY_THREADS;
+  }
+  if (M <= 16) return ANY_SKINNY;
+  return small <= wide && small <= large ? ANY_64x64 : wide <= large ? ANY_64x128 : ANY_128x128;
+}
+
+template <int KIND>
 static int launch_any(const GemmParams& p, hipStream_t stream) {
-  if (p.M <= 16) {
-    g_last_kernel = "any_skinny";
+  const AnyForm form = any_form(p.batch, p.M, p.N, p.K, (int)sizeof(typename Epi<KIND>::Out), num_cus());
+  g_last_kernel = p.M <= 16 ? "any_skinny" : "any";
+  g_last_form = kAnyForms[form];
+  if (form == ANY_THREADS) return launch_scalar<KIND>(p, stream);
+  if (form == ANY_SKINNY) {
     const int strips = (p.N + 15) / 16;
     const long long items = (long long)strips * p.batch, grid = (items + 7) / 8 * 8;
     if (grid > 0x7fffffffLL) return fail(TI_ERR_INVALID_ARG, "too many output strips (%lld)", items);
@@ -246,20 +304,8 @@ static int launch_any(const GemmParams& p, hipStream_t stream) {
     if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
     return TI_OK;
   }
-  g_last_kernel = "any";
-  // Bound by latency and by what the steps of the workgroups of a CU take from one another, us a step of 128 bytes: 64x64 0.5 a
-  // workgroup and 0.9 at least, 64x128 0.84 and 1.1, 128x128 1.38 and 1.4 (1001 bytes of K: 4 x 2000 x 2000 64.6 / 54.1 / 44.2 us on the
-  // three; 2 x 1000 x 1000 x 5001 37.1 / 45.9 / 56.3; 18 x 130 x 64 x 130 4.9 / 6.6 / 9.3; 64 x 777 x 80 x 777 32.1 / 33.2 / 27.1).
-  const long long cus = num_cus();
-  auto price = [&](int bm, int bn, int resident, double each, double least) {
-    const long long tiles = (long long)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) * p.batch, slots = cus * resident;
-    const long long rest = (tiles % slots + cus - 1) / cus;
-    const double last = rest == 0 ? 0.0 : rest * each > least ? rest * each : least;
-    return (double)(tiles / slots) * resident * each + last;
-  };
-  const double small = price(64, 64, 5, 0.5, 0.9), wide = price(64, 128, 3, 0.84, 1.1), large = price(128, 128, 2, 1.38, 1.4);
-  if (small <= wide && small <= large) return launch_any_tiles<AnyCfg<64, 64, KIND>>(p, stream);
-  if (wide <= large) return launch_any_tiles<AnyCfg<64, 128, KIND>>(p, stream);
+  if (form == ANY_64x64) return launch_any_tiles<AnyCfg<64, 64, KIND>>(p, stream);
+  if (form == ANY_64x128) return launch_any_tiles<AnyCfg<64, 128, KIND>>(p, stream);
   return launch_any_tiles<AnyCfg<128, 128, KIND>>(p, stream);
 }
 

@@ -2275,8 +2275,8 @@ static int skinny_waves(const GemmParams& p) {
   return (int)nw;
 }
 
-// Any-shape fallback of the linears (K not a multiple of 16 or operands not 16-byte aligned; batched products: bmm_any.h):
-// one thread per output element, scalar loop over K.
+// Any-shape fallback of the linears (K not a multiple of 16 or operands not 16-byte aligned; of batched products those of a short K
+// and few outputs, see bmm_any.h): one thread per output element, scalar loop over K.
 template <int KIND>
 __global__ __launch_bounds__(256) void gemm_scalar_kernel(GemmParams p) {
   using E = Epi<KIND>;
@@ -2910,12 +2910,7 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
       return launch_any<KIND>(p, stream);
     } else {
       g_last_kernel = "scalar";
-      const long long total = (long long)p.M * p.N;
-      dim3 grid((unsigned)((total + 255) / 256), 1, p.batch);
-      hipLaunchKernelGGL(gemm_scalar_kernel<KIND>, grid, dim3(256), 0, stream, p);
-      hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
-      return TI_OK;
+      return launch_scalar<KIND>(p, stream);
     }
   }
   if constexpr (KIND == EPI_F32_SCALE || KIND == EPI_S32_RAW) {

@@ -191,12 +191,17 @@ def _pad_inner(a, b, K):
     return torch.nn.functional.pad(a, (0, pad)), _padded_weight(b, pad), K + pad
 
 
-def _pad_products(a, b, batch, M, N, K):
+def _pad_products(a, b, batch, M, N, K, out_bytes):
     """Batched products with such a K have kernels that read rows where they lie (csrc/bmm_any.h).  Copies padded as above
-    are ahead of those only where the products are many to a byte, or where K is long enough to be cut into slices."""
+    are ahead of those only where the products are many to a byte (4 x 2048 x 2048 x 4097; a short K sooner: 64 x 1664 x 1664 x 25
+    int8 95 us against 152), where K is long enough to be cut into slices, or where K is at most 128 and the outputs are
+    many and of 32 bits, which then leave as whole lines (21 x 1958 x 1958 x 17 117 us against 206, 19 x 1319 x 2039 x 100
+    77 / 124; 708 products of 2^26 and more: the line is 1.02 times the better of the two)."""
     pad = -K % 64
-    if K % 16 == 0 or batch * M * N * K < (1 << 26) or not (
-            M * N >= 1024 * (M + N) or (K >= 2048 and M > 16 and _bmm_ws_bytes(batch, M, N, K + pad) > 0)):
+    if K % 16 == 0 or batch * M * N * K < (1 << 26):
+        return a, b, K
+    scores = out_bytes == 4 and K <= 128 and 4 * batch * M * N >= 24000000 and M * N >= 100 * (M + N)
+    if not (scores or M * N >= (700 if K < 32 else 1024) * (M + N) or (K >= 2048 and M > 16 and _bmm_ws_bytes(batch, M, N, K + pad) > 0)):
         return a, b, K
     return torch.nn.functional.pad(a, (0, pad)), torch.nn.functional.pad(b, (0, pad)), K + pad
 
@@ -319,7 +324,7 @@ def _bmm(op, kind, a, b, out_dtype, alpha):
     if out.numel() == 0:
         return out
     if K & 15:
-        a, b, K = _pad_products(a, b, batch, M, N, K)
+        a, b, K = _pad_products(a, b, batch, M, N, K, out.element_size())
     idx = dev.index
     switch = idx != _current_device()
     if switch:
