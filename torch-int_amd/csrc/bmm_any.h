@@ -72,10 +72,11 @@ struct Run {
 };
 
 // Work item of a workgroup: the ids congruent modulo 8 share an XCD, whose L2 then keeps the operand that the tiles of a batch
-// have in common.  -1 for the ids beyond the last item (the grid is a multiple of 8).
+// have in common.  -1 for the ids beyond the last item (the grid is a multiple of 8, xcd_grid).
+static constexpr int XCD_ROW_BITS = 20;
 __device__ __forceinline__ long long item_on_xcd(long long items) {
-  const long long per = (items + 7) / 8, item = (long long)(blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  return (long long)(blockIdx.x >> 3) < per && item < items ? item : -1;
+  const long long id = ((long long)blockIdx.y << XCD_ROW_BITS) + blockIdx.x, per = (items + 7) / 8, item = (id & 7) * per + (id >> 3);
+  return (id >> 3) < per && item < items ? item : -1;
 }
 
 // Tiles of BM x BN on four waves (2 x 2), K in steps of 128 bytes through registers into two LDS stages; rows as in
@@ -227,12 +228,22 @@ __global__ __launch_bounds__(1024) void gemm_any_skinny_kernel(GemmParams p, int
 
 // ------------------------------------------------------------------ host side
 
+// The grid of so many items: one row, or rows of 2^20 workgroups where one would have 2^32 threads or more, of which a launch starts only the
+// remainder, without an error (65535 batches of 16448 x 1 outputs: 65280 of 16.8 million workgroups).
+static inline int xcd_grid(long long items, int threads, dim3& grid) {
+  const long long groups = (items + 7) / 8 * 8, rows = (groups >> XCD_ROW_BITS) + 1;
+  if (groups * threads < 1LL << 32) grid = dim3((unsigned)groups);
+  else if (rows <= 65535) grid = dim3(1u << XCD_ROW_BITS, (unsigned)rows);
+  else return fail(TI_ERR_INVALID_ARG, "too many output tiles (%lld)", items);
+  return TI_OK;
+}
+
 template <class Cfg>
 static int launch_any_tiles(const GemmParams& p, hipStream_t stream) {
   const int tiles_m = (p.M + Cfg::BM - 1) / Cfg::BM, tiles_n = (p.N + Cfg::BN - 1) / Cfg::BN;
-  const long long items = (long long)tiles_m * tiles_n * p.batch, grid = (items + 7) / 8 * 8;
-  if (grid > 0x7fffffffLL) return fail(TI_ERR_INVALID_ARG, "too many output tiles (%lld)", items);
-  hipLaunchKernelGGL(gemm_any_kernel<Cfg>, dim3((unsigned)grid), dim3(Cfg::NT), Cfg::LDS_BYTES, stream, p, tiles_m, tiles_n);
+  dim3 grid;
+  if (int rc = xcd_grid((long long)tiles_m * tiles_n * p.batch, Cfg::NT, grid)) return rc;
+  hipLaunchKernelGGL(gemm_any_kernel<Cfg>, grid, dim3(Cfg::NT), Cfg::LDS_BYTES, stream, p, tiles_m, tiles_n);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
   return TI_OK;
@@ -291,14 +302,15 @@ static int launch_any(const GemmParams& p, hipStream_t stream) {
   if (form == ANY_THREADS) return launch_scalar<KIND>(p, stream);
   if (form == ANY_SKINNY) {
     const int strips = (p.N + 15) / 16;
-    const long long items = (long long)strips * p.batch, grid = (items + 7) / 8 * 8;
-    if (grid > 0x7fffffffLL) return fail(TI_ERR_INVALID_ARG, "too many output strips (%lld)", items);
+    const long long items = (long long)strips * p.batch;
     // waves to cover the latency of the loads, each with a block of K at least
     long long waves = (4096 + items - 1) / items;
     const long long most = (p.K + 255) / 256;
     waves = waves > most ? most : waves;
     waves = waves > 16 ? 16 : waves < 1 ? 1 : waves;
-    hipLaunchKernelGGL(gemm_any_skinny_kernel<KIND>, dim3((unsigned)grid), dim3((unsigned)(64 * waves)),
+    dim3 grid;
+    if (int rc = xcd_grid(items, (int)(64 * waves), grid)) return rc;
+    hipLaunchKernelGGL(gemm_any_skinny_kernel<KIND>, grid, dim3((unsigned)(64 * waves)),
                        (size_t)(waves - 1) * 1024, stream, p, strips);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));

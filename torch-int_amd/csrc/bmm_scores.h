@@ -161,9 +161,9 @@ template <int KIND, int KB>
 static int launch_scores_k(const GemmParams& p, hipStream_t stream) {
   auto launch = [&](auto kern, int bm, int bn, int each) -> int {
     const int tiles_m = (p.M + bm - 1) / bm, tiles_n = (p.N + bn - 1) / bn;
-    const long long groups = ((long long)tiles_m * tiles_n * p.batch + each - 1) / each, grid = (groups + 7) / 8 * 8;
-    if (grid > 0x7fffffffLL) return fail(TI_ERR_INVALID_ARG, "too many output tiles (%lld)", groups * each);
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), 0, stream, p, tiles_m, tiles_n);
+    dim3 grid;
+    if (int rc = xcd_grid(((long long)tiles_m * tiles_n * p.batch + each - 1) / each, 256, grid)) return rc;
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, p, tiles_m, tiles_n);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
     return TI_OK;
