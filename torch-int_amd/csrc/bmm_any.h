@@ -284,7 +284,7 @@ static inline AnyForm any_form(long long batch, long long M, long long N, long l
     auto longer = [](double a, double b) { return a > b ? a : b; };
     const double steps = small < wide ? (small < large ? small : large) : wide < large ? wide : large;
     const double outputs = (double)M * N * batch, threads = (double)((M * N + 255) / 256 * 256) * batch;
-    const double by_threads = longer(2.0 + 0.064 * K, 2.1 + threads * (0.77 + 0.74 * K) * 1e-6);
+    const double by_threads = longer((M <= 16 ? 1.75 : 2.0) + 0.064 * K, 2.1 + threads * (0.77 + 0.74 * K) * 1e-6);
     const double others = M <= 16  ? longer(3.0, 3.1 + strips * 4e-4)
                           : K < 16 ? longer(4.2, 2.1 + 2.6 * steps + 1.5e-7 * outputs * out_bytes) * (1.0 + 1.0 / K)
                                    : longer(4.3, 2.7 + 2.0 * steps + 2.1e-7 * outputs * out_bytes);
