@@ -81,7 +81,7 @@ const char* ti_last_kernel(void);
 /* Diagnostics: which of the pipelined kernels that was, where one family has several ("pipe_128x128", "pipe_256x256" and
  * "splitk_128x128"): "gemm_pipe" (64-byte steps), "gemm_pipe2" (128-byte steps, 32x32 blocks), "gemm_pipe16" and "gemm_pipe16q" (64-
  * and 128-byte steps, 16x16 blocks); of "any" and "any_skinny" the tile ("64x64", "64x128", "128x128"), "strips of 16" or "a thread to
- * an output"; "" for the others.  Of two problems or launches, the last product's. */
+ * an output", of "scores" "16x32 to a wave", "32x32 to a wave", "rows through the LDS" or that with ", non-temporal stores"; "" for the others.  Of two problems or launches, the last product's. */
 const char* ti_last_kernel_form(void);
 
 /* Diagnostic: what the calling thread's last linear or group did in the weight-streaming kernel of few rows: 0 = it

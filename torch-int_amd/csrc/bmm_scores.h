@@ -147,14 +147,52 @@ __global__ __launch_bounds__(256) void gemm_scores_lds_kernel(GemmParams p, int 
 // with plain stores, 85 with these.
 static inline bool scores_stream(const GemmParams& p) { return (double)p.M * p.N * p.batch > 64e6 && p.N % 32 == 0; }
 
+// Sizes that the tiled kernels had before these, and on which they are ahead (us, tiles / so).
+static inline bool scores_left(long long batch, long long M, long long N, long long K, long long cus) {
+  const long long t64 = (M + 63) / 64 * ((N + 63) / 64) * batch, t128 = (M + 127) / 128 * ((N + 127) / 128) * batch;
+  const long long t256 = (M + 255) / 256 * ((N + 255) / 256) * batch;
+  const double outputs = (double)M * N * batch;
+  // Rows of more than 96 bytes on 64x64 tiles.  A small wave loads three times the bytes an output, which queue from a second wave to a SIMD on
+  // at K = 128 (1 x 1151 x 1151 4.03 / 5.09, 65 x 116 x 116 3.76 / 4.56, 6 x 305 x 305 3.41 / 3.81; with one to a SIMD ahead, 8 x 244 x 244 3.41 / 3.16); rows
+  // through the LDS are then few workgroups of 128x128 (12 x 368 x 368 x 128 4.21 / 5.45).  Not where most of those tiles is padding.
+  if (K > 96 && 2 * t128 < cus) {
+    if (K > 112 && (M + 15) / 16 * ((N + 31) / 32) * batch > 4 * cus && outputs > 0.5 * 4096.0 * (double)t64) return true;
+    if (outputs > 1.6e6) return true;
+  }
+  // K that 64 does not divide, rows of whole lines: one round of 256x256 tiles with the same padding as four of 128x128 each, more than a
+  // quarter of it (204 x 160 x 160 x 80 10.6 / 12.3, 228 x 223 x 192 x 80 12.4 / 13.1; full ones 16 x 1024 x 1024 x 112 14.9 / 13.6).  (128x128 tiles
+  // that fill two to a CU would have some 5 % as well: 5 x 1217 x 1216 x 80 8.69 / 9.36; 27 x 512 x 512 x 80, which stays,
+  // 8.67 / 8.81.)
+  if (K > 64 && K % 64 != 0 && N % 32 == 0 && 4 * t256 > 3 * cus && t256 <= cus && t128 == 4 * t256 &&
+      outputs < 0.72 * 65536.0 * (double)t256)
+    return true;
+  return false;
+}
+
 // Whether the problem is one of these (operands in aligned 16-byte chunks; the caller checked that).  Not a few hundred keys of many
 // heads that fill most of that cache, in whole lines and whole steps of the persistent tiles: alone the scores are ahead here too, but they
-// leave more of it dirty to the product behind them (scores, then P.V, us, tiles / scores: 160 x 512 x 512 x 128 53.8 / 56.3,
-// 160 x 448 x 448 x 128 49.1 / 51.8; 64 x 768 x 768 x 64 48.8 / 48.8, with the softmax 80.9 / 75.0).
+// leave more of it dirty to the launch behind them.  Scores and P.V, and with the softmax between them, us, tiles / scores: 160 x 512 x 512 x 128
+// 51.6 / 57.0 and 83.1 / 89.0, 226 x 448 x 448 x 64 60.3 / 64.5 and 98.8 / 104.3, 286 x 448 x 448 x 128 91.1 / 94.0 and 148 / 145; others of
+// these sizes would be ahead, the smaller and those whose last round of tiles is short: 160 x 448 x 448 x 128 72.7 / 68.1 with the softmax, 120 x 576 x 576 x 128
+// 107 / 82, 240 x 384 x 384 x 64 80.9 / 74.5.
 static inline bool scores_take(const GemmParams& p) {
   if (p.M <= 16 || p.K <= 0 || p.K > 128 || p.lda != p.K || p.ldb != p.K || p.out_d != 0) return false;
   if (p.N == 128 && p.K == 128 && p.M >= 512 && (long long)((p.M + 255) / 256) * p.batch >= 2 * num_cus()) return false;  // tiles of 256x128: launch_kind
-  return !((double)p.M * p.N * p.batch > 30e6 && !scores_stream(p) && p.N % 32 == 0 && p.K % 64 == 0 && p.M > 128 && p.N > 128 && p.N < 640);
+  if ((double)p.M * p.N * p.batch > 30e6 && !scores_stream(p) && p.N % 32 == 0 && p.K % 64 == 0 && p.M > 128 && p.N > 128 && p.N < 640) return false;
+  return !scores_left(p.batch, p.M, p.N, p.K, num_cus());
+}
+
+enum ScoresForm { SCORES_16x32 = 0, SCORES_32x32, SCORES_LDS, SCORES_LDS_STREAM };
+static constexpr const char* kScoresForms[] = {"16x32 to a wave", "32x32 to a wave", "rows through the LDS", "rows through the LDS, non-temporal stores"};
+
+// Few outputs: the smallest waves, up to two to a SIMD (13 x 158 x 158 x 64 2.9 us, with 32 x 32 outputs to a wave 3.2, through the LDS
+// 4.8; 132 x 120 x 120 x 64, four to a SIMD, 4.9 / 4.7 / 6.0).  Then 32 x 32 while the bytes loaded for each output weigh less than the LDS
+// and its barrier, the sooner the longer K: 213 x 341 x 341 x 64 19.3, through the LDS 20.2, 243 x 667 x 667 x 64 157 / 131; 20 x 462 x 462 x 80
+// 7.7 / 8.0, 13 x 741 x 741 x 80 9.8 / 9.5; 24 x 256 x 256 x 128 5.3 / 5.7, 245 x 87 x 87 x 128 7.0 / 6.3.
+static inline ScoresForm scores_form(const GemmParams& p) {
+  if ((long long)((p.M + 15) / 16) * ((p.N + 31) / 32) * p.batch <= 8LL * num_cus()) return SCORES_16x32;
+  if ((double)p.M * p.N * p.batch <= (p.K <= 64 ? 24e6 : p.K <= 96 ? 5e6 : 1.6e6)) return SCORES_32x32;
+  return scores_stream(p) ? SCORES_LDS_STREAM : SCORES_LDS;
 }
 
 template <int KIND, int KB>
@@ -168,15 +206,12 @@ static int launch_scores_k(const GemmParams& p, hipStream_t stream) {
     if (e != hipSuccess) return fail(TI_ERR_LAUNCH, "gemm launch: %s", hipGetErrorString(e));
     return TI_OK;
   };
-  // Few outputs: the smallest waves, up to two to a SIMD (13 x 158 x 158 x 64 2.9 us, with 32 x 32 outputs to a wave 3.2, through the LDS
-  // 4.8; 132 x 120 x 120 x 64, four to a SIMD, 4.9 / 4.7 / 6.0).  Then 32 x 32 while the bytes loaded for each output weigh less than the LDS
-  // and its barrier, the sooner the longer K: 213 x 341 x 341 x 64 19.3, through the LDS 20.2, 243 x 667 x 667 x 64 157 / 131; 20 x 462 x 462 x 80
-  // 7.7 / 8.0, 13 x 741 x 741 x 80 9.8 / 9.5; 24 x 256 x 256 x 128 5.3 / 5.7, 245 x 87 x 87 x 128 7.0 / 6.3.
-  if ((long long)((p.M + 15) / 16) * ((p.N + 31) / 32) * p.batch <= 8LL * num_cus())
-    return launch(gemm_scores_kernel<KIND, KB, 1, 2>, 16, 32, 4);
-  if ((double)p.M * p.N * p.batch <= (p.K <= 64 ? 24e6 : p.K <= 96 ? 5e6 : 1.6e6)) return launch(gemm_scores_kernel<KIND, KB, 2, 2>, 32, 32, 4);
-  return scores_stream(p) ? launch(gemm_scores_lds_kernel<KIND, KB, true>, 128, 128, 1)
-                          : launch(gemm_scores_lds_kernel<KIND, KB, false>, 128, 128, 1);
+  const ScoresForm form = scores_form(p);
+  g_last_form = kScoresForms[form];
+  if (form == SCORES_16x32) return launch(gemm_scores_kernel<KIND, KB, 1, 2>, 16, 32, 4);
+  if (form == SCORES_32x32) return launch(gemm_scores_kernel<KIND, KB, 2, 2>, 32, 32, 4);
+  return form == SCORES_LDS_STREAM ? launch(gemm_scores_lds_kernel<KIND, KB, true>, 128, 128, 1)
+                                   : launch(gemm_scores_lds_kernel<KIND, KB, false>, 128, 128, 1);
 }
 
 template <int KIND>
