@@ -49,6 +49,12 @@ struct KWavesUnit {
   static constexpr int TM = 1, TN = Cfg::TN / Cfg::PARTS, WTM = 16, WTN = TN * 16;
 };
 
+// Four consecutive columns of an fp32 output or bias; single values where it does not begin on 16 bytes.
+__device__ __forceinline__ v4f load_f32x4(const float* at, bool aligned) {
+  if (aligned) return *reinterpret_cast<const v4f*>(at);
+  return v4f{at[0], at[1], at[2], at[3]};
+}
+
 template <class Cfg>
 __global__ __launch_bounds__(Cfg::NT, (Cfg::WAVES_PER_SIMD)) void gemm_kwaves_kernel(GemmParams p, int tiles_m, int tiles_n,
                                                                                      GemmGroup grp) {
@@ -131,12 +137,63 @@ __global__ __launch_bounds__(Cfg::NT, (Cfg::WAVES_PER_SIMD)) void gemm_kwaves_ke
         for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[s][j], fa[s][i], acc[i][j], 0, 0, 0);
   }
 
+  // What an fp32 tile that is added to holds, and the bias: of all units of a wave at once, on their way while the sums meet.  Fetched unit
+  // by unit behind the sums (store_tile16), each waited for memory by itself, three times on the tallest tiles: warm weights, us, so / on 64x64 tiles over the
+  // whole of K, which these rows had before / now: 804 x 2048 x 2048 14.7 / 12.1 / 11.3, 324 x 3072 x 768 8.7 / 7.8 / 6.2, 300 x 4096 x 4096 13.9, now 11.5.
+  using E = Epi<Cfg::KIND>;
+  using Unit = KWavesUnit<Cfg>;
+  constexpr bool ADDS_F32 = E::kAccumulate && sizeof(typename E::Out) == 4;
+  constexpr int UNITS = ADDS_F32 ? (TM * Cfg::PARTS + NW - 1) / NW : 1;  // of a wave, one column part
+  static_assert(NW % Cfg::PARTS == 0, "a wave's units have the same columns");
+  const bool vec_ok = (reinterpret_cast<uintptr_t>(p.C) & 15) == 0 && (reinterpret_cast<uintptr_t>(p.bias) & 15) == 0;
+  const int col = n0 + wave % Cfg::PARTS * Unit::WTN + 4 * g;  // whole columns (kwaves_pick)
+  auto unit_at = [&](int k, int j) {
+    const int m = m0 + (wave + k * NW) / Cfg::PARTS * 16 + r;
+    return static_cast<float*>(p.C) + out_index(p, m < p.M ? m : p.M - 1, col + j * 16);
+  };
+  v4f old[UNITS][Unit::TN], bias[Unit::TN];
+  if constexpr (ADDS_F32) {
+#pragma unroll
+    for (int j = 0; j < Unit::TN; ++j) {
+      bias[j] = load_f32x4(static_cast<const float*>(p.bias) + col + j * 16, vec_ok);
+#pragma unroll
+      for (int k = 0; k < UNITS; ++k) old[k][j] = load_f32x4(unit_at(k, j), vec_ok);  // rows beyond the last: row M - 1, not used
+    }
+  }
+
   // ---- the waves' sums, over the rings (every copy of this wave has landed and been read)
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) *reinterpret_cast<v4i*>(ring + ((i * TN + j) * 64 + lane) * 16) = acc[i][j];
   __syncthreads();
+  if constexpr (ADDS_F32) {
+#pragma unroll
+    for (int k = 0; k < UNITS; ++k) {
+      const int u = wave + k * NW, i = u / Cfg::PARTS, c = u - i * Cfg::PARTS;
+      if (u >= TM * Cfg::PARTS || m0 + 16 * i >= p.M) break;
+      const char* first = smem + ((i * TN + c * Unit::TN) * 64 + lane) * 16;
+#pragma unroll
+      for (int j = 0; j < Unit::TN; ++j) {
+        v4i sum = *reinterpret_cast<const v4i*>(first + j * 1024);
+#pragma unroll
+        for (int w = 1; w < NW; ++w) sum += *reinterpret_cast<const v4i*>(first + w * Cfg::RING + j * 1024);
+        v4f out;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) out[v] = old[k][j][v] + E::apply(sum[v], E::bias_term(bias[j][v], p.beta), p.alpha);
+        if (m0 + 16 * i + r < p.M) {
+          float* at = unit_at(k, j);
+          if (vec_ok) {
+            *reinterpret_cast<v4f*>(at) = out;
+          } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) at[v] = out[v];
+          }
+        }
+      }
+    }
+    return;
+  }
   GemmParams q = p;
   if constexpr (Cfg::GROUPED) {
     q.bias = grp.bias[b];
@@ -144,7 +201,6 @@ __global__ __launch_bounds__(Cfg::NT, (Cfg::WAVES_PER_SIMD)) void gemm_kwaves_ke
     q.alpha = grp.alpha[b];
     q.beta = grp.beta[b];
   }
-  using Unit = KWavesUnit<Cfg>;
   for (int u = wave; u < TM * Cfg::PARTS; u += NW) {
     const int i = u / Cfg::PARTS, c = u - i * Cfg::PARTS;
     if (m0 + 16 * i >= p.M) break;
