@@ -233,6 +233,26 @@ enum KWavesTile {
   KWAVES_64x64_PAIRS
 };
 
+// Wide outputs of a long K on which the kernels that had them are ahead, if only with weights that the last-level cache holds: several rows
+// of tiles read the same long rows of weights, and the tallest tiles have few copies in flight for them.  us, those / so, cold and warm weights:
+// 40 million weights of a K beyond 5120 160 x 7168 x 7680 25.2 / 27.1 and 22.4 / 23.6, in the mean of 65 to 192 rows of 7168 to 8192 on both sides 1.05 and
+// 1.08 times the time.  80 columns 240 x 5120 x 7680 23.8 / 25.4 and 20.7 / 24.6, 150 x 10240 x 5120 23.2 / 23.7 and 19.5 / 22.1, 100 rows 21.5 / 20.5 and
+// 17.5 / 19.3, 70 x 17920 x 2560 15.9 / 15.5 and 12.6 / 13.6, 700 x 2560 x 2048 10.7 / 11.2 and 10.7 / 10.7.  64 columns of widths that 2560 does not divide 120 x 13312 x
+// 5120 24.5 / 26.0 and 19.8 / 19.7.  One row of 80x80 or 96x80 tiles of 17920 and 20480 columns at K = 5120 stays: 96 x 20480 x 5120 28.8 / 28.3 and 20.2 / 22.3.
+// (The epilogue that adds to fp32 is ahead on nearly all of them: its slices do not meet in one launch.)
+static inline bool kwaves_behind(KWavesTile tile, long long N, long long K) {
+  if (K > 5120 && N * K >= 40000000) return true;
+  switch (tile) {
+    case KWAVES_64x80: return K > 7168 || (K > 4096 && N > 5120);
+    case KWAVES_96x80:
+      if (K < 2560) return true;
+      [[fallthrough]];
+    case KWAVES_80x80: return N > 5120 && (N <= 10240 ? K > 2560 : K <= 4096);
+    case KWAVES_128x64: return K > 4096 && N > 5120 && N % 2560 != 0;
+    default: return false;
+  }
+}
+
 // The tile of such a linear (or of `problems` of one shape in one launch), or none.  The first of the list that is one round of the CUs: a
 // step takes as long as the panel rows of its tile, and the round as long as its steps (us, 0.0022 a panel row and step and some 3.5).  Below
 // five eighths of a round the CUs stand idle (128 x 1024 x 4096 on 32x32), and in a second round larger tiles of other kernels are ahead (cold, us: 768 x
@@ -244,7 +264,7 @@ enum KWavesTile {
 // Widths: the measured ones, multiples of 2560 and 1024 (but for those that three divides, which have 192 and 288 columns wide tiles of their own), or of
 // 768 on both sides; K = 1024 and other widths stay with the kernels that had them, whose tests reach their forms there, and so do 257 to 512 rows of K
 // from 3072 on without an accumulating epilogue, of which this kernel would take 0.6 to 0.9 of the time (multiples of 2560 do not).
-static inline KWavesTile kwaves_pick(long long M, long long N, long long K, bool accumulates, int problems = 1) {
+static inline KWavesTile kwaves_pick(long long M, long long N, long long K, bool accumulates, int problems = 1, bool adds_f32 = false) {
   if (M <= TI_ROWS_MAX_M || M > 4096 || N < 768 || N > 20480 || K > 8192) return KWAVES_NONE;
   if (problems > 1 && K < 2048) return KWAVES_NONE;
   const bool short_rows = N % 768 == 0 && K % 768 == 0 && K <= 3072;
@@ -261,6 +281,7 @@ static inline KWavesTile kwaves_pick(long long M, long long N, long long K, bool
     if (N % f.bn != 0) continue;
     const long long tiles = (M + f.bm - 1) / f.bm * (N / f.bn) * problems;
     if (tiles > cus || K < f.k_from || K > f.k_to) continue;
+    if (problems == 1 && !adds_f32 && kwaves_behind(f.tile, N, K)) return KWAVES_NONE;
     return 8 * tiles >= 5 * cus ? f.tile : KWAVES_NONE;
   }
   return problems > 1 && (M + 63) / 64 * (N / 64) * problems <= 2 * cus ? KWAVES_64x64_PAIRS : KWAVES_NONE;

@@ -3010,7 +3010,8 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
     return launch_pipe<PipeCfg<128, 128, 2, 2, 4, KIND, SWAP>>(p, stream);
   }
   if constexpr (Epi<KIND>::kHasBias) {
-    const KWavesTile tile = p.batch == 1 && p.lda == p.K && p.ldb == p.K ? kwaves_pick(p.M, p.N, p.K, Epi<KIND>::kAccumulate) : KWAVES_NONE;
+    const KWavesTile tile = p.batch == 1 && p.lda == p.K && p.ldb == p.K ? kwaves_pick(p.M, p.N, p.K, Epi<KIND>::kAccumulate, 1, KIND == EPI_F32_BIAS_ACC)
+                                                                            : KWAVES_NONE;
     if (tile != KWAVES_NONE) {
       g_last_kernel = kwaves_name(tile);
       return launch_kwaves<KIND, false>(tile, p, stream);
