@@ -139,6 +139,9 @@ int ti_selftest_fused_slot(int64_t* table, uint32_t* live_mask, int cap, int64_t
 int ti_selftest_rows_pick(int64_t M, int64_t N, int64_t K, int cus, int* tiling);
 int ti_selftest_rows_slot(int64_t* table, signed char* state, int cap, int64_t stream, int* fresh);
 int ti_selftest_placement(const int32_t* words);
+/* ... and whether the LayerNorm-quantiser fetches gamma and beta together with the row (csrc/ln_q.hip), for an int32 addend (mode 0), one of
+ * the stream's type (1), none (2) or an fp32 one on an fp16 stream (3). */
+int ti_selftest_ln_early(int mode, int half, int64_t rows, int H, int cus);
 
 /* Diagnostic (no counterpart in the reference; computes nothing): one launch that issues the instruction mix of
  * the tiled GEMM mainloop `iters` times per wave on the first MiB of `data` (device memory, at least 1 MiB, 16-byte

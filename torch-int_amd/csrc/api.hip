@@ -496,6 +496,7 @@ int ti_selftest_rows_pick(int64_t M, int64_t N, int64_t K, int cus, int* tiling)
 int ti_selftest_rows_slot(int64_t* table, signed char* state, int cap, int64_t stream, int* fresh) {
   return rows_slot_for_test(reinterpret_cast<long long*>(table), state, cap, stream, fresh);
 }
+int ti_selftest_ln_early(int mode, int half, int64_t rows, int H, int cus) { return ln_early_for_test(mode, half, rows, H, cus); }
 int ti_selftest_placement(const int32_t* words) { return placement_of(words); }
 
 int64_t ti_diag_mfma_loop_ops(int64_t iters) { return iters > 0 ? diag_mfma_loop_ops(iters) : 0; }

@@ -185,17 +185,29 @@ __global__ __launch_bounds__(256) void ln_q_rows_generic_kernel(const void* __re
     }
 }
 
+// Whether gamma and beta come with the row, us after / with it.  Up to a row to a CU there is nothing else to do: 192 x 2048 fp16 read only 2.36 / 2.22,
+// 192 x 5120 with the int32 addend 4.36 / 4.02.  Many rows hide a latency behind one another, but not the two of a row that starts late:
+// 2048 x 2048 fp16 with an addend 7.63 / 7.06, 2048 x 5120 read only 9.46 / 8.74, 4096 x 5120 15.0 / 13.5, 2048 x 2048 fp32 read only 6.03 / 5.45.  Between
+// them two to four rows start together on a CU, and the loads for gamma and beta of all stand before some rows': 512 x 2048 fp32 read only 2.96 / 3.25,
+// 320 x 5120 fp32 with an addend 6.04 / 6.39; rows of up to 1024, of which a CU holds more: 832 x 768 2.69 / 2.80, 2048 x 768 fp16 with the int32 addend 4.95 / 4.87.
+// Not where the row by itself is bound by HBM: an fp32 stream with an addend (2048 x 5120 24.4 / 24.7), or one that is only read from 2049 elements on
+// (4096 x 2560 12.4 / 12.9, 7018 x 3072 22.0 / 22.6, 4096 x 5120 level); nor a short fp16 row before there are many more (2560 x 768 read only 1.007 times the
+// time, 4096 0.99), nor 2560 fp16 elements that are only read while the CUs hold all rows at once, eight each (2048 rows 6.21 / 6.38; 2560 rows 0.98 times).
+static inline bool ln_early(int mode, bool half, long long rows, int H, int cus) {
+  if (rows <= cus) return true;
+  if (!half) return mode == MODE_PLAIN && H <= 2048 && rows >= (H <= 1024 ? 2048 : 1024);
+  if (H <= 768 && (mode == MODE_PLAIN || mode == MODE_ADD)) return rows >= 4096;
+  if (H > 2048 && H <= 2560 && mode == MODE_PLAIN) return rows > 8ll * cus;
+  return rows >= (H <= 1024 ? 2048 : 1024);
+}
+// CPU-testable face of it.
+int ln_early_for_test(int mode, int half, long long rows, int H, int cus) { return ln_early(mode, half != 0, rows, H, cus) ? 1 : 0; }
+
 template <int NC, class T>
 static void launch_rows(int mode, const void* in, float scale, const T* res, const T* gamma, const T* beta, float eps,
                         T* r_out, int8_t* q_out, long long rows, int H, hipStream_t stream) {
   const dim3 grid((unsigned)rows), block(256);
-  // Gamma and beta with the row, us after / with it.  Up to a row to a CU there is nothing else to do: 192 x 2048 fp16 read only 2.36 / 2.22,
-  // 192 x 5120 with the int32 addend 4.36 / 4.02.  Many rows hide a latency behind one another, but not the two of a row that starts late:
-  // 2048 x 2048 fp16 with an addend 7.63 / 7.06, 2048 x 5120 read only 9.46 / 8.74, 4096 x 5120 15.0 / 13.5, 2048 x 2048 fp32 read only 6.03 / 5.45; an fp32
-  // stream with an addend is bound by HBM and stays (2048 x 5120 24.4 / 24.7).  Between them two to four rows start together on a CU, and the loads for gamma and beta of all stand before some rows':
-  // 512 x 2048 fp32 read only 2.96 / 3.25, 320 x 5120 fp32 with an addend 6.04 / 6.39; rows of up to 1024, of which a CU holds more: 832 x 768 2.69 / 2.80,
-  // 2048 x 768 fp16 with the int32 addend 4.95 / 4.87.
-  const bool early = rows <= compute_units() || ((mode == MODE_PLAIN || sizeof(T) == 2) && rows >= (NC == 1 ? 2048 : 1024));
+  const bool early = ln_early(mode, sizeof(T) == 2, rows, H, compute_units());
 #define TI_LN_LAUNCH(MODE)                                                                                        \
   if (early)                                                                                                      \
     hipLaunchKernelGGL((ln_q_rows_kernel<NC, MODE, true, T>), grid, block, 0, stream, in, scale, res, gamma, beta, eps, \

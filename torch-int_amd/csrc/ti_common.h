@@ -292,6 +292,7 @@ int set_fused_split(int enable);  // one-launch split-K on (1) / off (0) / uncha
 int rows_pick_for_test(long long M, long long N, long long K, int cus, int* tiling);
 int rows_slot_for_test(long long* table, signed char* state, int cap, long long stream, int* fresh);
 int placement_of(const volatile int* words);
+int ln_early_for_test(int mode, int half, long long rows, int H, int cus);
 int last_rows(int* tiling, int* slices);
 int compute_units();  // of the current device
 const char* last_gemm_kernel();  // kernel family of the calling thread's last launch_gemm ("" before the first)
