@@ -54,7 +54,8 @@ int ti_init(void);
  * loop over workgroups when the output has too few tiles to fill the chip
  * (16 < M <= 1024 with a long K, or the last rows of a larger M: see ti_linear_row_split; 0 up to 16 rows, whose slices
  * meet in memory of the library's own, 67 MiB per device: 2 MiB for each of 33 streams);
- * 0 when no split is worthwhile.  Passing a smaller or NULL workspace is always legal and
+ * 0 when no split is worthwhile.  An upper bound: of some 65 to 1024 rows many run whole on a kernel whose waves share K
+ * ("mid_waves_<tile>" of ti_last_kernel) and use none of it.  Passing a smaller or NULL workspace is always legal and
  * only selects another kernel, one that needs less or does not split. */
 int64_t ti_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
 /* The same for ti_linear_a8_w8_bfp32_ofp32_acc, which may want other slices; it does with the former as well. */
@@ -243,27 +244,27 @@ int ti_linear_a8_w8_b8_o8_heads(const int8_t* x, const int8_t* w, const int8_t* 
  * s8(rint(clamp(alpha[i]*(x . w[i]^T) + beta[i]*bias[i]))).  w, bias, out, alpha, beta are HOST arrays of
  * `count` device pointers / scalars.  The q, k and v projections of one attention block
  * (torch_int/models/opt.py:108-126 calls them one after the other); for M <= 16 with K % 1024 == 0 all
- * weights are streamed by a single launch, for M > 128 with N % 160 == 0 or N % 288 == 0 and K % 128 == 0 the
- * problems are the batches of one persistent tiled launch, other shapes run problem by problem.  Results are those of
- * `count` separate calls. */
+ * weights are streamed by a single launch, some of 65 to 512 rows run in one launch of waves that share K, for M > 128 with
+ * N % 128 == 0, N % 160 == 0 or N % 288 == 0 and K % 128 == 0 the problems may be the batches of one persistent tiled launch
+ * (ti_linear_group_is_one_launch), other shapes run problem by problem.  Results are those of `count` separate calls. */
 int ti_linear_a8_w8_b8_o8_group(const int8_t* x, const int8_t* const* w, const int8_t* const* bias,
                                 int8_t* const* out, const float* alpha, const float* beta, int64_t count,
                                 int64_t M, int64_t N, int64_t K, void* stream);
 
 /* ti_linear_a8_w8_b8_o8_group with every output stored head-major as by ti_linear_a8_w8_b8_o8_heads: the
  * q, k and v projections of a prefill (torch_int/models/opt.py:108-126 followed by the `_shape` permutations,
- * :80-81) as one call.  When N is a multiple of 160 or 288, K of 128 and M > 128, the problems run as the
- * batches of one persistent launch; other shapes run problem by problem.  Results are those of `count`
+ * :80-81) as one call.  The launches are those of ti_linear_a8_w8_b8_o8_group; results are those of `count`
  * separate calls. */
 int ti_linear_a8_w8_b8_o8_group_heads(const int8_t* x, const int8_t* const* w, const int8_t* const* bias,
                                       int8_t* const* out, const float* alpha, const float* beta, int64_t count,
                                       int64_t M, int64_t N, int64_t K, int64_t T, int64_t head_dim, void* stream);
 
 /* Diagnostic (no counterpart in the reference): 1 when a group call of `count` problems of that shape runs as ONE
- * launch on the current device (the streaming kernel for M <= 16 with K % 1024 == 0; a persistent tiled launch when
- * the 256x160, 256x288 or 256x128 tiles divide N, K % 128 == 0, M > 128, and the cost model does not price the
- * problems' own one-round tilings below it), 0 when it loops over the problems - without the split-K workspace that
- * separate ti_linear_a8_w8_b8_o8 calls could be given, so a caller that holds one does better with those. */
+ * launch on the current device (the streaming kernel for M <= 16 with K % 1024 == 0; waves that share K for some 65 to 512 rows
+ * of the widths that kernel takes; a persistent tiled launch when the 256x160, 256x288, 256x256 or 256x128 tiles divide N, K % 128 == 0,
+ * M > 128, and the cost model does not price the problems one after the other below it), 0 when it loops over the problems -
+ * without the split-K workspace that separate ti_linear_a8_w8_b8_o8 calls could be given, so a caller that holds one does
+ * better with those. */
 int ti_linear_group_is_one_launch(int64_t M, int64_t N, int64_t K, int count);
 
 /* replaces linear_relu_a8_w8_b8_o8 (linear.cu:476-625; linear.h:28-33):

@@ -3056,6 +3056,8 @@ int launch_kind(const GemmParams& p, void* workspace, long long workspace_bytes,
     // many rows, a few of them beyond the last multiple of 256: two problems (see row_split_rows)
     long long need = 0;
     const int r = row_split_rows(p.M, p.N, p.K, &need);
+    if constexpr (Epi<KIND>::kHasBias)  // rows that run without slices need no room for them
+      if (r > 0 && kwaves_pick(r, p.N, p.K, Epi<KIND>::kAccumulate, 1, KIND == EPI_F32_BIAS_ACC) != KWAVES_NONE) need = 0;
     if (r > 0 && (need == 0 || (workspace != nullptr && workspace_bytes >= need))) {
       GemmParams head = p;
       head.M = p.M - r;
