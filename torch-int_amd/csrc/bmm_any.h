@@ -170,7 +170,7 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p, int tiles_m
 }
 
 // Up to 16 rows (decode steps): a workgroup owns 16 rows of B, its waves take 256-byte blocks of K in turn and meet in the LDS.
-// Bound by the bytes of B: 200 heads, 1 x 128 x 2003 386 -> 17.8 us, 320 heads, 1 x 128 x 2047 89.7 (copies padded by zeros) -> 29.5.
+// Bound by the bytes of B: 200 heads, 1 x 128 x 2003 408 -> 13.5 us, 320 heads, 1 x 128 x 2047 79.4 (copies padded by zeros) -> 23.2.
 static constexpr int ANY_BLOCKS = 2;  // blocks of a wave in flight
 template <int KIND>
 __global__ __launch_bounds__(1024) void gemm_any_skinny_kernel(GemmParams p, int strips) {
@@ -265,7 +265,8 @@ static constexpr const char* kAnyForms[] = {"a thread to an output", "strips of 
 
 // Tiles: bound by latency and by what the steps of the workgroups of a CU take from one another, us a step of 128 bytes: 64x64 0.5 a
 // workgroup and 0.9 at least, 64x128 0.84 and 1.1, 128x128 1.38 and 1.4 (1001 bytes of K: 4 x 2000 x 2000 64.6 / 54.1 / 44.2 us on the
-// three; 2 x 1000 x 1000 x 5001 37.1 / 45.9 / 56.3; 18 x 130 x 64 x 130 4.9 / 6.6 / 9.3; 64 x 777 x 80 x 777 32.1 / 33.2 / 27.1).
+// three; 2 x 1000 x 1000 x 5001 37.1 / 45.9 / 56.3; 18 x 130 x 64 x 130 4.9 / 6.6 / 9.3; 64 x 777 x 80 x 777 32.1 / 33.2 / 27.1).  Five of 64x64 to a CU for 32-bit
+// outputs as well, of which registers allow four: of 6957 products, 49 to 2047 bytes of K, the choice is 1.020 times the best, priced at four 1.023.
 //
 // A short K of few outputs is a chain of a few latencies, which a thread to an output has fewer of: us, so / on the tiles 13 x 18 x 80 x 15
 // 3.0 / 4.4, 5 x 40 x 128 x 24 3.5 / 4.1, 3 x 33 x 80 x 33 4.25 / 4.26; on the strips 64 x 1 x 128 x 7 2.5 / 3.1, 4 x 1 x 128 x 20 3.0 / 3.0.  Beyond

@@ -254,16 +254,18 @@ static inline bool kwaves_behind(KWavesTile tile, long long N, long long K) {
 }
 
 // The tile of such a linear (or of `problems` of one shape in one launch), or none.  The first of the list that is one round of the CUs: a
-// step takes as long as the panel rows of its tile, and the round as long as its steps (us, 0.0022 a panel row and step and some 3.5).  Below
+// step takes as long as the panel rows of its tile, and the round as long as its steps (us, cold weights, 0.0022 a panel row and step and some 3.5; 0.0034 where the
+// outputs are wider than 10240: 96 x 16384 x 4096 20.3, 96 x 20480 x 5120 28.3).  Below
 // five eighths of a round the CUs stand idle (128 x 1024 x 4096 on 32x32), and in a second round larger tiles of other kernels are ahead (cold, us: 768 x
 // 4096 x 4096 24.5, 26.2 here), but for groups, whose other choice are problems one after the other: there, two workgroups of two waves share a CU (pairs;
 // three 300 x 2048 x 2048 19.2 apart, 13.2 so).  The tallest tiles are where the others walk K on few CUs, too: not for a short K (512 x 3072 x 768 7.3, on
 // 128x64 7.8) nor for a long one (1024 x 2048 x 8192 27.8, on 128x64 28.1); 128x80 are level with those others (128 x 20480 x 5120 32.7 / 32.2, 1024 x 2560 x 2560
 // 16.2 / 16.9).
 // K beyond 8192: the slices are ahead, or level (128 x 2560 x 10240 19.1 / 20, 256 x 4096 x 16384 34.6 / 34).
-// Widths: the measured ones, multiples of 2560 and 1024 (but for those that three divides, which have 192 and 288 columns wide tiles of their own), or of
-// 768 on both sides; K = 1024 and other widths stay with the kernels that had them, whose tests reach their forms there, and so do 257 to 512 rows of K
-// from 3072 on without an accumulating epilogue, of which this kernel would take 0.6 to 0.9 of the time (multiples of 2560 do not).
+// Widths: multiples of 2560 and 1024 (but for those that three divides, which have 192 and 288 columns wide tiles of their own), less what kwaves_behind
+// leaves, or of 768 on both sides.  K = 1024, other widths and 257 to 512 rows of K from 3072 on without an accumulating epilogue (multiples of 2560 are taken) stay
+// with the kernels that had them: a line drawn where the tests of those kernels reach their forms, not by time, of which this kernel would take 0.6 to 0.9 there (384 x 4096 x 4096 17.6, 14.9 so).
+// The 96x64 tiles of a K of 768 are level to behind with weights and old outputs that the cache holds, for fp32 outputs alone (324 x 3072 x 768 warm 6.1 / 6.4, cold level).
 static inline KWavesTile kwaves_pick(long long M, long long N, long long K, bool accumulates, int problems = 1, bool adds_f32 = false) {
   if (M <= TI_ROWS_MAX_M || M > 4096 || N < 768 || N > 20480 || K > 8192) return KWAVES_NONE;
   if (problems > 1 && K < 2048) return KWAVES_NONE;

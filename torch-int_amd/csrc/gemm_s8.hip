@@ -455,8 +455,10 @@ int launch_splitk_raw(int tile, const GemmParams& q, hipStream_t stream) {
   if (tile == SPLIT_128) return launch_pipe<PipeCfg<128, 128, 2, 2, 4, EPI_S32_RAW, false>>(q, stream);
   if (tile == SPLIT_256x160) return launch_pipe16q<Pipe16QCfg<256, 160, 4, 2, EPI_S32_RAW>>(q, stream);
   // Ten waves of 32x80 rather than four of 80x80: with one wave to a SIMD, what a wave reads and copies and what it multiplies come one after the other.
-  // Cold weights, us, four / ten: 300 x 5120 x 20480 int8 55.4 / 50.6, fp32 56.5 / 54.3, 320 rows int32 58.0 / 52.0, 257 rows 49.3 / 48.3,
-  // 160 x 20480 x 5120 40.4 / 39.4; weights that the last-level cache holds 43.4 / 43.9.  2x5 waves level, 5x1 of 32x160 behind, a fourth stage 0.3 behind.
+  // Cold weights, us, four / ten: 300 x 5120 x 20480 int8 51.3 / 48.6, fp32 52.3 / 49.7, 320 rows int32 53.5 / 50.4, 257 rows 47.7 / 46.3, 160 x 20480 x 5120
+  // 38.7 / 38.4, 770 to 800 x 3200 x 20480 76.4 / 71.6.  Weights that the last-level cache holds are copied as fast either way, and ten waves read more
+  // fragments: 1.00 to 1.03 times the time (300 x 5120 x 20480 43.7 / 44.7), 400 x 6400 x 12800 47.4 / 49.2 (cold 51.3 / 51.9).
+  // 2x5 waves level, 5x1 of 32x160 behind, a fourth stage 0.3 behind.
   if (tile == SPLIT_160x160) return launch_pipe16q<Pipe16QCfg<160, 160, 5, 2, EPI_S32_RAW>>(q, stream);
   if (tile == SPLIT_128x80) return launch_pipe16q<Pipe16QCfg<128, 80, 4, 1, EPI_S32_RAW>>(q, stream);
   if (tile == SPLIT_128x160) return launch_pipe16q<Pipe16QCfg<128, 160, 4, 2, EPI_S32_RAW>>(q, stream);

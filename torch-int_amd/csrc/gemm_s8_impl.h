@@ -2466,10 +2466,11 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmParams p, const 
 // (its four waves read 7 fragments from the LDS per 10 MFMAs); with K = 20480 the larger tiles win
 // (512x5120x20480: 79 against 64 us).  More than three LDS stages did not help it (four to six: +1 to +3 %).
 //
-// 160x160 tiles (four waves of 80x80, 10 fragment reads per 25 MFMAs; raw-int32 slices only) for the row counts that they
+// 160x160 tiles (ten waves of 32x80, launch_splitk_raw; raw-int32 slices only) for the row counts that they
 // cover with fewer padded rows than 128-row tiles do: 129 to 160, 257 to 320, 385 to 480, 769 to 800.  257 rows on three
 // 128-row tiles multiply half as much padding as rows.  Bound by the matrix pipe and by the partial tiles' way through the
 // last-level cache, cold weights, us: 257x5120x20480 57.3 -> 48.7, 300x5120x20480 59.1 -> 54.8, 320x5120x20480 60.3 -> 58.8.
+// These figures, the price and the lines below are of four waves of 80x80, which the ten replaced (0.94 to 1.01 times the time, cold).
 // The prices come out some 6 % low for these tiles and 8 % high for the split ones they are up against, so they have to
 // be 15 % cheaper: of 520 shapes (widths 1280 to 20480, 129 to 800 rows) the 212 that this takes run at 0.69 to 1.06 times what
 // they would, while without it 800x2560x10240 took 44.4 us instead of 39.8 and 770x6400x5120 55.3 instead of 36.5.  One row of
@@ -2649,8 +2650,8 @@ static inline bool one_launch_split(int tile, int splits, long long M, long long
   // Rows that end inside a tile: 128x128 tiles (72 to 1000 rows of widths 2048 to 16384, cold, 44 shapes against two launches and
   // 64-byte steps: 0.69 to 1.01 times the time, 0.83 in the mean; 400x4096x4096 23.3 -> 17.7 us, 1000x2048x8192 37.0 -> 27.8), and
   // 128x192 ones from three row tiles on (800x768x3072 18.4 -> 16.1, 350 rows 15.0 / 14.7, but 200 rows 13.9 / 14.4).  The others
-  // gained nothing: 128x80 0.99 times the two launches, 128x160 0.98, 256x160 1.01, and 160x160 1.22: with one wave to a SIMD
-  // and 253 registers the adding wave fetches five of its 25 blocks at a time.
+  // gained nothing: 128x80 0.99 times the two launches, 128x160 0.98, 256x160 1.01, and 160x160 1.22: on four waves of 80x80,
+  // one to a SIMD with 253 registers, of which the adding wave fetches five of its 25 blocks at a time (on the ten of 32x80 that run now: not measured).
   if (tile == SPLIT_160x160 || (M % bm != 0 && tile != SPLIT_128 && !(tile == SPLIT_128x192 && M > 320))) return false;
   // up to four slices: the wave that arrives last reads the others' accumulators one slice after the other,
   // and beyond four that tail costs more than the reduction launch it saves (measured: 2 slices -3 to -12 %,
